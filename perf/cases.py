@@ -185,3 +185,52 @@ def tolerance(case):
     # measured against a float64 evaluation of the same integers and scales: 2.1e-4 for fp16, 2.9e-4 with a bias, which
     # rounds once more, 1.7e-3 for bf16).
     return {"rel": 8e-4} if case["dtype"] == "float16" else {"rel": 7e-3}
+
+
+def _levels(case, n, k, gen):
+    """The layer of ``_layer`` in float64: its dequantised weight [n, k] and its bias, by the definition of the
+    quantiser (float32 levels, ties to even, scales stored in fp16), in plain torch."""
+    weight = torch.randn((n, k), generator=gen, device="cuda", dtype=torch.float16) * 0.02
+    bias = torch.randn((n,), generator=gen, device="cuda").to(DTYPES[case["dtype"]]) if case.get("bias") else None
+    top = 15 if case["kind"] == "linear4" else 3
+    w = weight.float().reshape(n, k // case["group"], case["group"])
+    if case["mode"] == "sym":
+        zero = torch.full_like(w[:, :, :1], (top + 1) // 2)      # also the divisor of the scale
+        scale = w.abs().amax(2, keepdim=True).clamp_min(1e-9) / zero[0, 0]
+    else:
+        low = w.amin(2, keepdim=True)
+        scale = (w.amax(2, keepdim=True) - low).clamp_min(1e-9) / torch.full_like(low, top)
+        zero = torch.round(-low / scale).clamp_(0, top)
+    codes = torch.round(w / scale).add_(zero).clamp_(0, top)
+    return (codes.sub_(zero).double() * scale.half().double()).reshape(n, k), bias
+
+
+def _quantised(x):
+    """The activation as the int8 path sees it, in float64: per-token scale, ties to even.  (Tensor divisors here and
+    above: torch turns a division by a Python number into a product with its rounded reciprocal.)"""
+    x = x.float()
+    amax = x.abs().amax(1, keepdim=True).clamp_min(1e-9)
+    scale = amax / torch.full_like(amax, 127.0)
+    return torch.round(x / scale).clamp_(-127, 127).double() * scale.double()
+
+
+def exact(case, seed):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seed)
+    kind, rows, dtype = case["kind"], case["rows"], case["dtype"]
+    if kind == "block":
+        w = {name: _levels(case, n, k, gen)[0] for name, (n, k) in BLOCK_LAYERS.items()}
+        x_attn, x_out, x_ffn = (_quantised(_activation(rows, HIDDEN, dtype, gen)) for _ in range(3))
+        x_down = _quantised(_activation(rows, FFN, dtype, gen))
+        inputs = {"q": x_attn, "k": x_attn, "v": x_attn, "o": x_out, "gate": x_ffn, "up": x_ffn, "down": x_down}
+        return {name: x @ w[name].t() for name, x in inputs.items()}
+    if kind == "grouped":
+        outs = []
+        for m, n, k in _grouped_shapes(case):
+            w, _ = _levels(case, n, k, gen)
+            outs.append(_quantised(_activation(m, k, dtype, gen)) @ w.t())
+        return outs
+    w, bias = _levels(case, case["n"], case["k"], gen)
+    x = _activation(rows, case["k"], dtype, gen)
+    y = (x.double() if kind == "linear16" else _quantised(x)) @ w.t()
+    return y if bias is None else y + bias.double()
