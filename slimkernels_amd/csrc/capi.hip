@@ -900,7 +900,7 @@ int slimk_w4a8_gemm(const int8_t* q, int ldq, const float* s_a, const int32_t* r
 
 int slimk_w2a16_gemm_auto_split_k(int M, int N, int K, int group_size) {
     if (M <= 0 || N <= 0 || !shape_ok(K, group_size) || K % 128 != 0) return 0;
-    return w2a8::w2a16_auto_split(M, strips_of(N), K / w2a8::kStepK, group_size / w2a8::kStepK);
+    return w2a8::w2a16_plan(M, strips_of(N), K / w2a8::kStepK, group_size / w2a8::kStepK, 0).split;
 }
 
 size_t slimk_w2a16_gemm_workspace_bytes(int M, int N, int K, int group_size, int split_k) {
@@ -928,7 +928,7 @@ int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
         return fail(SLIMK_ERR_MISALIGNED, "w2a16_gemm: x, w_r, s_r, zp_r must be 16-byte aligned; ldx %% 8 == 0; out 2-byte aligned");
     const int gs = group_size / w2a8::kStepK, steps = K / w2a8::kStepK;
     const int granules = steps / (gs > 2 ? gs : 2);
-    if (split_k <= 0) split_k = w2a8::w2a16_auto_split(M, strips_of(N), steps, gs);
+    if (split_k <= 0) split_k = w2a8::w2a16_plan(M, strips_of(N), steps, gs, 0).split;
     if (split_k > 64 || (split_k > 1 && split_k * 4 > granules))
         return fail(SLIMK_ERR_BAD_SHAPE, "split_k=%d: at most 64 and at most a quarter of the %d K granules", split_k, granules);
 

@@ -14,6 +14,8 @@
 // k-values of one MFMA therefore come in the order 0,2,1,3,4,6,5,7; the activation operand is put in
 // the same order with two v_perm_b32 per register pair.
 //
+// Launches of more than 32 token rows go to gemm_w2a16_tiled.hip where that is predicted to be faster (w2a16_plan).
+//
 // Work split: a workgroup is 4, 8 or 16 wavefronts that take as many K-parts of ONE strip of 64 channels and
 // 16 token rows and add their sums up through LDS; blockIdx.y splits K further across workgroups when the
 // strips alone would leave CUs idle (fp32 partial sums to a workspace, summed in split order by a second
@@ -286,14 +288,31 @@ __global__ __launch_bounds__(kWaves * 64, XBF && GS < 4 ? 4 : 1) void w2a16_grou
     w2a16_body<GS, kWaves, ZP, false, OutT, XBF>(p, local % units, 0, local / units, lp, red);
 }
 
+// Adds up the partial sums in split order: four neighbouring values of a row per thread, the splits' loads independent
+// of each other (one value per thread and its row and column by a 64-bit division: the second launch of a
+// 300 x 4096 x 14336 call).
 template <typename OutT>
-__global__ __launch_bounds__(256) void w2a16_reduce_kernel(const float* __restrict__ ws, int split, int M, int N,
+__global__ __launch_bounds__(128) void w2a16_reduce_kernel(const float* __restrict__ ws, int split, int M, int N,
                                                            uint16_t* __restrict__ out, int ldo) {
+    const int n = (int)(blockIdx.x * 128 + threadIdx.x) * 4;
+    if (n >= N) return;
     const size_t total = (size_t)M * N;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
-        float v = ws[i];
-        for (int s = 1; s < split; ++s) v += ws[(size_t)s * total + i];
-        out[(i / N) * ldo + i % N] = OutT::cast(v);
+    for (int m = (int)blockIdx.y; m < M; m += (int)gridDim.y) {
+        const float* src = ws + (size_t)m * N + n;
+        uint16_t* dst = out + (size_t)m * ldo + n;
+        if ((N & 3) == 0) {
+            v4f v = *reinterpret_cast<const v4f*>(src);
+#pragma unroll 4
+            for (int s = 1; s < split; ++s) v += *reinterpret_cast<const v4f*>(src + (size_t)s * total);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[i] = OutT::cast(v[i]);
+        } else {
+            for (int i = 0; i < 4 && n + i < N; ++i) {
+                float v = src[i];
+                for (int s = 1; s < split; ++s) v += src[(size_t)s * total + i];
+                dst[i] = OutT::cast(v);
+            }
+        }
     }
 }
 
@@ -332,7 +351,7 @@ void launch_gs(const W2A16Params& p, int waves, bool out_bf16, dim3 grid, hipStr
 // K splits across workgroups: one unless the strips (x blocks of 16 token rows) alone leave most CUs idle;
 // then enough for about one workgroup per CU, every K-part at least two granules (256 reduction elements at
 // group size <= 128) long.
-int w2a16_auto_split(int M, int strips, int steps, int gs) {
+int w2a16_few_rows_split(int M, int strips, int steps, int gs) {
     const int granule = gs > kChunkSteps ? gs : kChunkSteps;
     const int n_gran = steps / granule;
     const long long base = (long long)strips * ((M + 15) / 16);
@@ -386,19 +405,22 @@ hipError_t launch_w2a16_grouped(const W2A16Group& gp, int gs, bool zp, bool out_
 }
 
 hipError_t launch_w2a16(const W2A16Params& p, int gs, bool out_bf16, hipStream_t stream) {
-    const dim3 grid((unsigned)p.strips, (unsigned)p.split, (unsigned)((p.M + 15) / 16));
-    const int waves = w2a16_waves(p.M, p.strips, p.steps, gs, p.split);
-    if (gs == 1) launch_gs<1>(p, waves, out_bf16, grid, stream);
-    else if (gs == 2) launch_gs<2>(p, waves, out_bf16, grid, stream);
-    else launch_gs<4>(p, waves, out_bf16, grid, stream);
+    if (const int rb = w2a16_plan(p.M, p.strips, p.steps, gs, p.split).rb) {
+        if (hipError_t e = launch_w2a16_tiled(p, rb, gs, out_bf16, stream); e != hipSuccess) return e;
+    } else {
+        const dim3 grid((unsigned)p.strips, (unsigned)p.split, (unsigned)((p.M + 15) / 16));
+        const int waves = w2a16_waves(p.M, p.strips, p.steps, gs, p.split);
+        if (gs == 1) launch_gs<1>(p, waves, out_bf16, grid, stream);
+        else if (gs == 2) launch_gs<2>(p, waves, out_bf16, grid, stream);
+        else launch_gs<4>(p, waves, out_bf16, grid, stream);
+    }
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     if (p.split > 1) {
-        const size_t total = (size_t)p.M * p.N;
-        const unsigned blocks = (unsigned)((total + 255) / 256 > 4096 ? 4096 : (total + 255) / 256);
+        const dim3 blocks((unsigned)((p.N + 511) / 512), (unsigned)std::min(p.M, 32768));
         if (out_bf16)
-            w2a16_reduce_kernel<OutBF16><<<dim3(blocks), dim3(256), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo);
+            w2a16_reduce_kernel<OutBF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo);
         else
-            w2a16_reduce_kernel<OutF16><<<dim3(blocks), dim3(256), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo);
+            w2a16_reduce_kernel<OutF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo);
     }
     return hipGetLastError();
 }

@@ -50,6 +50,7 @@ class W2A8Weight:
     # lazily created split-K workspaces (uint8), one per stream the weight is used on: calls that share a workspace
     # must not overlap in time, and work on one stream does not
     workspaces: dict = dataclasses.field(default_factory=dict)
+    partials16: dict = dataclasses.field(default_factory=dict)   # the same for the weight-only form's partial sums
 
     @property
     def device(self):
@@ -310,15 +311,16 @@ def w2a16_gemm(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *, split
         out = torch.empty((M, w.N), dtype=out_dtype, device=dev)
     with torch.cuda.device(dev):
         ws_bytes = L.slimk_w2a16_gemm_workspace_bytes(M, w.N, K, w.group_size, split_k)
-        ws = getattr(w, "_partials16", None)      # its own buffer: the W2A8 workspace holds counters that must stay zero
+        stream = _stream_ptr(dev)
+        # its own buffer, one per stream as there: the W2A8 workspace holds counters that must stay zero
+        ws = w.partials16.get(stream) if ws_bytes else None
         if ws_bytes and (ws is None or ws.numel() < ws_bytes):
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            w._partials16 = ws
+            ws = w.partials16[stream] = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         _lib.check(L.slimk_w2a16_gemm(
             x.data_ptr(), x.stride(0), _DT[x.dtype], w.w_r.data_ptr(), w.s_r.data_ptr(),
             w.zp_r.data_ptr() if w.zp_r is not None else None, w.zp_const, M, w.N, K, w.group_size,
             out.data_ptr(), out.stride(0), _DT[out.dtype],
-            ws.data_ptr() if ws_bytes else None, ws.numel() if ws_bytes else 0, split_k, _stream_ptr(dev)))
+            ws.data_ptr() if ws_bytes else None, ws.numel() if ws_bytes else 0, split_k, stream))
     return out
 
 
