@@ -292,6 +292,25 @@ int slimk_w2a8_gemm_fused(const void* x, int ldx, int x_dtype,
  * workgroup take that road, which is how the tests reach it; results do not depend on the value. */
 int slimk_w2a8_set_fused_spin_limit(int polls);
 
+/* The whole layer for many token rows: x [M][ldx] fp16 or bf16 -> out, the activation quantisation included, through
+ * the digit form of the GEMM (csrc/gemm_mx.hip): q is split into an fp4 and an fp6 digit and multiplied on the
+ * block-scaled matrix cores at twice the int8 rate; the group sums are the exact integers of the int8 path, the scaled
+ * sums are fp32 as there.  Two launches on `stream`.
+ *  - slimk_w2a8_linear_route: 1 where this form is the faster one for a layer call (activation quantisation + GEMM),
+ *    else 0 (per_group_zp: whether the weight carries zp_r).
+ *  - activations: scratch of slimk_w2a8_linear_activation_bytes(...) bytes (no initialisation; 0: the form does not
+ *    take the shape: K > 32512, or 2 GiB and more of digits or weights), needed until the call's work is done.
+ *  - workspace: as for slimk_w2a8_gemm (zeroed once with slimk_w2a8_workspace_init; none where the query returns 0).
+ * x 16-byte aligned, ldx % 8 == 0.  No upstream counterpart (the model-level caller is llama.py:15-19). */
+int slimk_w2a8_linear_route(int M, int N, int K, int group_size, int per_group_zp);
+size_t slimk_w2a8_linear_activation_bytes(int M, int N, int K, int group_size);
+size_t slimk_w2a8_linear_workspace_bytes(int M, int N, int K, int group_size);
+int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
+                      const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                      int M, int N, int K, int group_size,
+                      void* out, int ldo, int out_dtype,
+                      void* activations, size_t activation_bytes, void* workspace, size_t workspace_bytes, void* stream);
+
 /* One problem of a grouped launch: the arguments of slimk_w2a8_gemm that describe data. */
 typedef struct slimk_w2a8_problem {
     const int8_t* q;

@@ -10,6 +10,7 @@
 #include <string>
 
 #include "../../include/slimk_w2a8.h"
+#include "mx_launch.h"
 #include "w2a8_launch.h"
 
 // The library-owned split-K workspace of slimk_w2a8_gemm_static (see static_workspace() below).
@@ -597,6 +598,83 @@ int slimk_w2a8_gemm_static(const int8_t* q, int ldq, const float* s_a, const int
     // device's first split-K call, its counters cleared) only when the launch splits K
     return gemm_impl(q, ldq, s_a, rowsum, ldr, w_r, s_r, zp_r, zp_const, M, N, K, group_size, out, ldo, out_dtype,
                      nullptr, SLIMK_DUMP_NONE, nullptr, kStaticWorkspaceBytes, kernel, split_k, stream, true);
+}
+
+// ---- the digit form (gemm_mx.hip).  The activation scratch: digit fragments, group sums, token scales.
+static size_t mx_frag_bytes(int M, int K) {
+    return (size_t)w2a8::mx_row_blocks(M) * (size_t)w2a8::mx_padded_steps(K) * w2a8::mx::kFragBytes;
+}
+static size_t mx_sums_bytes(int M, int K, int group_size) { return ((size_t)M * (K / group_size) * 4 + 16 + 255) / 256 * 256; }
+
+size_t slimk_w2a8_linear_activation_bytes(int M, int N, int K, int group_size) {
+    if (M <= 0 || N <= 0 || !shape_ok(K, group_size) || K > w2a8::mx::kMaxK) return 0;
+    const size_t weights = w2a8::weight_bytes(strips_of(N), K / w2a8::kStepK);
+    // (the kernels address fragments, group sums and weights through 32-bit offsets)
+    if (mx_frag_bytes(M + 128, K) > 0x7fffffffu || weights > 0x7fffffffu) return 0;
+    return mx_frag_bytes(M, K) + mx_sums_bytes(M, K, group_size) + ((size_t)M * 4 + 255) / 256 * 256;
+}
+
+size_t slimk_w2a8_linear_workspace_bytes(int M, int N, int K, int group_size) {
+    if (slimk_w2a8_linear_activation_bytes(M, N, K, group_size) == 0) return 0;
+    const w2a8::MxPlan plan = w2a8::mx_plan(M, N, K, group_size);
+    if (plan.split <= 1) return 0;
+    return kCounterBlockBytes + (size_t)plan.split * plan.tiles * plan.rb * w2a8::mx::kFragRows * 256 * sizeof(float);
+}
+
+// Where the digit form beats act_quant + the kernel that slimk_w2a8_gemm would take, both timed with their quantisation:
+// 128-row tiles that fill the chip (two per CU and more), groups of 64 and 128.  Its GEMM saves in proportion to M * N * K,
+// its quantisation costs a little more in proportion to M * K, so N decides: 2048 x 28672 x 8192 in groups of 64
+// 578 -> 509 us, 4096 x 14336 x 4096 257 -> 242, 4096 x 5120 x 5120 139 -> 132, but 4096 x 4096 x 14336 255 -> 258
+// (per-group zero-points: 304 -> 296).  Groups of 256, where the int8 kernel drains half as often, are level (2048 x 14336 x 4096 127 / 128 us).
+int slimk_w2a8_linear_route(int M, int N, int K, int group_size, int per_group_zp) {
+    if (slimk_w2a8_linear_activation_bytes(M, N, K, group_size) == 0) return 0;
+    if (group_size > 128 || N < (group_size == 128 && !per_group_zp ? 5120 : 4096)) return 0;
+    return w2a8::mx_plan(M, N, K, group_size).rb == 4 ? 1 : 0;
+}
+
+int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
+                      const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                      int M, int N, int K, int group_size,
+                      void* out, int ldo, int out_dtype,
+                      void* activations, size_t activation_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!x || !w_r || !s_r || !out || !activations) return fail(SLIMK_ERR_NULL_POINTER, "linear: NULL buffer");
+    if (M <= 0 || N <= 0) return fail(SLIMK_ERR_BAD_SHAPE, "M=%d, N=%d must be positive", M, N);
+    if (int rc = check_kg(K, group_size)) return rc;
+    if (x_dtype != SLIMK_F16 && x_dtype != SLIMK_BF16) return fail(SLIMK_ERR_BAD_ENUM, "x_dtype=%d", x_dtype);
+    if (out_dtype != SLIMK_F16 && out_dtype != SLIMK_BF16) return fail(SLIMK_ERR_BAD_ENUM, "out_dtype=%d", out_dtype);
+    if (zp_const < 0 || zp_const > 3) return fail(SLIMK_ERR_BAD_SHAPE, "zp_const=%d must be 0..3", zp_const);
+    if (ldx < K || ldo < N) return fail(SLIMK_ERR_BAD_SHAPE, "ldx=%d / ldo=%d too small for K=%d / N=%d", ldx, ldo, K, N);
+    const size_t need_act = slimk_w2a8_linear_activation_bytes(M, N, K, group_size);
+    if (need_act == 0) return fail(SLIMK_ERR_UNSUPPORTED, "linear: M=%d, N=%d, K=%d not supported", M, N, K);
+    if (!aligned16(x) || ldx % 8 != 0 || !aligned16(w_r) || !aligned16(s_r) || (zp_r && !aligned16(zp_r)) ||
+        !aligned16(activations) || (reinterpret_cast<uintptr_t>(out) & 1u))
+        return fail(SLIMK_ERR_MISALIGNED, "linear: x, w_r, s_r, zp_r, activations must be 16-byte aligned; ldx %% 8 == 0; out 2-byte aligned");
+    if (activation_bytes < need_act)
+        return fail(SLIMK_ERR_WORKSPACE, "activation scratch of %zu bytes is smaller than the %zu needed", activation_bytes, need_act);
+    const w2a8::MxPlan plan = w2a8::mx_plan(M, N, K, group_size);
+
+    char* const act = reinterpret_cast<char*>(activations);
+    w2a8::MxParams p{};
+    uint8_t* frag = reinterpret_cast<uint8_t*>(act);
+    uint32_t* rs = reinterpret_cast<uint32_t*>(act + mx_frag_bytes(M, K));
+    float* s_a = reinterpret_cast<float*>(act + mx_frag_bytes(M, K) + mx_sums_bytes(M, K, group_size));
+    p.frag = frag; p.rs = rs; p.s_a = s_a;
+    p.w_r = w_r; p.s_r = s_r; p.zp_r = zp_r; p.out = out; p.ldo = ldo;
+    p.M = M; p.N = N; p.K = K; p.G = K / group_size; p.steps = K / w2a8::kStepK; p.strips = strips_of(N);
+    p.zp_const = zp_const; p.group_shift = group_size == 256 ? 1 : 0;
+    p.split = plan.split; p.stages_per_split = plan.stages_per_split;
+    if (plan.split > 1) {
+        const size_t need = slimk_w2a8_linear_workspace_bytes(M, N, K, group_size);
+        if (!workspace || workspace_bytes < need)
+            return fail(SLIMK_ERR_WORKSPACE, "linear needs a workspace of %zu bytes (got %zu)", need, workspace ? workspace_bytes : (size_t)0);
+        if (!aligned16(workspace)) return fail(SLIMK_ERR_MISALIGNED, "workspace must be 16-byte aligned");
+        p.ws_counter = reinterpret_cast<unsigned*>(workspace);
+        p.ws_partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + kCounterBlockBytes);
+    }
+    hipStream_t st = (hipStream_t)stream;
+    if (int rc = hip_result(w2a8::launch_mx_quant(x, ldx, x_dtype == SLIMK_BF16, M, K, group_size, frag, rs, s_a, st), "linear quantisation"))
+        return rc;
+    return hip_result(w2a8::launch_mx_gemm(p, plan.rb, group_size == 64 ? 1 : 2, out_dtype == SLIMK_BF16, st), "linear gemm");
 }
 
 int slimk_w2a8_gemm_fused(const void* x, int ldx, int x_dtype,

@@ -1,0 +1,662 @@
+// The digit form of the W2A8 GEMM for gfx950: int8 activations times 2-bit weights on the block-scaled matrix cores
+// (v_mfma_f32_32x32x64_f8f6f4) for many token rows, exact.
+//
+// Why not the int8 matrix cores (tiled_bodies.h): there every accumulator costs a conversion and an fma per scale
+// group, and that and the unpacking hold the matrix cores to 0.53 of their rate in the main loop.  The fp4 / fp6 forms of
+// the f8f6f4 instruction run at twice the int8 rate, so an activation may cost two of them: q in -127..127 is split
+// exactly into two digits,
+//     q = 32 * a4 + 8 * a6,   a4 = fp4 (e2m1) nearest to q / 32,   a6 = fp6 (e2m3) of the rest, |rest| <= 16,
+// and a code c in 0..3 IS the fp4 number c / 2 once its two bits lie at the bottom of a nibble.  Products are
+// multiples of 1/16 and the group sums of q * c stay below 2^18, so the fp32 accumulators hold them exactly: the drain is
+// one fma per element and group instead of two instructions, and a packed weight dword becomes operands in 6
+// instructions per 16 codes.
+//
+// Measured: 38 cycles per 32x32x64 instruction with the 4 drain fmas of groups of 128 beside it, 49 with the 8 of
+// groups of 64 (32 alone) in a probe; in the kernel 469 against the int8 kernel's 551 thousand cycles at
+// 4096 x 14336 x 4096, at 2.16 against 2.42 GHz (the faster matrix instructions run into the power limit): 217
+// against 228 us; with the quantisation 257 -> 242 us, 2048 x 28672 x 8192 in groups of 64 578 -> 509 us.  What is left over the
+// matrix cores' own 235 thousand cycles is the vector instructions beside them (185 per 32 of them), prologue and
+// epilogue of a tile, and the half-empty last round of tiles.
+//
+// The zero-point leaves through the group sums of q: -zp * scale * rowsum goes into the running sums first, as a
+// matrix product over the groups (uniform zero-points: rowsum in two exact fp16 digits times the fp16 scales,
+// eight groups per instruction; per-group ones: fp32 products, two groups per instruction).
+//
+// Activation fragments (written by mx_quant_kernel): one of 2560 bytes per 32 rows x 64 elements, in operand order.
+// Lane l holds row l & 31, elements 32 * (l >> 5) .. + 31: 16 bytes of fp4 digits at 16 * l, the first 16 bytes of its
+// fp6 digits at 1024 + 16 * l, the other 8 at 2048 + 8 * l.  Slot j of the 32 is element 8 * (j / 8) + (j % 8) / 2 +
+// 4 * (j % 2): the order in which the weight dwords of the streaming layout come apart into nibbles.
+#include <algorithm>
+
+#include "mx_launch.h"
+
+namespace w2a8 {
+
+namespace {
+
+using namespace mx;
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef int v6i __attribute__((ext_vector_type(6)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+constexpr int kFp6 = 2, kFp4 = 4;          // operand formats of the f8f6f4 instructions
+constexpr int kScaleOne = 127, kScale4 = 129;   // 2^(x - 127)
+
+// ---- activations: per-token quantisation straight into digit fragments.  One row per workgroup, 32 elements per
+// thread (an fp6 conversion takes 32), the row read once, whole cache lines at a time: a thread's 64 bytes are four
+// lines' worth of address work per lane otherwise, so the row turns through LDS, its 16-byte pieces rotated by c / 16
+// inside each set of four (the readers' pieces then lie in all banks).  The quotients are those of
+// act_quant_keep_kernel, bit for bit.  32 consecutive rows go to one XCD, so that the 16-byte pieces of a fragment meet
+// in one L2.
+template <bool BF16>
+__global__ __launch_bounds__(1024) void mx_quant_kernel(const uint16_t* __restrict__ x, int ldx, int M, int K, int group_size,
+                                                        uint8_t* __restrict__ frag, uint32_t* __restrict__ rs,
+                                                        float* __restrict__ s_a) {
+    __shared__ float red[16];
+    const int xcd = blockIdx.x & 7, kth = blockIdx.x >> 3;
+    const int m = M >= 256 ? (((kth >> 5) << 3) + xcd) * 32 + (kth & 31) : (int)blockIdx.x;
+    if (m >= M) return;   // (uniform: the grid is rounded up to whole sets of rows)
+    const int tid = threadIdx.x;
+    const bool on = tid * 32 < K;
+    extern __shared__ __attribute__((aligned(16))) v4u row[];   // K / 8 pieces
+    const int threads = (int)blockDim.x, pieces = K / 8;
+    const auto place = [](int c) { return (c & ~3) | ((c + (c >> 4)) & 3); };
+    const auto widen = [](uint32_t w, float& a, float& b) {
+        a = BF16 ? __uint_as_float(w << 16) : half_bits_to_float((uint16_t)(w & 0xffffu));
+        b = BF16 ? __uint_as_float(w & 0xffff0000u) : half_bits_to_float((uint16_t)(w >> 16));
+    };
+    float amax = 0.0f;
+    {
+        const v4u* src = reinterpret_cast<const v4u*>(x + (size_t)m * ldx);
+        v4u raw[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) raw[i] = i * threads + tid < pieces ? src[i * threads + tid] : v4u{0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int c = i * threads + tid;
+            if (c < pieces) row[place(c)] = raw[i];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float a, b;
+                widen(raw[i][k], a, b);
+                amax = fmaxf(amax, fmaxf(fabsf(a), fabsf(b)));
+            }
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+    const int waves = (int)blockDim.x >> 6;
+    if ((tid & 63) == 0) red[tid >> 6] = amax;
+    __syncthreads();
+    amax = red[0];
+    for (int w = 1; w < waves; ++w) amax = fmaxf(amax, red[w]);
+    const float s = fmaxf(amax, 1e-9f) / 127.0f;
+    if (tid == 0) s_a[m] = s;
+    const float inv_s = 1.0f / s;
+
+    float f[32];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const v4u raw = on ? row[place(tid * 4 + i)] : v4u{0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) widen(raw[k], f[8 * i + 2 * k], f[8 * i + 2 * k + 1]);
+    }
+    float sumf = 0.0f;   // (whole numbers below 2^24: exact)
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        f[i] = fminf(fmaxf(rne_quotient(f[i], s, inv_s), -127.0f), 127.0f);
+        sumf += f[i];
+    }
+    v4u hi;
+    v16f lo_even, lo_odd;   // the rests in slot order: the conversion takes its two inputs alternately
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        uint32_t w = 0;
+#define SLIMK_MX_PAIR(B)                                                                                       \
+        w = (uint32_t)__builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, f[8 * d + B], f[8 * d + 4 + B], 32.0f, B);
+        SLIMK_MX_PAIR(0) SLIMK_MX_PAIR(1) SLIMK_MX_PAIR(2) SLIMK_MX_PAIR(3)
+#undef SLIMK_MX_PAIR
+#define SLIMK_MX_REST(B)                                                                                       \
+        {                                                                                                      \
+            const v2f back = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 32.0f, B);                            \
+            lo_even[4 * d + B] = f[8 * d + B] - back[0];                                                       \
+            lo_odd[4 * d + B] = f[8 * d + 4 + B] - back[1];                                                    \
+        }
+        SLIMK_MX_REST(0) SLIMK_MX_REST(1) SLIMK_MX_REST(2) SLIMK_MX_REST(3)
+#undef SLIMK_MX_REST
+        hi[d] = w;
+    }
+    const v6i lo = __builtin_bit_cast(v6i, __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(lo_even, lo_odd, 8.0f));
+    if (on) {
+        const int steps2 = mx_padded_steps(K);
+        uint8_t* dst = frag + ((size_t)(m >> 5) * steps2 + (tid >> 1)) * kFragBytes;
+        const int fl = (tid & 1) * 32 + (m & 31);
+        *reinterpret_cast<v4u*>(dst + fl * 16) = hi;
+        *reinterpret_cast<v4i*>(dst + 1024 + fl * 16) = v4i{lo[0], lo[1], lo[2], lo[3]};
+        *reinterpret_cast<v2i*>(dst + 2048 + fl * 8) = v2i{lo[4], lo[5]};
+    }
+    const int tpg = group_size / 32;   // threads per scale group: 2, 4 or 8 (all of a group's threads are on or off)
+    for (int off = 1; off < tpg; off <<= 1) sumf += __shfl_xor(sumf, off, 64);
+    if (on && tid % tpg == 0) {
+        const float h = rintf(sumf * 0.0078125f) * 128.0f;   // |sum| <= 256 * 127: both digits are exact in fp16
+        const _Float16 dh = (_Float16)h, dl = (_Float16)(sumf - h);
+        rs[(size_t)m * (K / group_size) + tid / tpg] =
+            (uint32_t)__builtin_bit_cast(uint16_t, dh) | ((uint32_t)__builtin_bit_cast(uint16_t, dl) << 16);
+    }
+}
+
+__device__ __forceinline__ v16f mfma_hi(v4i a, v4i b, v16f c) {   // 4 * a4 * c/2
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(v8i{a[0], a[1], a[2], a[3], 0, 0, 0, 0}, v8i{b[0], b[1], b[2], b[3], 0, 0, 0, 0},
+                                                           c, kFp4, kFp4, 0, kScale4, 0, kScaleOne);
+}
+__device__ __forceinline__ v16f mfma_lo(v4i a, v2i a2, v4i b, v16f c) {   // a6 * c/2
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(v8i{a[0], a[1], a[2], a[3], a2[0], a2[1], 0, 0},
+                                                           v8i{b[0], b[1], b[2], b[3], 0, 0, 0, 0}, c, kFp6, kFp4, 0, 0, 0, 0);
+}
+
+// The four raw dwords of a lane (16 elements of its quad x 4 channels) as the operands of the unit's two blocks of 32
+// channels.  Two dwords' nibbles are interleaved first (a nibble then holds two channels' codes of one element), the
+// masks leave one channel's code at the bottom of each nibble, and the row swap hands each half-wave both quads'
+// elements of its own channel: block nb's lane l holds channel nb * 32 + (l & 31), elements 32 * (l >> 5) .. + 31.
+__device__ __forceinline__ void unpack_unit(const v4i& raw, v4i (&b)[2]) {
+    const v4u r = __builtin_bit_cast(v4u, raw);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        uint32_t x = (r[2 * h] & 0x0f0f0f0fu) | ((r[2 * h + 1] << 4) & 0xf0f0f0f0u);
+        uint32_t y = ((r[2 * h] >> 4) & 0x0f0f0f0fu) | (r[2 * h + 1] & 0xf0f0f0f0u);
+        asm("" : "+v"(x), "+v"(y));   // (keeps the masks below from being folded back into the two merges: 6 more instructions)
+        const v2u lo = __builtin_bit_cast(v2u, __builtin_amdgcn_permlane16_swap(x & 0x33333333u, (x >> 2) & 0x33333333u, false, false));
+        // (field 3 is stored with its high bit flipped)
+        const v2u hi = __builtin_bit_cast(v2u, __builtin_amdgcn_permlane16_swap(y & 0x33333333u, ((y >> 2) & 0x33333333u) ^ 0x22222222u, false, false));
+        b[0][h] = (int)lo[0];
+        b[0][2 + h] = (int)lo[1];
+        b[1][h] = (int)hi[0];
+        b[1][2 + h] = (int)hi[1];
+    }
+}
+
+// Workgroup = 4 waves side by side along the channels (a strip of 64 each) x RB blocks of 32 token rows; per stage of
+// 128 elements the activation fragments come into a three-slot LDS ring (LDS-direct, two stages ahead, shared by the
+// waves), the wave's own weight units and scales into two wave-private slots (a wave moves a stage's units to registers
+// before it asks for the units two stages on).
+// GS = 64-element steps per drain: 1 (groups of 64) or 2 (128; groups of 256 drain twice with the same scale).
+template <int RB, int GS, bool SPLIT, bool ZP, typename OutT>
+__device__ __forceinline__ void mx_body(const MxParams& p) {
+    constexpr int kABytes = RB * kStageSteps * kFragBytes;       // 20 or 10 KiB
+    constexpr int kALoads = (kABytes / 1024 + 3) / 4;            // LDS-direct loads of 1 KiB per wave and stage: 5 or 3
+    constexpr int kASlot = kABytes;
+    constexpr int kSpare = kALoads * 4 * 1024 > kABytes ? 1024 : 0;   // RB = 2: where the two surplus loads land
+    constexpr int kWBytes = kStripsPerWg * kStageSteps * kUnitBytes;
+    constexpr int kSBytes = kStripsPerWg * 256;
+    constexpr int kLds = 3 * kASlot + 2 * (kWBytes + kSBytes) + kSpare;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
+    constexpr int kBM = RB * kFragRows;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, half = lane >> 5;
+    // tile order as in tiled_bodies.h: channel tiles that divide by eight go to the XCDs in bands, token tile major
+    const int tiles_n = (p.strips + kStripsPerWg - 1) / kStripsPerWg, tiles_m = (p.M + kBM - 1) / kBM;
+    const int total = tiles_m * tiles_n, per_xcd = (total + 7) / 8;
+    const int xcd = (int)(blockIdx.x & 7), local = (int)(blockIdx.x >> 3);
+    int tile;
+    if (tiles_n % 8 == 0) {
+        const int band = tiles_n / 8;
+        tile = (local / band) * tiles_n + xcd * band + local % band;
+    } else if (tiles_m >= 2 && tiles_m <= 4) {
+        int n_tile, m_tile_i;
+        if (!xcd_place((int)blockIdx.x, tiles_n, tiles_m, n_tile, m_tile_i)) return;
+        tile = m_tile_i * tiles_n + n_tile;
+    } else {
+        tile = xcd * per_xcd + local;
+    }
+    if (local >= per_xcd || tile >= total) return;
+    const int m_tile = (tile / tiles_n) * kBM;
+    const int strip_raw = (tile % tiles_n) * kStripsPerWg + wave;
+    const int strip = min(strip_raw, p.strips - 1);   // a surplus wave recomputes the last strip and stores nothing
+    const bool strip_ok = strip_raw < p.strips;
+
+    const int steps2 = (p.steps + 1) / 2 * 2;
+    const int all_stages = steps2 / 2;
+    const int stage0 = SPLIT ? (int)blockIdx.y * p.stages_per_split : 0;
+    const int n_stages = SPLIT ? min(p.stages_per_split, all_stages - stage0) : all_stages;
+
+    const int row_blocks = (p.M + kFragRows - 1) / kFragRows;
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(p.frag), 0, (int)((size_t)row_blocks * steps2 * kFragBytes), 0x00020000);
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t*>(p.w_r), 0, (int)min(weight_bytes(p.strips, p.steps), (size_t)0x7fffffff), 0x00020000);
+    const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(p.s_r), 0, (int)min((size_t)p.strips * p.G * 128, (size_t)0x7fffffff), 0x00020000);
+
+    // activations: chunk c = wave + 4 i of 1 KiB; a row block's two fragments of a stage are 5 chunks in one piece
+    uint32_t a_off[kALoads];
+#pragma unroll
+    for (int i = 0; i < kALoads; ++i) {
+        const int c = min(wave + 4 * i, kABytes / 1024 - 1), rb = c / 5;
+        a_off[i] = (uint32_t)(m_tile / kFragRows + rb) * (uint32_t)(steps2 * kFragBytes) + (uint32_t)(c % 5) * 1024u + lane * 16u;
+    }
+    const uint32_t run_pitch = (uint32_t)p.strips * (kRunSteps * kUnitBytes), strip_off = (uint32_t)strip * (kRunSteps * kUnitBytes);
+    const uint32_t s_pitch = (uint32_t)p.strips * 128;     // bytes between groups
+    const uint32_t s_voff = (GS == 1 ? half * s_pitch : 0u) + (lane & 31) * 4;
+    uint8_t* const a_lds = lds;
+    uint8_t* const w_lds = lds + 3 * kASlot + wave * (kStageSteps * kUnitBytes);
+    uint8_t* const s_lds = lds + 3 * kASlot + 2 * kWBytes + wave * 256;
+
+#define SLIMK_LDS_PTR(ptr) ((__attribute__((address_space(3))) void*)(ptr))
+    auto fetch_a = [&](int stage, int slot) {
+#pragma unroll
+        for (int i = 0; i < kALoads; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, SLIMK_LDS_PTR(a_lds + (wave + 4 * i < kABytes / 1024 ? slot * kASlot + (wave + 4 * i) * 1024 : kLds - 1024)),
+                                                     16, a_off[i],
+                                                     (stage0 + stage) * (kStageSteps * kFragBytes), 0, 0);
+    };
+    auto fetch_w = [&](int stage, int slot) {
+        const int st = (stage0 + stage) * kStageSteps;
+        const uint32_t off = (uint32_t)(st / kRunSteps) * run_pitch + (uint32_t)(st % kRunSteps) * kUnitBytes + strip_off;
+#pragma unroll
+        for (int s = 0; s < kStageSteps; ++s)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, SLIMK_LDS_PTR(w_lds + slot * kWBytes + s * kUnitBytes), 16, lane * 16,
+                                                     off + s * kUnitBytes, 0, 0);
+        const int g = GS == 1 ? st : (stage0 + stage) >> p.group_shift;   // (past the last group: reads as zero)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(s_rsrc, SLIMK_LDS_PTR(s_lds + slot * kSBytes), 4, s_voff,
+                                                 g * s_pitch + (uint32_t)strip * 128, 0, 0);
+    };
+    constexpr int kLoads = kALoads + kStageSteps + 1;      // LDS-direct loads of a wave per stage
+
+    float t[RB][2][16];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) t[rb][nb][j] = 0.0f;
+
+    fetch_a(0, 0);
+    fetch_w(0, 0);
+    fetch_a(min(1, n_stages - 1), 1);
+    fetch_w(min(1, n_stages - 1), 1);
+
+    // ---- the zero-point term of this workgroup's groups: t = -sum_g zp * scale * rowsum
+    const int sub = (lane >> 4) & 1, c16 = lane & 15;      // channel nb * 32 + col = sub-block 2 nb + sub, column c16
+    const int g_lo = GS == 1 ? stage0 * 2 : stage0 >> p.group_shift;
+    const int g_hi = min(p.G, GS == 1 ? (stage0 + n_stages) * 2 : (stage0 + n_stages + p.group_shift) >> p.group_shift);
+    const __amdgpu_buffer_rsrc_t rs_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t*>(p.rs), 0, (int)((size_t)p.M * p.G * 4 + 16), 0x00020000);
+    const uint32_t s_lane = ((uint32_t)strip * 64 + c16 * 4 + sub) * 2;
+    auto group_scale = [&](int g, int nb) {                // fp16 bits; zero past the workgroup's groups
+        const uint32_t off = g < g_hi ? (uint32_t)g * s_pitch + s_lane + nb * 4 : 0xfffffff0u;
+        return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(s_rsrc, off, 0, 0);
+    };
+    if (!ZP) {
+        for (int g0 = g_lo; g0 < g_hi; g0 += 8) {
+            const int g = g0 + half * 4;
+            uint16_t sc[2][4];
+            v4u r[RB];
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sc[nb][i] = group_scale(g + i, nb);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+                r[rb] = __builtin_amdgcn_raw_buffer_load_b128(rs_rsrc, ((uint32_t)(m_tile + rb * 32 + col) * (uint32_t)p.G + g) * 4u, 0, 0);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)   // (past the workgroup's groups: other rows' sums, or whatever follows the last)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r[rb][i] = g + i < g_hi ? r[rb][i] : 0u;
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                v4u bb;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) bb[i] = (uint32_t)sc[nb][i] * 0x10001u;
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) {
+                    v16f c;
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) c[j] = t[rb][nb][j];
+                    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, r[rb]), __builtin_bit_cast(v8h, bb), c, 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) t[rb][nb][j] = c[j];
+                }
+            }
+        }
+        const float f = -(float)p.zp_const;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) t[rb][nb][j] *= f;
+    } else {
+        constexpr int kRound = 4;   // pairs of groups whose loads are in flight together
+        for (int g0 = g_lo; g0 < g_hi; g0 += 2 * kRound) {
+            uint16_t sc[kRound][2];
+            uint32_t zz[kRound], r[kRound][RB];
+#pragma unroll
+            for (int b = 0; b < kRound; ++b) {
+                const int g = g0 + 2 * b + half;
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) sc[b][nb] = group_scale(g, nb);
+                zz[b] = reinterpret_cast<const uint32_t*>(p.zp_r)[((size_t)min(g, p.G - 1) * p.strips + strip) * 16 + c16] >> (8 * sub);
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+                    r[b][rb] = __builtin_amdgcn_raw_buffer_load_b32(rs_rsrc, ((uint32_t)(m_tile + rb * 32 + col) * (uint32_t)p.G + min(g, p.G - 1)) * 4u, 0, 0);
+            }
+#pragma unroll
+            for (int b = 0; b < kRound; ++b)
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) {
+                    const float zs = -(float)((zz[b] >> (16 * nb)) & 0xffu) * half_bits_to_float(sc[b][nb]);
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) {
+                        const float rsum = half_bits_to_float((uint16_t)(r[b][rb] & 0xffffu)) + half_bits_to_float((uint16_t)(r[b][rb] >> 16));
+                        v16f c;
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) c[j] = t[rb][nb][j];
+                        c = __builtin_amdgcn_mfma_f32_32x32x2f32(rsum, zs, c, 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) t[rb][nb][j] = c[j];
+                    }
+                }
+        }
+    }
+
+    // ---- main loop.  A unit of work is (row block, channel block) and, with GS = 1, the step: its instructions go into
+    // accumulator set u & 1 while the other set is folded into the running sums; the last unit of a stage is folded at
+    // the top of the next.
+    constexpr int kGroups = kStageSteps / GS;              // drains of a block per stage
+    constexpr int kUnits = RB * 2 * kGroups;
+    constexpr int kAq = RB == 4 ? 4 : 3;                   // fragments in registers (64-row tiles: three waves per SIMD)
+    v16f acc[2];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[0][j] = acc[1][j] = 0.0f;
+    float sc_prev = 0.0f;
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+
+    int slot = 0, wslot = 0;
+    v4i raw[kStageSteps];
+    uint16_t sraw[kGroups][2];
+    auto read_w = [&](int ws) {                            // the wave's units and scales of a stage, LDS -> registers
+        const uint8_t* w_st = w_lds + ws * kWBytes + lane * 16;
+        const uint8_t* s_st = s_lds + ws * kSBytes + (c16 * 4 + sub) * 2;
+#pragma unroll
+        for (int s = 0; s < kStageSteps; ++s) raw[s] = *reinterpret_cast<const v4i*>(w_st + s * kUnitBytes);
+#pragma unroll
+        for (int gi = 0; gi < kGroups; ++gi)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) sraw[gi][nb] = *reinterpret_cast<const uint16_t*>(s_st + gi * 128 + nb * 4);
+    };
+    read_w(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    for (int stage = 0; stage < n_stages; ++stage) {
+        const uint8_t* a_st = a_lds + slot * kASlot + lane * 16;
+        const uint8_t* a_st8 = a_lds + slot * kASlot + 2048 + lane * 8;
+        struct Frag { v4i hi, lo; v2i lo2; };
+        auto lds_frag = [&](int f) {                       // f = 2 * row block + step
+            Frag r;
+            r.hi = *reinterpret_cast<const v4i*>(a_st + f * kFragBytes);
+            r.lo = *reinterpret_cast<const v4i*>(a_st + f * kFragBytes + 1024);
+            // (volatile: two of these merged into one read would land outside the operands they belong to)
+            r.lo2 = *(const volatile __attribute__((address_space(3))) v2i*)(a_st8 + f * kFragBytes);
+            return r;
+        };
+        Frag aq[kAq];
+        aq[0] = lds_frag(0);
+        aq[1] = lds_frag(1);
+        // two stages on: every wave is past its reads of that activation slot, this wave past those of its weight slot
+        fetch_a(min(stage + 2, n_stages - 1), slot == 0 ? 2 : slot - 1);
+        fetch_w(min(stage + 2, n_stages - 1), wslot);
+        float sc[kGroups][2];
+#pragma unroll
+        for (int gi = 0; gi < kGroups; ++gi)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) sc[gi][nb] = half_bits_to_float(sraw[gi][nb]) * 16.0f;
+        v4i b[kStageSteps][2];
+#pragma unroll
+        for (int s = 0; s < kStageSteps; ++s) unpack_unit(raw[s], b[s]);
+
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+            // order: row block, then (channel block, step group)
+            const int rb = u / (2 * kGroups), nb = (u / kGroups) % 2, gi = u % kGroups;
+            const int pu = (u + kUnits - 1) % kUnits;
+            const int prb = pu / (2 * kGroups), pnb = (pu / kGroups) % 2, pgi = pu % kGroups;
+            const float scale = u == 0 ? sc_prev : sc[pgi][pnb];
+            if (u % (2 * kGroups) == 0) {
+                if (rb + 1 < RB) {
+                    aq[(2 * rb + 2) % kAq] = lds_frag(2 * rb + 2);
+                    if (kAq == 4) aq[(2 * rb + 3) % kAq] = lds_frag(2 * rb + 3);
+                } else {
+                    // everything but this stage's own requests has landed: the next stage's weights are this wave's alone
+                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+                    read_w(wslot ^ 1);
+                }
+            }
+            // The previous unit is folded beside all but the first of this unit's instructions: its last result is not
+            // there yet when that one issues.
+            constexpr int kMfmas = 2 * GS;
+#pragma unroll
+            for (int i = 0; i < kMfmas; ++i) {
+                const int st = gi * GS + i / 2;
+                const Frag& a = aq[(2 * rb + st) % kAq];
+                v16f zero;
+#pragma unroll
+                for (int j = 0; j < 16; ++j) zero[j] = 0.0f;
+                const v16f c = i == 0 ? zero : acc[u & 1];
+                acc[u & 1] = i % 2 == 0 ? mfma_hi(a.hi, b[st][nb], c) : mfma_lo(a.lo, a.lo2, b[st][nb], c);
+                if (kAq == 3 && rb + 1 < RB && nb == 1 && st == 0 && i % 2 == 1)   // (step 0's last use in this row block)
+                    aq[(2 * rb + 3) % kAq] = lds_frag(2 * rb + 3);
+                __builtin_amdgcn_sched_barrier(0);
+                if (i > 0) {
+#pragma unroll
+                    for (int j = 16 * (i - 1) / (kMfmas - 1); j < 16 * i / (kMfmas - 1); ++j)
+                        t[prb][pnb][j] = __builtin_fmaf(acc[(u & 1) ^ 1][j], scale, t[prb][pnb][j]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        sc_prev = sc[kGroups - 1][1];
+        // (the wave's requests for the next stage landed above) meet the other waves
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        slot = slot == 2 ? 0 : slot + 1;
+        wslot ^= 1;
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+        t[RB - 1][1][j] = __builtin_fmaf(acc[(kUnits - 1) & 1][j], sc_prev, t[RB - 1][1][j]);
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");   // the last (repeated) requests have landed: LDS is free
+
+    uint16_t* out = reinterpret_cast<uint16_t*>(p.out);
+    if (SPLIT) {
+        // publish the partial sums, the last workgroup of the tile adds them up in split order: as in tiled_bodies.h
+        // (write-through 16-byte stores, each followed by the idle cycles its data registers need before reuse)
+        constexpr int kTileBytes = kBM * 256 * 4;
+        constexpr int kCoherent = 17;  // sc0 | sc1
+        const int n_split = (int)gridDim.y;
+        const __amdgpu_buffer_rsrc_t ws_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            p.ws_partial, 0, (int)((size_t)n_split * total * kTileBytes), 0x00020000);
+        const uint32_t ws_lane = (uint32_t)wave * (RB * 2 * 4 * 1024) + lane * 16;
+        const uint32_t ws_tile = (uint32_t)tile * kTileBytes, ws_pitch = (uint32_t)total * kTileBytes;
+        uint32_t ws_off[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            ws_off[rb] = ws_lane + rb * 8192 + blockIdx.y * ws_pitch + ws_tile;
+            asm volatile("" : "+v"(ws_off[rb]));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float* tv = &t[rb][i / 4][(i % 4) * 4];
+                const v4f v = {tv[0], tv[1], tv[2], tv[3]};
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), ws_rsrc, ws_off[rb] + i * 1024, 0, kCoherent);
+                asm volatile("s_nop 1" ::: "memory");
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        if (tid == 0) {
+            const unsigned prev = __hip_atomic_fetch_add(p.ws_counter + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *reinterpret_cast<uint32_t*>(lds) = (prev == (unsigned)(n_split - 1));
+        }
+        __syncthreads();
+        const bool last = *reinterpret_cast<uint32_t*>(lds) != 0;
+        if (!last) return;
+        __syncthreads();   // (the verdict is read before the output staging overwrites it)
+        constexpr int kChunk = 2;   // row blocks whose fragments are in flight together
+#pragma unroll
+        for (int rb0 = 0; rb0 < RB; rb0 += kChunk) {
+#pragma unroll
+            for (int rb = 0; rb < kChunk; ++rb)
+#pragma unroll
+                for (int j = 0; j < 32; ++j) t[rb0 + rb][j / 16][j % 16] = 0.0f;
+            for (int sp = 0; sp < n_split; ++sp) {
+                v4f v[kChunk][8];
+#pragma unroll
+                for (int rb = 0; rb < kChunk; ++rb)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        v[rb][i] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                            ws_rsrc, ws_lane + (rb0 + rb) * 8192 + i * 1024, sp * ws_pitch + ws_tile, kCoherent));
+#pragma unroll
+                for (int rb = 0; rb < kChunk; ++rb)
+#pragma unroll
+                    for (int j = 0; j < 32; ++j) t[rb0 + rb][j / 16][j % 16] += v[rb][j / 4][j % 4];
+            }
+        }
+        if (tid == 0) __hip_atomic_store(p.ws_counter + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+
+    // ---- epilogue: out = cast(t * s_a[m]); lane (col, half), element j: row (j & 3) + 8 * (j >> 2) + 4 * half
+    if (!strip_ok) return;
+    const bool wide = (p.N & 7) == 0 && (p.ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
+    constexpr int kPitch = 72;   // floats: the half-waves' rows (4 apart) fall into different halves of the banks
+    static_assert(32 * kPitch * 4 * kStripsPerWg <= kLds, "output staging exceeds the stage buffers");
+    float* stage_out = reinterpret_cast<float*>(lds) + wave * (32 * kPitch);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        float sa[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sa[j] = p.s_a[min(m_tile + rb * 32 + (j & 3) + 8 * (j >> 2) + 4 * half, p.M - 1)];
+        if (wide) {
+            // 8 channels = one 16-byte store per lane: the values turn through the wave's corner of LDS
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    stage_out[((j & 3) + 8 * (j >> 2) + 4 * half) * kPitch + nb * 32 + col] = t[rb][nb][j] * sa[j];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = i * 8 + (lane >> 3), cg = lane & 7;
+                const v4f lo = *reinterpret_cast<const v4f*>(stage_out + row * kPitch + cg * 8);
+                const v4f hi = *reinterpret_cast<const v4f*>(stage_out + row * kPitch + cg * 8 + 4);
+                v4u v;
+                v.x = (uint32_t)OutT::cast(lo.x) | ((uint32_t)OutT::cast(lo.y) << 16);
+                v.y = (uint32_t)OutT::cast(lo.z) | ((uint32_t)OutT::cast(lo.w) << 16);
+                v.z = (uint32_t)OutT::cast(hi.x) | ((uint32_t)OutT::cast(hi.y) << 16);
+                v.w = (uint32_t)OutT::cast(hi.z) | ((uint32_t)OutT::cast(hi.w) << 16);
+                const int m = m_tile + rb * 32 + row, n = strip * kStripN + cg * 8;
+                if (m < p.M && n < p.N) *reinterpret_cast<v4u*>(out + (size_t)m * p.ldo + n) = v;
+            }
+        } else {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const int m = m_tile + rb * 32 + (j & 3) + 8 * (j >> 2) + 4 * half, n = strip * kStripN + nb * 32 + col;
+                    if (m < p.M && n < p.N) out[(size_t)m * p.ldo + n] = OutT::cast(t[rb][nb][j] * sa[j]);
+                }
+        }
+    }
+}
+
+// 128-row tiles: two workgroups per CU (80 KiB of LDS and 256 registers each), 64-row tiles three
+template <int RB, int GS, bool SPLIT, bool ZP, typename OutT>
+__global__ __launch_bounds__(256, RB == 4 ? 2 : 3) void mx_gemm_kernel(const MxParams p) {
+    mx_body<RB, GS, SPLIT, ZP, OutT>(p);
+}
+
+template <int RB, int GS>
+void launch_rb_gs(const MxParams& p, bool out_bf16, dim3 grid, hipStream_t stream) {
+    const dim3 block(256);
+#define SLIMK_MX_LAUNCH(SPLITV, ZPV)                                                                       \
+    do {                                                                                                   \
+        if (out_bf16) mx_gemm_kernel<RB, GS, SPLITV, ZPV, OutBF16><<<grid, block, 0, stream>>>(p);         \
+        else mx_gemm_kernel<RB, GS, SPLITV, ZPV, OutF16><<<grid, block, 0, stream>>>(p);                   \
+    } while (0)
+    const bool zp = p.zp_r != nullptr;
+    if (p.split > 1) {
+        if (zp) SLIMK_MX_LAUNCH(true, true);
+        else SLIMK_MX_LAUNCH(true, false);
+    } else {
+        if (zp) SLIMK_MX_LAUNCH(false, true);
+        else SLIMK_MX_LAUNCH(false, false);
+    }
+#undef SLIMK_MX_LAUNCH
+}
+
+}  // namespace
+
+MxPlan mx_plan(int M, int N, int K, int group_size) {
+    const int tiles_n = ((N + kStripN - 1) / kStripN + kStripsPerWg - 1) / kStripsPerWg;
+    const int tiles128 = tiles_n * ((M + 127) / 128);
+    MxPlan plan;
+    plan.rb = tiles128 >= 2 * 256 ? 4 : 2;
+    plan.tiles = plan.rb == 4 ? tiles128 : tiles_n * ((M + 63) / 64);
+    const int stages = mx_padded_steps(K) / 2;
+    // K splits of 64-row tiles: how evenly the workgroups fill the CUs, how well a CU runs with one, two or three of
+    // them, and the stages' worth a workgroup spends outside its stages
+    int best = 1;
+    if (plan.rb == 2 && plan.tiles <= 400) {
+        double best_score = -1.0;
+        for (int split : {1, 2, 3, 4, 6, 8}) {
+            const int per = (stages + split - 1) / split;
+            if (split > 1 && per < 8) break;
+            const long long wgs = (long long)plan.tiles * ((stages + per - 1) / per);
+            const long long n = (wgs + 255) / 256;
+            const double fill = (double)wgs / (256.0 * (double)n), together = n == 1 ? 0.7 : (n == 2 ? 0.9 : 1.0);
+            const double score = fill * together * (double)per / ((double)per + 10.0);
+            if (score > best_score * 1.0001) {
+                best_score = score;
+                best = split;
+            }
+        }
+    }
+    int per = (stages + best - 1) / best;
+    if (group_size == 256) per = (per + 1) / 2 * 2;   // (a split owns whole groups)
+    plan.stages_per_split = per;
+    plan.split = (stages + per - 1) / per;
+    return plan;
+}
+
+hipError_t launch_mx_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size, uint8_t* frag, uint32_t* rs,
+                           float* s_a, hipStream_t stream) {
+    const dim3 grid((unsigned)(M >= 256 ? (M + 255) / 256 * 256 : M)), block((unsigned)((K / 32 + 63) / 64 * 64));
+    if (x_bf16) mx_quant_kernel<true><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, rs, s_a);
+    else mx_quant_kernel<false><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, rs, s_a);
+    return hipGetLastError();
+}
+
+hipError_t launch_mx_gemm(const MxParams& p, int rb, int gs, bool out_bf16, hipStream_t stream) {
+    const int bm = rb * kFragRows;
+    const int tiles = ((p.strips + kStripsPerWg - 1) / kStripsPerWg) * ((p.M + bm - 1) / bm);
+    const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)p.split);
+    if (rb == 4) {
+        if (gs == 1) launch_rb_gs<4, 1>(p, out_bf16, grid, stream);
+        else launch_rb_gs<4, 2>(p, out_bf16, grid, stream);
+    } else {
+        if (gs == 1) launch_rb_gs<2, 1>(p, out_bf16, grid, stream);
+        else launch_rb_gs<2, 2>(p, out_bf16, grid, stream);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace w2a8

@@ -288,6 +288,44 @@ def w2a8_linear_fused(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *
     return out
 
 
+def w2a8_linear_digits(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *,
+                       out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """out[M, N] for many token rows x [M, K] fp16 / bf16: the activations are quantised as by ``quantize_act_int8``,
+    split into an fp4 and an fp6 digit each, and multiplied on the block-scaled matrix cores (exact group sums, the
+    scaled sums in fp32).  The layers take it where ``linear_digits_applies``."""
+    L = _lib.lib()
+    _require_cuda(x, "x")
+    if x.dim() != 2 or x.dtype not in _DT:
+        raise ValueError("x must be a 2-D float16 or bfloat16 tensor [M, K]")
+    if out_dtype not in _DT:
+        raise ValueError("out_dtype must be torch.float16 or torch.bfloat16")
+    M, K = x.shape
+    if K != w.K:
+        raise ValueError(f"activation K={K} does not match weight K={w.K}")
+    if x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < K or x.data_ptr() % 16 != 0:
+        x = x.contiguous()
+        if x.data_ptr() % 16 != 0:      # contiguous already, but not at a 16-byte boundary
+            x = x.clone()
+    dev = x.device
+    if out is None:
+        out = torch.empty((M, w.N), dtype=out_dtype, device=dev)
+    with torch.cuda.device(dev):
+        act = torch.empty(L.slimk_w2a8_linear_activation_bytes(M, w.N, K, w.group_size), dtype=torch.uint8, device=dev)
+        ws = _workspace(w, L.slimk_w2a8_linear_workspace_bytes(M, w.N, K, w.group_size))
+        _lib.check(L.slimk_w2a8_linear(
+            x.data_ptr(), x.stride(0), _DT[x.dtype], w.w_r.data_ptr(), w.s_r.data_ptr(),
+            w.zp_r.data_ptr() if w.zp_r is not None else None, w.zp_const, M, w.N, K, w.group_size,
+            out.data_ptr(), out.stride(0), _DT[out.dtype], act.data_ptr(), act.numel(),
+            ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream_ptr(dev)))
+    return out
+
+
+def linear_digits_applies(M: int, w: W2A8Weight) -> bool:
+    """Whether a layer call of M token rows goes through ``w2a8_linear_digits`` (the rule and what it was measured
+    against stand at slimk_w2a8_linear_route)."""
+    return bool(_lib.lib().slimk_w2a8_linear_route(M, w.N, w.K, w.group_size, 0 if w.zp_r is None else 1))
+
+
 def w2a16_gemm(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *, split_k: int = 0,
                out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The weight-only form: out[M, N] = x @ dequant(W)^T with the fp16 or bf16 activations x [M, K] as they are (no
@@ -500,6 +538,8 @@ class W2A8Linear(torch.nn.Module):
             # one token row: one launch with the quantisation inside the GEMM (measured 6.1 us against 8.0 us at
             # 4096 x 4096; from two rows on the separate act-quant launch is as fast or faster)
             y = w2a8_linear_fused(x2, self.weight, self.out_dtype)
+        elif linear_digits_applies(x2.shape[0], self.weight):
+            y = w2a8_linear_digits(x2, self.weight, self.out_dtype)
         else:
             # prefill-sized inputs on symmetric weights go to the tiled kernel, which reads no group sums: leave them out
             qa = quantize_act_int8(x2, self.weight.group_size, rowsum=needs_rowsum(x2.shape[0], self.weight))

@@ -1,0 +1,91 @@
+"""The digit form of a layer call (csrc/gemm_mx.hip): activations split into an fp4 and an fp6 digit, exact group sums on
+the block-scaled matrix cores.  Held to the oracle within the output criterion of the path: every element within one
+ULP or rtol 1e-3, or within the fp32 re-association bound (the zero-point term is added first and in one piece, K may be
+split across workgroups)."""
+import numpy as np
+import pytest
+import torch
+
+from slimkernels_amd import _lib, workloads
+import parity_utils as pu
+
+FAKE = 0x10000
+
+
+def test_every_int8_value_is_the_sum_of_its_two_digits():
+    fp4 = np.array([0, 0.5, 1, 1.5, 2, 3, 4, 6])                     # e2m1
+    fp6 = np.array([(m / 8 if e == 0 else (1 + m / 8) * 2.0 ** (e - 1)) for e in range(4) for m in range(8)])   # e2m3
+    for q in range(-127, 128):
+        a4 = np.sign(q) * fp4[np.argmin(np.abs(fp4 - abs(q) / 32))]
+        assert abs(q - 32 * a4) <= 16
+        assert abs(q - 32 * a4) / 8 in fp6, q
+
+
+def test_validation_and_sizes():
+    L = _lib.lib()
+    # (x, ldx, x_dtype, w_r, s_r, zp_r, zp_const, M, N, K, group, out, ldo, out_dtype, act, act_bytes, ws, ws_bytes, stream)
+    names = ["x", "ldx", "xdt", "w", "s", "zp", "zpc", "M", "N", "K", "g", "out", "ldo", "odt", "act", "actb", "ws", "wsb", "st"]
+    ok = [FAKE, 4096, 0, FAKE, FAKE, None, 2, 64, 256, 4096, 128, FAKE, 256, 0, FAKE, 1 << 30, None, 0, None]
+
+    def call(**kw):
+        a = list(ok)
+        for k, v in kw.items():
+            a[names.index(k)] = v
+        return L.slimk_w2a8_linear(*a)
+
+    assert call(x=None) == 1 and call(act=None) == 1
+    assert call(M=0) == 2 and call(g=100) == 2 and call(zpc=4) == 2 and call(ldx=4000) == 2 and call(ldo=100) == 2
+    assert call(xdt=2) == 4 and call(odt=5) == 4
+    assert call(ldx=4100) == 3 and call(x=FAKE + 2) == 3 and call(act=FAKE + 4) == 3 and call(out=FAKE + 1) == 3
+    assert call(actb=1000) == 5
+    assert L.slimk_w2a8_linear_workspace_bytes(64, 256, 4096, 128) > 0 and call() == 5      # few tiles: K is split
+    assert call(K=32768 + 64, ldx=40000, g=64) == 7                                          # a row no longer fits a workgroup
+    assert L.slimk_w2a8_linear_activation_bytes(64, 256, 32768 + 64, 64) == 0
+    assert L.slimk_w2a8_linear_route(4096, 4096, 32768 + 64, 64, 0) == 0
+    # digits: 2560 bytes per 32 rows x 64 elements, an odd step count rounded up; then sums and token scales
+    assert L.slimk_w2a8_linear_activation_bytes(33, 256, 192, 64) == 2 * 4 * 2560 + 512 + 256
+    assert L.slimk_w2a8_linear_route(1, 4096, 4096, 128, 0) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,g,mode,out", [
+    (1, 64, 64, 64, "sym", "float16"),             # one row, one step: half a stage
+    (31, 100, 192, 64, "asym", "bfloat16"),        # an odd number of steps, a ragged N, per-group zero-points
+    (33, 256, 128, 128, "ref", "float16"),         # one stage; uniform zero-point 1
+    (64, 320, 1088, 64, "sym", "bfloat16"),        # two channel tiles, one of a single strip; an odd number of steps
+    (65, 1001, 768, 256, "asym", "float16"),       # groups of two stages, three to a split-free launch; 2-byte stores
+    (77, 256, 4096, 128, "sym", "float16"),        # K split across workgroups
+    (130, 264, 3328, 256, "sym", "bfloat16"),      # split in whole groups of 256
+    (257, 72, 2048, 64, "asym", "float16"),        # rows dealt to the XCDs (from 256 on), split
+    (1025, 14592, 320, 64, "sym", "float16"),      # 128-row tiles (513 of them), the last one a single row
+    (1000, 16640, 256, 128, "asym", "bfloat16"),   # 128-row tiles with per-group zero-points
+])
+def test_digits_against_the_oracle(gpu_ops, oracle, M, N, K, g, mode, out):
+    from slimkernels_amd.torch.ops import w2a8_linear_digits
+    print(f"digits M={M} N={N} K={K} g={g} {mode} {out}", flush=True)
+    case = pu.small_case(M, N, K, g, mode, seed=M + N, out_dtype=out, outliers=M % 2 == 1)
+    packed, scales, zero = pu.quantized_weight(case)
+    x = workloads.make_activation(case)
+    bf16 = out == "bfloat16"
+    big = M * N * (K // g) > 1 << 26               # (the oracle's group sums would be gigabytes: the strict criterion alone)
+    ref = oracle.reference_forward(x, packed, scales, zero, g, out_bf16=bf16, want_acc=not big)
+    w, xd = pu.device_inputs(gpu_ops, case, packed, scales, zero, x)
+    y = w2a8_linear_digits(xd, w, pu.torch_dtype(case))
+    bound = None
+    if not big:
+        # the zero-point term and the sum of q * code are each larger than their difference: their magnitudes bound it
+        zp = np.broadcast_to(np.asarray(zero, np.int64), (K // g, N))
+        rs = ref["q"].reshape(M, K // g, g).astype(np.int64).sum(2)
+        folded = np.abs(rs)[:, None, :] * zp.T[None]
+        bound = pu.reorder_bound(np.abs(ref["acc"].astype(np.int64)) + 2 * folded, scales, ref["s_a"])
+    if big:
+        # every element within one ULP or rtol 1e-3 but a few whose terms cancel, which the sums' magnitude bounds:
+        # K / g * 2^-24 * s_a * sum_g scale * 127 * 3 * g, far below a dropped term
+        bound = (K // g * 2.0 ** -24 * ref["s_a"].astype(np.float64)[:, None] * 3 * 127 * g *
+                 np.asarray(scales, np.float64).sum(0)[None, :])
+    pu.assert_out_close(pu.out_tensor_bits(y), ref["out_bits"], bf16, reorder_bound=bound, what="digits")
+    # a strided activation and reused scratch give the same bits
+    wide = torch.zeros((M, K + 64), dtype=xd.dtype, device="cuda")
+    wide[:, :K] = xd
+    y2 = w2a8_linear_digits(wide[:, :K], w, pu.torch_dtype(case))
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
