@@ -15,9 +15,11 @@ computes on the CPU.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import collections
 import dataclasses
+import functools
 from typing import Optional
 
 import numpy as np
@@ -28,8 +30,29 @@ from .. import _lib
 _DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 
 
+# A decode call's kernel runs for 4-5 us, so what the host does around its launch decides how many calls a second one
+# process makes: the stream pointer and the current device come straight from torch's native accessors (0.2 us; building
+# a Stream object and entering torch.cuda.device took 4 us a call), and the library's pure functions of the
+# shape are asked once per shape.
+_raw_stream = torch._C._cuda_getCurrentRawStream
+_current_device = torch._C._cuda_getDevice
+_HERE = contextlib.nullcontext()
+
+
 def _stream_ptr(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index
+    return _raw_stream(_current_device() if index is None else index)
+
+
+def _on(device):
+    """torch.cuda.device(device), for nothing where that device is already the current one."""
+    return _HERE if device.index is None or device.index == _current_device() else torch.cuda.device(device)
+
+
+@functools.lru_cache(maxsize=4096)
+def _query(name: str, *args) -> int:
+    """A size or route the library computes from the shape alone."""
+    return getattr(_lib.lib(), name)(*args)
 
 
 def _require_cuda(t: torch.Tensor, name: str):
@@ -110,7 +133,7 @@ def repack_w2(packed, scales, zp=None, group_size: int = 128, zp_const: int = 2,
     s_r = torch.empty(sb // 2, dtype=torch.float16, device=dev)
     zp_r = torch.empty(L.slimk_w2a8_repacked_zp_bytes(N, K, group_size), dtype=torch.uint8, device=dev) \
         if zp_d is not None else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(L.slimk_w2a8_repack(packed_d.data_ptr(), packed_d.stride(0), scales_d.data_ptr(),
                                        zp_d.data_ptr() if zp_d is not None else None, N, K, group_size,
                                        w_r.data_ptr(), s_r.data_ptr(),
@@ -140,7 +163,7 @@ def quantize_weight_gpu(weight_nk: torch.Tensor, group_size: int = 128, mode: st
     packed = torch.empty((N, K // 4), dtype=torch.uint8, device=dev)
     scales = torch.empty((K // group_size, N), dtype=torch.float16, device=dev)
     zero = torch.empty((K // group_size, N), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(L.slimk_w2a8_quantize_weight(w.data_ptr(), w.stride(0), _DT[w.dtype], N, K, group_size, modes[mode],
                                                 packed.data_ptr(), packed.stride(0), scales.data_ptr(), zero.data_ptr(),
                                                 _stream_ptr(dev)))
@@ -178,7 +201,7 @@ def quantize_act_int8(x: torch.Tensor, group_size: int = 128, copies: int = 1, r
     q = torch.empty((M, max(copies, 1) * K), dtype=torch.int8, device=x.device)
     s_a = torch.empty((M,), dtype=torch.float32, device=x.device)
     rs = torch.empty((max(copies, 1) * max(K // group_size, 1), ldr), dtype=torch.int32, device=x.device) if rowsum else None
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.check(L.slimk_w2a8_act_quant_rep(x.data_ptr(), x.stride(0), _DT[x.dtype], M, K, group_size, copies,
                                               q.data_ptr(), q.stride(0), s_a.data_ptr(),
                                               rs.data_ptr() if rs is not None else None, ldr, _stream_ptr(x.device)))
@@ -190,7 +213,7 @@ def needs_rowsum(M: int, w: "W2A8Weight") -> bool:
     everything but the tiled kernel and the kernel for 33..128 rows on the symmetric levels (uniform zero-point 2) does."""
     if w.zp_r is not None or w.zp_const != 2 or w.group_size > 256:
         return True
-    return _lib.lib().slimk_w2a8_gemm_auto_route(M, w.N, w.K, w.group_size) not in (2, 4)
+    return _query("slimk_w2a8_gemm_auto_route", M, w.N, w.K, w.group_size) not in (2, 4)
 
 
 def _workspace(w: W2A8Weight, nbytes: int) -> Optional[torch.Tensor]:
@@ -228,8 +251,8 @@ def w2a8_gemm(qa: QuantizedActivation, w: W2A8Weight, out_dtype=torch.float16, *
         acc, mode = torch.empty((M, w.N), dtype=torch.int32, device=dev), _lib.DUMP_SUM
     elif dump is not None:
         raise ValueError("dump must be None, 'groups' or 'sum'")
-    with torch.cuda.device(dev):
-        ws_bytes = L.slimk_w2a8_gemm_workspace_bytes(M, w.N, K, w.group_size, kern, split_k)
+    with _on(dev):
+        ws_bytes = _query("slimk_w2a8_gemm_workspace_bytes", M, w.N, K, w.group_size, kern, split_k)
         ws = _workspace(w, ws_bytes)
         _lib.check(L.slimk_w2a8_gemm(
             qa.q.data_ptr(), qa.q.stride(0), qa.s_a.data_ptr(),
@@ -277,8 +300,8 @@ def w2a8_linear_fused(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *
     dev = x.device
     if out is None:
         out = torch.empty((M, w.N), dtype=out_dtype, device=dev)
-    with torch.cuda.device(dev):
-        ws_bytes = L.slimk_w2a8_gemm_fused_workspace_bytes(M, w.N, K, w.group_size, split_k)
+    with _on(dev):
+        ws_bytes = _query("slimk_w2a8_gemm_fused_workspace_bytes", M, w.N, K, w.group_size, split_k)
         ws = _workspace(w, ws_bytes)
         _lib.check(L.slimk_w2a8_gemm_fused(
             x.data_ptr(), x.stride(0), _DT[x.dtype], w.w_r.data_ptr(), w.s_r.data_ptr(),
@@ -309,9 +332,9 @@ def w2a8_linear_digits(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, 
     dev = x.device
     if out is None:
         out = torch.empty((M, w.N), dtype=out_dtype, device=dev)
-    with torch.cuda.device(dev):
-        act = torch.empty(L.slimk_w2a8_linear_activation_bytes(M, w.N, K, w.group_size), dtype=torch.uint8, device=dev)
-        ws = _workspace(w, L.slimk_w2a8_linear_workspace_bytes(M, w.N, K, w.group_size))
+    with _on(dev):
+        act = torch.empty(_query("slimk_w2a8_linear_activation_bytes", M, w.N, K, w.group_size), dtype=torch.uint8, device=dev)
+        ws = _workspace(w, _query("slimk_w2a8_linear_workspace_bytes", M, w.N, K, w.group_size))
         _lib.check(L.slimk_w2a8_linear(
             x.data_ptr(), x.stride(0), _DT[x.dtype], w.w_r.data_ptr(), w.s_r.data_ptr(),
             w.zp_r.data_ptr() if w.zp_r is not None else None, w.zp_const, M, w.N, K, w.group_size,
@@ -323,7 +346,7 @@ def w2a8_linear_digits(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, 
 def linear_digits_applies(M: int, w: W2A8Weight) -> bool:
     """Whether a layer call of M token rows goes through ``w2a8_linear_digits`` (the rule and what it was measured
     against stand at slimk_w2a8_linear_route)."""
-    return bool(_lib.lib().slimk_w2a8_linear_route(M, w.N, w.K, w.group_size, 0 if w.zp_r is None else 1))
+    return bool(_query("slimk_w2a8_linear_route", M, w.N, w.K, w.group_size, 0 if w.zp_r is None else 1))
 
 
 def w2a16_gemm(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *, split_k: int = 0,
@@ -347,8 +370,8 @@ def w2a16_gemm(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *, split
     dev = x.device
     if out is None:
         out = torch.empty((M, w.N), dtype=out_dtype, device=dev)
-    with torch.cuda.device(dev):
-        ws_bytes = L.slimk_w2a16_gemm_workspace_bytes(M, w.N, K, w.group_size, split_k)
+    with _on(dev):
+        ws_bytes = _query("slimk_w2a16_gemm_workspace_bytes", M, w.N, K, w.group_size, split_k)
         stream = _stream_ptr(dev)
         # its own buffer, one per stream as there: the W2A8 workspace holds counters that must stay zero
         ws = w.partials16.get(stream) if ws_bytes else None
@@ -378,7 +401,7 @@ def w2a16_gemm_grouped(problems, out_dtype=torch.float16):
     if xdt not in _DT or out_dtype not in _DT:
         raise ValueError("activations and out_dtype must be torch.float16 or torch.bfloat16")
     outs, keep = [], []
-    with torch.cuda.device(dev):
+    with _on(dev):
         for lo in range(0, len(probs), _lib.MAX_GROUP):
             chunk = probs[lo:lo + _lib.MAX_GROUP]
             arr = (_lib.Problem16 * len(chunk))()
@@ -420,7 +443,7 @@ def w2a8_gemm_grouped(problems, out_dtype=torch.float16, *, dump: Optional[str] 
     if dump not in (None, "groups", "sum"):
         raise ValueError("dump must be None, 'groups' or 'sum'")
     outs, accs = [], []
-    with torch.cuda.device(dev):
+    with _on(dev):
         for lo in range(0, len(probs), _lib.MAX_GROUP):
             chunk = probs[lo:lo + _lib.MAX_GROUP]
             arr = (_lib.Problem * len(chunk))()
@@ -530,8 +553,7 @@ class W2A8Linear(torch.nn.Module):
         return cls(load_w2_weight(path, device), bias, out_dtype)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1])
+        x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         if x2.dtype not in _DT:
             x2 = x2.to(self.out_dtype)
         if x2.shape[0] == 1 and fused_applies(1, x2.shape[1]):
@@ -546,7 +568,7 @@ class W2A8Linear(torch.nn.Module):
             y = w2a8_gemm(qa, self.weight, self.out_dtype)
         if self.bias is not None:
             y = y + self.bias
-        return y.reshape(*lead, self.out_features)
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.out_features)
 
 
 class W2A16Linear(W2A8Linear):
@@ -554,11 +576,10 @@ class W2A16Linear(W2A8Linear):
     weight-only kernel, meant for a few token rows; the weight object and the constructors are W2A8Linear's."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1])
+        x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         if x2.dtype not in _DT:
             x2 = x2.to(torch.float16)
         y = w2a16_gemm(x2, self.weight, self.out_dtype)
         if self.bias is not None:
             y = y + self.bias
-        return y.reshape(*lead, self.out_features)
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.out_features)

@@ -12,7 +12,7 @@ import torch
 
 from .. import w4 as host_w4
 from .. import _lib
-from .ops import (QuantizedActivation, W2A8Weight, _DT, _require_cuda, _stream_ptr, _workspace, fused_applies, quantize_act_int8, repack_w2,
+from .ops import (QuantizedActivation, W2A8Weight, _DT, _on, _query, _require_cuda, _stream_ptr, _workspace, fused_applies, quantize_act_int8, repack_w2,
                   w2a8_gemm, w2a8_linear_fused)
 
 
@@ -72,7 +72,7 @@ def quantize_weight4_gpu(weight_nk: torch.Tensor, group_size: int = 128, mode: s
     planes = torch.empty((N, K // 2), dtype=torch.uint8, device=dev)
     scales2 = torch.empty((2 * G, N), dtype=torch.float16, device=dev)
     zp2 = torch.empty((2 * G, N), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(L.slimk_w2a8_quantize_weight4(w.data_ptr(), w.stride(0), _DT[w.dtype], N, K, group_size, modes[mode],
                                                  planes.data_ptr(), planes.stride(0), scales2.data_ptr(), zp2.data_ptr(),
                                                  _stream_ptr(dev)))
@@ -153,8 +153,8 @@ def w4a8_gemm_one_pass(qa: QuantizedActivation, w: W4A8Weight, out_dtype=torch.f
     if out is None:
         out = torch.empty((M, w.N), dtype=out_dtype, device=dev)
     L = _lib.lib()
-    with torch.cuda.device(dev):
-        ws = _workspace(w.planes, L.slimk_w4a8_gemm_workspace_bytes(M, w.N, K, w.group_size, split_k))
+    with _on(dev):
+        ws = _workspace(w.planes, _query("slimk_w4a8_gemm_workspace_bytes", M, w.N, K, w.group_size, split_k))
         # zero-points other than 8 enter through the row sums of the activations
         zp_r = None if w.uniform_zp8 else w.planes.zp_r
         _lib.check(L.slimk_w4a8_gemm(qa.q.data_ptr(), qa.q.stride(0), qa.s_a.data_ptr(),
@@ -215,14 +215,13 @@ class W4A8Linear(torch.nn.Module):
         return cls(repack_w4(packed4, scales, zero, group_size, device=device), bias, out_dtype)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1])
+        x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         if x2.dtype not in _DT:
             x2 = x2.to(self.out_dtype)
         y = w4a8_linear(x2, self.weight, self.out_dtype)
         if self.bias is not None:
             y = y + self.bias
-        return y.reshape(*lead, self.out_features)
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.out_features)
 
 
 def w4matmul_splitk(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor) -> torch.Tensor:
