@@ -295,36 +295,44 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
         return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(s_rsrc, off, 0, 0);
     };
     if (!ZP) {
-        for (int g0 = g_lo; g0 < g_hi; g0 += 8) {
+        // eight groups per turn (a half-wave four of them), the next turn's operands asked for ahead
+        struct Operands { v2u sc[4]; v4u r[RB]; };
+        auto load = [&](int g0) {
+            Operands o;
             const int g = g0 + half * 4;
-            uint16_t sc[2][4];
-            v4u r[RB];
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) sc[nb][i] = group_scale(g + i, nb);
+            for (int i = 0; i < 4; ++i)   // the four sub-blocks' scales; zero past the workgroup's groups
+                o.sc[i] = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(
+                    s_rsrc, g + i < g_hi ? (uint32_t)(g + i) * s_pitch + ((uint32_t)strip * 64 + c16 * 4) * 2 : 0xfffffff0u, 0, 0));
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
-                r[rb] = __builtin_amdgcn_raw_buffer_load_b128(rs_rsrc, ((uint32_t)(m_tile + rb * 32 + col) * (uint32_t)p.G + g) * 4u, 0, 0);
+                o.r[rb] = __builtin_amdgcn_raw_buffer_load_b128(rs_rsrc, ((uint32_t)(m_tile + rb * 32 + col) * (uint32_t)p.G + g) * 4u, 0, 0);
+            return o;
+        };
+        Operands cur = load(g_lo);
+        for (int g0 = g_lo; g0 < g_hi; g0 += 8) {
+            const Operands next = load(g0 + 8);
+            const int g = g0 + half * 4;
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)   // (past the workgroup's groups: other rows' sums, or whatever follows the last)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) r[rb][i] = g + i < g_hi ? r[rb][i] : 0u;
+                for (int i = 0; i < 4; ++i) cur.r[rb][i] = g + i < g_hi ? cur.r[rb][i] : 0u;
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
                 v4u bb;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) bb[i] = (uint32_t)sc[nb][i] * 0x10001u;
+                for (int i = 0; i < 4; ++i) bb[i] = ((cur.sc[i][nb] >> (16 * sub)) & 0xffffu) * 0x10001u;
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb) {
                     v16f c;
 #pragma unroll
                     for (int j = 0; j < 16; ++j) c[j] = t[rb][nb][j];
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, r[rb]), __builtin_bit_cast(v8h, bb), c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, cur.r[rb]), __builtin_bit_cast(v8h, bb), c, 0, 0, 0);
 #pragma unroll
                     for (int j = 0; j < 16; ++j) t[rb][nb][j] = c[j];
                 }
             }
+            cur = next;
         }
         const float f = -(float)p.zp_const;
 #pragma unroll
@@ -541,11 +549,19 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
     constexpr int kPitch = 72;   // floats: the half-waves' rows (4 apart) fall into different halves of the banks
     static_assert(32 * kPitch * 4 * kStripsPerWg <= kLds, "output staging exceeds the stage buffers");
     float* stage_out = reinterpret_cast<float*>(lds) + wave * (32 * kPitch);
+    // the token scales, four rows a load, all in flight together (rows past M: zero, or what the scratch holds behind them)
+    const __amdgpu_buffer_rsrc_t sa_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.s_a), 0, (p.M + 3) / 4 * 16, 0x00020000);
+    v4f sa4[RB][4];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            sa4[rb][i] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(sa_rsrc, (m_tile + rb * 32 + i * 8 + 4 * half) * 4, 0, 0));
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
         float sa[16];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) sa[j] = p.s_a[min(m_tile + rb * 32 + (j & 3) + 8 * (j >> 2) + 4 * half, p.M - 1)];
+        for (int j = 0; j < 16; ++j) sa[j] = sa4[rb][j >> 2][j & 3];
         if (wide) {
             // 8 channels = one 16-byte store per lane: the values turn through the wave's corner of LDS
 #pragma unroll
@@ -605,32 +621,44 @@ void launch_rb_gs(const MxParams& p, bool out_bf16, dim3 grid, hipStream_t strea
 
 }  // namespace
 
+// The predicted time of a layer call in this form (us, quantisation included): start-up, quantisation, the round trip of
+// the partial sums, and stages per workgroup times what one, two or more workgroups of a CU take for a stage together.
+// Least squares on the logarithm over 340 timed plans (24 matrices of 2048..28672 channels, K = 4096..28672, groups of
+// 64 and 128, 96..2048 rows): 6.6 % rms.
+float mx_predicted_time(int M, int N, int K, int group_size, int rb, int split) {
+    const int stages = mx_padded_steps(K) / 2, per = (stages + split - 1) / split;
+    const int tiles = ((N + 255) / 256) * ((M + rb * kFragRows - 1) / (rb * kFragRows));
+    const int n = (tiles * split + 255) / 256;
+    const float each = rb == 2 ? (n == 1 ? 0.774f : n == 2 ? 1.014f : 0.463f * (float)n)
+                               : (n == 1 ? 1.019f : n == 2 ? 1.563f : 0.787f * (float)n);
+    const float sums = split > 1 ? 0.0834e-6f * 8.0f * (float)split * (float)M * (float)N : 0.0f;
+    return 12.57f + 1.124e-6f * (float)M * (float)K + sums + ((float)per + 3.24f) * each * (group_size == 64 ? 1.325f : 1.0f);
+}
+
+// 128-row tiles where they fill the chip; otherwise the tile height and K split with the smallest predicted time
+// (1024 x 14336 x 4096: 448 128-row tiles unsplit 74 us, 64-row tiles 94; 512 x 8192 x 28672: 128-row tiles in four splits
+// 142 us, unsplit 243, 64-row tiles 150..233).
 MxPlan mx_plan(int M, int N, int K, int group_size) {
     const int tiles_n = ((N + kStripN - 1) / kStripN + kStripsPerWg - 1) / kStripsPerWg;
-    const int tiles128 = tiles_n * ((M + 127) / 128);
-    MxPlan plan;
-    plan.rb = tiles128 >= 2 * 256 ? 4 : 2;
-    plan.tiles = plan.rb == 4 ? tiles128 : tiles_n * ((M + 63) / 64);
     const int stages = mx_padded_steps(K) / 2;
-    // K splits of 64-row tiles: how evenly the workgroups fill the CUs, how well a CU runs with one, two or three of
-    // them, and the stages' worth a workgroup spends outside its stages
-    int best = 1;
-    if (plan.rb == 2 && plan.tiles <= 400) {
-        double best_score = -1.0;
+    MxPlan plan{4, tiles_n * ((M + 127) / 128), 1, stages};
+    if (plan.tiles >= 2 * 256) return plan;
+    int best_split = 1;
+    float best = 1e30f;
+    for (int rb = 2; rb <= 4; rb += 2) {
+        const int tiles = tiles_n * ((M + rb * kFragRows - 1) / (rb * kFragRows));
         for (int split : {1, 2, 3, 4, 6, 8}) {
-            const int per = (stages + split - 1) / split;
-            if (split > 1 && per < 8) break;
-            const long long wgs = (long long)plan.tiles * ((stages + per - 1) / per);
-            const long long n = (wgs + 255) / 256;
-            const double fill = (double)wgs / (256.0 * (double)n), together = n == 1 ? 0.7 : (n == 2 ? 0.9 : 1.0);
-            const double score = fill * together * (double)per / ((double)per + 10.0);
-            if (score > best_score * 1.0001) {
-                best_score = score;
-                best = split;
+            if (split > 1 && (stages / split < 6 || tiles * split > 1100)) break;
+            const float time = mx_predicted_time(M, N, K, group_size, rb, split);
+            if (time < best) {
+                best = time;
+                best_split = split;
+                plan.rb = rb;
+                plan.tiles = tiles;
             }
         }
     }
-    int per = (stages + best - 1) / best;
+    int per = (stages + best_split - 1) / best_split;
     if (group_size == 256) per = (per + 1) / 2 * 2;   // (a split owns whole groups)
     plan.stages_per_split = per;
     plan.split = (stages + per - 1) / per;

@@ -34,6 +34,7 @@ __host__ __device__ inline int mx_padded_steps(int K) { return (K / kStepK + 1) 
 // what a launch looks like: row blocks per workgroup tile (2 or 4), tiles, K splits and stages per split
 struct MxPlan { int rb, tiles, split, stages_per_split; };
 MxPlan mx_plan(int M, int N, int K, int group_size);
+float mx_predicted_time(int M, int N, int K, int group_size, int rb, int split);
 
 hipError_t launch_mx_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size, uint8_t* frag, uint32_t* rs,
                            float* s_a, hipStream_t stream);

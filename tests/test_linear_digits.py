@@ -47,6 +47,53 @@ def test_validation_and_sizes():
     assert L.slimk_w2a8_linear_route(1, 4096, 4096, 128, 0) == 0
 
 
+def test_routes_only_name_what_the_kernels_take():
+    import random
+    L = _lib.lib()
+    rng = random.Random(5)
+    routed = 0
+    for _ in range(3000):
+        g = rng.choice([64, 128, 256])
+        K = g * rng.randint(1, 40960 // g)
+        M, N = int(2 ** rng.uniform(0, 13)), int(2 ** rng.uniform(0, 15))
+        zp = rng.randint(0, 1)
+        if L.slimk_w2a8_linear_route(M, N, K, g, zp):
+            routed += 1
+            assert M >= 96 and g <= 128 and K <= 32512
+            assert L.slimk_w2a8_linear_activation_bytes(M, N, K, g) >= (M + 31) // 32 * ((K + 127) // 128) * 2 * 2560
+            assert L.slimk_w2a8_linear_workspace_bytes(M, N, K, g) < 1 << 28
+        if K % 128 == 0:      # the weight-only form's own choice of a split is one that a caller may ask for
+            split = L.slimk_w2a16_gemm_auto_split_k(M, N, K, g)
+            assert split == 1 or 1 < split <= 64 and split * 4 <= K // max(g, 128)
+    assert routed > 100
+
+
+@pytest.mark.gpu
+def test_recorded_into_a_graph(gpu_ops):
+    """Split calls of both tiled forms replay to the eager bits, with eager work between the replays."""
+    from slimkernels_amd.torch.ops import w2a8_linear_digits
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(9)
+    w = gpu_ops.W2A8Linear.from_float(torch.randn((320, 4096), generator=gen, device="cuda", dtype=torch.float16), 128, "asym").weight
+    x = torch.randn((200, 4096), generator=gen, device="cuda", dtype=torch.float16)
+    assert _lib.lib().slimk_w2a8_linear_workspace_bytes(200, 320, 4096, 128) > 0
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        want = [w2a8_linear_digits(x, w), gpu_ops.w2a16_gemm(x, w, split_k=4)]
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        got = [w2a8_linear_digits(x, w), gpu_ops.w2a16_gemm(x, w, split_k=4)]
+    for _ in range(3):
+        for y in got:
+            y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for y, e in zip(got, want):
+            assert torch.equal(y.view(torch.int16), e.view(torch.int16))
+        w2a8_linear_digits(x[:100], w)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,g,mode,out", [
     (1, 64, 64, 64, "sym", "float16"),             # one row, one step: half a stage
