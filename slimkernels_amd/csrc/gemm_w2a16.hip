@@ -405,8 +405,8 @@ hipError_t launch_w2a16_grouped(const W2A16Group& gp, int gs, bool zp, bool out_
 }
 
 hipError_t launch_w2a16(const W2A16Params& p, int gs, bool out_bf16, hipStream_t stream) {
-    if (const int rb = w2a16_plan(p.M, p.strips, p.steps, gs, p.split).rb) {
-        if (hipError_t e = launch_w2a16_tiled(p, rb, gs, out_bf16, stream); e != hipSuccess) return e;
+    if (const W2A16Plan plan = w2a16_plan(p.M, p.strips, p.steps, gs, p.split); plan.rb) {
+        if (hipError_t e = launch_w2a16_tiled(p, plan.rb, plan.halves, gs, out_bf16, stream); e != hipSuccess) return e;
     } else {
         const dim3 grid((unsigned)p.strips, (unsigned)p.split, (unsigned)((p.M + 15) / 16));
         const int waves = w2a16_waves(p.M, p.strips, p.steps, gs, p.split);

@@ -50,18 +50,22 @@ __device__ __forceinline__ CodeTable code_table(int z) {
     return {__builtin_amdgcn_perm(v23, v01, 0x07050301u), __builtin_amdgcn_perm(v23, v01, 0x06040200u)};
 }
 
-template <int RB, bool ZP, bool PARTIAL, typename OutT, bool XBF>
+// KP = 2: eight waves, the second four on the second half of the workgroup's steps in a ring of their own; the halves
+// meet in LDS (half the partial sums of a split launch with as many waves on a CU).
+template <int RB, int KP, bool ZP, bool PARTIAL, typename OutT, bool XBF>
 __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int steps_per_split, const int group_shift) {
     constexpr int kBM = RB * 32;
     constexpr int kASlot = RB * 4096, kWSlot = kStripsPerWg * kUnitBytes, kSSlot = kStripsPerWg * 256;
     constexpr int kSlot = kASlot + kWSlot + kSSlot * (ZP ? 2 : 1);
-    constexpr int kLds = 3 * kSlot;
+    constexpr int kLds = 3 * kSlot;   // a ring
     constexpr int kPitch = 72;   // floats of an output staging row
     static_assert(32 * kPitch * 4 * kStripsPerWg <= kLds, "output staging exceeds the stage buffers");
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
+    __shared__ __attribute__((aligned(16))) uint8_t lds_all[KP * kLds];
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kh = KP == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & (kStripsPerWg - 1);
+    uint8_t* const lds = lds_all + kh * kLds;
     const int col = lane & 31, half = lane >> 5, c16 = lane & 15, sub = (lane >> 4) & 1;
     // token tiles of a channel tile next to each other on one XCD: they read the same weights
     const int tiles_n = (p.strips + kStripsPerWg - 1) / kStripsPerWg, tiles_m = (p.M + kBM - 1) / kBM;
@@ -71,8 +75,10 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
     const int strip_raw = n_tile * kStripsPerWg + wave;
     const int strip = min(strip_raw, p.strips - 1);   // a surplus wave recomputes the last strip and stores nothing
     const bool strip_ok = strip_raw < p.strips;
-    const int step0 = PARTIAL ? (int)blockIdx.y * steps_per_split : 0;
-    const int n_steps = PARTIAL ? min(steps_per_split, p.steps - step0) : p.steps;
+    // (KP = 2: an even number of steps in every split, so that the halves meet at the same barriers)
+    const int wg_step0 = PARTIAL ? (int)blockIdx.y * steps_per_split : 0;
+    const int wg_steps = PARTIAL ? max(0, min(steps_per_split, p.steps - wg_step0)) : p.steps;
+    const int n_steps = wg_steps / KP, step0 = wg_step0 + kh * n_steps;
 
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(p.x), 0, (int)min(((size_t)(p.M - 1) * p.ldx + p.K) * 2, (size_t)0x7fffffff), 0x00020000);
@@ -225,6 +231,29 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
 #pragma unroll
     for (int j = 0; j < 16; ++j) t[RB - 1][1][j] = __builtin_fmaf(acc[1][j], sc_prev, t[RB - 1][1][j]);
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");   // the last (repeated) requests have landed: LDS is free
+    if constexpr (KP == 2) {   // the second half's running sums, lane-linear, into the first half's
+        constexpr int kSums = RB * 8 * 1024;   // bytes of a wave
+        static_assert(kStripsPerWg * kSums <= KP * kLds, "the halves' exchange exceeds the rings");
+        v4f* const meet = reinterpret_cast<v4f*>(lds_all + wave * kSums) + lane;
+        if (kh == 1) {
+#pragma unroll
+            for (int i = 0; i < RB * 8; ++i) {
+                const float* tv = &t[i / 8][(i / 4) % 2][(i % 4) * 4];
+                meet[i * 64] = v4f{tv[0], tv[1], tv[2], tv[3]};
+            }
+        }
+        __syncthreads();
+        if (kh == 0) {
+#pragma unroll
+            for (int i = 0; i < RB * 8; ++i) {
+                const v4f v = meet[i * 64];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) t[i / 8][(i / 4) % 2][(i % 4) * 4 + j] += v[j];
+            }
+        }
+        __syncthreads();       // (the output staging goes over the same memory)
+        if (kh == 1) return;
+    }
     if (!strip_ok) return;
 
     if constexpr (PARTIAL) {   // fp32 partial sums [split][M][N]: 128 bytes of a row per half-wave and store
@@ -276,58 +305,64 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
     }
 }
 
-template <int RB, bool ZP, bool PARTIAL, typename OutT, bool XBF>
-__global__ __launch_bounds__(256, RB == 4 ? 2 : 3) void w2a16_tiled_kernel(const W2A16Params p, const int steps_per_split, const int group_shift) {
-    w2a16_tiled_body<RB, ZP, PARTIAL, OutT, XBF>(p, steps_per_split, group_shift);
+// (four-wave workgroups: two of 128 or three of 64 rows per CU; eight-wave ones, 64 rows only: one)
+template <int RB, int KP, bool ZP, bool PARTIAL, typename OutT, bool XBF>
+__global__ __launch_bounds__(KP * 256, RB == 4 || KP == 2 ? 2 : 3) void w2a16_tiled_kernel(const W2A16Params p, const int steps_per_split, const int group_shift) {
+    w2a16_tiled_body<RB, KP, ZP, PARTIAL, OutT, XBF>(p, steps_per_split, group_shift);
 }
 
-template <int RB, bool ZP, bool XBF>
+template <int RB, int KP, bool ZP, bool XBF>
 void launch_rb(const W2A16Params& p, bool out_bf16, dim3 grid, int sps, int shift, hipStream_t stream) {
-    const dim3 block(256);
-    if (p.split > 1) w2a16_tiled_kernel<RB, ZP, true, OutF16, XBF><<<grid, block, 0, stream>>>(p, sps, shift);
-    else if (out_bf16) w2a16_tiled_kernel<RB, ZP, false, OutBF16, XBF><<<grid, block, 0, stream>>>(p, sps, shift);
-    else w2a16_tiled_kernel<RB, ZP, false, OutF16, XBF><<<grid, block, 0, stream>>>(p, sps, shift);
+    const dim3 block(KP * 256);
+    if (p.split > 1) w2a16_tiled_kernel<RB, KP, ZP, true, OutF16, XBF><<<grid, block, 0, stream>>>(p, sps, shift);
+    else if (out_bf16) w2a16_tiled_kernel<RB, KP, ZP, false, OutBF16, XBF><<<grid, block, 0, stream>>>(p, sps, shift);
+    else w2a16_tiled_kernel<RB, KP, ZP, false, OutF16, XBF><<<grid, block, 0, stream>>>(p, sps, shift);
 }
 
 }  // namespace
 
-// rb: row blocks of 32 per workgroup tile (2 or 4).  With p.split > 1 the partial sums go to p.ws (a split may turn out
-// empty: its workgroups then write zeros).
-hipError_t launch_w2a16_tiled(const W2A16Params& p, int rb, int gs, bool out_bf16, hipStream_t stream) {
+// rb: row blocks of 32 per workgroup tile (2 or 4); halves: K parts inside a workgroup (1, or 2 with rb = 2).  With
+// p.split > 1 the partial sums go to p.ws (a split may turn out empty: its workgroups then write zeros).
+hipError_t launch_w2a16_tiled(const W2A16Params& p, int rb, int halves, int gs, bool out_bf16, hipStream_t stream) {
     const int tiles_n = (p.strips + kStripsPerWg - 1) / kStripsPerWg, tiles_m = (p.M + rb * 32 - 1) / (rb * 32);
     const dim3 grid((unsigned)xcd_grid(tiles_n, tiles_m), (unsigned)p.split);
-    const int sps = (p.steps + p.split - 1) / p.split, shift = gs == 1 ? 0 : (gs == 2 ? 1 : 2);
+    // (K is a multiple of 128: an even number of steps, dealt out in pairs)
+    const int sps = (p.steps / 2 + p.split - 1) / p.split * 2, shift = gs == 1 ? 0 : (gs == 2 ? 1 : 2);
     const bool zp = p.zp_r != nullptr;
-#define SLIMK_W2A16_TILED(RBV)                                                          \
-    do {                                                                                \
-        if (zp) {                                                                       \
-            if (p.x_bf16) launch_rb<RBV, true, true>(p, out_bf16, grid, sps, shift, stream);   \
-            else launch_rb<RBV, true, false>(p, out_bf16, grid, sps, shift, stream);    \
-        } else {                                                                        \
-            if (p.x_bf16) launch_rb<RBV, false, true>(p, out_bf16, grid, sps, shift, stream);  \
-            else launch_rb<RBV, false, false>(p, out_bf16, grid, sps, shift, stream);   \
-        }                                                                               \
+#define SLIMK_W2A16_TILED(RBV, KPV)                                                              \
+    do {                                                                                         \
+        if (zp) {                                                                                \
+            if (p.x_bf16) launch_rb<RBV, KPV, true, true>(p, out_bf16, grid, sps, shift, stream);   \
+            else launch_rb<RBV, KPV, true, false>(p, out_bf16, grid, sps, shift, stream);        \
+        } else {                                                                                 \
+            if (p.x_bf16) launch_rb<RBV, KPV, false, true>(p, out_bf16, grid, sps, shift, stream);  \
+            else launch_rb<RBV, KPV, false, false>(p, out_bf16, grid, sps, shift, stream);       \
+        }                                                                                        \
     } while (0)
-    if (rb == 4) SLIMK_W2A16_TILED(4);
-    else SLIMK_W2A16_TILED(2);
+    if (rb == 4) SLIMK_W2A16_TILED(4, 1);
+    else if (halves == 2) SLIMK_W2A16_TILED(2, 2);
+    else SLIMK_W2A16_TILED(2, 1);
 #undef SLIMK_W2A16_TILED
     return hipGetLastError();
 }
 
 // Which kernel, which tile height and how many K splits: the smallest predicted time.  The few-rows kernel runs 16 rows
 // x one strip per workgroup, 0.02 us for each and 4096 reduction elements.  A 64-row workgroup of this kernel takes
-// 0.65 us a step alone on a CU, two side by side 1.0, three and more 0.47 each (128-row ones 0.97, 1.7 and 0.85 each); a
-// split writes and reads its partial sums at about 5 TB/s, plus the second launch.  Within 6 % of the measured times
+// 0.65 us a step alone on a CU, two side by side 1.0, three and more 0.47 each (128-row ones 0.97, 1.7 and 0.85 each),
+// an eight-wave one with two K halves 1.03 for a step of both and 2 us for their meeting: ahead while one round of them
+// covers the problem, as it needs half the splits (300 x 4096 x 14336: three splits of two halves 51.6 us, six splits
+// 55.0 on the same card; 768 x 5120 x 5120 unsplit 47.9, in two splits 56.2; in two rounds it loses, 400 x 2048 x 20480 in six
+// 67.5 against 64.9).  A split writes and reads its partial sums at about 5 TB/s, plus the second launch.  Within 6 % of the measured times
 // of fourteen shapes (64..1024 rows, 1024..28672 channels, K = 4096..14336) at one to eight splits: 300 x 4096 x 14336 89 -> 53 us,
 // 128 x 14336 x 4096 39 -> 31, 1024 x 14336 x 4096 275 -> 115, 100 x 28672 x 8192 132 -> 74; 64 x 4096 x 4096 stays with
 // the few-rows kernel (8.4 against 13 us).
 W2A16Plan w2a16_plan(int M, int strips, int steps, int gs, int split) {
-    W2A16Plan plan{0, split > 0 ? split : w2a16_few_rows_split(M, strips, steps, gs)};
+    W2A16Plan plan{0, split > 0 ? split : w2a16_few_rows_split(M, strips, steps, gs), 1};
     if (M <= 32) return plan;
     const float few_rows = 3.5f + 0.02f * (float)strips * (float)((M + 15) / 16) * (float)steps / 64.0f;
     const int tiles_n = (strips + kStripsPerWg - 1) / kStripsPerWg;
     const int cap = std::max(1, steps / (gs > 2 ? gs : 2) / 4);   // (what an explicit request is held to)
-    float best = few_rows, best_tiled = 1e30f;
+    float best = few_rows;
     for (int rb = 2; rb <= 4; rb += 2) {
         const int tiles = tiles_n * ((M + rb * 32 - 1) / (rb * 32));
         for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
@@ -338,9 +373,10 @@ W2A16Plan w2a16_plan(int M, int strips, int steps, int gs, int split) {
                                        : (wgs == 1 ? 0.97f : wgs == 2 ? 1.7f : 0.85f * (float)wgs);
             const float sums = s > 1 ? 3.0f + (float)s * (float)M * (float)strips * (64.0f * 8.0f / 5e6f) : 0.0f;
             const float time = 2.5f + (float)((steps + s - 1) / s) * each + sums;
-            if (time < best_tiled) {
-                best_tiled = time;
-                if (time < best || plan.rb) { best = time; plan.rb = rb; plan.split = s; }
+            const float halves = rb == 2 && tiles * s <= 256 ? 4.5f + (float)((steps / 2 + s - 1) / s) * 1.03f + sums : 1e30f;
+            if (std::min(time, halves) < best) {
+                best = std::min(time, halves);
+                plan = {rb, s, halves < time ? 2 : 1};
             }
             if (split > 0) break;
         }

@@ -114,11 +114,11 @@ struct W2A16Params {
 };
 hipError_t launch_w2a16(const W2A16Params& p, int gs, bool out_bf16, hipStream_t stream);
 // Many token rows (gemm_w2a16_tiled.hip): row blocks of 32 per workgroup tile (2 or 4; 0: the few-rows kernel is the
-// faster one) and K splits (split > 0: as requested); the launch (with p.split > 1 the partial sums only).
-struct W2A16Plan { int rb, split; };
+// faster one), K splits (split > 0: as requested) and K parts inside a workgroup (1 or 2); the launch (with p.split > 1 the partial sums only).
+struct W2A16Plan { int rb, split, halves; };
 W2A16Plan w2a16_plan(int M, int strips, int steps, int gs, int split);
 int w2a16_few_rows_split(int M, int strips, int steps, int gs);
-hipError_t launch_w2a16_tiled(const W2A16Params& p, int rb, int gs, bool out_bf16, hipStream_t stream);
+hipError_t launch_w2a16_tiled(const W2A16Params& p, int rb, int halves, int gs, bool out_bf16, hipStream_t stream);
 // Several weight-only problems in one launch (each unsplit; the activation type, zero-point mode and output type are
 // the launch's): problem i owns workgroups wg_begin[i] .. wg_begin[i+1]-1, sets of strips x blocks of 16 token rows;
 // a workgroup of `waves` wavefronts holds waves >> log_parts[i] strips of problem i, each in 1 << log_parts[i] K-parts.
