@@ -639,8 +639,10 @@ static float int8_layer_time(int M, int N, int K, int group_size) {
 //  * 512 and more 128-row tiles (two per CU): the GEMM saves in proportion to M * N * K, the quantisation costs a little
 //    more in proportion to M * K, so N decides: 2048 x 28672 x 8192 in groups of 64 578 -> 509 us, 4096 x 14336 x 4096
 //    257 -> 242, 4096 x 5120 x 5120 139 -> 132, but 4096 x 4096 x 14336 255 -> 258 (per-group zero-points: 304 -> 296).
-//  * fewer tiles, more than 256 rows: the smaller predicted time, with 3 % in hand (45 timed calls: 6.7 % faster than
-//    the int8 path on average where always picking the faster one would give 7.2 %, worst 1 % slower;
+//  * fewer tiles, more than 256 rows: the smaller predicted time, with 3 % in hand, inside the range the predictions were
+//    fitted on, 4096 channels and elements and more (45 timed calls: 6.7 % faster than the int8 path on average where
+//    always picking the faster one would give 7.2 %, worst 1 % slower; narrower matrices are mostly quantisation:
+//    2622 x 1922 x 8960 94 -> 104 us;
 //    1024 x 14336 x 4096 g 64 101 -> 87 us, 512 x 28672 x 8192 g 64 186 -> 153, 512 x 8192 x 28672 162 -> 142, 1900 x 7168 x 8192 152 -> 134).
 //  * 96..256 rows: long reductions only, in groups of 128 (128 x 8192 x 28672 63.5 -> 56 us, 256 x 8192 x 20480 74.5 -> 66,
 //    96 x 4096 x 28672 51 -> 44; in groups of 64 128 x 4096 x 28672 57 / 58 and with K = 14336 256 x 4096 37.5 / 38.5).
@@ -650,6 +652,7 @@ int slimk_w2a8_linear_route(int M, int N, int K, int group_size, int per_group_z
     if (M <= 256) return group_size == 128 && K >= 20480 && N >= 4096 ? 1 : 0;
     const w2a8::MxPlan plan = w2a8::mx_plan(M, N, K, group_size);
     if (plan.rb == 4 && plan.tiles >= 2 * 256) return N >= (group_size == 128 && !per_group_zp ? 5120 : 4096) ? 1 : 0;
+    if (N < 4096 || K < 4096) return 0;
     return w2a8::mx_predicted_time(M, N, K, group_size, plan.rb, plan.split) < 0.97f * int8_layer_time(M, N, K, group_size) ? 1 : 0;
 }
 
