@@ -294,23 +294,24 @@ __global__ __launch_bounds__(kWaves * 64, XBF && GS < 4 ? 4 : 1) void w2a16_grou
 template <typename OutT>
 __global__ __launch_bounds__(128) void w2a16_reduce_kernel(const float* __restrict__ ws, int split, int M, int N,
                                                            uint16_t* __restrict__ out, int ldo) {
-    const int n = (int)(blockIdx.x * 128 + threadIdx.x) * 4;
-    if (n >= N) return;
     const size_t total = (size_t)M * N;
+    const int t = (int)(blockIdx.x * 128 + threadIdx.x);
     for (int m = (int)blockIdx.y; m < M; m += (int)gridDim.y) {
-        const float* src = ws + (size_t)m * N + n;
-        uint16_t* dst = out + (size_t)m * ldo + n;
+        const float* src = ws + (size_t)m * N;
+        uint16_t* dst = out + (size_t)m * ldo;
         if ((N & 3) == 0) {
-            v4f v = *reinterpret_cast<const v4f*>(src);
+            if (t * 4 >= N) return;
+            v4f v = *reinterpret_cast<const v4f*>(src + t * 4);
 #pragma unroll 4
-            for (int s = 1; s < split; ++s) v += *reinterpret_cast<const v4f*>(src + (size_t)s * total);
+            for (int s = 1; s < split; ++s) v += *reinterpret_cast<const v4f*>(src + (size_t)s * total + t * 4);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) dst[i] = OutT::cast(v[i]);
+            for (int i = 0; i < 4; ++i) dst[t * 4 + i] = OutT::cast(v[i]);
         } else {
-            for (int i = 0; i < 4 && n + i < N; ++i) {
-                float v = src[i];
-                for (int s = 1; s < split; ++s) v += src[(size_t)s * total + i];
-                dst[i] = OutT::cast(v);
+            for (int n = t; n < N; n += (int)gridDim.x * 128) {
+                float v = src[n];
+#pragma unroll 4
+                for (int s = 1; s < split; ++s) v += src[(size_t)s * total + n];
+                dst[n] = OutT::cast(v);
             }
         }
     }
@@ -416,7 +417,8 @@ hipError_t launch_w2a16(const W2A16Params& p, int gs, bool out_bf16, hipStream_t
     }
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     if (p.split > 1) {
-        const dim3 blocks((unsigned)((p.N + 511) / 512), (unsigned)std::min(p.M, 32768));
+        const int per_thread = p.N % 4 == 0 ? 4 : 1;
+        const dim3 blocks((unsigned)((p.N + 128 * per_thread - 1) / (128 * per_thread)), (unsigned)std::min(p.M, 32768));
         if (out_bf16)
             w2a16_reduce_kernel<OutBF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo);
         else
