@@ -394,6 +394,10 @@ int slimk_w4a8_gemm(const int8_t* q, int ldq, const float* s_a, const int32_t* r
  * `b = ((b >> 4) & 0b11).to(tl.float16); accumulator = tl.dot(a, b, accumulator)`), which has no scales,
  * no zero-point and reads one field per word. */
 int slimk_w2a16_gemm_auto_split_k(int M, int N, int K, int group_size);
+/* What a call with this split_k runs: the token rows of a workgroup tile of the many-rows kernel (64 or 128; 0: the
+ * few-rows kernel), the K splits across workgroups (fewer than asked for where some would have no work) and the parts of
+ * K inside a workgroup of the many-rows kernel (1 or 2).  Launches nothing. */
+int slimk_w2a16_gemm_plan(int M, int N, int K, int group_size, int split_k, int* tile_rows, int* splits, int* halves);
 size_t slimk_w2a16_gemm_workspace_bytes(int M, int N, int K, int group_size, int split_k);
 int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
                      const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,

@@ -1005,6 +1005,18 @@ int slimk_w2a16_gemm_auto_split_k(int M, int N, int K, int group_size) {
     return w2a8::w2a16_plan(M, strips_of(N), K / w2a8::kStepK, group_size / w2a8::kStepK, 0).split;
 }
 
+int slimk_w2a16_gemm_plan(int M, int N, int K, int group_size, int split_k, int* tile_rows, int* splits, int* halves) {
+    if (!tile_rows || !splits || !halves) return fail(SLIMK_ERR_NULL_POINTER, "w2a16_gemm_plan: NULL result");
+    if (M <= 0 || N <= 0) return fail(SLIMK_ERR_BAD_SHAPE, "M=%d, N=%d must be positive", M, N);
+    if (int rc = check_kg(K, group_size)) return rc;
+    if (K % 128 != 0) return fail(SLIMK_ERR_UNSUPPORTED, "w2a16_gemm: K=%d must be a multiple of 128", K);
+    const w2a8::W2A16Plan plan = w2a8::w2a16_plan(M, strips_of(N), K / w2a8::kStepK, group_size / w2a8::kStepK, split_k);
+    *tile_rows = plan.rb * 32;
+    *splits = plan.split;
+    *halves = plan.halves;
+    return SLIMK_OK;
+}
+
 size_t slimk_w2a16_gemm_workspace_bytes(int M, int N, int K, int group_size, int split_k) {
     if (split_k <= 0) split_k = slimk_w2a16_gemm_auto_split_k(M, N, K, group_size);
     if (split_k <= 1 || M <= 0 || N <= 0) return 0;

@@ -405,8 +405,11 @@ hipError_t launch_w2a16_grouped(const W2A16Group& gp, int gs, bool zp, bool out_
     return hipGetLastError();
 }
 
-hipError_t launch_w2a16(const W2A16Params& p, int gs, bool out_bf16, hipStream_t stream) {
-    if (const W2A16Plan plan = w2a16_plan(p.M, p.strips, p.steps, gs, p.split); plan.rb) {
+hipError_t launch_w2a16(const W2A16Params& asked, int gs, bool out_bf16, hipStream_t stream) {
+    const W2A16Plan plan = w2a16_plan(asked.M, asked.strips, asked.steps, gs, asked.split);
+    W2A16Params p = asked;
+    p.split = plan.split;   // (at most what was asked for, which the workspace was sized by)
+    if (plan.rb) {
         if (hipError_t e = launch_w2a16_tiled(p, plan.rb, plan.halves, gs, out_bf16, stream); e != hipSuccess) return e;
     } else {
         const dim3 grid((unsigned)p.strips, (unsigned)p.split, (unsigned)((p.M + 15) / 16));

@@ -75,9 +75,9 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
     const int strip_raw = n_tile * kStripsPerWg + wave;
     const int strip = min(strip_raw, p.strips - 1);   // a surplus wave recomputes the last strip and stores nothing
     const bool strip_ok = strip_raw < p.strips;
-    // (KP = 2: an even number of steps in every split, so that the halves meet at the same barriers)
+    // (KP = 2: an even number of steps in every split, so that the halves meet at the same barriers; no split is empty)
     const int wg_step0 = PARTIAL ? (int)blockIdx.y * steps_per_split : 0;
-    const int wg_steps = PARTIAL ? max(0, min(steps_per_split, p.steps - wg_step0)) : p.steps;
+    const int wg_steps = PARTIAL ? min(steps_per_split, p.steps - wg_step0) : p.steps;
     const int n_steps = wg_steps / KP, step0 = wg_step0 + kh * n_steps;
 
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -321,13 +321,21 @@ void launch_rb(const W2A16Params& p, bool out_bf16, dim3 grid, int sps, int shif
 
 }  // namespace
 
+// K is a multiple of 128, an even number of steps, dealt out to the splits in pairs.  Where rounding up to whole pairs
+// would leave the last splits empty (146 pairs in 16 splits: ten each, the sixteenth would start past the end) there are
+// only as many as have work.
+static int pairs_per_split(int steps, int split) { return (steps / 2 + split - 1) / split; }
+static int splits_with_work(int steps, int split) {
+    const int per = pairs_per_split(steps, split);
+    return (steps / 2 + per - 1) / per;
+}
+
 // rb: row blocks of 32 per workgroup tile (2 or 4); halves: K parts inside a workgroup (1, or 2 with rb = 2).  With
-// p.split > 1 the partial sums go to p.ws (a split may turn out empty: its workgroups then write zeros).
+// p.split > 1, one of splits_with_work, the partial sums go to p.ws.
 hipError_t launch_w2a16_tiled(const W2A16Params& p, int rb, int halves, int gs, bool out_bf16, hipStream_t stream) {
     const int tiles_n = (p.strips + kStripsPerWg - 1) / kStripsPerWg, tiles_m = (p.M + rb * 32 - 1) / (rb * 32);
     const dim3 grid((unsigned)xcd_grid(tiles_n, tiles_m), (unsigned)p.split);
-    // (K is a multiple of 128: an even number of steps, dealt out in pairs)
-    const int sps = (p.steps / 2 + p.split - 1) / p.split * 2, shift = gs == 1 ? 0 : (gs == 2 ? 1 : 2);
+    const int sps = pairs_per_split(p.steps, p.split) * 2, shift = gs == 1 ? 0 : (gs == 2 ? 1 : 2);
     const bool zp = p.zp_r != nullptr;
 #define SLIMK_W2A16_TILED(RBV, KPV)                                                              \
     do {                                                                                         \
@@ -368,6 +376,7 @@ W2A16Plan w2a16_plan(int M, int strips, int steps, int gs, int split) {
         for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
             if (split > 0) s = split;
             if (s > cap && split <= 0) break;
+            s = splits_with_work(steps, s);
             const int wgs = (tiles * s + 255) / 256;
             const float each = rb == 2 ? (wgs == 1 ? 0.65f : wgs == 2 ? 1.0f : 0.47f * (float)wgs)
                                        : (wgs == 1 ? 0.97f : wgs == 2 ? 1.7f : 0.85f * (float)wgs);

@@ -114,7 +114,8 @@ struct W2A16Params {
 };
 hipError_t launch_w2a16(const W2A16Params& p, int gs, bool out_bf16, hipStream_t stream);
 // Many token rows (gemm_w2a16_tiled.hip): row blocks of 32 per workgroup tile (2 or 4; 0: the few-rows kernel is the
-// faster one), K splits (split > 0: as requested) and K parts inside a workgroup (1 or 2); the launch (with p.split > 1 the partial sums only).
+// faster one), K splits (split > 0: as requested, fewer where some would have no work) and K parts inside a workgroup (1 or
+// 2); the launch (with p.split > 1 the partial sums only).
 struct W2A16Plan { int rb, split, halves; };
 W2A16Plan w2a16_plan(int M, int strips, int steps, int gs, int split);
 int w2a16_few_rows_split(int M, int strips, int steps, int gs);

@@ -10,6 +10,7 @@ import torch
 from slimkernels_amd import workloads
 import parity_utils as pu
 from test_w2a16 import _check
+from test_w2a16_plan import plan
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +65,9 @@ def test_w2a16_many_rows_against_the_oracle(gpu_ops, oracle, M, N, K, g, mode, x
 def test_w2a16_many_rows_with_zero_points_beyond_the_codes(gpu_ops, oracle, xdt):
     _run(gpu_ops, oracle, 300, 16448, 256, 64, "asym", xdt, "bfloat16", 1,
          zero=lambda shape: np.random.default_rng(3).integers(0, 256, shape).astype(np.uint8))
+
+
+def test_w2a16_many_rows_with_a_split_count_that_does_not_divide(gpu_ops, oracle):
+    """48 pairs of steps in nine splits: six each, so the ninth has no work and is not launched."""
+    assert plan(33, 16384, 6144, 128, 9) == (64, 8, 1)
+    _run(gpu_ops, oracle, 33, 16384, 6144, 128, "asym", "float16", "float16", 9)
