@@ -600,11 +600,13 @@ int slimk_w2a8_gemm_static(const int8_t* q, int ldq, const float* s_a, const int
                      nullptr, SLIMK_DUMP_NONE, nullptr, kStaticWorkspaceBytes, kernel, split_k, stream, true);
 }
 
-// ---- the digit form (gemm_mx.hip).  The activation scratch: digit fragments, group sums, token scales.
+// ---- the digit form (gemm_mx.hip).  The activation scratch: digit fragments, centring sums, token scales.
 static size_t mx_frag_bytes(int M, int K) {
     return (size_t)w2a8::mx_row_blocks(M) * (size_t)w2a8::mx_padded_steps(K) * w2a8::mx::kFragBytes;
 }
-static size_t mx_sums_bytes(int M, int K, int group_size) { return ((size_t)M * (K / group_size) * 4 + 16 + 255) / 256 * 256; }
+static size_t mx_sums_bytes(int M, int K, int group_size) {
+    return ((size_t)M * (K / (group_size == 64 ? 64 : 128)) * 4 + 255) / 256 * 256;
+}
 
 size_t slimk_w2a8_linear_activation_bytes(int M, int N, int K, int group_size) {
     if (M <= 0 || N <= 0 || !shape_ok(K, group_size) || K > w2a8::mx::kMaxK) return 0;
@@ -680,9 +682,9 @@ int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
     char* const act = reinterpret_cast<char*>(activations);
     w2a8::MxParams p{};
     uint8_t* frag = reinterpret_cast<uint8_t*>(act);
-    uint32_t* rs = reinterpret_cast<uint32_t*>(act + mx_frag_bytes(M, K));
+    float* cs = reinterpret_cast<float*>(act + mx_frag_bytes(M, K));
     float* s_a = reinterpret_cast<float*>(act + mx_frag_bytes(M, K) + mx_sums_bytes(M, K, group_size));
-    p.frag = frag; p.rs = rs; p.s_a = s_a;
+    p.frag = frag; p.cs = cs; p.s_a = s_a;
     p.w_r = w_r; p.s_r = s_r; p.zp_r = zp_r; p.out = out; p.ldo = ldo;
     p.M = M; p.N = N; p.K = K; p.G = K / group_size; p.steps = K / w2a8::kStepK; p.strips = strips_of(N);
     p.zp_const = zp_const; p.group_shift = group_size == 256 ? 1 : 0;
@@ -696,7 +698,7 @@ int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
         p.ws_partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + kCounterBlockBytes);
     }
     hipStream_t st = (hipStream_t)stream;
-    if (int rc = hip_result(w2a8::launch_mx_quant(x, ldx, x_dtype == SLIMK_BF16, M, K, group_size, frag, rs, s_a, st), "linear quantisation"))
+    if (int rc = hip_result(w2a8::launch_mx_quant(x, ldx, x_dtype == SLIMK_BF16, M, K, group_size, zp_r ? 2 : zp_const, frag, cs, s_a, st), "linear quantisation"))
         return rc;
     return hip_result(w2a8::launch_mx_gemm(p, plan.rb, group_size == 64 ? 1 : 2, out_dtype == SLIMK_BF16, st), "linear gemm");
 }

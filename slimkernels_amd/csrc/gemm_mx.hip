@@ -11,16 +11,22 @@
 // one fma per element and group instead of two instructions, and a packed weight dword becomes operands in 6
 // instructions per 16 codes.
 //
-// Measured: 38 cycles per 32x32x64 instruction with the 4 drain fmas of groups of 128 beside it, 49 with the 8 of
-// groups of 64 (32 alone) in a probe; in the kernel 469 against the int8 kernel's 551 thousand cycles at
-// 4096 x 14336 x 4096, at 2.16 against 2.42 GHz (the faster matrix instructions run into the power limit): 217
-// against 228 us; with the quantisation 257 -> 242 us, 2048 x 28672 x 8192 in groups of 64 578 -> 509 us.  What is left over the
-// matrix cores' own 235 thousand cycles is the vector instructions beside them (185 per 32 of them), prologue and
-// epilogue of a tile, and the half-empty last round of tiles.
+// The zero-point is in the accumulators from the start: the first matrix instruction of a group takes -zp * sum q / 16 of
+// its rows as the addend (the quantising kernel writes it, one fp32 per row and group), a multiple of 1/16 like the
+// products, so what is folded is the exact sum of q * (code - zp) and the running sums go through the oracle's values, bit
+// for bit where K is not split.  (Taken off the running sums in one piece in front of the loop instead, the offset
+// is about a hundred times the result on activations whose mean is not zero, and up to 2.3 % of the fp16 outputs rounded
+// the other way.)  Per-group zero-points: centred on 2 in that way, what is missing of two groups at a time goes onto the
+// running sums as a matrix product (groups of 128: two stages' at a time).  The addends cost LDS reads (16 or 32 of 16
+// bytes a wave and stage of 128 rows) and no vector instruction, and the pass over the groups in front of the loop is gone.
 //
-// The zero-point leaves through the group sums of q: -zp * scale * rowsum goes into the running sums first, as a
-// matrix product over the groups (uniform zero-points: rowsum in two exact fp16 digits times the fp16 scales,
-// eight groups per instruction; per-group ones: fp32 products, two groups per instruction).
+// Measured: 38 cycles per 32x32x64 instruction with the 4 drain fmas of groups of 128 beside it, 49 with the 8 of
+// groups of 64 (32 alone) in a probe; on random operands the faster matrix instructions run into the power limit
+// (2.16 against the int8 kernel's 2.42 GHz).  Layer calls with their quantisation on one card, us: the int8 path / this
+// kernel with the offset in front of the loop / this kernel: 4096 x 14336 x 4096 246 / 245 / 241, with per-group zero-points
+// 277 / 267 / 263; 2048 x 28672 x 8192 in groups of 64 577 / 525 / 523, with per-group zero-points 724 / 640 / 595;
+// 1024 x 14336 x 4096 81 / 75 / 73.  What is left over the matrix cores' own time is the vector instructions beside them
+// (185 per 32 of them), prologue and epilogue of a tile, and the half-empty last round of tiles.
 //
 // Activation fragments (written by mx_quant_kernel): one of 2560 bytes per 32 rows x 64 elements, in operand order.
 // Lane l holds row l & 31, elements 32 * (l >> 5) .. + 31: 16 bytes of fp4 digits at 16 * l, the first 16 bytes of its
@@ -43,7 +49,7 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 
 constexpr int kFp6 = 2, kFp4 = 4;          // operand formats of the f8f6f4 instructions
 constexpr int kScaleOne = 127, kScale4 = 129;   // 2^(x - 127)
@@ -56,7 +62,7 @@ constexpr int kScaleOne = 127, kScale4 = 129;   // 2^(x - 127)
 // in one L2.
 template <bool BF16>
 __global__ __launch_bounds__(1024) void mx_quant_kernel(const uint16_t* __restrict__ x, int ldx, int M, int K, int group_size,
-                                                        uint8_t* __restrict__ frag, uint32_t* __restrict__ rs,
+                                                        uint8_t* __restrict__ frag, float* __restrict__ cs, float centre,
                                                         float* __restrict__ s_a) {
     __shared__ float red[16];
     const int xcd = blockIdx.x & 7, kth = blockIdx.x >> 3;
@@ -141,14 +147,9 @@ __global__ __launch_bounds__(1024) void mx_quant_kernel(const uint16_t* __restri
         *reinterpret_cast<v4i*>(dst + 1024 + fl * 16) = v4i{lo[0], lo[1], lo[2], lo[3]};
         *reinterpret_cast<v2i*>(dst + 2048 + fl * 8) = v2i{lo[4], lo[5]};
     }
-    const int tpg = group_size / 32;   // threads per scale group: 2, 4 or 8 (all of a group's threads are on or off)
-    for (int off = 1; off < tpg; off <<= 1) sumf += __shfl_xor(sumf, off, 64);
-    if (on && tid % tpg == 0) {
-        const float h = rintf(sumf * 0.0078125f) * 128.0f;   // |sum| <= 256 * 127: both digits are exact in fp16
-        const _Float16 dh = (_Float16)h, dl = (_Float16)(sumf - h);
-        rs[(size_t)m * (K / group_size) + tid / tpg] =
-            (uint32_t)__builtin_bit_cast(uint16_t, dh) | ((uint32_t)__builtin_bit_cast(uint16_t, dl) << 16);
-    }
+    const int tpd = group_size == 64 ? 2 : 4;   // threads per drain of the GEMM (all of a drain's threads are on or off)
+    for (int off = 1; off < tpd; off <<= 1) sumf += __shfl_xor(sumf, off, 64);
+    if (on && tid % tpd == 0) cs[(size_t)(tid / tpd) * M + m] = sumf * centre;
 }
 
 __device__ __forceinline__ v16f mfma_hi(v4i a, v4i b, v16f c) {   // 4 * a4 * c/2
@@ -186,7 +187,7 @@ __device__ __forceinline__ void unpack_unit(const v4i& raw, v4i (&b)[2]) {
 // waves), the wave's own weight units and scales into two wave-private slots (a wave moves a stage's units to registers
 // before it asks for the units two stages on).
 // GS = 64-element steps per drain: 1 (groups of 64) or 2 (128; groups of 256 drain twice with the same scale).
-template <int RB, int GS, bool SPLIT, bool ZP, typename OutT>
+template <int RB, int GS, bool SPLIT, bool ZP, int WGS, typename OutT>
 __device__ __forceinline__ void mx_body(const MxParams& p) {
     constexpr int kABytes = RB * kStageSteps * kFragBytes;       // 20 or 10 KiB
     constexpr int kALoads = (kABytes / 1024 + 3) / 4;            // LDS-direct loads of 1 KiB per wave and stage: 5 or 3
@@ -194,7 +195,10 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
     constexpr int kSpare = kALoads * 4 * 1024 > kABytes ? 1024 : 0;   // RB = 2: where the two surplus loads land
     constexpr int kWBytes = kStripsPerWg * kStageSteps * kUnitBytes;
     constexpr int kSBytes = kStripsPerWg * 256;
-    constexpr int kLds = 3 * kASlot + 2 * (kWBytes + kSBytes) + kSpare;
+    constexpr int kGroups = kStageSteps / GS;                    // drains of a block per stage
+    constexpr int kCBytes = RB * kGroups * kFragRows * 4;
+    constexpr int kCSlots = ZP && GS == 2 ? 3 : 2;              // (3: the zero-point correction takes two stages' sums)
+    constexpr int kLds = 3 * kASlot + 2 * (kWBytes + kSBytes) + kCSlots * kCBytes + kSpare;
     __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
     constexpr int kBM = RB * kFragRows;
 
@@ -234,13 +238,17 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
         const_cast<uint32_t*>(p.w_r), 0, (int)min(weight_bytes(p.strips, p.steps), (size_t)0x7fffffff), 0x00020000);
     const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(p.s_r), 0, (int)min((size_t)p.strips * p.G * 128, (size_t)0x7fffffff), 0x00020000);
+    const int drains = p.steps / GS;                       // of the whole reduction
+    const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(p.cs), 0, (int)((size_t)p.M * drains * 4), 0x00020000);
 
     // activations: chunk c = wave + 4 i of 1 KiB; a row block's two fragments of a stage are 5 chunks in one piece
+    // (all of it the wave's: in scalar registers beside the lane's 16 bytes; a row block past the last repeats it)
     uint32_t a_off[kALoads];
 #pragma unroll
     for (int i = 0; i < kALoads; ++i) {
         const int c = min(wave + 4 * i, kABytes / 1024 - 1), rb = c / 5;
-        a_off[i] = (uint32_t)(m_tile / kFragRows + rb) * (uint32_t)(steps2 * kFragBytes) + (uint32_t)(c % 5) * 1024u + lane * 16u;
+        a_off[i] = (uint32_t)min(m_tile / kFragRows + rb, row_blocks - 1) * (uint32_t)(steps2 * kFragBytes) + (uint32_t)(c % 5) * 1024u;
     }
     const uint32_t run_pitch = (uint32_t)p.strips * (kRunSteps * kUnitBytes), strip_off = (uint32_t)strip * (kRunSteps * kUnitBytes);
     const uint32_t s_pitch = (uint32_t)p.strips * 128;     // bytes between groups
@@ -248,14 +256,18 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
     uint8_t* const a_lds = lds;
     uint8_t* const w_lds = lds + 3 * kASlot + wave * (kStageSteps * kUnitBytes);
     uint8_t* const s_lds = lds + 3 * kASlot + 2 * kWBytes + wave * 256;
+    uint8_t* const c_lds = lds + 3 * kASlot + 2 * (kWBytes + kSBytes);
+    // centring sums: a stage's RB x kGroups pieces of 32 rows, two pieces a load (waves past the last one repeat an earlier
+    // wave's load); drains past the end of K read as zero
+    const int c_piece = wave % (kCBytes / 256) * 2 + half, c_rb = c_piece / kGroups, c_gi = c_piece % kGroups;
+    const uint32_t c_off = ((uint32_t)c_gi * (uint32_t)p.M + (uint32_t)(m_tile + c_rb * kFragRows + col)) * 4u;
 
 #define SLIMK_LDS_PTR(ptr) ((__attribute__((address_space(3))) void*)(ptr))
     auto fetch_a = [&](int stage, int slot) {
 #pragma unroll
         for (int i = 0; i < kALoads; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, SLIMK_LDS_PTR(a_lds + (wave + 4 * i < kABytes / 1024 ? slot * kASlot + (wave + 4 * i) * 1024 : kLds - 1024)),
-                                                     16, a_off[i],
-                                                     (stage0 + stage) * (kStageSteps * kFragBytes), 0, 0);
+                                                     16, lane * 16, a_off[i] + (uint32_t)((stage0 + stage) * (kStageSteps * kFragBytes)), 0, 0);
     };
     auto fetch_w = [&](int stage, int slot) {
         const int st = (stage0 + stage) * kStageSteps;
@@ -268,7 +280,11 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(s_rsrc, SLIMK_LDS_PTR(s_lds + slot * kSBytes), 4, s_voff,
                                                  g * s_pitch + (uint32_t)strip * 128, 0, 0);
     };
-    constexpr int kLoads = kALoads + kStageSteps + 1;      // LDS-direct loads of a wave per stage
+    auto fetch_c = [&](int stage, int slot) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(c_rsrc, SLIMK_LDS_PTR(c_lds + slot * kCBytes + wave % (kCBytes / 256) * 256), 4, c_off,
+                                                 (uint32_t)((stage0 + stage) * kGroups) * (uint32_t)p.M * 4u, 0, 0);
+    };
+    constexpr int kLoads = kALoads + kStageSteps + 1;      // a wave's requests for activations, weights and scales per stage
 
     float t[RB][2][16];
 #pragma unroll
@@ -278,116 +294,33 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
 #pragma unroll
             for (int j = 0; j < 16; ++j) t[rb][nb][j] = 0.0f;
 
+    fetch_c(0, 0);
     fetch_a(0, 0);
     fetch_w(0, 0);
     fetch_a(min(1, n_stages - 1), 1);
     fetch_w(min(1, n_stages - 1), 1);
 
-    // ---- the zero-point term of this workgroup's groups: t = -sum_g zp * scale * rowsum
     const int sub = (lane >> 4) & 1, c16 = lane & 15;      // channel nb * 32 + col = sub-block 2 nb + sub, column c16
-    const int g_lo = GS == 1 ? stage0 * 2 : stage0 >> p.group_shift;
-    const int g_hi = min(p.G, GS == 1 ? (stage0 + n_stages) * 2 : (stage0 + n_stages + p.group_shift) >> p.group_shift);
-    const __amdgpu_buffer_rsrc_t rs_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint32_t*>(p.rs), 0, (int)((size_t)p.M * p.G * 4 + 16), 0x00020000);
-    const uint32_t s_lane = ((uint32_t)strip * 64 + c16 * 4 + sub) * 2;
-    auto group_scale = [&](int g, int nb) {                // fp16 bits; zero past the workgroup's groups
-        const uint32_t off = g < g_hi ? (uint32_t)g * s_pitch + s_lane + nb * 4 : 0xfffffff0u;
-        return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(s_rsrc, off, 0, 0);
-    };
-    if (!ZP) {
-        // eight groups per turn (a half-wave four of them), the next turn's operands asked for ahead
-        struct Operands { v2u sc[4]; v4u r[RB]; };
-        auto load = [&](int g0) {
-            Operands o;
-            const int g = g0 + half * 4;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)   // the four sub-blocks' scales; zero past the workgroup's groups
-                o.sc[i] = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(
-                    s_rsrc, g + i < g_hi ? (uint32_t)(g + i) * s_pitch + ((uint32_t)strip * 64 + c16 * 4) * 2 : 0xfffffff0u, 0, 0));
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-                o.r[rb] = __builtin_amdgcn_raw_buffer_load_b128(rs_rsrc, ((uint32_t)(m_tile + rb * 32 + col) * (uint32_t)p.G + g) * 4u, 0, 0);
-            return o;
-        };
-        Operands cur = load(g_lo);
-        for (int g0 = g_lo; g0 < g_hi; g0 += 8) {
-            const Operands next = load(g0 + 8);
-            const int g = g0 + half * 4;
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)   // (past the workgroup's groups: other rows' sums, or whatever follows the last)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) cur.r[rb][i] = g + i < g_hi ? cur.r[rb][i] : 0u;
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                v4u bb;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) bb[i] = ((cur.sc[i][nb] >> (16 * sub)) & 0xffffu) * 0x10001u;
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb) {
-                    v16f c;
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) c[j] = t[rb][nb][j];
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, cur.r[rb]), __builtin_bit_cast(v8h, bb), c, 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) t[rb][nb][j] = c[j];
-                }
-            }
-            cur = next;
-        }
-        const float f = -(float)p.zp_const;
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) t[rb][nb][j] *= f;
-    } else {
-        constexpr int kRound = 4;   // pairs of groups whose loads are in flight together
-        for (int g0 = g_lo; g0 < g_hi; g0 += 2 * kRound) {
-            uint16_t sc[kRound][2];
-            uint32_t zz[kRound], r[kRound][RB];
-#pragma unroll
-            for (int b = 0; b < kRound; ++b) {
-                const int g = g0 + 2 * b + half;
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb) sc[b][nb] = group_scale(g, nb);
-                zz[b] = reinterpret_cast<const uint32_t*>(p.zp_r)[((size_t)min(g, p.G - 1) * p.strips + strip) * 16 + c16] >> (8 * sub);
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb)
-                    r[b][rb] = __builtin_amdgcn_raw_buffer_load_b32(rs_rsrc, ((uint32_t)(m_tile + rb * 32 + col) * (uint32_t)p.G + min(g, p.G - 1)) * 4u, 0, 0);
-            }
-#pragma unroll
-            for (int b = 0; b < kRound; ++b)
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb) {
-                    const float zs = -(float)((zz[b] >> (16 * nb)) & 0xffu) * half_bits_to_float(sc[b][nb]);
-#pragma unroll
-                    for (int rb = 0; rb < RB; ++rb) {
-                        const float rsum = half_bits_to_float((uint16_t)(r[b][rb] & 0xffffu)) + half_bits_to_float((uint16_t)(r[b][rb] >> 16));
-                        v16f c;
-#pragma unroll
-                        for (int j = 0; j < 16; ++j) c[j] = t[rb][nb][j];
-                        c = __builtin_amdgcn_mfma_f32_32x32x2f32(rsum, zs, c, 0, 0, 0);
-#pragma unroll
-                        for (int j = 0; j < 16; ++j) t[rb][nb][j] = c[j];
-                    }
-                }
-        }
-    }
 
-    // ---- main loop.  A unit of work is (row block, channel block) and, with GS = 1, the step: its instructions go into
-    // accumulator set u & 1 while the other set is folded into the running sums; the last unit of a stage is folded at
-    // the top of the next.
-    constexpr int kGroups = kStageSteps / GS;              // drains of a block per stage
+    // ---- main loop.  A unit of work is (row block, drain of the stage, channel block): its instructions start from the
+    // rows' centring sums and go into accumulator set u & 1 while the other set is folded into the running sums; the last
+    // unit of a stage is folded at the top of the next.
     constexpr int kUnits = RB * 2 * kGroups;
-    constexpr int kAq = RB == 4 ? 4 : 3;                   // fragments in registers (64-row tiles: three waves per SIMD)
+    // Two workgroups on a CU (256 registers a lane): both channel blocks of a row block start from one copy of its centring
+    // sums, and the next stage's raw weights are read ahead.  Three (168): each unit's sums are read into its accumulators
+    // as soon as these are folded, the raw weights at the top of their stage.
+    constexpr bool kShare = WGS == 2, kAhead = WGS == 2;
     v16f acc[2];
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[0][j] = acc[1][j] = 0.0f;
     float sc_prev = 0.0f;
+    const __amdgpu_buffer_rsrc_t z_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(ZP ? p.zp_r : reinterpret_cast<const uint8_t*>(p.s_r)), 0,
+        (int)min((size_t)p.strips * p.G * 64, (size_t)0x7fffffff), 0x00020000);
+    float sc_last[2] = {0.0f, 0.0f};                       // ZP, GS = 2: the scales of the stage before
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 
-    int slot = 0, wslot = 0;
+    int slot = 0, wslot = 0, cslot = 0;
     v4i raw[kStageSteps];
     uint16_t sraw[kGroups][2];
     auto read_w = [&](int ws) {                            // the wave's units and scales of a stage, LDS -> registers
@@ -400,25 +333,51 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) sraw[gi][nb] = *reinterpret_cast<const uint16_t*>(s_st + gi * 128 + nb * 4);
     };
-    read_w(0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (kAhead) {
+        read_w(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
     for (int stage = 0; stage < n_stages; ++stage) {
         const uint8_t* a_st = a_lds + slot * kASlot + lane * 16;
         const uint8_t* a_st8 = a_lds + slot * kASlot + 2048 + lane * 8;
         struct Frag { v4i hi, lo; v2i lo2; };
-        auto lds_frag = [&](int f) {                       // f = 2 * row block + step
-            Frag r;
-            r.hi = *reinterpret_cast<const v4i*>(a_st + f * kFragBytes);
-            r.lo = *reinterpret_cast<const v4i*>(a_st + f * kFragBytes + 1024);
+        Frag aq[kStageSteps];                              // a row block's two fragments, refilled behind their last use
+        auto load_hi = [&](int rb, int st) { aq[st].hi = *reinterpret_cast<const v4i*>(a_st + (2 * rb + st) * kFragBytes); };
+        auto load_lo = [&](int rb, int st) {
+            aq[st].lo = *reinterpret_cast<const v4i*>(a_st + (2 * rb + st) * kFragBytes + 1024);
             // (volatile: two of these merged into one read would land outside the operands they belong to)
-            r.lo2 = *(const volatile __attribute__((address_space(3))) v2i*)(a_st8 + f * kFragBytes);
-            return r;
+            aq[st].lo2 = *(const volatile __attribute__((address_space(3))) v2i*)(a_st8 + (2 * rb + st) * kFragBytes);
         };
-        Frag aq[kAq];
-        aq[0] = lds_frag(0);
-        aq[1] = lds_frag(1);
-        // two stages on: every wave is past its reads of that activation slot, this wave past those of its weight slot
+        // the centring sums of the lane's 16 accumulator rows: the first addend of the units of (row block, drain) rc
+        v16f start;
+        auto load_start = [&](int rc, v16f& to) {
+            const v4f* c_st = reinterpret_cast<const v4f*>(c_lds + cslot * kCBytes + rc * (kFragRows * 4) + half * 16);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const v4f v = c_st[2 * i];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) to[4 * i + j] = v[j];
+            }
+        };
+        if (!kAhead) read_w(wslot);
+        load_start(0, kShare ? start : acc[0]);
+#pragma unroll
+        for (int st = 0; st < kStageSteps; ++st) {
+            load_hi(0, st);
+            load_lo(0, st);
+        }
+        // The centring sums one stage on go where the stage before had them: every wave is past its reads.  They are asked
+        // for first, so that the wait for all but the requests below covers them.  The rest two stages on: every wave is
+        // past its reads of that activation slot, this wave past those of its weight slot.
+        uint32_t z_zp = 0u;   // ZP: the zero-points of a drain (half 0: GS = 1 the stage's first, GS = 2 that of the stage before)
+        if constexpr (ZP) {
+            const int d = GS == 1 ? 2 * (stage0 + stage) + half : max(stage0 + stage - 1 + half, 0);
+            z_zp = __builtin_amdgcn_raw_buffer_load_b32(z_rsrc, (((uint32_t)(d >> p.group_shift) * (uint32_t)p.strips + strip) * 16 + c16) * 4, 0, 0);
+        }
+        const int cnext = cslot == kCSlots - 1 ? 0 : cslot + 1;
+        fetch_c(min(stage + 1, n_stages - 1), cnext);
         fetch_a(min(stage + 2, n_stages - 1), slot == 0 ? 2 : slot - 1);
+        if (!kAhead) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         fetch_w(min(stage + 2, n_stages - 1), wslot);
         float sc[kGroups][2];
 #pragma unroll
@@ -431,20 +390,14 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
 
 #pragma unroll
         for (int u = 0; u < kUnits; ++u) {
-            // order: row block, then (channel block, step group)
-            const int rb = u / (2 * kGroups), nb = (u / kGroups) % 2, gi = u % kGroups;
+            const int rb = u / (2 * kGroups), gi = (u / 2) % kGroups, nb = u % 2;
             const int pu = (u + kUnits - 1) % kUnits;
-            const int prb = pu / (2 * kGroups), pnb = (pu / kGroups) % 2, pgi = pu % kGroups;
+            const int prb = pu / (2 * kGroups), pgi = (pu / 2) % kGroups, pnb = pu % 2;
             const float scale = u == 0 ? sc_prev : sc[pgi][pnb];
-            if (u % (2 * kGroups) == 0) {
-                if (rb + 1 < RB) {
-                    aq[(2 * rb + 2) % kAq] = lds_frag(2 * rb + 2);
-                    if (kAq == 4) aq[(2 * rb + 3) % kAq] = lds_frag(2 * rb + 3);
-                } else {
-                    // everything but this stage's own requests has landed: the next stage's weights are this wave's alone
-                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
-                    read_w(wslot ^ 1);
-                }
+            if (u == kUnits - 2 * kGroups) {
+                // everything but this stage's own requests has landed: the next stage's weights are this wave's alone
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+                if (kAhead) read_w(wslot ^ 1);
             }
             // The previous unit is folded beside all but the first of this unit's instructions: its last result is not
             // there yet when that one issues.
@@ -452,14 +405,14 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
 #pragma unroll
             for (int i = 0; i < kMfmas; ++i) {
                 const int st = gi * GS + i / 2;
-                const Frag& a = aq[(2 * rb + st) % kAq];
-                v16f zero;
-#pragma unroll
-                for (int j = 0; j < 16; ++j) zero[j] = 0.0f;
-                const v16f c = i == 0 ? zero : acc[u & 1];
+                const Frag& a = aq[st];
+                const v16f c = i == 0 && kShare ? start : acc[u & 1];
                 acc[u & 1] = i % 2 == 0 ? mfma_hi(a.hi, b[st][nb], c) : mfma_lo(a.lo, a.lo2, b[st][nb], c);
-                if (kAq == 3 && rb + 1 < RB && nb == 1 && st == 0 && i % 2 == 1)   // (step 0's last use in this row block)
-                    aq[(2 * rb + 3) % kAq] = lds_frag(2 * rb + 3);
+                if (kShare && i == 0 && nb == 1 && u + 1 < kUnits) load_start(u / 2 + 1, start);
+                if (rb + 1 < RB && nb == 1) {
+                    if (i % 2 == 0) load_hi(rb + 1, st);
+                    else load_lo(rb + 1, st);
+                }
                 __builtin_amdgcn_sched_barrier(0);
                 if (i > 0) {
 #pragma unroll
@@ -467,13 +420,65 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
                         t[prb][pnb][j] = __builtin_fmaf(acc[(u & 1) ^ 1][j], scale, t[prb][pnb][j]);
                 }
                 __builtin_amdgcn_sched_barrier(0);
+                if (!kShare && i == kMfmas - 1 && u + 1 < kUnits) {
+                    load_start((u + 1) / 2, acc[(u & 1) ^ 1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
         sc_prev = sc[kGroups - 1][1];
+        if constexpr (ZP) {
+            // Per-group zero-points: (2 - zp) * scale * rowsum of two drains at a time, a half-wave supplying a drain, as a
+            // matrix product onto the running sums.  The row sum (15 bits) comes apart into two bf16 numbers, 8 * (zp - 2) *
+            // scale (19 bits) into three, exactly, and their six products are exact in fp32: half the matrix core's time
+            // of v_mfma_f32_32x32x2_f32 and a vector load fewer in flight (4096 x 14336 x 4096 278 -> 263 us).
+            // (groups of 128: an odd number of stages ends with its last one alone, which half 1 supplies)
+            if (GS == 1 || (stage & 1) || stage == n_stages - 1) {
+                const bool on = GS == 1 || half == 1 || (stage & 1);
+                const uint8_t* const c_st = GS == 1 ? c_lds + cslot * kCBytes + half * (kFragRows * 4)
+                                                    : c_lds + (half == 1 || !(stage & 1) ? cslot : cslot == 0 ? kCSlots - 1 : cslot - 1) * kCBytes;
+                const auto upper = [](float v) { return __float_as_uint(v) & 0xffff0000u; };
+                v4u zb[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const float scale0 = GS == 1 ? sc[0][i] : sc_last[i], scale1 = sc[kGroups - 1][i];   // (16 times the scales)
+                    const float scale = half == 1 ? scale1 : scale0;
+                    float z = on ? ((float)((z_zp >> (8 * (2 * i + sub))) & 0xffu) - 2.0f) * 0.5f * scale : 0.0f;
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        const uint32_t u = upper(z);
+                        zb[i][d] = u | (u >> 16);
+                        z -= __uint_as_float(u);
+                    }
+                    zb[i][3] = 0u;
+                }
+#pragma unroll
+                for (int rb = RB - 1; rb >= 0; --rb) {
+                    const float sum = *reinterpret_cast<const float*>(c_st + rb * (kGroups * kFragRows * 4) + col * 4);
+                    const uint32_t u = upper(sum);
+                    const uint32_t pair = (u >> 16) | upper(sum - __uint_as_float(u));
+                    const v4u za = {pair, pair, pair, 0u};
+#pragma unroll
+                    for (int i = 1; i >= 0; --i) {
+                        v16f c;
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) c[j] = t[rb][i][j];
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, za), __builtin_bit_cast(v8b, zb[i]), c, 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) t[rb][i][j] = c[j];
+                    }
+                }
+            }
+            if (GS == 2) {
+                sc_last[0] = sc[0][0];
+                sc_last[1] = sc[0][1];
+            }
+        }
         // (the wave's requests for the next stage landed above) meet the other waves
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         slot = slot == 2 ? 0 : slot + 1;
         wslot ^= 1;
+        cslot = cnext;
     }
 #pragma unroll
     for (int j = 0; j < 16; ++j)
@@ -594,19 +599,19 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
     }
 }
 
-// 128-row tiles: two workgroups per CU (80 KiB of LDS and 256 registers each), 64-row tiles three
-template <int RB, int GS, bool SPLIT, bool ZP, typename OutT>
-__global__ __launch_bounds__(256, RB == 4 ? 2 : 3) void mx_gemm_kernel(const MxParams p) {
-    mx_body<RB, GS, SPLIT, ZP, OutT>(p);
+// 128-row tiles: two workgroups per CU (80 KiB of LDS and 256 registers each); 64-row tiles two or three
+template <int RB, int GS, bool SPLIT, bool ZP, int WGS, typename OutT>
+__global__ __launch_bounds__(256, WGS) void mx_gemm_kernel(const MxParams p) {
+    mx_body<RB, GS, SPLIT, ZP, WGS, OutT>(p);
 }
 
-template <int RB, int GS>
+template <int RB, int GS, int WGS>
 void launch_rb_gs(const MxParams& p, bool out_bf16, dim3 grid, hipStream_t stream) {
     const dim3 block(256);
 #define SLIMK_MX_LAUNCH(SPLITV, ZPV)                                                                       \
     do {                                                                                                   \
-        if (out_bf16) mx_gemm_kernel<RB, GS, SPLITV, ZPV, OutBF16><<<grid, block, 0, stream>>>(p);         \
-        else mx_gemm_kernel<RB, GS, SPLITV, ZPV, OutF16><<<grid, block, 0, stream>>>(p);                   \
+        if (out_bf16) mx_gemm_kernel<RB, GS, SPLITV, ZPV, WGS, OutBF16><<<grid, block, 0, stream>>>(p);    \
+        else mx_gemm_kernel<RB, GS, SPLITV, ZPV, WGS, OutF16><<<grid, block, 0, stream>>>(p);              \
     } while (0)
     const bool zp = p.zp_r != nullptr;
     if (p.split > 1) {
@@ -665,11 +670,12 @@ MxPlan mx_plan(int M, int N, int K, int group_size) {
     return plan;
 }
 
-hipError_t launch_mx_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size, uint8_t* frag, uint32_t* rs,
+hipError_t launch_mx_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size, int centre, uint8_t* frag, float* cs,
                            float* s_a, hipStream_t stream) {
     const dim3 grid((unsigned)(M >= 256 ? (M + 255) / 256 * 256 : M)), block((unsigned)((K / 32 + 63) / 64 * 64));
-    if (x_bf16) mx_quant_kernel<true><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, rs, s_a);
-    else mx_quant_kernel<false><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, rs, s_a);
+    const float f = -(float)centre / 16.0f;   // (the accumulators hold sums of q * code / 16)
+    if (x_bf16) mx_quant_kernel<true><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a);
+    else mx_quant_kernel<false><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a);
     return hipGetLastError();
 }
 
@@ -678,11 +684,14 @@ hipError_t launch_mx_gemm(const MxParams& p, int rb, int gs, bool out_bf16, hipS
     const int tiles = ((p.strips + kStripsPerWg - 1) / kStripsPerWg) * ((p.M + bm - 1) / bm);
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)p.split);
     if (rb == 4) {
-        if (gs == 1) launch_rb_gs<4, 1>(p, out_bf16, grid, stream);
-        else launch_rb_gs<4, 2>(p, out_bf16, grid, stream);
+        if (gs == 1) launch_rb_gs<4, 1, 2>(p, out_bf16, grid, stream);
+        else launch_rb_gs<4, 2, 2>(p, out_bf16, grid, stream);
+    } else if (tiles * p.split <= 2 * 256) {
+        if (gs == 1) launch_rb_gs<2, 1, 2>(p, out_bf16, grid, stream);
+        else launch_rb_gs<2, 2, 2>(p, out_bf16, grid, stream);
     } else {
-        if (gs == 1) launch_rb_gs<2, 1>(p, out_bf16, grid, stream);
-        else launch_rb_gs<2, 2>(p, out_bf16, grid, stream);
+        if (gs == 1) launch_rb_gs<2, 1, 3>(p, out_bf16, grid, stream);
+        else launch_rb_gs<2, 2, 3>(p, out_bf16, grid, stream);
     }
     return hipGetLastError();
 }

@@ -15,7 +15,7 @@ constexpr int kMaxK = 32512;         // the quantising kernel holds a row in 64 
 
 struct MxParams {
     const uint8_t* frag;    // activation digits: [row block][steps rounded up to even][2560]
-    const uint32_t* rs;     // [M][G] (+ 16 bytes) group sums of q as two fp16 digits (low half: a multiple of 128, high half: the rest)
+    const float* cs;        // [K / (64 or 128)][M] centring sums: -centre / 16 * the sum of q over the elements of a drain
     const float* s_a;       // [M]
     const uint32_t* w_r;    // repacked codes
     const uint16_t* s_r;    // [G][strips][16][4] fp16 bits
@@ -36,7 +36,8 @@ struct MxPlan { int rb, tiles, split, stages_per_split; };
 MxPlan mx_plan(int M, int N, int K, int group_size);
 float mx_predicted_time(int M, int N, int K, int group_size, int rb, int split);
 
-hipError_t launch_mx_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size, uint8_t* frag, uint32_t* rs,
+// centre: the zero-point the group sums start from (the layer's, or 2 where it has one per group)
+hipError_t launch_mx_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size, int centre, uint8_t* frag, float* cs,
                            float* s_a, hipStream_t stream);
 hipError_t launch_mx_gemm(const MxParams& p, int rb, int gs, bool out_bf16, hipStream_t stream);
 

@@ -1,7 +1,7 @@
 """The digit form of a layer call (csrc/gemm_mx.hip): activations split into an fp4 and an fp6 digit, exact group sums on
 the block-scaled matrix cores.  Held to the oracle within the output criterion of the path: every element within one
-ULP or rtol 1e-3, or within the fp32 re-association bound (the zero-point term is added first and in one piece, K may be
-split across workgroups)."""
+ULP or rtol 1e-3, or within the fp32 re-association bound (per-group zero-points reach the running sums in terms of their
+own, K may be split across workgroups); with a uniform zero-point and K in one piece the outputs are the oracle's bits."""
 import numpy as np
 import pytest
 import torch
@@ -136,3 +136,80 @@ def test_digits_against_the_oracle(gpu_ops, oracle, M, N, K, g, mode, out):
     wide[:, :K] = xd
     y2 = w2a8_linear_digits(wide[:, :K], w, pu.torch_dtype(case))
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+
+
+def _activation(case, kind):
+    """What a ReLU or a gating leaves (no value below zero), and values around 3: both have a mean far from zero."""
+    x = workloads.make_activation(case)
+    return {"relu": np.maximum(x, np.float16(0)), "shifted": (x.astype(np.float32) + 3 * np.abs(x).mean()).astype(np.float16)}[kind]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["relu", "shifted"])
+@pytest.mark.parametrize("M,N,K,g,mode,out", [
+    (40, 8256, 1024, 128, "sym", "float16"),       # 64-row tiles, four of them two row blocks short
+    (513, 4160, 1088, 64, "ref", "bfloat16"),      # an odd number of steps; uniform zero-point 1
+    (300, 16640, 512, 64, "sym", "bfloat16"),      # 325 64-row tiles
+    (600, 16640, 512, 128, "sym", "float16"),      # 128-row tiles
+])
+def test_activations_with_a_mean_uniform_zero_points(gpu_ops, oracle, M, N, K, g, mode, out, kind):
+    """The zero-point is in the group sums: without K splits every output is the oracle's, bit for bit."""
+    from slimkernels_amd.torch.ops import w2a8_linear_digits
+    print(f"digits, bits of the oracle M={M} N={N} K={K} g={g} {mode} {out} {kind}", flush=True)
+    assert _lib.lib().slimk_w2a8_linear_workspace_bytes(M, N, K, g) == 0
+    case = pu.small_case(M, N, K, g, mode, seed=M + N, out_dtype=out)
+    packed, scales, zero = pu.quantized_weight(case)
+    x = _activation(case, kind)
+    ref = oracle.reference_forward(x, packed, scales, zero, g, out_bf16=out == "bfloat16", want_acc=False)
+    w, xd = pu.device_inputs(gpu_ops, case, packed, scales, zero, x)
+    y = w2a8_linear_digits(xd, w, pu.torch_dtype(case))
+    np.testing.assert_array_equal(pu.out_tensor_bits(y), np.ascontiguousarray(ref["out_bits"]).view(np.uint16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["relu", "shifted"])
+@pytest.mark.parametrize("M,N,K,g,mode", [
+    (300, 4096, 4096, 128, "sym"),
+    (300, 4096, 4096, 64, "asym"),
+    (256, 2048, 8192, 128, "asym"),
+    (1024, 8192, 2048, 128, "asym"),
+    (1024, 8192, 2112, 64, "asym"),
+])
+def test_activations_with_a_mean_are_no_less_exact_than_on_the_int8_path(gpu_ops, oracle, M, N, K, g, mode, kind):
+    """Against float64 from the same integers and scales: no more outputs than the int8 path has are other than the
+    correctly rounded ones (0.1 % of the outputs apart, which is what the two paths' own splits of K may add), and every
+    output is within its rounding and the rounding of the running sums.  These never hold more than the zero-point terms of
+    two drains beside the groups so far, and a term of a group costs at most 2^-24 of what they hold."""
+    from slimkernels_amd.torch.ops import w2a8_linear_digits
+    print(f"digits against float64 M={M} N={N} K={K} g={g} {mode} {kind}", flush=True)
+    case = pu.small_case(M, N, K, g, mode, seed=M + N)
+    packed, scales, zero = pu.quantized_weight(case)
+    x = _activation(case, kind)
+    w, xd = pu.device_inputs(gpu_ops, case, packed, scales, zero, x)
+    qa = gpu_ops.quantize_act_int8(xd, g)
+    # float64 products of a group are whole numbers below 2^53: exact
+    G = K // g
+    q = qa.q.double().reshape(M, G, g).transpose(0, 1).contiguous()
+    sc = torch.from_numpy(np.asarray(scales, np.float16)).cuda().double()
+    zp = torch.from_numpy(np.broadcast_to(np.asarray(zero), (G, N)).astype(np.float64)).cuda()
+    codes = torch.from_numpy(oracle.np_unpack(packed)).cuda().double().reshape(N, G, g)
+    want = torch.zeros((M, N), dtype=torch.float64, device="cuda")
+    held = torch.zeros_like(want)                  # the sum over the groups of what the running sums hold, at most
+    for i in range(G):
+        term = (q[i] @ (codes[:, i] - zp[i][:, None]).t().contiguous()) * sc[i]
+        want += term
+        offset = (2 - zp[i]).abs() * sc[i] * q[i].sum(1, keepdim=True).abs()
+        held += want.abs() + term.abs() + 2 * offset
+    s_a = qa.s_a.double()[:, None]
+    want, held = want * s_a, held * s_a
+    best = want.half()
+    digits = w2a8_linear_digits(xd, w)
+    off = {"digits": (digits != best).sum().item(), "int8": (gpu_ops.w2a8_gemm(qa, w) != best).sum().item()}
+    print(f"  not correctly rounded: {off} of {M * N}", flush=True)
+    assert off["digits"] <= off["int8"] + M * N // 1000, off
+    # half an ULP, the product with the token scale, and three roundings a drain (the fold and the two terms of a pair; a
+    # split's sums are added once more, which the third covers)
+    ulp = torch.from_numpy(pu.ulp_of(want.float().cpu().numpy(), False)).cuda()
+    tol = 0.5 * ulp * (1 + 2.0 ** -12) + 2.0 ** -24 * (3 * held + want.abs())
+    bad = (digits.double() - want).abs() > tol
+    assert not bad.any(), int(bad.sum())
