@@ -33,9 +33,9 @@ _DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 # A decode call's kernel runs for 4-5 us, so what the host does around its launch decides how many calls a second one
 # process makes: the stream pointer and the current device come straight from torch's native accessors (0.2 us; building
 # a Stream object and entering torch.cuda.device took 4 us a call), and the library's pure functions of the
-# shape are asked once per shape.
-_raw_stream = torch._C._cuda_getCurrentRawStream
-_current_device = torch._C._cuda_getDevice
+# shape are asked once per shape.  (None on a torch without GPU support, where no call gets as far as using them.)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
 _HERE = contextlib.nullcontext()
 
 
