@@ -71,3 +71,17 @@ def test_w2a16_many_rows_with_a_split_count_that_does_not_divide(gpu_ops, oracle
     """48 pairs of steps in nine splits: six each, so the ninth has no work and is not launched."""
     assert plan(33, 16384, 6144, 128, 9) == (64, 8, 1)
     _run(gpu_ops, oracle, 33, 16384, 6144, 128, "asym", "float16", "float16", 9)
+
+
+def test_w2a16_partial_sums_are_not_kept(gpu_ops):
+    """A call whose K is split leaves nothing behind on the weight or in the allocator."""
+    w = gpu_ops.W2A16Linear.from_float(torch.randn((4096, 8192), device="cuda", dtype=torch.float16), 128).weight
+    x = torch.randn((300, 8192), device="cuda", dtype=torch.float16)
+    assert plan(300, 4096, 8192, 128)[1] > 1
+    out = torch.empty((300, 4096), device="cuda", dtype=torch.float16)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    gpu_ops.w2a16_gemm(x, w, out=out)
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_allocated() == before
+    assert torch.equal(out, gpu_ops.w2a16_gemm(x, w))
