@@ -298,9 +298,11 @@ int slimk_w2a8_set_fused_spin_limit(int polls);
  * sums are fp32 as there.  Two launches on `stream`.
  *  - slimk_w2a8_linear_route: 1 where this form is the faster one for a layer call (activation quantisation + GEMM),
  *    else 0 (per_group_zp: whether the weight carries zp_r).
- *  - activations: scratch of slimk_w2a8_linear_activation_bytes(...) bytes (no initialisation; 0: the form does not
+ *  - activations: scratch of slimk_w2a8_linear_activation_bytes(...) bytes, a multiple of 256 (no initialisation; 0: the form does not
  *    take the shape: K > 32512, or 2 GiB and more of digits or weights), needed until the call's work is done.
- *  - workspace: as for slimk_w2a8_gemm (zeroed once with slimk_w2a8_workspace_init; none where the query returns 0).
+ *  - workspace: 16-byte aligned scratch of slimk_w2a8_linear_workspace_bytes(...) bytes (none where the query returns 0),
+ *    no initialisation (the first launch zeroes the arrival counters in it), needed until the call's work is done.  A
+ *    workspace of slimk_w2a8_gemm serves too, its counters are left at zero.
  * x 16-byte aligned, ldx % 8 == 0.  No upstream counterpart (the model-level caller is llama.py:15-19). */
 int slimk_w2a8_linear_route(int M, int N, int K, int group_size, int per_group_zp);
 size_t slimk_w2a8_linear_activation_bytes(int M, int N, int K, int group_size);

@@ -698,7 +698,8 @@ int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
         p.ws_partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + kCounterBlockBytes);
     }
     hipStream_t st = (hipStream_t)stream;
-    if (int rc = hip_result(w2a8::launch_mx_quant(x, ldx, x_dtype == SLIMK_BF16, M, K, group_size, zp_r ? 2 : zp_const, frag, cs, s_a, st), "linear quantisation"))
+    if (int rc = hip_result(w2a8::launch_mx_quant(x, ldx, x_dtype == SLIMK_BF16, M, K, group_size, zp_r ? 2 : zp_const, frag, cs, s_a,
+                                                     p.ws_counter, p.ws_counter ? plan.tiles : 0, st), "linear quantisation"))
         return rc;
     return hip_result(w2a8::launch_mx_gemm(p, plan.rb, group_size == 64 ? 1 : 2, out_dtype == SLIMK_BF16, st), "linear gemm");
 }

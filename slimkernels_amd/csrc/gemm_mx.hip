@@ -63,12 +63,14 @@ constexpr int kScaleOne = 127, kScale4 = 129;   // 2^(x - 127)
 template <bool BF16>
 __global__ __launch_bounds__(1024) void mx_quant_kernel(const uint16_t* __restrict__ x, int ldx, int M, int K, int group_size,
                                                         uint8_t* __restrict__ frag, float* __restrict__ cs, float centre,
-                                                        float* __restrict__ s_a) {
+                                                        float* __restrict__ s_a, unsigned* __restrict__ counters, int n_counters) {
     __shared__ float red[16];
     const int xcd = blockIdx.x & 7, kth = blockIdx.x >> 3;
     const int m = M >= 256 ? (((kth >> 5) << 3) + xcd) * 32 + (kth & 31) : (int)blockIdx.x;
     if (m >= M) return;   // (uniform: the grid is rounded up to whole sets of rows)
     const int tid = threadIdx.x;
+    if (m == 0)   // the arrival counters of a split GEMM behind this launch
+        for (int i = tid; i < n_counters; i += (int)blockDim.x) counters[i] = 0u;
     const bool on = tid * 32 < K;
     extern __shared__ __attribute__((aligned(16))) v4u row[];   // K / 8 pieces
     const int threads = (int)blockDim.x, pieces = K / 8;
@@ -671,11 +673,11 @@ MxPlan mx_plan(int M, int N, int K, int group_size) {
 }
 
 hipError_t launch_mx_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size, int centre, uint8_t* frag, float* cs,
-                           float* s_a, hipStream_t stream) {
+                           float* s_a, unsigned* counters, int n_counters, hipStream_t stream) {
     const dim3 grid((unsigned)(M >= 256 ? (M + 255) / 256 * 256 : M)), block((unsigned)((K / 32 + 63) / 64 * 64));
     const float f = -(float)centre / 16.0f;   // (the accumulators hold sums of q * code / 16)
-    if (x_bf16) mx_quant_kernel<true><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a);
-    else mx_quant_kernel<false><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a);
+    if (x_bf16) mx_quant_kernel<true><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a, counters, n_counters);
+    else mx_quant_kernel<false><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a, counters, n_counters);
     return hipGetLastError();
 }
 

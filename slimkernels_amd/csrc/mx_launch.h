@@ -22,7 +22,7 @@ struct MxParams {
     const uint8_t* zp_r;    // [G][strips][16][4] or nullptr
     void* out;              // [M][ldo] fp16 / bf16 bits
     float* ws_partial;      // split-K partial tiles
-    unsigned* ws_counter;   // arrival counters (zero between calls)
+    unsigned* ws_counter;   // arrival counters (the quantising kernel zeroes them)
     int ldo, M, N, K, G, steps, strips, zp_const;
     int group_shift;        // 1 with groups of 256 (two stages share a scale), else 0
     int split;              // K splits (grid.y)
@@ -36,9 +36,10 @@ struct MxPlan { int rb, tiles, split, stages_per_split; };
 MxPlan mx_plan(int M, int N, int K, int group_size);
 float mx_predicted_time(int M, int N, int K, int group_size, int rb, int split);
 
-// centre: the zero-point the group sums start from (the layer's, or 2 where it has one per group)
+// centre: the zero-point the group sums start from (the layer's, or 2 where it has one per group); counters: n_counters
+// words to be zeroed
 hipError_t launch_mx_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size, int centre, uint8_t* frag, float* cs,
-                           float* s_a, hipStream_t stream);
+                           float* s_a, unsigned* counters, int n_counters, hipStream_t stream);
 hipError_t launch_mx_gemm(const MxParams& p, int rb, int gs, bool out_bf16, hipStream_t stream);
 
 }  // namespace w2a8

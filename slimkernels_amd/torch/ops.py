@@ -335,13 +335,21 @@ def w2a8_linear_digits(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, 
     if out is None:
         out = torch.empty((M, w.N), dtype=out_dtype, device=dev)
     with _on(dev):
-        act = torch.empty(_query("slimk_w2a8_linear_activation_bytes", M, w.N, K, w.group_size), dtype=torch.uint8, device=dev)
-        ws = _workspace(w, _query("slimk_w2a8_linear_workspace_bytes", M, w.N, K, w.group_size))
-        _lib.check(L.slimk_w2a8_linear(
-            x.data_ptr(), x.stride(0), _DT[x.dtype], w.w_r.data_ptr(), w.s_r.data_ptr(),
-            w.zp_r.data_ptr() if w.zp_r is not None else None, w.zp_const, M, w.N, K, w.group_size,
-            out.data_ptr(), out.stride(0), _DT[out.dtype], act.data_ptr(), act.numel(),
-            ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream_ptr(dev)))
+        # Scratch of the call's own, given back when the launches are queued: digits (a multiple of 256 bytes) and, where K
+        # is split, the partial sums (88 MB for 300 x 28672 x 8192).  The next call on the stream gets it again, behind them.
+        act_bytes = _query("slimk_w2a8_linear_activation_bytes", M, w.N, K, w.group_size)
+        ws_bytes = _query("slimk_w2a8_linear_workspace_bytes", M, w.N, K, w.group_size)
+        stream = _stream_ptr(dev)
+        scratch = _raw_alloc(act_bytes + ws_bytes, stream) if act_bytes else None
+        try:
+            _lib.check(L.slimk_w2a8_linear(
+                x.data_ptr(), x.stride(0), _DT[x.dtype], w.w_r.data_ptr(), w.s_r.data_ptr(),
+                w.zp_r.data_ptr() if w.zp_r is not None else None, w.zp_const, M, w.N, K, w.group_size,
+                out.data_ptr(), out.stride(0), _DT[out.dtype], scratch, act_bytes,
+                scratch + act_bytes if ws_bytes else None, ws_bytes, stream))
+        finally:
+            if scratch is not None:
+                _raw_free(scratch)
     return out
 
 

@@ -213,3 +213,32 @@ def test_activations_with_a_mean_are_no_less_exact_than_on_the_int8_path(gpu_ops
     tol = 0.5 * ulp * (1 + 2.0 ** -12) + 2.0 ** -24 * (3 * held + want.abs())
     bad = (digits.double() - want).abs() > tol
     assert not bad.any(), int(bad.sum())
+
+
+@pytest.mark.gpu
+def test_split_call_keeps_nothing_and_takes_dirty_scratch(gpu_ops):
+    """The partial sums of a split call are the call's own memory, whatever it held; nothing stays behind on the weight or in
+    the allocator, and the arrival counters are left at zero."""
+    from slimkernels_amd.torch.ops import _raw_stream, w2a8_linear_digits
+    L = _lib.lib()
+    M, N, K, g = 300, 4096, 4096, 128
+    w = gpu_ops.W2A8Linear.from_float(torch.randn((N, K), device="cuda", dtype=torch.float16), g, "sym").weight
+    x = torch.randn((M, K), device="cuda", dtype=torch.float16)
+    act_bytes, ws_bytes = L.slimk_w2a8_linear_activation_bytes(M, N, K, g), L.slimk_w2a8_linear_workspace_bytes(M, N, K, g)
+    assert act_bytes % 256 == 0 and ws_bytes > _lib.COUNTER_BLOCK_BYTES
+    out = torch.empty((M, N), device="cuda", dtype=torch.float16)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    w2a8_linear_digits(x, w, out=out)
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_allocated() == before and not w.workspaces
+    act = torch.full((act_bytes,), 0xff, device="cuda", dtype=torch.uint8)
+    ws = torch.full((ws_bytes,), 0xff, device="cuda", dtype=torch.uint8)
+    for _ in range(2):
+        dirty = torch.zeros_like(out)
+        _lib.check(L.slimk_w2a8_linear(x.data_ptr(), K, _lib.F16, w.w_r.data_ptr(), w.s_r.data_ptr(), None, w.zp_const, M, N, K, g,
+                                       dirty.data_ptr(), N, _lib.F16, act.data_ptr(), act_bytes, ws.data_ptr(), ws_bytes,
+                                       _raw_stream(torch.cuda.current_device())))
+        assert torch.equal(dirty, out)
+    tiles = N // 256 * ((M + 127) // 128)          # (64-row tiles would be more)
+    assert not ws[:4 * tiles].any()
