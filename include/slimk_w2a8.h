@@ -386,20 +386,24 @@ int slimk_w4a8_gemm(const int8_t* q, int ldq, const float* s_a, const int32_t* r
  * fp32 result:
  *   out[m][n] = cast( sum_g scales[g][n] * sum_{k in g} x[m][k] * (code[n][k] - zp[g][n]) ).
  * Same repacked weight operands as slimk_w2a8_gemm (w_r, s_r, zp_r / zp_const).  Built for few token rows
- * (the weight stream bounds the time); any M works, 16 rows at a time, each re-reading the weights.
- * K % 128 == 0; x_dtype SLIMK_F16 or SLIMK_BF16 (bf16: the codes enter the matrix core as 1 + code / 4 and the
- * group's activation sum, a fifth MFMA, takes the offset and the zero-point off in fp32); x 16-byte aligned,
- * ldx % 8 == 0.  split_k: K splits across workgroups, 0 = choose; with more than one the caller supplies
- * slimk_w2a16_gemm_workspace_bytes(...) bytes of workspace (fp32 partial sums, summed in split order by a
- * second kernel: results do not depend on timing).  The workspace needs no initialisation.
+ * (the weight stream bounds the time): 16 rows a workgroup, each re-reading the weights; above 32 rows, where it is
+ * predicted to be faster, a tiled kernel of 64 or 128 rows.
+ * K % 128 == 0; x_dtype SLIMK_F16 or SLIMK_BF16 (few rows, bf16: the codes enter the matrix core as 1 + code / 4 and the
+ * group's activation sum, a fifth MFMA, takes the offset and the zero-point off in fp32; the tiled kernel's operand is
+ * code - zp in either type); x 16-byte aligned, ldx % 8 == 0.  split_k: K splits across workgroups, 0 = choose; with more
+ * than one the caller supplies slimk_w2a16_gemm_workspace_bytes(...) bytes of workspace (fp32 partial sums, summed in split
+ * order by a second kernel: results do not depend on timing), no initialisation.  The choice splits many prompts of
+ * 33 rows and more, unless the workspace at hand is too small (or NULL) for it: then it is that of the few-rows
+ * kernel, one for most shapes, which takes none.
  * Replaces the upstream notebook kernel w2matmul(a, b, c) (slimkernels/triton/gemm_splitk.ipynb cell 1:
  * `b = ((b >> 4) & 0b11).to(tl.float16); accumulator = tl.dot(a, b, accumulator)`), which has no scales,
  * no zero-point and reads one field per word. */
 int slimk_w2a16_gemm_auto_split_k(int M, int N, int K, int group_size);
-/* What a call with this split_k runs: the token rows of a workgroup tile of the many-rows kernel (64 or 128; 0: the
- * few-rows kernel), the K splits across workgroups (fewer than asked for where some would have no work) and the parts of
- * K inside a workgroup of the many-rows kernel (1 or 2).  Launches nothing. */
-int slimk_w2a16_gemm_plan(int M, int N, int K, int group_size, int split_k, int* tile_rows, int* splits, int* halves);
+/* What a call with this split_k and a workspace of this size runs: the token rows of a workgroup tile of the many-rows
+ * kernel (64 or 128; 0: the few-rows kernel), the K splits across workgroups (fewer than asked for where some would have no
+ * work) and the parts of K inside a workgroup of the many-rows kernel (1 or 2).  Launches nothing. */
+int slimk_w2a16_gemm_plan(int M, int N, int K, int group_size, int split_k, size_t workspace_bytes,
+                          int* tile_rows, int* splits, int* halves);
 size_t slimk_w2a16_gemm_workspace_bytes(int M, int N, int K, int group_size, int split_k);
 int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
                      const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,

@@ -1008,11 +1008,22 @@ int slimk_w2a16_gemm_auto_split_k(int M, int N, int K, int group_size) {
     return w2a8::w2a16_plan(M, strips_of(N), K / w2a8::kStepK, group_size / w2a8::kStepK, 0).split;
 }
 
-int slimk_w2a16_gemm_plan(int M, int N, int K, int group_size, int split_k, int* tile_rows, int* splits, int* halves) {
+// The K splits of a call that leaves the choice to the library: the plan's, or where the workspace at hand does not hold their
+// partial sums the few-rows rule's (one for most shapes, which takes none).
+static int w2a16_choose_split(int M, int N, int K, int group_size, size_t workspace_bytes) {
+    const int strips = strips_of(N), steps = K / w2a8::kStepK, gs = group_size / w2a8::kStepK;
+    const int split = w2a8::w2a16_plan(M, strips, steps, gs, 0).split;
+    if (split <= 1 || (size_t)split * (size_t)M * (size_t)N * sizeof(float) <= workspace_bytes) return split;
+    return w2a8::w2a16_few_rows_split(M, strips, steps, gs);
+}
+
+int slimk_w2a16_gemm_plan(int M, int N, int K, int group_size, int split_k, size_t workspace_bytes,
+                          int* tile_rows, int* splits, int* halves) {
     if (!tile_rows || !splits || !halves) return fail(SLIMK_ERR_NULL_POINTER, "w2a16_gemm_plan: NULL result");
     if (M <= 0 || N <= 0) return fail(SLIMK_ERR_BAD_SHAPE, "M=%d, N=%d must be positive", M, N);
     if (int rc = check_kg(K, group_size)) return rc;
     if (K % 128 != 0) return fail(SLIMK_ERR_UNSUPPORTED, "w2a16_gemm: K=%d must be a multiple of 128", K);
+    if (split_k <= 0) split_k = w2a16_choose_split(M, N, K, group_size, workspace_bytes);
     const w2a8::W2A16Plan plan = w2a8::w2a16_plan(M, strips_of(N), K / w2a8::kStepK, group_size / w2a8::kStepK, split_k);
     *tile_rows = plan.rb * 32;
     *splits = plan.split;
@@ -1045,7 +1056,8 @@ int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
         return fail(SLIMK_ERR_MISALIGNED, "w2a16_gemm: x, w_r, s_r, zp_r must be 16-byte aligned; ldx %% 8 == 0; out 2-byte aligned");
     const int gs = group_size / w2a8::kStepK, steps = K / w2a8::kStepK;
     const int granules = steps / (gs > 2 ? gs : 2);
-    if (split_k <= 0) split_k = w2a8::w2a16_plan(M, strips_of(N), steps, gs, 0).split;
+    if (split_k <= 0)
+        split_k = w2a16_choose_split(M, N, K, group_size, workspace && aligned16(workspace) ? workspace_bytes : 0);
     if (split_k > 64 || (split_k > 1 && split_k * 4 > granules))
         return fail(SLIMK_ERR_BAD_SHAPE, "split_k=%d: at most 64 and at most a quarter of the %d K granules", split_k, granules);
 

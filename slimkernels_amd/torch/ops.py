@@ -363,7 +363,7 @@ def w2a16_gemm(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *, split
                out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The weight-only form: out[M, N] = x @ dequant(W)^T with the fp16 or bf16 activations x [M, K] as they are (no
     activation quantisation), the 2-bit codes widened in front of the fp16 resp. bf16 matrix cores, fp32 sums.
-    Built for few token rows; K must be a multiple of 128."""
+    Any number of token rows (above 32 a tiled kernel takes over where it is faster); K must be a multiple of 128."""
     L = _lib.lib()
     _require_cuda(x, "x")
     if x.dim() != 2 or x.dtype not in _DT:
@@ -587,7 +587,7 @@ class W2A8Linear(torch.nn.Module):
 
 class W2A16Linear(W2A8Linear):
     """The same layer with the activations left in fp16 or bf16 (weight-only quantisation): forward runs the
-    weight-only kernel, meant for a few token rows; the weight object and the constructors are W2A8Linear's."""
+    weight-only kernels, for any number of token rows; the weight object and the constructors are W2A8Linear's."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])

@@ -7,10 +7,10 @@ import pytest
 from slimkernels_amd import _lib
 
 
-def plan(M, N, K, g, split_k=0):
+def plan(M, N, K, g, split_k=0, workspace=1 << 62):
     """(token rows of a tile, 0: the few-rows kernel; K splits; K parts inside a workgroup)"""
     out = [ctypes.c_int() for _ in range(3)]
-    _lib.check(_lib.lib().slimk_w2a16_gemm_plan(M, N, K, g, split_k, *[ctypes.byref(v) for v in out]))
+    _lib.check(_lib.lib().slimk_w2a16_gemm_plan(M, N, K, g, split_k, workspace, *[ctypes.byref(v) for v in out]))
     return tuple(v.value for v in out)
 
 
@@ -53,3 +53,17 @@ def test_no_plan_has_an_empty_split():
             # the launch asks for the plan again with the split it was given: the same split comes out
             assert plan(M, N, K, g, splits)[1] == splits
     assert tiled > 500
+
+
+def test_a_call_without_workspace_is_taken_where_the_few_rows_rule_takes_none():
+    """The library's own choice of a split must fit the workspace at hand: prompts that ran unsplit with NULL still do."""
+    L = _lib.lib()
+    for M, N, K in ((300, 14336, 4096), (300, 4096, 14336), (436, 14336, 12288)):
+        need = L.slimk_w2a16_gemm_workspace_bytes(M, N, K, 128, 0)
+        assert need > 0 and plan(M, N, K, 128)[1] * M * N * 4 == need
+        for short in (0, need - 1):
+            assert plan(M, N, K, 128, 0, short) == plan(M, N, K, 128, 1)
+        assert plan(M, N, K, 128, 0, need) == plan(M, N, K, 128)
+    # (explicit requests are not changed, and a few rows still ask for what they need)
+    assert plan(300, 14336, 4096, 128, 2, 0)[1] == 2
+    assert plan(1, 4096, 14336, 128, 0, 0) == plan(1, 4096, 14336, 128) and plan(1, 4096, 14336, 128)[1] > 1

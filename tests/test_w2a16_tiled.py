@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from slimkernels_amd import workloads
+from slimkernels_amd import _lib, workloads
 import parity_utils as pu
 from test_w2a16 import _check
 from test_w2a16_plan import plan
@@ -85,3 +85,17 @@ def test_w2a16_partial_sums_are_not_kept(gpu_ops):
     torch.cuda.synchronize()
     assert torch.cuda.memory_allocated() == before
     assert torch.equal(out, gpu_ops.w2a16_gemm(x, w))
+
+
+def test_w2a16_prompt_without_workspace(gpu_ops):
+    """NULL for the workspace of a prompt the library would rather split: it runs unsplit, with the bits of split_k = 1."""
+    L = _lib.lib()
+    M, N, K, g = 300, 14336, 4096, 128
+    w = gpu_ops.W2A16Linear.from_float(torch.randn((N, K), device="cuda", dtype=torch.float16), g).weight
+    x = torch.randn((M, K), device="cuda", dtype=torch.float16)
+    assert plan(M, N, K, g)[1] > 1 and plan(M, N, K, g, 0, 0)[1] == 1
+    out = torch.zeros((M, N), device="cuda", dtype=torch.float16)
+    stream = torch.cuda.current_stream()
+    _lib.check(L.slimk_w2a16_gemm(x.data_ptr(), K, _lib.F16, w.w_r.data_ptr(), w.s_r.data_ptr(), None, w.zp_const, M, N, K, g,
+                                  out.data_ptr(), N, _lib.F16, None, 0, 0, stream.cuda_stream))
+    assert torch.equal(out, gpu_ops.w2a16_gemm(x, w, split_k=1))
