@@ -305,6 +305,8 @@ int slimk_w2a8_set_fused_spin_limit(int polls);
  *    workspace of slimk_w2a8_gemm serves too, its counters are left at zero.
  * x 16-byte aligned, ldx % 8 == 0.  No upstream counterpart (the model-level caller is llama.py:15-19). */
 int slimk_w2a8_linear_route(int M, int N, int K, int group_size, int per_group_zp);
+/* What such a call runs: the token rows of a workgroup tile (64 or 128) and the K splits across workgroups.  Launches nothing. */
+int slimk_w2a8_linear_plan(int M, int N, int K, int group_size, int* tile_rows, int* splits);
 size_t slimk_w2a8_linear_activation_bytes(int M, int N, int K, int group_size);
 size_t slimk_w2a8_linear_workspace_bytes(int M, int N, int K, int group_size);
 int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,

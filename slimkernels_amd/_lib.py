@@ -42,6 +42,7 @@ SIGNATURES = {
     "slimk_w2a8_gemm_fused_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "slimk_w2a8_set_fused_spin_limit": (_i, [_i]),
     "slimk_w2a8_linear_route": (_i, [_i, _i, _i, _i, _i]),
+    "slimk_w2a8_linear_plan": (_i, [_i, _i, _i, _i, _vp, _vp]),
     "slimk_w2a8_linear_activation_bytes": (_sz, [_i, _i, _i, _i]),
     "slimk_w2a8_linear_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "slimk_w2a8_linear": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _i, _i, _vp, _sz, _vp, _sz, _vp]),

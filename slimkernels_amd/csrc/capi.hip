@@ -624,38 +624,58 @@ size_t slimk_w2a8_linear_workspace_bytes(int M, int N, int K, int group_size) {
 }
 
 // What act_quant and the int8 tiled kernel take for more than 256 rows in fewer than 512 128-row tiles (64-row tiles,
-// the split tiled_fast_auto_split chooses), in the form of mx_predicted_time; 3.4 % rms on 36 timed calls.
-static float int8_layer_time(int M, int N, int K, int group_size) {
+// the split tiled_fast_auto_split chooses), in the form of mx_predicted_time; 4.6 % rms on 364 timed calls, 4.3 % on 328
+// others.
+static float int8_layer_time(int M, int N, int K, int group_size, int per_group_zp) {
     const int strips = strips_of(N), steps = K / w2a8::kStepK, gs = group_size / w2a8::kStepK;
     const int split = w2a8::tiled_fast_auto_split(M, strips, steps, gs);
     const int wgs = (int)w2a8::tiled_fast_workspace_tiles(M, strips, gs) * split, n = (wgs + 255) / 256;
     const int stages = (steps + 1) / 2, per = (stages + split - 1) / split;
-    const float each = n == 1 ? 0.812f : n == 2 ? 1.115f : n == 3 ? 1.584f : 0.506f * (float)n;
-    const float sums = split > 1 ? 1.29f + 0.0811e-6f * 8.0f * (float)split * (float)M * (float)N : 0.0f;
-    return 6.73f + 1.169e-6f * (float)M * (float)K + sums + ((float)per + 1.85f) * each * (group_size == 64 ? 1.314f : 1.0f);
+    float each = n == 1 ? 0.746f : n == 2 ? 1.127f : n == 3 ? 1.536f : 0.505f * (float)n;
+    if (group_size == 64) each *= 1.268f;
+    if (per_group_zp) each *= group_size == 64 ? 1.306f : 1.205f;
+    const float sums = split > 1 ? 4.39f + 0.054e-6f * 8.0f * (float)split * (float)M * (float)N : 0.0f;
+    return 5.36f + 0.968e-6f * (float)M * (float)K + sums + ((float)per + 3.44f) * each;
 }
 
 // Where the digit form beats act_quant + the kernel that slimk_w2a8_gemm would take, both timed with their quantisation;
-// groups of 64 and 128 (with 256, where the int8 kernel drains half as often, they are level: 2048 x 14336 x 4096
+// groups of 64 and 128 (with 256, where the int8 kernel drains half as often, they were level: 2048 x 14336 x 4096
 // 127 / 128 us).
 //  * 512 and more 128-row tiles (two per CU): the GEMM saves in proportion to M * N * K, the quantisation costs a little
-//    more in proportion to M * K, so N decides: 2048 x 28672 x 8192 in groups of 64 578 -> 509 us, 4096 x 14336 x 4096
-//    257 -> 242, 4096 x 5120 x 5120 139 -> 132, but 4096 x 4096 x 14336 255 -> 258 (per-group zero-points: 304 -> 296).
-//  * fewer tiles, more than 256 rows: the smaller predicted time, with 3 % in hand, inside the range the predictions were
-//    fitted on, 4096 channels and elements and more (45 timed calls: 6.7 % faster than the int8 path on average where
-//    always picking the faster one would give 7.2 %, worst 1 % slower; narrower matrices are mostly quantisation:
-//    2622 x 1922 x 8960 94 -> 104 us;
-//    1024 x 14336 x 4096 g 64 101 -> 87 us, 512 x 28672 x 8192 g 64 186 -> 153, 512 x 8192 x 28672 162 -> 142, 1900 x 7168 x 8192 152 -> 134).
-//  * 96..256 rows: long reductions only, in groups of 128 (128 x 8192 x 28672 63.5 -> 56 us, 256 x 8192 x 20480 74.5 -> 66,
-//    96 x 4096 x 28672 51 -> 44; in groups of 64 128 x 4096 x 28672 57 / 58 and with K = 14336 256 x 4096 37.5 / 38.5).
+//    more in proportion to M * K, so N decides: 4096 x 14336 x 4096 246 -> 241 us, 2048 x 28672 x 8192 in groups of 64
+//    577 -> 523, but 4096 x 4096 x 14336 260 -> 263 (per-group zero-points: 304 -> 283).  Symmetric levels with K < 512 are mostly
+//    launch and quantisation: level at K = 384, up to 3 % slower at 256 (2317 x 8400 x 256 24.3 -> 25.1).  95 routed calls of 70 drawn
+//    shapes, K = 256..16384: 18 % faster on average, the slowest 2 % faster.
+//  * fewer tiles, more than 256 rows: the smaller predicted time, with 6 % in hand, inside the range the predictions were
+//    first fitted on, 4096 channels and elements and more.  174 routed calls of shapes that took no part in the fit: 16 %
+//    faster on average, the slowest 2048 x 4096 x 11008 115.6 -> 120.0 us and 264 x 14336 x 4096 with per-group zero-points
+//    47.5 -> 48.1; 512 x 28672 x 8192 in groups of 64 184 -> 149, with per-group zero-points 239 -> 169.  (With 3 % in hand
+//    1300 x 4096 x 14336 in groups of 64 would go 130 -> 138 and 512 x 4096 x 14336 53 -> 55.)
+//  * 96..256 rows: long reductions only, in groups of 128 (128 x 8192 x 28672 62 -> 54 us, 96 x 4096 x 28672 50 -> 41).
 int slimk_w2a8_linear_route(int M, int N, int K, int group_size, int per_group_zp) {
     if (slimk_w2a8_linear_activation_bytes(M, N, K, group_size) == 0) return 0;
     if (group_size > 128 || M < 96) return 0;
     if (M <= 256) return group_size == 128 && K >= 20480 && N >= 4096 ? 1 : 0;
     const w2a8::MxPlan plan = w2a8::mx_plan(M, N, K, group_size);
-    if (plan.rb == 4 && plan.tiles >= 2 * 256) return N >= (group_size == 128 && !per_group_zp ? 5120 : 4096) ? 1 : 0;
+    if (plan.rb == 4 && plan.tiles >= 2 * 256) {
+        if (!per_group_zp && K < 512) return 0;
+        return N >= (group_size == 128 && !per_group_zp ? 5120 : 4096) ? 1 : 0;
+    }
     if (N < 4096 || K < 4096) return 0;
-    return w2a8::mx_predicted_time(M, N, K, group_size, plan.rb, plan.split) < 0.97f * int8_layer_time(M, N, K, group_size) ? 1 : 0;
+    return w2a8::mx_predicted_time(M, N, K, group_size, per_group_zp, plan.rb, plan.split) <
+                   0.94f * int8_layer_time(M, N, K, group_size, per_group_zp) ? 1 : 0;
+}
+
+int slimk_w2a8_linear_plan(int M, int N, int K, int group_size, int* tile_rows, int* splits) {
+    if (!tile_rows || !splits) return fail(SLIMK_ERR_NULL_POINTER, "linear_plan: NULL result");
+    if (M <= 0 || N <= 0) return fail(SLIMK_ERR_BAD_SHAPE, "M=%d, N=%d must be positive", M, N);
+    if (int rc = check_kg(K, group_size)) return rc;
+    if (slimk_w2a8_linear_activation_bytes(M, N, K, group_size) == 0)
+        return fail(SLIMK_ERR_UNSUPPORTED, "linear: M=%d, N=%d, K=%d not supported", M, N, K);
+    const w2a8::MxPlan plan = w2a8::mx_plan(M, N, K, group_size);
+    *tile_rows = plan.rb * w2a8::mx::kFragRows;
+    *splits = plan.split;
+    return SLIMK_OK;
 }
 
 int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,

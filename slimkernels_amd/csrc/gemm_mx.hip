@@ -629,17 +629,20 @@ void launch_rb_gs(const MxParams& p, bool out_bf16, dim3 grid, hipStream_t strea
 }  // namespace
 
 // The predicted time of a layer call in this form (us, quantisation included): start-up, quantisation, the round trip of
-// the partial sums, and stages per workgroup times what one, two or more workgroups of a CU take for a stage together.
-// Least squares on the logarithm over 340 timed plans (24 matrices of 2048..28672 channels, K = 4096..28672, groups of
-// 64 and 128, 96..2048 rows): 6.6 % rms.
-float mx_predicted_time(int M, int N, int K, int group_size, int rb, int split) {
+// the partial sums, and stages per workgroup times what one, two or more workgroups of a CU take for a stage together, more
+// of it in groups of 64 (twice the drains) and with per-group zero-points.  Least squares on the logarithm over 3482 timed
+// plans of drawn shapes and of thirteen decoder matrices (2048..28672 channels, K = 2048..28672, groups of 64 and 128,
+// 96..2048 rows, symmetric and per-group zero-points): 6.0 % rms, 5.7 % on 2690 plans of other shapes.
+float mx_predicted_time(int M, int N, int K, int group_size, int per_group_zp, int rb, int split) {
     const int stages = mx_padded_steps(K) / 2, per = (stages + split - 1) / split;
     const int tiles = ((N + 255) / 256) * ((M + rb * kFragRows - 1) / (rb * kFragRows));
     const int n = (tiles * split + 255) / 256;
-    const float each = rb == 2 ? (n == 1 ? 0.774f : n == 2 ? 1.014f : 0.463f * (float)n)
-                               : (n == 1 ? 1.019f : n == 2 ? 1.563f : 0.787f * (float)n);
-    const float sums = split > 1 ? 0.0834e-6f * 8.0f * (float)split * (float)M * (float)N : 0.0f;
-    return 12.57f + 1.124e-6f * (float)M * (float)K + sums + ((float)per + 3.24f) * each * (group_size == 64 ? 1.325f : 1.0f);
+    float each = rb == 2 ? (n == 1 ? 0.644f : n == 2 ? 0.899f : 0.4365f * (float)n)
+                         : (n == 1 ? 0.984f : n == 2 ? 1.473f : 0.766f * (float)n);
+    if (group_size == 64) each *= 1.249f;
+    if (per_group_zp) each *= group_size == 64 ? 1.155f : 1.113f;
+    const float sums = split > 1 ? 0.088e-6f * 8.0f * (float)split * (float)M * (float)N : 0.0f;
+    return 13.77f + 1.056e-6f * (float)M * (float)K + sums + ((float)per + 2.81f) * each;
 }
 
 // 128-row tiles where they fill the chip; otherwise the tile height and K split with the smallest predicted time
@@ -656,7 +659,7 @@ MxPlan mx_plan(int M, int N, int K, int group_size) {
         const int tiles = tiles_n * ((M + rb * kFragRows - 1) / (rb * kFragRows));
         for (int split : {1, 2, 3, 4, 6, 8}) {
             if (split > 1 && (stages / split < 6 || tiles * split > 1100)) break;
-            const float time = mx_predicted_time(M, N, K, group_size, rb, split);
+            const float time = mx_predicted_time(M, N, K, group_size, 0, rb, split);
             if (time < best) {
                 best = time;
                 best_split = split;

@@ -34,7 +34,7 @@ __host__ __device__ inline int mx_padded_steps(int K) { return (K / kStepK + 1) 
 // what a launch looks like: row blocks per workgroup tile (2 or 4), tiles, K splits and stages per split
 struct MxPlan { int rb, tiles, split, stages_per_split; };
 MxPlan mx_plan(int M, int N, int K, int group_size);
-float mx_predicted_time(int M, int N, int K, int group_size, int rb, int split);
+float mx_predicted_time(int M, int N, int K, int group_size, int per_group_zp, int rb, int split);
 
 // centre: the zero-point the group sums start from (the layer's, or 2 where it has one per group); counters: n_counters
 // words to be zeroed
