@@ -120,10 +120,10 @@ def test_digits_against_the_oracle(gpu_ops, oracle, M, N, K, g, mode, out):
     y = w2a8_linear_digits(xd, w, pu.torch_dtype(case))
     bound = None
     if not big:
-        # the zero-point term and the sum of q * code are each larger than their difference: their magnitudes bound it
+        # per-group zero-points: the sums centred on 2 and the rest (zp - 2) * rowsum are each larger than their difference
         zp = np.broadcast_to(np.asarray(zero, np.int64), (K // g, N))
         rs = ref["q"].reshape(M, K // g, g).astype(np.int64).sum(2)
-        folded = np.abs(rs)[:, None, :] * zp.T[None]
+        folded = np.abs(rs)[:, None, :] * np.abs(zp - (2 if mode == "asym" else zp)).T[None]
         bound = pu.reorder_bound(np.abs(ref["acc"].astype(np.int64)) + 2 * folded, scales, ref["s_a"])
     if big:
         # every element within one ULP or rtol 1e-3 but a few whose terms cancel, which the sums' magnitude bounds:
@@ -131,6 +131,8 @@ def test_digits_against_the_oracle(gpu_ops, oracle, M, N, K, g, mode, out):
         bound = (K // g * 2.0 ** -24 * ref["s_a"].astype(np.float64)[:, None] * 3 * 127 * g *
                  np.asarray(scales, np.float64).sum(0)[None, :])
     pu.assert_out_close(pu.out_tensor_bits(y), ref["out_bits"], bf16, reorder_bound=bound, what="digits")
+    if mode != "asym" and g < 256 and _lib.lib().slimk_w2a8_linear_workspace_bytes(M, N, K, g) == 0:
+        np.testing.assert_array_equal(pu.out_tensor_bits(y), np.ascontiguousarray(ref["out_bits"]).view(np.uint16))
     # a strided activation and reused scratch give the same bits
     wide = torch.zeros((M, K + 64), dtype=xd.dtype, device="cuda")
     wide[:, :K] = xd

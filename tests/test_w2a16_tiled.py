@@ -46,7 +46,7 @@ def _run(gpu_ops, oracle, M, N, K, g, mode, xdt, out, split, zero=None):
 
 
 @pytest.mark.parametrize("M,N,K,g,mode,xdt,out,split", [
-    (300, 16448, 256, 128, "sym", "float16", "float16", 1),       # 64-row tiles, four steps, one strip in the last channel tile
+    (300, 16448, 256, 128, "sym", "float16", "float16", 1),       # 128-row tiles, four steps, one strip in the last channel tile
     (1000, 16384, 512, 128, "ref", "float16", "bfloat16", 0),     # 128-row tiles
     (1000, 16384, 512, 64, "asym", "bfloat16", "bfloat16", 0),
     (250, 16384, 2048, 64, "asym", "bfloat16", "bfloat16", 1),    # two K halves in a workgroup
