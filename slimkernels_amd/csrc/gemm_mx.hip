@@ -245,12 +245,13 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
         const_cast<float*>(p.cs), 0, (int)((size_t)p.M * drains * 4), 0x00020000);
 
     // activations: chunk c = wave + 4 i of 1 KiB; a row block's two fragments of a stage are 5 chunks in one piece
-    // (all of it the wave's: in scalar registers beside the lane's 16 bytes; a row block past the last repeats it)
+    // (all of it the wave's, below 2 GiB: in scalar registers beside the lane's 16 bytes.  Said outright: with offsets that the
+    // compiler computed in vector registers each load was a loop over their values.  A row block past the last repeats it)
     uint32_t a_off[kALoads];
 #pragma unroll
     for (int i = 0; i < kALoads; ++i) {
         const int c = min(wave + 4 * i, kABytes / 1024 - 1), rb = c / 5;
-        a_off[i] = (uint32_t)min(m_tile / kFragRows + rb, row_blocks - 1) * (uint32_t)(steps2 * kFragBytes) + (uint32_t)(c % 5) * 1024u;
+        a_off[i] = (uint32_t)__builtin_amdgcn_readfirstlane(min(m_tile / kFragRows + rb, row_blocks - 1) * (steps2 * kFragBytes) + c % 5 * 1024);
     }
     const uint32_t run_pitch = (uint32_t)p.strips * (kRunSteps * kUnitBytes), strip_off = (uint32_t)strip * (kRunSteps * kUnitBytes);
     const uint32_t s_pitch = (uint32_t)p.strips * 128;     // bytes between groups
