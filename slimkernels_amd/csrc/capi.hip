@@ -624,18 +624,18 @@ size_t slimk_w2a8_linear_workspace_bytes(int M, int N, int K, int group_size) {
 }
 
 // What act_quant and the int8 tiled kernel take for more than 256 rows in fewer than 512 128-row tiles (64-row tiles,
-// the split tiled_fast_auto_split chooses), in the form of mx_predicted_time; 4.6 % rms on 364 timed calls, 4.3 % on 328
+// the split tiled_fast_auto_split chooses), in the form of mx_predicted_time; 4.5 % rms on 364 timed calls, 4.2 % on 328
 // others.
 static float int8_layer_time(int M, int N, int K, int group_size, int per_group_zp) {
     const int strips = strips_of(N), steps = K / w2a8::kStepK, gs = group_size / w2a8::kStepK;
     const int split = w2a8::tiled_fast_auto_split(M, strips, steps, gs);
     const int wgs = (int)w2a8::tiled_fast_workspace_tiles(M, strips, gs) * split, n = (wgs + 255) / 256;
     const int stages = (steps + 1) / 2, per = (stages + split - 1) / split;
-    float each = n == 1 ? 0.746f : n == 2 ? 1.127f : n == 3 ? 1.536f : 0.505f * (float)n;
-    if (group_size == 64) each *= 1.268f;
-    if (per_group_zp) each *= group_size == 64 ? 1.306f : 1.205f;
-    const float sums = split > 1 ? 4.39f + 0.054e-6f * 8.0f * (float)split * (float)M * (float)N : 0.0f;
-    return 5.36f + 0.968e-6f * (float)M * (float)K + sums + ((float)per + 3.44f) * each;
+    float each = n == 1 ? 0.74f : n == 2 ? 1.118f : n == 3 ? 1.536f : 0.501f * (float)n;
+    if (group_size == 64) each *= 1.271f;
+    if (per_group_zp) each *= group_size == 64 ? 1.298f : 1.205f;
+    const float sums = split > 1 ? 4.15f + 0.0562e-6f * 8.0f * (float)split * (float)M * (float)N : 0.0f;
+    return 5.57f + 1.104e-6f * (float)M * (float)K + sums + ((float)per + 3.4f) * each;
 }
 
 // Where the digit form beats act_quant + the kernel that slimk_w2a8_gemm would take, both timed with their quantisation;
@@ -647,10 +647,12 @@ static float int8_layer_time(int M, int N, int K, int group_size, int per_group_
 //    launch and quantisation: level at K = 384, up to 3 % slower at 256 (2317 x 8400 x 256 24.3 -> 25.1).  95 routed calls of 70 drawn
 //    shapes, K = 256..16384: 18 % faster on average, the slowest 2 % faster.
 //  * fewer tiles, more than 256 rows: the smaller predicted time, with 6 % in hand, inside the range the predictions were
-//    first fitted on, 4096 channels and elements and more.  174 routed calls of shapes that took no part in the fit: 16 %
-//    faster on average, the slowest 2048 x 4096 x 11008 115.6 -> 120.0 us and 264 x 14336 x 4096 with per-group zero-points
-//    47.5 -> 48.1; 512 x 28672 x 8192 in groups of 64 184 -> 149, with per-group zero-points 239 -> 169.  (With 3 % in hand
-//    1300 x 4096 x 14336 in groups of 64 would go 130 -> 138 and 512 x 4096 x 14336 53 -> 55.)
+//    first fitted on, 4096 channels and elements and more.  200 routed calls of shapes that took no part in the fit: 16 %
+//    faster on average, the slowest level (264 x 14336 x 4096 with per-group zero-points 47.6 / 47.9 us); on normal
+//    activations without outliers (other toggling, another clock) 281 routed calls of thirteen decoder matrices 13 %
+//    faster, the slowest 1500 x 8192 x 8192 120.5 -> 124.0.  512 x 28672 x 8192 in
+//    groups of 64 184 -> 146, with per-group zero-points 236 -> 165.  (With 3 % in hand 1300 x 4096 x 11008 in groups of
+//    64 would go 111 -> 115.)
 //  * 96..256 rows: long reductions only, in groups of 128 (128 x 8192 x 28672 62 -> 54 us, 96 x 4096 x 28672 50 -> 41).
 int slimk_w2a8_linear_route(int M, int N, int K, int group_size, int per_group_zp) {
     if (slimk_w2a8_linear_activation_bytes(M, N, K, group_size) == 0) return 0;

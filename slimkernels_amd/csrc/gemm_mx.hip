@@ -633,17 +633,17 @@ void launch_rb_gs(const MxParams& p, bool out_bf16, dim3 grid, hipStream_t strea
 // the partial sums, and stages per workgroup times what one, two or more workgroups of a CU take for a stage together, more
 // of it in groups of 64 (twice the drains) and with per-group zero-points.  Least squares on the logarithm over 3482 timed
 // plans of drawn shapes and of thirteen decoder matrices (2048..28672 channels, K = 2048..28672, groups of 64 and 128,
-// 96..2048 rows, symmetric and per-group zero-points): 6.0 % rms, 5.7 % on 2690 plans of other shapes.
+// 96..2048 rows, symmetric and per-group zero-points): 5.9 % rms, 5.7 % on 2690 plans of other shapes.
 float mx_predicted_time(int M, int N, int K, int group_size, int per_group_zp, int rb, int split) {
     const int stages = mx_padded_steps(K) / 2, per = (stages + split - 1) / split;
     const int tiles = ((N + 255) / 256) * ((M + rb * kFragRows - 1) / (rb * kFragRows));
     const int n = (tiles * split + 255) / 256;
-    float each = rb == 2 ? (n == 1 ? 0.644f : n == 2 ? 0.899f : 0.4365f * (float)n)
-                         : (n == 1 ? 0.984f : n == 2 ? 1.473f : 0.766f * (float)n);
-    if (group_size == 64) each *= 1.249f;
-    if (per_group_zp) each *= group_size == 64 ? 1.155f : 1.113f;
-    const float sums = split > 1 ? 0.088e-6f * 8.0f * (float)split * (float)M * (float)N : 0.0f;
-    return 13.77f + 1.056e-6f * (float)M * (float)K + sums + ((float)per + 2.81f) * each;
+    float each = rb == 2 ? (n == 1 ? 0.596f : n == 2 ? 0.857f : 0.4234f * (float)n)
+                         : (n == 1 ? 0.977f : n == 2 ? 1.463f : 0.757f * (float)n);
+    if (group_size == 64) each *= 1.257f;
+    if (per_group_zp) each *= group_size == 64 ? 1.145f : 1.129f;
+    const float sums = split > 1 ? 0.0886e-6f * 8.0f * (float)split * (float)M * (float)N : 0.0f;
+    return 13.7f + 1.119e-6f * (float)M * (float)K + sums + ((float)per + 2.87f) * each;
 }
 
 // 128-row tiles where they fill the chip; otherwise the tile height and K split with the smallest predicted time

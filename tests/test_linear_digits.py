@@ -249,7 +249,7 @@ def test_split_call_keeps_nothing_and_takes_dirty_scratch(gpu_ops):
 def test_route_knows_short_reductions_and_per_group_zero_points():
     """512 and more 128-row tiles: with K < 512 symmetric layers stay on the int8 path (2317 x 8400 x 256 24.3 against 25.1
     us), layers with per-group zero-points do not (32.3 against 25.6).  Fewer tiles: the two paths' predictions know the
-    zero-points too (600 x 11008 x 4096: 46.7 / 45.8 us symmetric, 52.9 / 51.0 with zero-points)."""
+    zero-points too (600 x 11008 x 4096: 46.4 / 44.2 us symmetric, less than the 6 % in hand, 52.9 / 48.7 with zero-points)."""
     route = _lib.lib().slimk_w2a8_linear_route
     for M, N, g in ((2317, 8400, 128), (7173, 6000, 128), (2189, 22352, 64)):
         assert [route(M, N, 256, g, zp) for zp in (0, 1)] == [0, 1]

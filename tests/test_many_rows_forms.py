@@ -40,7 +40,8 @@ def _weight(gpu_ops, N, K, g, mode, gen):
     (999, 8201, 1024, 128, "asym", 64, 1),
     (999, 8200, 1152, 128, "sym", 64, 1),
     (999, 3001, 6144, 64, "asym", 64, 4),        # the same with K split
-    (1000, 3000, 6144, 128, "sym", 64, 4),
+    (900, 3000, 6144, 128, "sym", 64, 4),
+    (300, 4100, 4096, 128, "asym", 64, 3),       # two workgroups a CU with K split
     (999, 14593, 1088, 64, "sym", 128, 1),       # 128-row tiles, nine stages
     (999, 14593, 1088, 64, "asym", 128, 1),
     (1000, 14592, 1152, 128, "sym", 128, 1),
