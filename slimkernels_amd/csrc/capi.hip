@@ -642,8 +642,8 @@ static float int8_layer_time(int M, int N, int K, int group_size, int per_group_
 // groups of 64 and 128 (with 256, where the int8 kernel drains half as often, they were level: 2048 x 14336 x 4096
 // 127 / 128 us).
 //  * 512 and more 128-row tiles (two per CU): the GEMM saves in proportion to M * N * K, the quantisation costs a little
-//    more in proportion to M * K, so N decides: 4096 x 14336 x 4096 246 -> 241 us, 2048 x 28672 x 8192 in groups of 64
-//    577 -> 523, but 4096 x 4096 x 14336 260 -> 263 (per-group zero-points: 304 -> 283).  Symmetric levels with K < 512 are mostly
+//    more in proportion to M * K, so N decides: 4096 x 14336 x 4096 244 -> 237 us, 2048 x 28672 x 8192 in groups of 64
+//    575 -> 512, but 4096 x 4096 x 14336 level at 257 (per-group zero-points: 301 -> 279).  Symmetric levels with K < 512 are mostly
 //    launch and quantisation: level at K = 384, up to 3 % slower at 256 (2317 x 8400 x 256 24.3 -> 25.1).  95 routed calls of 70 drawn
 //    shapes, K = 256..16384: 18 % faster on average, the slowest 2 % faster.
 //  * fewer tiles, more than 256 rows: the smaller predicted time, with 6 % in hand, inside the range the predictions were

@@ -22,11 +22,12 @@
 //
 // Measured: 38 cycles per 32x32x64 instruction with the 4 drain fmas of groups of 128 beside it, 49 with the 8 of
 // groups of 64 (32 alone) in a probe; on random operands the faster matrix instructions run into the power limit
-// (2.16 against the int8 kernel's 2.42 GHz).  Layer calls with their quantisation on one card, us: the int8 path / this
-// kernel with the offset in front of the loop / this kernel: 4096 x 14336 x 4096 246 / 245 / 241, with per-group zero-points
-// 277 / 267 / 263; 2048 x 28672 x 8192 in groups of 64 577 / 525 / 523, with per-group zero-points 724 / 640 / 595;
-// 1024 x 14336 x 4096 81 / 75 / 73.  What is left over the matrix cores' own time is the vector instructions beside them
-// (185 per 32 of them), prologue and epilogue of a tile, and the half-empty last round of tiles.
+// (4096 x 14336 x 4096: 448 thousand cycles at 2.07 GHz against the int8 kernel's 556 at 2.43).  Layer calls with their
+// quantisation in one run on one card, us: the int8 path / this kernel with the offset in front of the loop / this kernel:
+// 4096 x 14336 x 4096 244 / 241 / 237, with per-group zero-points 276 / 263 / 257; 2048 x 28672 x 8192 in groups of 64
+// 575 / 515 / 512, with per-group zero-points 726 / 629 / 583; 1024 x 14336 x 4096 80 / 74 / 72.  What is left over the
+// matrix cores' own time is the vector instructions beside them (186 per 32 of them), prologue and epilogue of a tile, and the
+// half-empty last round of tiles.
 //
 // Activation fragments (written by mx_quant_kernel): one of 2560 bytes per 32 rows x 64 elements, in operand order.
 // Lane l holds row l & 31, elements 32 * (l >> 5) .. + 31: 16 bytes of fp4 digits at 16 * l, the first 16 bytes of its
@@ -434,7 +435,8 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
             // Per-group zero-points: (2 - zp) * scale * rowsum of two drains at a time, a half-wave supplying a drain, as a
             // matrix product onto the running sums.  The row sum (15 bits) comes apart into two bf16 numbers, 8 * (zp - 2) *
             // scale (19 bits) into three, exactly, and their six products are exact in fp32: half the matrix core's time
-            // of v_mfma_f32_32x32x2_f32 and a vector load fewer in flight (4096 x 14336 x 4096 278 -> 263 us).
+            // of v_mfma_f32_32x32x2_f32 and no vector load in flight beside the requests
+            // (4096 x 14336 x 4096 278 -> 263 us).
             // (groups of 128: an odd number of stages ends with its last one alone, which half 1 supplies)
             if (GS == 1 || (stage & 1) || stage == n_stages - 1) {
                 const bool on = GS == 1 || half == 1 || (stage & 1);

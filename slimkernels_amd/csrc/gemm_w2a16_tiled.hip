@@ -361,7 +361,7 @@ hipError_t launch_w2a16_tiled(const W2A16Params& p, int rb, int halves, int gs, 
 // covers the problem, as it needs half the splits (300 x 4096 x 14336: three splits of two halves 51.6 us, six splits
 // 55.0 on the same card; 768 x 5120 x 5120 unsplit 47.9, in two splits 56.2; in two rounds it loses, 400 x 2048 x 20480 in six
 // 67.5 against 64.9).  A split writes and reads its partial sums at about 5 TB/s, plus the second launch.  Within 6 % of the measured times
-// of fourteen shapes (64..1024 rows, 1024..28672 channels, K = 4096..14336) at one to eight splits: 300 x 4096 x 14336 89 -> 53 us,
+// of fourteen shapes (64..1024 rows, 1024..28672 channels, K = 4096..14336) at one to eight splits: 300 x 4096 x 14336 80 -> 49 us,
 // 128 x 14336 x 4096 39 -> 31, 1024 x 14336 x 4096 275 -> 115, 100 x 28672 x 8192 132 -> 74; 64 x 4096 x 4096 stays with
 // the few-rows kernel (8.4 against 13 us).
 W2A16Plan w2a16_plan(int M, int strips, int steps, int gs, int split) {
