@@ -5,8 +5,19 @@
 
 namespace w2a8 {
 
-size_t tiled_w4_tiles(int M, int strips) {
-    return (size_t)((strips + fast::kStrips - 1) / fast::kStrips) * (size_t)((M + 63) / 64);
+size_t tiled_w4_tiles(int M, int strips, int rows) {
+    return (size_t)((strips + fast::kStrips - 1) / fast::kStrips) * (size_t)((M + rows - 1) / rows);
+}
+
+// 128-row tiles of the one-pass W4 kernel unpack a weight unit once for twice the rows (5.3 vector instructions beside a
+// matrix instruction, not 6.5), but a lone workgroup hides nothing and the chip takes them in coarser rounds.  In units of
+// 32 stages, n workgroups on the fullest CU take about 24 n (64 rows) or 41 n us (128 rows; alone 50): measured on 31 shapes
+// (100..2048 rows, 1024..28672 channels, K = 1280..14336) the rule is never more than 1 % behind the better height.
+// 1000 x 14336 x 4096 98.6 -> 84.1 us (896 or 448 tiles), 1536 x 16384 x 4096 136.6 -> 123.0, 2048 x 28672 x 2048 182.1 ->
+// 150.6; kept on 64 rows: 600 x 14336 x 4096 69.2 / 74.5, 2000 x 6000 x 8192 140.1 / 148.2.
+bool tiled_w4_tall(int M, int strips) {
+    const int n64 = (int)((tiled_w4_tiles(M, strips, 64) + 255) / 256), n128 = (int)((tiled_w4_tiles(M, strips, 128) + 255) / 256);
+    return n128 >= 2 && 41 * n128 < 24 * n64;
 }
 
 // The split a score of three factors picks among 1, 2, 3, 4, 6 and 8 for `tiles` 64-row tiles of `stages` stages:

@@ -63,7 +63,13 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
     constexpr int kWDwords = kStrips * kStageSteps * 256 * kWPlanes;  // the four waves' weight units of a stage: 8 KiB a plane
     constexpr int kBufDwords = kStageDwords + kWDwords;
     constexpr int kBufs = 3;                       // stage s+2 is in flight while stage s is consumed
-    __shared__ __attribute__((aligned(16))) uint32_t lds[kBufs][kBufDwords];
+    // (128-row tiles with both planes: the weights, a wave's own, take two places in turn, a stage's units moving to
+    // registers before those two stages on are asked for: 80 KiB, two workgroups on a CU)
+    constexpr bool kTwoW = W4 && BM == 128;
+    constexpr int kAPitch = kTwoW ? kStageDwords : kBufDwords, kWPitch = kTwoW ? kWDwords : kBufDwords;
+    constexpr int kWBase = kTwoW ? kBufs * kStageDwords : kStageDwords;
+    constexpr int kLdsDwords = kTwoW ? kBufs * kStageDwords + 2 * kWDwords : kBufs * kBufDwords;
+    __shared__ __attribute__((aligned(16))) uint32_t lds[kLdsDwords];
     // GS = 64-element steps per scale group: 1, 2, or 4.  With 4 a group spans two stages: every token block keeps
     // its own int32 accumulators from the first stage of a group to the second (kLong), the drain happens in the
     // second stages only, and the stage loop runs over pairs of stages.
@@ -144,22 +150,22 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
     // Activations and this wave's weight units go straight from global memory into LDS (no registers
     // held while in flight), two stages ahead; the scales, a few bytes, go to registers one stage ahead.
     constexpr int kLdsLoads = kALoads + kStageSteps * kWPlanes;  // LDS-direct loads a wave issues per stage
-    auto fetch = [&](int stage, int buf) {
+    auto fetch = [&](int stage, int buf, int wbuf) {
 #pragma unroll
         for (int i = 0; i < kALoads; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                q_rsrc, (__attribute__((address_space(3))) void*)&lds[buf][(wave + 4 * i) * 256], 16, a_off[i],
+                q_rsrc, (__attribute__((address_space(3))) void*)&lds[buf * kAPitch + (wave + 4 * i) * 256], 16, a_off[i],
                 (stage0 + stage) * (kStageSteps * kStepK), 0, 0);
 #pragma unroll
         for (int s = 0; s < kStageSteps; ++s)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                w_rsrc, (__attribute__((address_space(3))) void*)&lds[buf][kStageDwords + (wave * kStageSteps + s) * 256], 16,
+                w_rsrc, (__attribute__((address_space(3))) void*)&lds[wbuf * kWPitch + kWBase + (wave * kStageSteps + s) * 256], 16,
                 lane * 16, unit_off((stage0 + stage) * kStageSteps + s), 0, 0);
         if constexpr (W4) {
 #pragma unroll
             for (int s = 0; s < kStageSteps; ++s)   // the lo digits of the same steps: p.steps units further on
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    w_rsrc, (__attribute__((address_space(3))) void*)&lds[buf][kStageDwords + kWDwords / 2 + (wave * kStageSteps + s) * 256], 16,
+                    w_rsrc, (__attribute__((address_space(3))) void*)&lds[wbuf * kWPitch + kWBase + kWDwords / 2 + (wave * kStageSteps + s) * 256], 16,
                     lane * 16, unit_off((stage0 + stage) * kStageSteps + s + p.steps), 0, 0);
         }
     };
@@ -187,8 +193,8 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
             for (int j = 0; j < 4; ++j) t[mb][pp][j] = 0.0f;
 
     fetch_scales(0);
-    fetch(0, 0);
-    fetch(min(1, n_stages - 1), 1);
+    fetch(0, 0, 0);
+    fetch(min(1, n_stages - 1), 1, 1);
 
     if (ZP) {
         // Zero-points other than the 2 the operand bytes are centred on: the missing term
@@ -260,11 +266,12 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
         sc_prev[pp] = 0.0f;
     }
 
-    int buf = 0;
+    int buf = 0, wbuf = 0;
     // one stage; kHalf (group of 256 only): 0 = first stage of a group, 1 = second
     auto run_stage = [&](const int stage, auto half_tag) {
         constexpr int kHalf = decltype(half_tag)::value;
-        const uint32_t* la = &lds[buf][lane * 4];
+        const uint32_t* la = &lds[buf * kAPitch + lane * 4];
+        const uint32_t* lw = kTwoW ? &lds[wbuf * kWPitch + kWBase + lane * 4] : la + kWBase;
         auto lds_a = [&](int r) {  // r-th fragment in consumption order: token block r / 2, step r % 2
             return *reinterpret_cast<const v4i*>(la + ((r % kStageSteps) * kMB + r / kStageSteps) * 256);
         };
@@ -286,18 +293,25 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
         v4i b[kStageSteps][4];
 #pragma unroll
         for (int s = 0; s < kStageSteps; ++s) {
-            const v4i w = *reinterpret_cast<const v4i*>(la + kStageDwords + (wave * kStageSteps + s) * 256);
-            const v4i wf = w ^ (int)0x2a2a2a2au;  // flip the high bit of fields 0..2: code -> two's complement of code - 2
-#pragma unroll
-            for (int pp = 0; pp < 3; ++pp) b[s][pp] = (wf << (6 - 2 * pp)) & (int)0xc0c0c0c0u;
-            b[s][3] = w & (int)0xc0c0c0c0u;  // field 3 is stored already flipped
+            const v4i w = *reinterpret_cast<const v4i*>(lw + (wave * kStageSteps + s) * 256);
             if constexpr (W4) {
+                // both digits of two fields in one register, the codes in its nibbles, then a nibble to the top of its byte
+                // and the high bits flipped (hi digits of fields 0..2: code -> two's complement of code - 2; lo digits of
+                // field 3, which are stored flipped: back to the code): 10 instructions per dword of each plane
+                // (digit by digit it was 16: 1000 x 14336 x 4096 on 64-row tiles 108 -> 100 us)
                 typedef unsigned v4w __attribute__((ext_vector_type(4)));
-                const v4w wl = __builtin_bit_cast(v4w, *reinterpret_cast<const v4i*>(la + kStageDwords + kWDwords / 2 + (wave * kStageSteps + s) * 256));
-                b[s][0] |= __builtin_bit_cast(v4i, (wl << 4) & 0x30303030u);
-                b[s][1] |= __builtin_bit_cast(v4i, (wl << 2) & 0x30303030u);
-                b[s][2] |= __builtin_bit_cast(v4i, wl & 0x30303030u);
-                b[s][3] |= __builtin_bit_cast(v4i, ((wl ^ 0x80808080u) >> 2) & 0x30303030u);  // stored flipped: back to the code
+                const v4w wh = __builtin_bit_cast(v4w, w);
+                const v4w wl = __builtin_bit_cast(v4w, *reinterpret_cast<const v4i*>(lw + kWDwords / 2 + (wave * kStageSteps + s) * 256));
+                const v4w even = ((wh << 2) & 0xccccccccu) | (wl & 0x33333333u), odd = (wh & 0xccccccccu) | ((wl >> 2) & 0x33333333u);
+                b[s][0] = __builtin_bit_cast(v4i, ((even << 4) & 0xf0f0f0f0u) ^ 0x80808080u);
+                b[s][1] = __builtin_bit_cast(v4i, ((odd << 4) & 0xf0f0f0f0u) ^ 0x80808080u);
+                b[s][2] = __builtin_bit_cast(v4i, (even & 0xf0f0f0f0u) ^ 0x80808080u);
+                b[s][3] = __builtin_bit_cast(v4i, (odd & 0xf0f0f0f0u) ^ 0x20202020u);
+            } else {
+                const v4i wf = w ^ (int)0x2a2a2a2au;  // flip the high bit of fields 0..2: code -> two's complement of code - 2
+#pragma unroll
+                for (int pp = 0; pp < 3; ++pp) b[s][pp] = (wf << (6 - 2 * pp)) & (int)0xc0c0c0c0u;
+                b[s][3] = w & (int)0xc0c0c0c0u;  // field 3 is stored already flipped
             }
         }
 
@@ -305,7 +319,9 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
         // (every wave is past the barrier that ended stage - 1); the last iterations re-read the last
         // stage into an idle buffer: harmless, and the number of loads in flight stays the same
         fetch_scales(min(stage + 1, n_stages - 1));
-        fetch(min(stage + 2, n_stages - 1), buf == 0 ? 2 : buf - 1);
+        const int ahead = buf == 0 ? 2 : buf - 1;
+        if (kTwoW) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (this wave's units are in registers)
+        fetch(min(stage + 2, n_stages - 1), ahead, kTwoW ? wbuf : ahead);
 
         // Work units in order: (token block, group of the stage).  The MFMAs of unit u go into
         // accumulator set u & 1 and are written before the drain of unit u - 1, so the matrix core
@@ -360,6 +376,7 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
 
         land();
         buf = buf == kBufs - 1 ? 0 : buf + 1;
+        wbuf ^= 1;
     };
     if constexpr (kLong) {
         for (int stage = 0; stage < n_stages; stage += 2) {  // whole groups: an even number of stages
@@ -434,10 +451,10 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
         __syncthreads();
         if (tid == 0) {
             const unsigned prev = __hip_atomic_fetch_add(p.ws_counter + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            lds[0][0] = (prev == (unsigned)(n_split - 1));
+            lds[0] = (prev == (unsigned)(n_split - 1));
         }
         __syncthreads();
-        if (lds[0][0] == 0) return;
+        if (lds[0] == 0) return;
         // one split at a time, four token blocks' fragments in flight together (one memory latency per split and
         // half tile; all eight blocks at once would not fit the registers next to the running sums)
         constexpr int kChunk = 4;
@@ -489,7 +506,7 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
         if (!strip_ok) return;
         constexpr int kPitch = 68;
         static_assert(32 * kPitch * 4 * kStrips <= (int)sizeof(lds), "output staging exceeds the stage buffers");
-        float* stage_out = reinterpret_cast<float*>(&lds[0][0]) + wave * (32 * kPitch);
+        float* stage_out = reinterpret_cast<float*>(&lds[0]) + wave * (32 * kPitch);
         typedef float v4f_t __attribute__((ext_vector_type(4)));
 #pragma unroll
         for (int rd = 0; rd < kMB / 2; ++rd) {
@@ -550,14 +567,23 @@ template <int GS, bool SPLIT, bool ZP, typename OutT, bool DUMP = false>
 __global__ __launch_bounds__(256, 2) void tiled_kernel_w4(const GemmParams p) {
     tiled_body<64, GS, SPLIT, ZP, OutT, true, DUMP>(p);
 }
+// ... and 128-row tiles, two workgroups on a CU as well
+template <int GS, bool ZP, typename OutT>
+__global__ __launch_bounds__(256, 2) void tiled_kernel_w4_bm128(const GemmParams p) {
+    tiled_body<128, GS, false, ZP, OutT, true>(p);
+}
 
 template <bool DUMP>
 static hipError_t launch_tiled_w4_impl(const GemmParams& p, int gs, bool out_bf16, hipStream_t stream) {
-    const int tiles = (int)tiled_w4_tiles(p.M, p.strips);
+    const bool tall = !DUMP && p.split <= 1 && tiled_w4_tall(p.M, p.strips);
+    const int tiles = (int)tiled_w4_tiles(p.M, p.strips, tall ? 128 : 64);
     const dim3 grid((tiles + 7) / 8 * 8, p.split > 1 ? p.split : 1), block(256);
 #define SLIMK_W4_LAUNCH(GSV, ZPV)                                                                         \
     do {                                                                                                  \
-        if (p.split > 1) {                                                                                \
+        if (tall) {                                                                                       \
+            if (out_bf16) tiled_kernel_w4_bm128<GSV, ZPV, OutBF16><<<grid, block, 0, stream>>>(p);        \
+            else tiled_kernel_w4_bm128<GSV, ZPV, OutF16><<<grid, block, 0, stream>>>(p);                  \
+        } else if (p.split > 1) {                                                                                \
             if (out_bf16) tiled_kernel_w4<GSV, true, ZPV, OutBF16, DUMP><<<grid, block, 0, stream>>>(p);  \
             else tiled_kernel_w4<GSV, true, ZPV, OutF16, DUMP><<<grid, block, 0, stream>>>(p);            \
         } else {                                                                                          \
