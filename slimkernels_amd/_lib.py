@@ -6,6 +6,7 @@ fails, an exception is raised.
 import ctypes
 import os
 import subprocess
+import sys
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.path.join(_CSRC, "libslimk_w2a8.so")
@@ -81,8 +82,9 @@ class SlimkError(RuntimeError):
 
 
 def build(verbose=False):
-    """Compile the library in-tree with hipcc for gfx950 (cross-compiles without a GPU)."""
-    subprocess.run(["make", "-C", _CSRC, "-B", "-j8", "libslimk_w2a8.so"], check=True,
+    """Compile the library in-tree with hipcc for gfx950 (cross-compiles without a GPU), and the native host side of the
+    torch calls beside it."""
+    subprocess.run(["make", "-C", _CSRC, "-B", "-j8", f"PYTHON={sys.executable}", "libslimk_w2a8.so", "../torch/_native.so"], check=True,
                    stdout=None if verbose else subprocess.DEVNULL,
                    stderr=None if verbose else subprocess.DEVNULL)
     return LIB_PATH

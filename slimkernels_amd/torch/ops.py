@@ -29,9 +29,27 @@ from .. import _lib
 
 _DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 
+# The calls a model makes per token take the native host side (_native.cpp) where their tensors are plain; it returns None
+# for everything else, which the general code of each function below takes as it is.
+_fast = None
 
-# A decode call's kernel runs for 4-5 us, so what the host does around its launch decides how many calls a second one
-# process makes: the stream pointer and the current device come straight from torch's native accessors (0.2 us; building
+
+def _host():
+    """The native host side, bound to the loaded library.  As with the library itself there is no doing without it."""
+    global _fast
+    if _fast is None:
+        L = _lib.lib()
+        try:
+            from . import _native
+        except ImportError as e:
+            raise ImportError(f"slimkernels_amd/torch/_native.so is missing or does not load ({e}): build it with "
+                              "`python -c 'import __graft_entry__ as g; g.build()'`") from e
+        _native.bind({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in _lib.SIGNATURES}, _lib.check)
+        _fast = _native
+    return _fast
+
+
+# In the general code the stream pointer and the current device come straight from torch's native accessors (0.2 us; building
 # a Stream object and entering torch.cuda.device took 4 us a call), and the library's pure functions of the
 # shape are asked once per shape.  (None on a torch without GPU support, where no call gets as far as using them.)
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -189,6 +207,9 @@ def quantize_act_int8(x: torch.Tensor, group_size: int = 128, copies: int = 1, r
     rowsum [copies * G, ...]): the operand of a reduction over copies * K, as the 4-bit weights take it.
     ``rowsum=False`` leaves the group sums out (faster on many rows); only the tiled kernel on weights with the
     symmetric levels takes such an activation (see ``needs_rowsum``)."""
+    parts = (_fast or _host()).quantize(x, group_size, copies, rowsum)
+    if parts is not None:
+        return QuantizedActivation(*parts, group_size)
     L = _lib.lib()
     _require_cuda(x, "x")
     if x.dim() != 2 or x.dtype not in _DT:
@@ -235,6 +256,10 @@ def w2a8_gemm(qa: QuantizedActivation, w: W2A8Weight, out_dtype=torch.float16, *
               split_k: int = 0, dump: Optional[str] = None, out: Optional[torch.Tensor] = None):
     """out[M, N] = dequant( q @ (codes - zp)^T ).  Returns out, or (out, acc) when ``dump`` is
     "groups" (int32 [M, N, G]) or "sum" (int32 [M, N])."""
+    if kernel == "auto" and split_k == 0 and dump is None and out is None:
+        y = (_fast or _host()).gemm(qa, w, out_dtype)
+        if y is not None:
+            return y
     L = _lib.lib()
     kern = {"auto": _lib.KERNEL_AUTO, "skinny": _lib.KERNEL_SKINNY, "tiled": _lib.KERNEL_TILED, "mid": _lib.KERNEL_MID}[kernel]
     M, K = qa.q.shape
@@ -364,6 +389,10 @@ def w2a16_gemm(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *, split
     """The weight-only form: out[M, N] = x @ dequant(W)^T with the fp16 or bf16 activations x [M, K] as they are (no
     activation quantisation), the 2-bit codes widened in front of the fp16 resp. bf16 matrix cores, fp32 sums.
     Any number of token rows (above 32 a tiled kernel takes over where it is faster); K must be a multiple of 128."""
+    if split_k == 0 and out is None and x.dim() == 2:
+        y = (_fast or _host()).linear16(x, w, out_dtype)
+        if y is not None:
+            return y
     L = _lib.lib()
     _require_cuda(x, "x")
     if x.dim() != 2 or x.dtype not in _DT:
@@ -448,6 +477,10 @@ def w2a8_gemm_grouped(problems, out_dtype=torch.float16, *, dump: Optional[str] 
     share group size and zero-point mode; returns the list of outputs.  More than 24 problems are
     issued as several launches.  With ``dump`` ("groups" or "sum") the verification instantiation of
     the grouped kernel runs and (outputs, int32 accumulator tensors) is returned."""
+    if dump is None:
+        outs = (_fast or _host()).grouped(problems, out_dtype)
+        if outs is not None:
+            return outs
     L = _lib.lib()
     probs = [(p[0], p[1], p[2] if len(p) > 2 else None) for p in problems]
     if not probs:
@@ -567,6 +600,9 @@ class W2A8Linear(torch.nn.Module):
         return cls(load_w2_weight(path, device), bias, out_dtype)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = (_fast or _host()).linear(x, self.weight, self.out_dtype)
+        if y is not None and (self.bias is None or self.bias.dim() <= 1):
+            return y if self.bias is None else y + self.bias
         x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         if x2.dtype not in _DT:
             x2 = x2.to(self.out_dtype)
@@ -590,6 +626,9 @@ class W2A16Linear(W2A8Linear):
     weight-only kernels, for any number of token rows; the weight object and the constructors are W2A8Linear's."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = (_fast or _host()).linear16(x, self.weight, self.out_dtype)
+        if y is not None and (self.bias is None or self.bias.dim() <= 1):
+            return y if self.bias is None else y + self.bias
         x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         if x2.dtype not in _DT:
             x2 = x2.to(torch.float16)
