@@ -413,6 +413,36 @@ int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
                      void* out, int ldo, int out_dtype,
                      void* workspace, size_t workspace_bytes, int split_k, void* stream);
 
+/* The GEMMs with a layer's bias: `bias` is [N] of out_dtype, 16-byte aligned, or NULL (then they are the functions they
+ * are named after; slimk_w2a8_gemm_bias has no dump).  The output is rounded to out_dtype first and the sum with the bias
+ * rounded again, so the result is bit for bit that of an addition of two tensors of out_dtype behind the GEMM. */
+int slimk_w2a8_gemm_bias(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum, int ldr,
+                         const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                         int M, int N, int K, int group_size,
+                         void* out, int ldo, int out_dtype,
+                         void* workspace, size_t workspace_bytes,
+                         int kernel, int split_k, const void* bias, void* stream);
+int slimk_w2a8_gemm_fused_bias(const void* x, int ldx, int x_dtype,
+                               const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                               int M, int N, int K, int group_size,
+                               void* out, int ldo, int out_dtype,
+                               void* workspace, size_t workspace_bytes, int split_k, const void* bias, void* stream);
+int slimk_w2a8_linear_bias(const void* x, int ldx, int x_dtype,
+                           const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                           int M, int N, int K, int group_size,
+                           void* out, int ldo, int out_dtype,
+                           void* activations, size_t activation_bytes, void* workspace, size_t workspace_bytes, const void* bias, void* stream);
+int slimk_w4a8_gemm_bias(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum, int ldr,
+                         const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r,
+                         int M, int N, int K, int group_size,
+                         void* out, int ldo, int out_dtype,
+                         void* workspace, size_t workspace_bytes, int split_k, const void* bias, void* stream);
+int slimk_w2a16_gemm_bias(const void* x, int ldx, int x_dtype,
+                          const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                          int M, int N, int K, int group_size,
+                          void* out, int ldo, int out_dtype,
+                          void* workspace, size_t workspace_bytes, int split_k, const void* bias, void* stream);
+
 /* One problem of a grouped weight-only launch: the arguments of slimk_w2a16_gemm that describe data. */
 typedef struct slimk_w2a16_problem {
     const void* x;       /* [M][ldx] fp16 or bf16 (the launch's x_dtype) */

@@ -57,6 +57,11 @@ SIGNATURES = {
     "slimk_w2a16_gemm_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "slimk_w2a16_gemm": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _i, _i, _vp, _sz, _i, _vp]),
     "slimk_w2a16_gemm_grouped": (_i, [_vp, _i, _i, _i, _i, _vp]),
+    "slimk_w2a8_gemm_bias": (_i, [_vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _i, _i, _vp, _sz, _i, _i, _vp, _vp]),
+    "slimk_w2a8_gemm_fused_bias": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _i, _i, _vp, _sz, _i, _vp, _vp]),
+    "slimk_w2a8_linear_bias": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _i, _i, _vp, _sz, _vp, _sz, _vp, _vp]),
+    "slimk_w4a8_gemm_bias": (_i, [_vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _i, _i, _vp, _sz, _i, _vp, _vp]),
+    "slimk_w2a16_gemm_bias": (_i, [_vp, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _i, _i, _vp, _sz, _i, _vp, _vp]),
     "slimk_w2a8_read_probe": (_i, [_vp, _sz, _vp, _vp]),
 }
 MAX_GROUP = 24

@@ -57,6 +57,18 @@ int check_extent(int M, int N, int K, int ldq) {
     return SLIMK_OK;
 }
 
+// a bias [N] of the output's type: read eight channels at a time
+int check_bias(const void* bias) {
+    if (!aligned16(bias)) return fail(SLIMK_ERR_MISALIGNED, "bias must be 16-byte aligned");
+    return SLIMK_OK;
+}
+
+// the bias behind a GEMM whose kernel does not add it
+int bias_behind(int rc, void* out, int ldo, int M, int N, const void* bias, int out_dtype, void* stream) {
+    if (rc != SLIMK_OK || !bias) return rc;
+    return hip_result(w2a8::launch_add_bias(out, ldo, M, N, reinterpret_cast<const uint16_t*>(bias), out_dtype == SLIMK_BF16, (hipStream_t)stream), "bias");
+}
+
 bool shape_ok(int K, int group_size) {
     return K > 0 && K % 64 == 0 && (group_size == 64 || group_size == 128 || group_size == 256) &&
            K % group_size == 0;
@@ -426,7 +438,7 @@ int gemm_impl(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum,
               void* out, int ldo, int out_dtype,
               int32_t* acc_dump, int dump_mode,
               void* workspace, size_t workspace_bytes,
-              int kernel, int split_k, void* stream, bool fit_split) {
+              int kernel, int split_k, void* stream, bool fit_split, const void* bias = nullptr) {
     if (!q || !s_a || !w_r || !s_r || !out) return fail(SLIMK_ERR_NULL_POINTER, "gemm: NULL buffer");
     if (M <= 0 || N <= 0) return fail(SLIMK_ERR_BAD_SHAPE, "M=%d, N=%d must be positive", M, N);
     if (int rc = check_kg(K, group_size)) return rc;
@@ -448,6 +460,7 @@ int gemm_impl(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum,
         !aligned16(s_r) || (zp_r && !aligned16(zp_r)))
         return fail(SLIMK_ERR_MISALIGNED, "gemm: q, rowsum, w_r, s_r, zp_r must be 16-byte aligned; ldq %% 16 == 0; ldr %% 4 == 0");
     if ((reinterpret_cast<uintptr_t>(out) & 1u) != 0) return fail(SLIMK_ERR_MISALIGNED, "gemm: out must be 2-byte aligned");
+    if (int rc = check_bias(bias)) return rc;
 
     const int kern = resolve_kernel(M, N, K, group_size, kernel);
     if (kern == SLIMK_KERNEL_SKINNY && M > kSkinnyMaxRows)
@@ -489,7 +502,9 @@ int gemm_impl(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum,
 
     w2a8::GemmParams p{};
     p.q = q; p.s_a = s_a; p.rowsum = rowsum; p.w_r = w_r; p.s_r = s_r; p.zp_r = zp_r;
-    p.out = out; p.acc_dump = dump_mode != SLIMK_DUMP_NONE ? acc_dump : nullptr;
+    p.out = out;
+    if (dump_mode != SLIMK_DUMP_NONE) p.acc_dump = acc_dump;
+    else p.bias = reinterpret_cast<const uint16_t*>(bias);
     p.ldq = ldq; p.ldr = ldr; p.ldo = ldo;
     p.M = M; p.N = N; p.K = K; p.G = G; p.steps = K / w2a8::kStepK; p.strips = strips_of(N);
     p.zp_const = zp_const; p.dump_mode = dump_mode;
@@ -525,16 +540,18 @@ int gemm_impl(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum,
     const bool asym = zp_r != nullptr;
     const bool out_bf16 = out_dtype == SLIMK_BF16;
     // a call with a dump runs the verification instantiation of the kernel the same call without one would run
-    const bool dump = p.acc_dump != nullptr;
+    const bool dump = dump_mode != SLIMK_DUMP_NONE;
     if (kern == SLIMK_KERNEL_MID)
-        return hip_result(dump ? w2a8::launch_mid_verify(p, gs, asym, out_bf16, st) : w2a8::launch_mid(p, gs, asym, out_bf16, st), "mid gemm");
+        return bias_behind(hip_result(dump ? w2a8::launch_mid_verify(p, gs, asym, out_bf16, st) : w2a8::launch_mid(p, gs, asym, out_bf16, st), "mid gemm"),
+                           out, ldo, M, N, bias, out_dtype, stream);
     if (kern == SLIMK_KERNEL_SKINNY && skinny_shared_applies(M, N, K, group_size))
         return hip_result(dump ? w2a8::launch_skinny_shared_verify(p, gs, skinny_shared_parts(M, N), asym, out_bf16, st)
                                : w2a8::launch_skinny_shared(p, gs, skinny_shared_parts(M, N), asym, out_bf16, st), "shared skinny gemm");
     if (kern == SLIMK_KERNEL_SKINNY)
         return hip_result(dump ? w2a8::launch_skinny_verify(p, gs, skinny_waves(M, N, K, split_k), asym, out_bf16, st)
                                : w2a8::launch_skinny(p, gs, skinny_waves(M, N, K, split_k), asym, out_bf16, st), "skinny gemm");
-    return hip_result(w2a8::launch_tiled(p, gs, asym, out_bf16, st), "tiled gemm");
+    const int rc = hip_result(w2a8::launch_tiled(p, gs, asym, out_bf16, st), "tiled gemm");
+    return w2a8::output_rows_whole(out, ldo, N) ? rc : bias_behind(rc, out, ldo, M, N, bias, out_dtype, stream);
 }
 
 // ---- the library-owned split-K workspace of slimk_w2a8_gemm_static: a device array of fixed size, one copy per GPU
@@ -585,6 +602,16 @@ int slimk_w2a8_gemm(const int8_t* q, int ldq, const float* s_a, const int32_t* r
                     int kernel, int split_k, void* stream) {
     return gemm_impl(q, ldq, s_a, rowsum, ldr, w_r, s_r, zp_r, zp_const, M, N, K, group_size, out, ldo, out_dtype,
                      acc_dump, dump_mode, workspace, workspace_bytes, kernel, split_k, stream, false);
+}
+
+int slimk_w2a8_gemm_bias(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum, int ldr,
+                         const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                         int M, int N, int K, int group_size,
+                         void* out, int ldo, int out_dtype,
+                         void* workspace, size_t workspace_bytes,
+                         int kernel, int split_k, const void* bias, void* stream) {
+    return gemm_impl(q, ldq, s_a, rowsum, ldr, w_r, s_r, zp_r, zp_const, M, N, K, group_size, out, ldo, out_dtype,
+                     nullptr, SLIMK_DUMP_NONE, workspace, workspace_bytes, kernel, split_k, stream, false, bias);
 }
 
 size_t slimk_w2a8_static_workspace_bytes(void) { return kStaticWorkspaceBytes; }
@@ -680,11 +707,11 @@ int slimk_w2a8_linear_plan(int M, int N, int K, int group_size, int* tile_rows, 
     return SLIMK_OK;
 }
 
-int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
-                      const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
-                      int M, int N, int K, int group_size,
-                      void* out, int ldo, int out_dtype,
-                      void* activations, size_t activation_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+static int w2a8_linear_impl(const void* x, int ldx, int x_dtype,
+                            const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                            int M, int N, int K, int group_size,
+                            void* out, int ldo, int out_dtype,
+                            void* activations, size_t activation_bytes, void* workspace, size_t workspace_bytes, const void* bias, void* stream) {
     if (!x || !w_r || !s_r || !out || !activations) return fail(SLIMK_ERR_NULL_POINTER, "linear: NULL buffer");
     if (M <= 0 || N <= 0) return fail(SLIMK_ERR_BAD_SHAPE, "M=%d, N=%d must be positive", M, N);
     if (int rc = check_kg(K, group_size)) return rc;
@@ -699,6 +726,7 @@ int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
         return fail(SLIMK_ERR_MISALIGNED, "linear: x, w_r, s_r, zp_r, activations must be 16-byte aligned; ldx %% 8 == 0; out 2-byte aligned");
     if (activation_bytes < need_act)
         return fail(SLIMK_ERR_WORKSPACE, "activation scratch of %zu bytes is smaller than the %zu needed", activation_bytes, need_act);
+    if (int rc = check_bias(bias)) return rc;
     const w2a8::MxPlan plan = w2a8::mx_plan(M, N, K, group_size);
 
     char* const act = reinterpret_cast<char*>(activations);
@@ -707,7 +735,7 @@ int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
     float* cs = reinterpret_cast<float*>(act + mx_frag_bytes(M, K));
     float* s_a = reinterpret_cast<float*>(act + mx_frag_bytes(M, K) + mx_sums_bytes(M, K, group_size));
     p.frag = frag; p.cs = cs; p.s_a = s_a;
-    p.w_r = w_r; p.s_r = s_r; p.zp_r = zp_r; p.out = out; p.ldo = ldo;
+    p.w_r = w_r; p.s_r = s_r; p.zp_r = zp_r; p.out = out; p.ldo = ldo; p.bias = reinterpret_cast<const uint16_t*>(bias);
     p.M = M; p.N = N; p.K = K; p.G = K / group_size; p.steps = K / w2a8::kStepK; p.strips = strips_of(N);
     p.zp_const = zp_const; p.group_shift = group_size == 256 ? 1 : 0;
     p.split = plan.split; p.stages_per_split = plan.stages_per_split;
@@ -723,14 +751,33 @@ int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
     if (int rc = hip_result(w2a8::launch_mx_quant(x, ldx, x_dtype == SLIMK_BF16, M, K, group_size, zp_r ? 2 : zp_const, frag, cs, s_a,
                                                      p.ws_counter, p.ws_counter ? plan.tiles : 0, st), "linear quantisation"))
         return rc;
-    return hip_result(w2a8::launch_mx_gemm(p, plan.rb, group_size == 64 ? 1 : 2, out_dtype == SLIMK_BF16, st), "linear gemm");
+    const int rc = hip_result(w2a8::launch_mx_gemm(p, plan.rb, group_size == 64 ? 1 : 2, out_dtype == SLIMK_BF16, st), "linear gemm");
+    return w2a8::output_rows_whole(out, ldo, N) ? rc : bias_behind(rc, out, ldo, M, N, bias, out_dtype, stream);
 }
 
-int slimk_w2a8_gemm_fused(const void* x, int ldx, int x_dtype,
-                          const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
-                          int M, int N, int K, int group_size,
-                          void* out, int ldo, int out_dtype,
-                          void* workspace, size_t workspace_bytes, int split_k, void* stream) {
+int slimk_w2a8_linear(const void* x, int ldx, int x_dtype,
+                      const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                      int M, int N, int K, int group_size,
+                      void* out, int ldo, int out_dtype,
+                      void* activations, size_t activation_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+    return w2a8_linear_impl(x, ldx, x_dtype, w_r, s_r, zp_r, zp_const, M, N, K, group_size, out, ldo, out_dtype,
+                            activations, activation_bytes, workspace, workspace_bytes, nullptr, stream);
+}
+
+int slimk_w2a8_linear_bias(const void* x, int ldx, int x_dtype,
+                           const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                           int M, int N, int K, int group_size,
+                           void* out, int ldo, int out_dtype,
+                           void* activations, size_t activation_bytes, void* workspace, size_t workspace_bytes, const void* bias, void* stream) {
+    return w2a8_linear_impl(x, ldx, x_dtype, w_r, s_r, zp_r, zp_const, M, N, K, group_size, out, ldo, out_dtype,
+                            activations, activation_bytes, workspace, workspace_bytes, bias, stream);
+}
+
+static int w2a8_gemm_fused_impl(const void* x, int ldx, int x_dtype,
+                                const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                                int M, int N, int K, int group_size,
+                                void* out, int ldo, int out_dtype,
+                                void* workspace, size_t workspace_bytes, int split_k, const void* bias, void* stream) {
     if (!x || !w_r || !s_r || !out) return fail(SLIMK_ERR_NULL_POINTER, "gemm_fused: NULL buffer");
     if (M <= 0 || N <= 0) return fail(SLIMK_ERR_BAD_SHAPE, "M=%d, N=%d must be positive", M, N);
     if (int rc = check_kg(K, group_size)) return rc;
@@ -743,6 +790,7 @@ int slimk_w2a8_gemm_fused(const void* x, int ldx, int x_dtype,
     if (!aligned16(x) || ldx % 8 != 0 || !aligned16(w_r) || !aligned16(s_r) || (zp_r && !aligned16(zp_r)) ||
         (reinterpret_cast<uintptr_t>(out) & 1u))
         return fail(SLIMK_ERR_MISALIGNED, "gemm_fused: x, w_r, s_r, zp_r must be 16-byte aligned; ldx %% 8 == 0; out 2-byte aligned");
+    if (int rc = check_bias(bias)) return rc;
     const int G = K / group_size;
     const bool in_workgroup = fused_in_workgroup(M, K);
     if (split_k <= 0) split_k = in_workgroup ? auto_split(M, N, K, group_size, SLIMK_KERNEL_SKINNY) : skinny_plain_split(N, K, group_size);
@@ -752,7 +800,7 @@ int slimk_w2a8_gemm_fused(const void* x, int ldx, int x_dtype,
 
     w2a8::GemmParams p{};
     p.x = reinterpret_cast<const uint16_t*>(x); p.ldx = ldx; p.x_bf16 = x_dtype == SLIMK_BF16 ? 1 : 0;
-    p.w_r = w_r; p.s_r = s_r; p.zp_r = zp_r; p.out = out; p.ldo = ldo;
+    p.w_r = w_r; p.s_r = s_r; p.zp_r = zp_r; p.out = out; p.ldo = ldo; p.bias = reinterpret_cast<const uint16_t*>(bias);
     p.M = M; p.N = N; p.K = K; p.G = G; p.steps = K / w2a8::kStepK; p.strips = strips_of(N);
     p.zp_const = zp_const; p.split = split_k; p.groups_per_split = gps;
     if (!in_workgroup) {
@@ -791,6 +839,24 @@ int slimk_w2a8_gemm_fused(const void* x, int ldx, int x_dtype,
     return hip_result(w2a8::launch_skinny_fused(p, group_size / w2a8::kStepK, skinny_waves(M, N, K, split_k), zp_r != nullptr,
                                                 out_dtype == SLIMK_BF16, (hipStream_t)stream),
                       "fused skinny gemm");
+}
+
+int slimk_w2a8_gemm_fused(const void* x, int ldx, int x_dtype,
+                          const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                          int M, int N, int K, int group_size,
+                          void* out, int ldo, int out_dtype,
+                          void* workspace, size_t workspace_bytes, int split_k, void* stream) {
+    return w2a8_gemm_fused_impl(x, ldx, x_dtype, w_r, s_r, zp_r, zp_const, M, N, K, group_size, out, ldo, out_dtype,
+                                workspace, workspace_bytes, split_k, nullptr, stream);
+}
+
+int slimk_w2a8_gemm_fused_bias(const void* x, int ldx, int x_dtype,
+                               const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                               int M, int N, int K, int group_size,
+                               void* out, int ldo, int out_dtype,
+                               void* workspace, size_t workspace_bytes, int split_k, const void* bias, void* stream) {
+    return w2a8_gemm_fused_impl(x, ldx, x_dtype, w_r, s_r, zp_r, zp_const, M, N, K, group_size, out, ldo, out_dtype,
+                                workspace, workspace_bytes, split_k, bias, stream);
 }
 
 size_t slimk_w2a8_gemm_fused_workspace_bytes(int M, int N, int K, int group_size, int split_k) {
@@ -979,11 +1045,11 @@ size_t slimk_w4a8_gemm_workspace_bytes(int M, int N, int K, int group_size, int 
     return kCounterBlockBytes + (size_t)split_k * tiles * 64 * 256 * sizeof(float);
 }
 
-int slimk_w4a8_gemm(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum, int ldr,
+static int w4a8_gemm_impl(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum, int ldr,
                     const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r,
                     int M, int N, int K, int group_size,
                     void* out, int ldo, int out_dtype,
-                    void* workspace, size_t workspace_bytes, int split_k, void* stream) {
+                    void* workspace, size_t workspace_bytes, int split_k, const void* bias, void* stream) {
     if (!q || !s_a || !w_r || !s_r || !out) return fail(SLIMK_ERR_NULL_POINTER, "w4a8_gemm: NULL buffer");
     if (zp_r && !rowsum) return fail(SLIMK_ERR_NULL_POINTER, "w4a8_gemm: per-group zero-points need the row sums");
     if (M <= 0 || N <= 0) return fail(SLIMK_ERR_BAD_SHAPE, "M=%d, N=%d must be positive", M, N);
@@ -999,6 +1065,7 @@ int slimk_w4a8_gemm(const int8_t* q, int ldq, const float* s_a, const int32_t* r
     if (int rc = check_extent(M, N, 2 * K, ldq)) return rc;
     if (!aligned16(q) || ldq % 16 != 0 || !aligned16(w_r) || !aligned16(s_r) || (reinterpret_cast<uintptr_t>(out) & 1u))
         return fail(SLIMK_ERR_MISALIGNED, "w4a8_gemm: q, w_r, s_r must be 16-byte aligned; ldq %% 16 == 0; out 2-byte aligned");
+    if (int rc = check_bias(bias)) return rc;
     const int stages = K / (2 * w2a8::kStepK);
     if (split_k <= 0) split_k = w2a8::tiled_w4_auto_split(M, strips_of(N), K / w2a8::kStepK);
     if (split_k > stages) return fail(SLIMK_ERR_BAD_SHAPE, "split_k=%d exceeds the %d stages of 128 reduction elements", split_k, stages);
@@ -1009,7 +1076,7 @@ int slimk_w4a8_gemm(const int8_t* q, int ldq, const float* s_a, const int32_t* r
     if (split_k > 1) split_k = (stages + sps - 1) / sps;   // effective split: whole stages per split
 
     w2a8::GemmParams p{};
-    p.q = q; p.s_a = s_a; p.w_r = w_r; p.s_r = s_r; p.out = out; p.ldq = ldq; p.ldo = ldo;
+    p.q = q; p.s_a = s_a; p.w_r = w_r; p.s_r = s_r; p.out = out; p.ldq = ldq; p.ldo = ldo; p.bias = reinterpret_cast<const uint16_t*>(bias);
     p.zp_r = zp_r; p.rowsum = zp_r ? rowsum : nullptr; p.ldr = ldr;
     p.M = M; p.N = N; p.K = K; p.G = K / group_size; p.steps = K / w2a8::kStepK; p.strips = strips_of(N);
     p.zp_const = 2; p.split = split_k; p.groups_per_split = split_k > 1 ? sps * (128 / group_size) : p.G;
@@ -1022,7 +1089,26 @@ int slimk_w4a8_gemm(const int8_t* q, int ldq, const float* s_a, const int32_t* r
         p.ws_counter = reinterpret_cast<unsigned*>(workspace);
         p.ws_partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + kCounterBlockBytes);
     }
-    return hip_result(w2a8::launch_tiled_w4(p, group_size / w2a8::kStepK, out_dtype == SLIMK_BF16, (hipStream_t)stream), "w4a8_gemm");
+    const int rc = hip_result(w2a8::launch_tiled_w4(p, group_size / w2a8::kStepK, out_dtype == SLIMK_BF16, (hipStream_t)stream), "w4a8_gemm");
+    return w2a8::output_rows_whole(out, ldo, N) ? rc : bias_behind(rc, out, ldo, M, N, bias, out_dtype, stream);
+}
+
+int slimk_w4a8_gemm(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum, int ldr,
+                    const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r,
+                    int M, int N, int K, int group_size,
+                    void* out, int ldo, int out_dtype,
+                    void* workspace, size_t workspace_bytes, int split_k, void* stream) {
+    return w4a8_gemm_impl(q, ldq, s_a, rowsum, ldr, w_r, s_r, zp_r, M, N, K, group_size, out, ldo, out_dtype,
+                          workspace, workspace_bytes, split_k, nullptr, stream);
+}
+
+int slimk_w4a8_gemm_bias(const int8_t* q, int ldq, const float* s_a, const int32_t* rowsum, int ldr,
+                         const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r,
+                         int M, int N, int K, int group_size,
+                         void* out, int ldo, int out_dtype,
+                         void* workspace, size_t workspace_bytes, int split_k, const void* bias, void* stream) {
+    return w4a8_gemm_impl(q, ldq, s_a, rowsum, ldr, w_r, s_r, zp_r, M, N, K, group_size, out, ldo, out_dtype,
+                          workspace, workspace_bytes, split_k, bias, stream);
 }
 
 int slimk_w2a16_gemm_auto_split_k(int M, int N, int K, int group_size) {
@@ -1059,11 +1145,11 @@ size_t slimk_w2a16_gemm_workspace_bytes(int M, int N, int K, int group_size, int
     return (size_t)split_k * (size_t)M * (size_t)N * sizeof(float);
 }
 
-int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
-                     const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
-                     int M, int N, int K, int group_size,
-                     void* out, int ldo, int out_dtype,
-                     void* workspace, size_t workspace_bytes, int split_k, void* stream) {
+static int w2a16_gemm_impl(const void* x, int ldx, int x_dtype,
+                           const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                           int M, int N, int K, int group_size,
+                           void* out, int ldo, int out_dtype,
+                           void* workspace, size_t workspace_bytes, int split_k, const void* bias, void* stream) {
     if (!x || !w_r || !s_r || !out) return fail(SLIMK_ERR_NULL_POINTER, "w2a16_gemm: NULL buffer");
     if (M <= 0 || N <= 0) return fail(SLIMK_ERR_BAD_SHAPE, "M=%d, N=%d must be positive", M, N);
     if (int rc = check_kg(K, group_size)) return rc;
@@ -1076,6 +1162,7 @@ int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
     if (!aligned16(x) || ldx % 8 != 0 || !aligned16(w_r) || !aligned16(s_r) || (zp_r && !aligned16(zp_r)) ||
         (reinterpret_cast<uintptr_t>(out) & 1u))
         return fail(SLIMK_ERR_MISALIGNED, "w2a16_gemm: x, w_r, s_r, zp_r must be 16-byte aligned; ldx %% 8 == 0; out 2-byte aligned");
+    if (int rc = check_bias(bias)) return rc;
     const int gs = group_size / w2a8::kStepK, steps = K / w2a8::kStepK;
     const int granules = steps / (gs > 2 ? gs : 2);
     if (split_k <= 0)
@@ -1085,7 +1172,7 @@ int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
 
     w2a8::W2A16Params p{};
     p.x = reinterpret_cast<const uint16_t*>(x); p.ldx = ldx;
-    p.w_r = w_r; p.s_r = s_r; p.zp_r = zp_r; p.out = out; p.ldo = ldo;
+    p.w_r = w_r; p.s_r = s_r; p.zp_r = zp_r; p.out = out; p.ldo = ldo; p.bias = reinterpret_cast<const uint16_t*>(bias);
     p.M = M; p.N = N; p.K = K; p.G = K / group_size; p.steps = steps; p.strips = strips_of(N);
     p.zp_const = zp_const; p.split = split_k; p.x_bf16 = x_dtype == SLIMK_BF16;
     if (split_k > 1) {
@@ -1097,6 +1184,24 @@ int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
         p.ws = reinterpret_cast<float*>(workspace);
     }
     return hip_result(w2a8::launch_w2a16(p, gs, out_dtype == SLIMK_BF16, (hipStream_t)stream), "w2a16_gemm");
+}
+
+int slimk_w2a16_gemm(const void* x, int ldx, int x_dtype,
+                     const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                     int M, int N, int K, int group_size,
+                     void* out, int ldo, int out_dtype,
+                     void* workspace, size_t workspace_bytes, int split_k, void* stream) {
+    return w2a16_gemm_impl(x, ldx, x_dtype, w_r, s_r, zp_r, zp_const, M, N, K, group_size, out, ldo, out_dtype,
+                           workspace, workspace_bytes, split_k, nullptr, stream);
+}
+
+int slimk_w2a16_gemm_bias(const void* x, int ldx, int x_dtype,
+                          const uint32_t* w_r, const uint16_t* s_r, const uint8_t* zp_r, int zp_const,
+                          int M, int N, int K, int group_size,
+                          void* out, int ldo, int out_dtype,
+                          void* workspace, size_t workspace_bytes, int split_k, const void* bias, void* stream) {
+    return w2a16_gemm_impl(x, ldx, x_dtype, w_r, s_r, zp_r, zp_const, M, N, K, group_size, out, ldo, out_dtype,
+                           workspace, workspace_bytes, split_k, bias, stream);
 }
 
 int slimk_w2a16_gemm_grouped(const slimk_w2a16_problem* problems, int count, int group_size, int x_dtype, int out_dtype,

@@ -36,6 +36,7 @@
 #include <algorithm>
 
 #include "mx_launch.h"
+#include "w2a8_launch.h"
 
 namespace w2a8 {
 
@@ -189,8 +190,9 @@ __device__ __forceinline__ void unpack_unit(const v4i& raw, v4i (&b)[2]) {
 // 128 elements the activation fragments come into a three-slot LDS ring (LDS-direct, two stages ahead, shared by the
 // waves), the wave's own weight units and scales into two wave-private slots (a wave moves a stage's units to registers
 // before it asks for the units two stages on).
+// BIAS: p.bias is added to the rounded outputs (whole 16-byte output rows only; instantiations of their own, as in tiled_bodies.h)
 // GS = 64-element steps per drain: 1 (groups of 64) or 2 (128; groups of 256 drain twice with the same scale).
-template <int RB, int GS, bool SPLIT, bool ZP, int WGS, typename OutT>
+template <int RB, int GS, bool SPLIT, bool ZP, int WGS, typename OutT, bool BIAS>
 __device__ __forceinline__ void mx_body(const MxParams& p) {
     constexpr int kABytes = RB * kStageSteps * kFragBytes;       // 20 or 10 KiB
     constexpr int kALoads = (kABytes / 1024 + 3) / 4;            // LDS-direct loads of 1 KiB per wave and stage: 5 or 3
@@ -561,6 +563,8 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
     float* stage_out = reinterpret_cast<float*>(lds) + wave * (32 * kPitch);
     // the token scales, four rows a load, all in flight together (rows past M: zero, or what the scratch holds behind them)
     const __amdgpu_buffer_rsrc_t sa_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.s_a), 0, (p.M + 3) / 4 * 16, 0x00020000);
+    out8 bias8 = {0, 0, 0, 0};
+    if constexpr (BIAS) bias8 = *reinterpret_cast<const out8*>(p.bias + min(strip * kStripN + (lane & 7) * 8, p.N - 8));
     v4f sa4[RB][4];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
@@ -589,6 +593,7 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
                 v.y = (uint32_t)OutT::cast(lo.z) | ((uint32_t)OutT::cast(lo.w) << 16);
                 v.z = (uint32_t)OutT::cast(hi.x) | ((uint32_t)OutT::cast(hi.y) << 16);
                 v.w = (uint32_t)OutT::cast(hi.z) | ((uint32_t)OutT::cast(hi.w) << 16);
+                if constexpr (BIAS) v = add_bias8<OutT>(v, bias8);
                 const int m = m_tile + rb * 32 + row, n = strip * kStripN + cg * 8;
                 if (m < p.M && n < p.N) *reinterpret_cast<v4u*>(out + (size_t)m * p.ldo + n) = v;
             }
@@ -605,18 +610,24 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
 }
 
 // 128-row tiles: two workgroups per CU (80 KiB of LDS and 256 registers each); 64-row tiles two or three
-template <int RB, int GS, bool SPLIT, bool ZP, int WGS, typename OutT>
+template <int RB, int GS, bool SPLIT, bool ZP, int WGS, typename OutT, bool BIAS>
 __global__ __launch_bounds__(256, WGS) void mx_gemm_kernel(const MxParams p) {
-    mx_body<RB, GS, SPLIT, ZP, WGS, OutT>(p);
+    mx_body<RB, GS, SPLIT, ZP, WGS, OutT, BIAS>(p);
 }
 
 template <int RB, int GS, int WGS>
 void launch_rb_gs(const MxParams& p, bool out_bf16, dim3 grid, hipStream_t stream) {
     const dim3 block(256);
-#define SLIMK_MX_LAUNCH(SPLITV, ZPV)                                                                       \
-    do {                                                                                                   \
-        if (out_bf16) mx_gemm_kernel<RB, GS, SPLITV, ZPV, WGS, OutBF16><<<grid, block, 0, stream>>>(p);    \
-        else mx_gemm_kernel<RB, GS, SPLITV, ZPV, WGS, OutF16><<<grid, block, 0, stream>>>(p);              \
+    const bool biased = p.bias != nullptr && output_rows_whole(p.out, p.ldo, p.N);
+#define SLIMK_MX_LAUNCH_OUT(SPLITV, ZPV, OUT)                                                                  \
+    do {                                                                                                       \
+        if (biased) mx_gemm_kernel<RB, GS, SPLITV, ZPV, WGS, OUT, true><<<grid, block, 0, stream>>>(p);        \
+        else mx_gemm_kernel<RB, GS, SPLITV, ZPV, WGS, OUT, false><<<grid, block, 0, stream>>>(p);              \
+    } while (0)
+#define SLIMK_MX_LAUNCH(SPLITV, ZPV)                                  \
+    do {                                                              \
+        if (out_bf16) SLIMK_MX_LAUNCH_OUT(SPLITV, ZPV, OutBF16);      \
+        else SLIMK_MX_LAUNCH_OUT(SPLITV, ZPV, OutF16);                \
     } while (0)
     const bool zp = p.zp_r != nullptr;
     if (p.split > 1) {
@@ -627,6 +638,7 @@ void launch_rb_gs(const MxParams& p, bool out_bf16, dim3 grid, hipStream_t strea
         else SLIMK_MX_LAUNCH(false, false);
     }
 #undef SLIMK_MX_LAUNCH
+#undef SLIMK_MX_LAUNCH_OUT
 }
 
 }  // namespace

@@ -257,7 +257,11 @@ __device__ __forceinline__ void w2a16_body(const W2A16Params& p, const int unit,
         const int n = strip * kStripN + pp * 16 + col;
         if (strip_ok && m < p.M && n < p.N) {
             if (PARTIAL) p.ws[((size_t)split_idx * p.M + m) * p.N + n] = v;
-            else reinterpret_cast<uint16_t*>(p.out)[(size_t)m * p.ldo + n] = OutT::cast(v);
+            else {
+                uint16_t o = OutT::cast(v);
+                if (__builtin_expect(p.bias != nullptr, 0)) o = add_bias<OutT>(o, p.bias[n]);
+                reinterpret_cast<uint16_t*>(p.out)[(size_t)m * p.ldo + n] = o;
+            }
         }
     }
 }
@@ -293,7 +297,7 @@ __global__ __launch_bounds__(kWaves * 64, XBF && GS < 4 ? 4 : 1) void w2a16_grou
 // 300 x 4096 x 14336 call).
 template <typename OutT>
 __global__ __launch_bounds__(128) void w2a16_reduce_kernel(const float* __restrict__ ws, int split, int M, int N,
-                                                           uint16_t* __restrict__ out, int ldo) {
+                                                           uint16_t* __restrict__ out, int ldo, const uint16_t* __restrict__ bias) {
     const size_t total = (size_t)M * N;
     const int t = (int)(blockIdx.x * 128 + threadIdx.x);
     for (int m = (int)blockIdx.y; m < M; m += (int)gridDim.y) {
@@ -304,14 +308,23 @@ __global__ __launch_bounds__(128) void w2a16_reduce_kernel(const float* __restri
             v4f v = *reinterpret_cast<const v4f*>(src + t * 4);
 #pragma unroll 4
             for (int s = 1; s < split; ++s) v += *reinterpret_cast<const v4f*>(src + (size_t)s * total + t * 4);
+            uint16_t o[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) dst[t * 4 + i] = OutT::cast(v[i]);
+            for (int i = 0; i < 4; ++i) o[i] = OutT::cast(v[i]);
+            if (bias) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = add_bias<OutT>(o[i], bias[t * 4 + i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[t * 4 + i] = o[i];
         } else {
             for (int n = t; n < N; n += (int)gridDim.x * 128) {
                 float v = src[n];
 #pragma unroll 4
                 for (int s = 1; s < split; ++s) v += src[(size_t)s * total + n];
-                dst[n] = OutT::cast(v);
+                uint16_t o = OutT::cast(v);
+                if (bias) o = add_bias<OutT>(o, bias[n]);
+                dst[n] = o;
             }
         }
     }
@@ -423,9 +436,11 @@ hipError_t launch_w2a16(const W2A16Params& asked, int gs, bool out_bf16, hipStre
         const int per_thread = p.N % 4 == 0 ? 4 : 1;
         const dim3 blocks((unsigned)((p.N + 128 * per_thread - 1) / (128 * per_thread)), (unsigned)std::min(p.M, 32768));
         if (out_bf16)
-            w2a16_reduce_kernel<OutBF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo);
+            w2a16_reduce_kernel<OutBF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo, p.bias);
         else
-            w2a16_reduce_kernel<OutF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo);
+            w2a16_reduce_kernel<OutF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo, p.bias);
+    } else if (plan.rb && p.bias && !output_rows_whole(p.out, p.ldo, p.N)) {
+        return launch_add_bias(p.out, p.ldo, p.M, p.N, p.bias, out_bf16, stream);
     }
     return hipGetLastError();
 }

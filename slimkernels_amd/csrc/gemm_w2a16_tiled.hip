@@ -67,6 +67,7 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & (kStripsPerWg - 1);
     uint8_t* const lds = lds_all + kh * kLds;
     const int col = lane & 31, half = lane >> 5, c16 = lane & 15, sub = (lane >> 4) & 1;
+    const uint16_t* const bias = early_bias(p.bias);
     // token tiles of a channel tile next to each other on one XCD: they read the same weights
     const int tiles_n = (p.strips + kStripsPerWg - 1) / kStripsPerWg, tiles_m = (p.M + kBM - 1) / kBM;
     int n_tile, m_tile_i;
@@ -272,6 +273,8 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
     uint16_t* out = reinterpret_cast<uint16_t*>(p.out);
     const bool wide = (p.N & 7) == 0 && (p.ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
     float* stage_out = reinterpret_cast<float*>(lds) + wave * (32 * kPitch);
+    out8 bias8 = {0, 0, 0, 0};
+    if (__builtin_expect(bias != nullptr, 0)) bias8 = *reinterpret_cast<const out8*>(bias + min(strip * kStripN + (lane & 7) * 8, p.N - 8));
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
         if (wide) {
@@ -279,7 +282,8 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-                for (int j = 0; j < 16; ++j) stage_out[((j & 3) + 8 * (j >> 2) + 4 * half) * kPitch + nb * 32 + col] = t[rb][nb][j];
+                for (int j = 0; j < 16; ++j)
+                    stage_out[((j & 3) + 8 * (j >> 2) + 4 * half) * kPitch + nb * 32 + col] = t[rb][nb][j];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int row = i * 8 + (lane >> 3), cg = lane & 7;
@@ -290,6 +294,7 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
                 v.y = (uint32_t)OutT::cast(lo.z) | ((uint32_t)OutT::cast(lo.w) << 16);
                 v.z = (uint32_t)OutT::cast(hi.x) | ((uint32_t)OutT::cast(hi.y) << 16);
                 v.w = (uint32_t)OutT::cast(hi.z) | ((uint32_t)OutT::cast(hi.w) << 16);
+                if (__builtin_expect(bias != nullptr, 0)) v = add_bias8<OutT>(v, bias8);
                 const int m = m_tile + rb * 32 + row, n = strip * kStripN + cg * 8;
                 if (m < p.M && n < p.N) *reinterpret_cast<v4u*>(out + (size_t)m * p.ldo + n) = v;
             }

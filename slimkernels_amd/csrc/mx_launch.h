@@ -21,6 +21,7 @@ struct MxParams {
     const uint16_t* s_r;    // [G][strips][16][4] fp16 bits
     const uint8_t* zp_r;    // [G][strips][16][4] or nullptr
     void* out;              // [M][ldo] fp16 / bf16 bits
+    const uint16_t* bias;   // [N] in the output's type, added to the rounded outputs, or nullptr
     float* ws_partial;      // split-K partial tiles
     unsigned* ws_counter;   // arrival counters (the quantising kernel zeroes them)
     int ldo, M, N, K, G, steps, strips, zp_const;

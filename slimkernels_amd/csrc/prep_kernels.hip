@@ -1,4 +1,6 @@
 // Weight repack, activation quantisation, fill and read-probe kernels (gfx950).
+#include <algorithm>
+
 #include "w2a8_launch.h"
 
 namespace w2a8 {
@@ -302,6 +304,33 @@ hipError_t launch_act_quant(const void* x, int ldx, bool x_bf16, int M, int K, i
     else
         act_quant_kernel<false><<<dim3(act_quant_grid(M)), dim3(256), 0, stream>>>((const uint16_t*)x, ldx, M, K, group_size, q,
                                                                   ldq, s_a, rowsum, ldr, copies);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------ a bias behind a GEMM
+// Where a GEMM's epilogue does not add it: the many-rows kernels' 2-byte stores (N or row pitch no whole 16-byte pieces: the
+// addition there cost calls without a bias 1 to 3 % in registers and branches) and the kernel for 33..256 rows (its registers
+// are full).
+template <typename OutT>
+__global__ __launch_bounds__(256) void add_bias_kernel(uint16_t* __restrict__ out, int ldo, int M, int N, const uint16_t* __restrict__ bias) {
+    const int n = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (n >= N) return;
+    const uint16_t b = bias[n];
+    const int step = (int)gridDim.y * 4;
+    for (int m0 = (int)blockIdx.y * 4; m0 < M; m0 += step) {   // four rows' values in flight together
+        uint16_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = out[(size_t)min(m0 + i, M - 1) * ldo + n];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (m0 + i < M) out[(size_t)(m0 + i) * ldo + n] = add_bias<OutT>(v[i], b);
+    }
+}
+
+hipError_t launch_add_bias(void* out, int ldo, int M, int N, const uint16_t* bias, bool bf16, hipStream_t stream) {
+    const dim3 grid((unsigned)((N + 255) / 256), (unsigned)std::min((M + 3) / 4, 32768));
+    if (bf16) add_bias_kernel<OutBF16><<<grid, dim3(256), 0, stream>>>((uint16_t*)out, ldo, M, N, bias);
+    else add_bias_kernel<OutF16><<<grid, dim3(256), 0, stream>>>((uint16_t*)out, ldo, M, N, bias);
     return hipGetLastError();
 }
 

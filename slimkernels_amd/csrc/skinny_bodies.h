@@ -247,6 +247,7 @@ __device__ __forceinline__ void skinny_body(const GemmParams& p, const int strip
     const int tile_id = strip * mblocks + mblk;  // index of this (strip, row block) in the split-K workspace
 
     // token scales for the epilogue, fetched first
+    const uint16_t* const bias_at = DUMP ? nullptr : early_bias(p.bias);
     float sa[NWK == 1 ? MB * J : kOutPerThread];
     auto load_sa = [&]() {
         if (NWK == 1) {  // this wave stores D fragments itself: rows mb*16 + quad*4 + j
@@ -630,7 +631,13 @@ __device__ __forceinline__ void skinny_body(const GemmParams& p, const int strip
 
     constexpr float kUnscale[4] = {1.0f, 0.25f, 0.0625f, 0.015625f};  // 4^-p, exact
 
+    const bool biased = __builtin_expect(bias_at != nullptr, 0);   // (its values loaded here, under the meeting of the waves: the main loop's registers are full)
     if (NWK == 1) {  // the wave owns the strip's whole K range: store the D fragments directly
+        uint16_t bias[4] = {0, 0, 0, 0};
+        if (__builtin_expect(biased, 0)) {
+#pragma unroll
+            for (int pp = 0; pp < 4; ++pp) bias[pp] = bias_at[min(strip * kStripN + pp * 16 + col, p.N - 1)];
+        }
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -639,13 +646,18 @@ __device__ __forceinline__ void skinny_body(const GemmParams& p, const int strip
                 for (int j = 0; j < J; ++j) {
                     const int m = mb * 16 + quad * 4 + j;
                     const int n = strip * kStripN + pp * 16 + col;
-                    if (m < M && n < p.N)
-                        out[(size_t)m * p.ldo + n] = OutT::cast((t[mb][pp][j] * kUnscale[pp]) * sa[mb * J + j]);
+                    if (m < M && n < p.N) {
+                        uint16_t v = OutT::cast((t[mb][pp][j] * kUnscale[pp]) * sa[mb * J + j]);
+                        if (__builtin_expect(biased, 0)) v = add_bias<OutT>(v, bias[pp]);
+                        out[(size_t)m * p.ldo + n] = v;
+                    }
                 }
         return;
     }
 
     // ---- meet the workgroup's waves in LDS (the metadata area is dead once every wave is here)
+    uint16_t bias = 0;   // (a thread's outputs are of one channel)
+    if (__builtin_expect(biased, 0)) bias = bias_at[min(strip * kStripN + (tid & 63), p.N - 1)];
     __syncthreads();
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -666,7 +678,9 @@ __device__ __forceinline__ void skinny_body(const GemmParams& p, const int strip
                 float v = sm.red[0][m][nl];
 #pragma unroll
                 for (int w = 1; w < NWP; ++w) v += sm.red[w][m][nl];
-                out[(size_t)m * p.ldo + n] = OutT::cast(v * sa[i]);
+                uint16_t o = OutT::cast(v * sa[i]);
+                if (__builtin_expect(biased, 0)) o = add_bias<OutT>(o, bias);
+                out[(size_t)m * p.ldo + n] = o;
             }
         }
         return;
@@ -721,7 +735,11 @@ __device__ __forceinline__ void skinny_body(const GemmParams& p, const int strip
             for (int u = 0; u < 4; ++u)
                 if (sp0 + u < p.split) v += part[u];
         }
-        if (m < M && n < p.N) out[(size_t)m * p.ldo + n] = OutT::cast(v * sa[i]);
+        if (m < M && n < p.N) {
+            uint16_t o = OutT::cast(v * sa[i]);
+            if (__builtin_expect(biased, 0)) o = add_bias<OutT>(o, bias);
+            out[(size_t)m * p.ldo + n] = o;
+        }
     }
     if (tid == 0) __hip_atomic_store(p.ws_counter + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -825,6 +843,7 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
     uint16_t* const out = reinterpret_cast<uint16_t*>(p.out) + (size_t)m0 * p.ldo;
 
     // token scales for the epilogue, fetched first
+    const uint16_t* const bias_at = DUMP ? nullptr : early_bias(p.bias);
     float sa[NK == 1 && !SPLIT ? J : kOutPerThread];
     if (NK == 1 && !SPLIT) {
 #pragma unroll
@@ -1022,21 +1041,35 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
     }
 
     constexpr float kUnscale[4] = {1.0f, 0.25f, 0.0625f, 0.015625f};  // 4^-p, exact
+    const bool biased = __builtin_expect(bias_at != nullptr, 0);
     if (NK == 1 && !SPLIT) {
         if (active) {
+            uint16_t bias[4] = {0, 0, 0, 0};
+            if (__builtin_expect(biased, 0)) {
+#pragma unroll
+                for (int pp = 0; pp < 4; ++pp) bias[pp] = bias_at[min(strip * kStripN + pp * 16 + col, p.N - 1)];
+            }
 #pragma unroll
             for (int pp = 0; pp < 4; ++pp)
 #pragma unroll
                 for (int j = 0; j < J; ++j) {
                     const int m = quad * 4 + j;
                     const int n = strip * kStripN + pp * 16 + col;
-                    if (m < M && n < p.N) out[(size_t)m * p.ldo + n] = OutT::cast((t[pp][j] * kUnscale[pp]) * sa[j]);
+                    if (m < M && n < p.N) {
+                        uint16_t v = OutT::cast((t[pp][j] * kUnscale[pp]) * sa[j]);
+                        if (__builtin_expect(biased, 0)) v = add_bias<OutT>(v, bias[pp]);
+                        out[(size_t)m * p.ldo + n] = v;
+                    }
                 }
         }
         return;
     }
 
     // ---- the k-parts of each strip meet in LDS (the metadata area is dead once every wave is here)
+    uint16_t bias[kOutPerThread];
+#pragma unroll
+    for (int i = 0; i < kOutPerThread; ++i)
+        bias[i] = __builtin_expect(biased, 0) ? bias_at[min((unit * NS + min((tid + kThreads * i) / kLive, NS - 1)) * kStripN + (tid & 63), p.N - 1)] : (uint16_t)0;
     __syncthreads();
 #pragma unroll
     for (int pp = 0; pp < 4; ++pp)
@@ -1056,7 +1089,9 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
                 float v = sm.red[sidx][m][nl];
 #pragma unroll
                 for (int kp = 1; kp < NK; ++kp) v += sm.red[kp * NS + sidx][m][nl];
-                out[(size_t)m * p.ldo + n] = OutT::cast(v * sa[i]);
+                uint16_t o = OutT::cast(v * sa[i]);
+                if (__builtin_expect(biased, 0)) o = add_bias<OutT>(o, bias[i]);
+                out[(size_t)m * p.ldo + n] = o;
             }
         }
         return;
@@ -1119,7 +1154,11 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
         const int sidx = e / kLive, w = e % kLive;
         const int m = w >> 6, nl = w & 63;
         const int n = (unit * NS + sidx) * kStripN + nl;
-        if (eon[i] && m < M && n < p.N) out[(size_t)m * p.ldo + n] = OutT::cast(v[i] * sa[i]);
+        if (eon[i] && m < M && n < p.N) {
+            uint16_t o = OutT::cast(v[i] * sa[i]);
+            if (__builtin_expect(biased, 0)) o = add_bias<OutT>(o, bias[i]);
+            out[(size_t)m * p.ldo + n] = o;
+        }
     }
     if (tid == 0) __hip_atomic_store(p.ws_counter + counter_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

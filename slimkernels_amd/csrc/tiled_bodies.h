@@ -48,10 +48,12 @@ constexpr int kAQueue = 4;                                 // activation fragmen
 // steps .. 2*steps-1; s_r rows 0 .. G-1 = 4 * scale) with the uniform zero-point 8.  Both digits of a step are fetched
 // and put together before the MFMA: the operand byte 64 * (hi - 2) | 16 * lo is 16 * (code - 8), and the hi plane's
 // scale times the 1/64 of the 2-bit path is scale / 16: one pass over K instead of two over 2K.
+// BIAS: p.bias [N] is added to the rounded outputs, on whole 16-byte output rows only (instantiations of their own: as a branch in
+// one kernel it cost calls without a bias 1 us, 512 x 4096 x 14336 51.6 -> 52.7).
 // DUMP: verification instantiation of the same body: every per-group int32 accumulator is also written out (exactly,
 // as the MFMA left it, before its conversion to fp32); nothing else changes, so the output bits are the production
 // instantiation's.
-template <int BM, int GS, bool SPLIT, bool ZP, typename OutT, bool W4 = false, bool DUMP = false>
+template <int BM, int GS, bool SPLIT, bool ZP, typename OutT, bool W4 = false, bool DUMP = false, bool BIAS = false>
 __device__ __forceinline__ void tiled_body(const GemmParams& p) {
     using namespace fast;
     constexpr int kBM = BM;
@@ -508,6 +510,8 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
         static_assert(32 * kPitch * 4 * kStrips <= (int)sizeof(lds), "output staging exceeds the stage buffers");
         float* stage_out = reinterpret_cast<float*>(&lds[0]) + wave * (32 * kPitch);
         typedef float v4f_t __attribute__((ext_vector_type(4)));
+        out8 bias8 = {0, 0, 0, 0};
+        if constexpr (BIAS) bias8 = *reinterpret_cast<const out8*>(p.bias + min(strip * kStripN + (lane & 7) * 8, p.N - 8));
 #pragma unroll
         for (int rd = 0; rd < kMB / 2; ++rd) {
 #pragma unroll
@@ -527,6 +531,7 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
                 v.y = (uint32_t)OutT::cast(lo.z) | ((uint32_t)OutT::cast(lo.w) << 16);
                 v.z = (uint32_t)OutT::cast(hi.x) | ((uint32_t)OutT::cast(hi.y) << 16);
                 v.w = (uint32_t)OutT::cast(hi.z) | ((uint32_t)OutT::cast(hi.w) << 16);
+                if constexpr (BIAS) v = add_bias8<OutT>(v, bias8);
                 const int m = m_tile + rd * 32 + row, n = strip * kStripN + cg * 8;
                 if (m < p.M && n < p.N) *reinterpret_cast<v4u_t*>(out + (size_t)m * p.ldo + n) = v;
             }
@@ -553,42 +558,50 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
 
 // 128-row tiles: two workgroups (eight waves) per CU; 64-row tiles need fewer registers: three (two with a group of
 // 256, whose token blocks each keep a set of int32 accumulators).
-template <int GS, bool SPLIT, bool ZP, typename OutT, bool DUMP = false>
+template <int GS, bool SPLIT, bool ZP, typename OutT, bool DUMP, bool BIAS>
 __global__ __launch_bounds__(256, 2) void tiled_kernel(const GemmParams p) {
-    tiled_body<128, GS, SPLIT, ZP, OutT, false, DUMP>(p);
+    tiled_body<128, GS, SPLIT, ZP, OutT, false, DUMP, BIAS>(p);
 }
-template <int GS, bool SPLIT, bool ZP, typename OutT, bool DUMP = false>
+template <int GS, bool SPLIT, bool ZP, typename OutT, bool DUMP, bool BIAS>
 __global__ __launch_bounds__(256, DUMP || GS == 4 ? 2 : 3) void tiled_kernel_bm64(const GemmParams p) {
-    tiled_body<64, GS, SPLIT, ZP, OutT, false, DUMP>(p);
+    tiled_body<64, GS, SPLIT, ZP, OutT, false, DUMP, BIAS>(p);
 }
 
 // 4-bit weights, one pass (64-row tiles: three stage buffers of 24 KiB leave room for two workgroups on a CU)
-template <int GS, bool SPLIT, bool ZP, typename OutT, bool DUMP = false>
+template <int GS, bool SPLIT, bool ZP, typename OutT, bool DUMP, bool BIAS>
 __global__ __launch_bounds__(256, 2) void tiled_kernel_w4(const GemmParams p) {
-    tiled_body<64, GS, SPLIT, ZP, OutT, true, DUMP>(p);
+    tiled_body<64, GS, SPLIT, ZP, OutT, true, DUMP, BIAS>(p);
 }
 // ... and 128-row tiles, two workgroups on a CU as well
-template <int GS, bool ZP, typename OutT>
+template <int GS, bool ZP, typename OutT, bool DUMP, bool BIAS>
 __global__ __launch_bounds__(256, 2) void tiled_kernel_w4_bm128(const GemmParams p) {
-    tiled_body<128, GS, false, ZP, OutT, true>(p);
+    tiled_body<128, GS, false, ZP, OutT, true, DUMP, BIAS>(p);
 }
+
+// the instantiation with or without a bias (a verification launch has none)
+#define SLIMK_TILED_PICK(KERNEL, ...)                                                     \
+    do {                                                                                  \
+        if (biased) KERNEL<__VA_ARGS__, DUMP, !DUMP><<<grid, block, 0, stream>>>(p);      \
+        else KERNEL<__VA_ARGS__, DUMP, false><<<grid, block, 0, stream>>>(p);             \
+    } while (0)
 
 template <bool DUMP>
 static hipError_t launch_tiled_w4_impl(const GemmParams& p, int gs, bool out_bf16, hipStream_t stream) {
+    const bool biased = !DUMP && p.bias != nullptr && output_rows_whole(p.out, p.ldo, p.N);
     const bool tall = !DUMP && p.split <= 1 && tiled_w4_tall(p.M, p.strips);
     const int tiles = (int)tiled_w4_tiles(p.M, p.strips, tall ? 128 : 64);
     const dim3 grid((tiles + 7) / 8 * 8, p.split > 1 ? p.split : 1), block(256);
 #define SLIMK_W4_LAUNCH(GSV, ZPV)                                                                         \
     do {                                                                                                  \
         if (tall) {                                                                                       \
-            if (out_bf16) tiled_kernel_w4_bm128<GSV, ZPV, OutBF16><<<grid, block, 0, stream>>>(p);        \
-            else tiled_kernel_w4_bm128<GSV, ZPV, OutF16><<<grid, block, 0, stream>>>(p);                  \
+            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel_w4_bm128, GSV, ZPV, OutBF16);        \
+            else SLIMK_TILED_PICK(tiled_kernel_w4_bm128, GSV, ZPV, OutF16);                  \
         } else if (p.split > 1) {                                                                                \
-            if (out_bf16) tiled_kernel_w4<GSV, true, ZPV, OutBF16, DUMP><<<grid, block, 0, stream>>>(p);  \
-            else tiled_kernel_w4<GSV, true, ZPV, OutF16, DUMP><<<grid, block, 0, stream>>>(p);            \
+            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel_w4, GSV, true, ZPV, OutBF16);  \
+            else SLIMK_TILED_PICK(tiled_kernel_w4, GSV, true, ZPV, OutF16);            \
         } else {                                                                                          \
-            if (out_bf16) tiled_kernel_w4<GSV, false, ZPV, OutBF16, DUMP><<<grid, block, 0, stream>>>(p); \
-            else tiled_kernel_w4<GSV, false, ZPV, OutF16, DUMP><<<grid, block, 0, stream>>>(p);           \
+            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel_w4, GSV, false, ZPV, OutBF16); \
+            else SLIMK_TILED_PICK(tiled_kernel_w4, GSV, false, ZPV, OutF16);           \
         }                                                                                                 \
     } while (0)
     const bool zp = p.zp_r != nullptr;   // per-group zero-points: the planes' (rows 0..G-1 hi, G..2G-1 lo) and p.rowsum
@@ -622,24 +635,25 @@ static hipError_t launch_tiled_impl(const GemmParams& p, int gs, bool asym, bool
     const dim3 grid((tiles + 7) / 8 * 8, p.split > 1 ? p.split : 1), block(256);
     const bool zp = asym || p.zp_const != 2;
     const bool split = p.split > 1;
+    const bool biased = !DUMP && p.bias != nullptr && output_rows_whole(p.out, p.ldo, p.N);
 #define SLIMK_TILED_LAUNCH_BM64(GSV, ZPV)                                                                     \
     do {                                                                                                      \
         if (split) {                                                                                          \
-            if (out_bf16) tiled_kernel_bm64<GSV, true, ZPV, OutBF16, DUMP><<<grid, block, 0, stream>>>(p);    \
-            else tiled_kernel_bm64<GSV, true, ZPV, OutF16, DUMP><<<grid, block, 0, stream>>>(p);              \
+            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel_bm64, GSV, true, ZPV, OutBF16);    \
+            else SLIMK_TILED_PICK(tiled_kernel_bm64, GSV, true, ZPV, OutF16);              \
         } else {                                                                                              \
-            if (out_bf16) tiled_kernel_bm64<GSV, false, ZPV, OutBF16, DUMP><<<grid, block, 0, stream>>>(p);   \
-            else tiled_kernel_bm64<GSV, false, ZPV, OutF16, DUMP><<<grid, block, 0, stream>>>(p);             \
+            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel_bm64, GSV, false, ZPV, OutBF16);   \
+            else SLIMK_TILED_PICK(tiled_kernel_bm64, GSV, false, ZPV, OutF16);             \
         }                                                                                                     \
     } while (0)
 #define SLIMK_TILED_LAUNCH(GSV, ZPV)                                                                          \
     do {                                                                                                      \
         if (bm == 128 && split) {                                                                             \
-            if (out_bf16) tiled_kernel<GSV, true, ZPV, OutBF16, DUMP><<<grid, block, 0, stream>>>(p);         \
-            else tiled_kernel<GSV, true, ZPV, OutF16, DUMP><<<grid, block, 0, stream>>>(p);                   \
+            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel, GSV, true, ZPV, OutBF16);         \
+            else SLIMK_TILED_PICK(tiled_kernel, GSV, true, ZPV, OutF16);                   \
         } else if (bm == 128) {                                                                               \
-            if (out_bf16) tiled_kernel<GSV, false, ZPV, OutBF16, DUMP><<<grid, block, 0, stream>>>(p);        \
-            else tiled_kernel<GSV, false, ZPV, OutF16, DUMP><<<grid, block, 0, stream>>>(p);                  \
+            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel, GSV, false, ZPV, OutBF16);        \
+            else SLIMK_TILED_PICK(tiled_kernel, GSV, false, ZPV, OutF16);                  \
         } else {                                                                                              \
             SLIMK_TILED_LAUNCH_BM64(GSV, ZPV);                                                                \
         }                                                                                                     \

@@ -63,7 +63,10 @@ struct GemmParams {
     const uint16_t* s_r;    // [G][strips][16][4] fp16 bits
     const uint8_t* zp_r;    // [G][strips][16][4] or nullptr
     void* out;              // [M][ldo] fp16 / bf16 bits
-    int32_t* acc_dump;      // verification output or nullptr
+    union {                 // (one or the other: 24 problems of a grouped launch fit the kernel arguments)
+        int32_t* acc_dump;      // dump_mode != 0: verification output
+        const uint16_t* bias;   // dump_mode == 0: [N] in the output's type, added to the rounded outputs, or nullptr
+    };
     float* ws_partial;      // split-K partial tiles
     unsigned* ws_counter;   // split-K arrival counters (zero between calls)
     int ldq, ldr, ldo;
@@ -141,12 +144,14 @@ __device__ __forceinline__ void dump_group_sum(const GemmParams& p, int m, int n
 // The output is defined as cast(fp32 product): the empty asm keeps the compiler from folding the
 // caller's fp32 multiply into a v_fma_mixlo_f16, which would round the exact product once.
 struct OutF16 {
+    static __device__ __forceinline__ float widen(uint16_t v) { return half_bits_to_float(v); }
     static __device__ __forceinline__ uint16_t cast(float v) {
         asm volatile("" : "+v"(v));
         return __builtin_bit_cast(uint16_t, (_Float16)v);
     }
 };
 struct OutBF16 {
+    static __device__ __forceinline__ float widen(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
     static __device__ __forceinline__ uint16_t cast(float v) {
         uint32_t x = __float_as_uint(v);
         if ((x & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((x >> 16) | 0x40u);
@@ -154,6 +159,30 @@ struct OutBF16 {
         return (uint16_t)(x >> 16);
     }
 };
+
+// A layer's bias in the kernels' epilogues: the output is rounded, then the sum with the bias is, so the bits are those of
+// a separate addition of two tensors of the output's type (which reads and writes the output once more, and is a launch: 4 us
+// for 4 x 9312 outputs, 8 for 616 x 12120).  The int8 tiled kernels and the digit form have instantiations of their own for
+// it; in the few-rows and weight-only kernels it is a branch marked unlikely, so that its code lies behind the rest.
+template <typename OutT>
+__device__ __forceinline__ uint16_t add_bias(uint16_t out, uint16_t bias) {
+    return OutT::cast(OutT::widen(out) + OutT::widen(bias));
+}
+// The bias pointer as the kernel starts: asked of the arguments at the end of a workgroup instead, its scalar load is a round
+// trip of its own in front of the stores (half a microsecond of 57 x 20728 x 9216, when the tiled kernel had it there).
+__device__ __forceinline__ const uint16_t* early_bias(const uint16_t* bias) {
+    asm volatile("" : "+s"(bias));
+    return bias;
+}
+// eight consecutive channels of an output row in 16 bytes (bias 16-byte aligned, channel a multiple of eight)
+typedef unsigned out8 __attribute__((ext_vector_type(4)));
+template <typename OutT>
+__device__ __forceinline__ out8 add_bias8(out8 v, out8 b) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        v[i] = (uint32_t)add_bias<OutT>((uint16_t)v[i], (uint16_t)b[i]) | ((uint32_t)add_bias<OutT>((uint16_t)(v[i] >> 16), (uint16_t)(b[i] >> 16)) << 16);
+    return v;
+}
 
 // Placement of a one-dimensional grid on the eight XCDs.  Workgroups go to the XCDs in turn, so blockIdx.x & 7 names
 // the XCD and blockIdx.x >> 3 the workgroup's place in that XCD's queue.  The work is `sets` sets of `members`

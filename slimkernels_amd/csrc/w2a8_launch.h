@@ -25,6 +25,13 @@ hipError_t launch_quantize_weight(const void* w, int ldw, bool w_bf16, int N, in
 hipError_t launch_quantize_weight4(const void* w, int ldw, bool w_bf16, int N, int K, int group_size, bool asym,
                                    uint8_t* packed, int ldp, uint16_t* scales, uint8_t* zp, hipStream_t stream);
 
+// out[m][n] = rounded(out[m][n] + bias[n]) in the outputs' type.  output_rows_whole: rows of `out` are whole 16-byte pieces, which
+// is where the many-rows kernels add p.bias themselves.
+hipError_t launch_add_bias(void* out, int ldo, int M, int N, const uint16_t* bias, bool bf16, hipStream_t stream);
+inline bool output_rows_whole(const void* out, int ldo, int N) {
+    return N % 8 == 0 && ldo % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+}
+
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t stream);
 
 hipError_t launch_read_probe(const void* src, size_t bytes, uint32_t* sink, hipStream_t stream);
@@ -105,6 +112,7 @@ struct W2A16Params {
     const uint16_t* s_r;    // [G][strips][16][4] fp16 bits
     const uint8_t* zp_r;    // [G][strips][16][4] or nullptr
     void* out;              // [M][ldo] fp16 / bf16 bits
+    const uint16_t* bias;   // [N] in the output's type, added to the rounded outputs, or nullptr
     float* ws;              // [split][M][N] partial sums when split > 1
     int ldx, ldo;
     int M, N, K;

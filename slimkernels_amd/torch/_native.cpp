@@ -14,6 +14,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
@@ -32,10 +33,10 @@ namespace {
 
 // ---- the C ABI, bound by address from the library that slimkernels_amd._lib loaded
 #define SLIMK_FUNCTIONS(X)                                                                                              \
-    X(slimk_w2a8_act_quant_rep) X(slimk_w2a8_gemm) X(slimk_w2a8_gemm_workspace_bytes) X(slimk_w2a8_gemm_auto_route)     \
-    X(slimk_w2a8_gemm_fused) X(slimk_w2a8_gemm_fused_workspace_bytes) X(slimk_w2a8_linear) X(slimk_w2a8_linear_route)   \
+    X(slimk_w2a8_act_quant_rep) X(slimk_w2a8_gemm_bias) X(slimk_w2a8_gemm_workspace_bytes) X(slimk_w2a8_gemm_auto_route)     \
+    X(slimk_w2a8_gemm_fused_bias) X(slimk_w2a8_gemm_fused_workspace_bytes) X(slimk_w2a8_linear_bias) X(slimk_w2a8_linear_route)   \
     X(slimk_w2a8_linear_activation_bytes) X(slimk_w2a8_linear_workspace_bytes) X(slimk_w2a8_gemm_grouped)               \
-    X(slimk_w2a16_gemm) X(slimk_w2a16_gemm_workspace_bytes) X(slimk_w4a8_gemm) X(slimk_w4a8_gemm_workspace_bytes)
+    X(slimk_w2a16_gemm_bias) X(slimk_w2a16_gemm_workspace_bytes) X(slimk_w4a8_gemm_bias) X(slimk_w4a8_gemm_workspace_bytes)
 #define X(name) decltype(&name) p_##name = nullptr;
 SLIMK_FUNCTIONS(X)
 #undef X
@@ -169,6 +170,28 @@ struct Scratch {
 };
 size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
+// A layer's bias.  The kernels add one that is laid out for them and that no derivative is asked of; any other vector is added
+// behind the call, as `y + bias` does; the rest goes the general way.
+struct Bias {
+    Ref keep;
+    const void* p = nullptr;
+    bool behind = false;
+    bool of(PyObject* o, int N, int dtype, at::Device device) {
+        if (o == Py_None) return true;
+        if (!plain(o)) return false;
+        Py_INCREF(o);
+        keep.take(o);
+        const at::Tensor& t = tensor(keep);
+        if (t.dim() > 1) return false;
+        p = t.data_ptr();
+        behind = dtype_code(t.scalar_type()) != dtype || t.dim() != 1 || t.size(0) != N || (N > 1 && t.stride(0) != 1) || t.device() != device ||
+                 (reinterpret_cast<uintptr_t>(p) & 15) != 0 || (t.requires_grad() && c10::GradMode::is_enabled()) || t._fw_grad(0).defined();
+        if (behind) p = nullptr;
+        return true;
+    }
+    at::Tensor add(at::Tensor&& y) const { return behind ? at::add(y, tensor(keep)) : std::move(y); }
+};
+
 at::Tensor output(at::IntArrayRef sizes, int dtype, at::Device device) {
     return at::empty(sizes, at::TensorOptions().dtype(dtype_of(dtype)).device(device));
 }
@@ -181,8 +204,8 @@ at::Tensor output_like(PyObject* x, int N, int dtype, at::Device device) {
 
 PyObject* none() { Py_RETURN_NONE; }
 // a call's result, or the exception that slimkernels_amd._lib.check raises for the library's code
-PyObject* finish(int rc, at::Tensor&& out) {
-    if (rc == SLIMK_OK) return THPVariable_Wrap(std::move(out));
+PyObject* finish(int rc, at::Tensor&& out, const Bias* bias = nullptr) {
+    if (rc == SLIMK_OK) return THPVariable_Wrap(bias ? bias->add(std::move(out)) : std::move(out));
     Py_XDECREF(PyObject_CallFunction(g_check, "i", rc));
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "slimk_w2a8 call failed");
     return nullptr;
@@ -237,7 +260,7 @@ int zp_kind(const Weight& w) { return w.per_group() ? 2 : w.zp_const != 2; }
 
 // quantisation into scratch and the GEMM behind it
 int quantise_and_gemm(const Rows& x, const Weight& w, int copies, const Answer& a, bool one_pass_w4, const uint8_t* zp, at::Tensor& out,
-                      int odt, void* ws, size_t ws_bytes, hipStream_t stream) {
+                      int odt, const void* bias, void* ws, size_t ws_bytes, hipStream_t stream) {
     const int K = x.K * copies, ldr = (x.M + 3) / 4 * 4;
     const size_t q_bytes = rounded((size_t)x.M * K), s_bytes = rounded((size_t)x.M * 4);
     const size_t sum_bytes = a.sums ? rounded((size_t)copies * (x.K / w.group) * ldr * 4) : 0;
@@ -252,21 +275,22 @@ int quantise_and_gemm(const Rows& x, const Weight& w, int copies, const Answer& 
     Py_BEGIN_ALLOW_THREADS
     rc = p_slimk_w2a8_act_quant_rep(x.p, x.ld, x.dtype, x.M, x.K, w.group, copies, q, K, s_a, sums, ldr, stream);
     if (rc == SLIMK_OK)
-        rc = one_pass_w4 ? p_slimk_w4a8_gemm(q, K, s_a, zp ? sums : nullptr, ldr, w_r, s_r, zp, x.M, w.N, x.K, w.group, y, w.N, odt, ws,
-                                             ws_bytes, 0, stream)
-                         : p_slimk_w2a8_gemm(q, K, s_a, sums, ldr, w_r, s_r, zp, w.zp_const, x.M, w.N, K, w.group, y, w.N, odt, nullptr,
-                                             SLIMK_DUMP_NONE, ws, ws_bytes, SLIMK_KERNEL_AUTO, 0, stream);
+        rc = one_pass_w4 ? p_slimk_w4a8_gemm_bias(q, K, s_a, zp ? sums : nullptr, ldr, w_r, s_r, zp, x.M, w.N, x.K, w.group, y, w.N, odt, ws,
+                                                  ws_bytes, 0, bias, stream)
+                         : p_slimk_w2a8_gemm_bias(q, K, s_a, sums, ldr, w_r, s_r, zp, w.zp_const, x.M, w.N, K, w.group, y, w.N, odt, ws,
+                                                  ws_bytes, SLIMK_KERNEL_AUTO, 0, bias, stream);
     Py_END_ALLOW_THREADS
     return rc;
 }
 
-// linear(x, weight, out_dtype): W2A8Linear without its bias
+// linear(x, weight, out_dtype, bias): W2A8Linear
 PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Rows x;
     Weight w;
-    const int odt = n == 3 ? dtype_code(args[2]) : -1;
-    if (odt < 0 || modes() || !x.of(args[0]) || !w.of(args[1]) || x.K != w.K) return none();
+    Bias bias;
+    const int odt = n == 4 ? dtype_code(args[2]) : -1;
+    if (odt < 0 || modes() || !x.of(args[0]) || !w.of(args[1]) || x.K != w.K || !bias.of(args[3], w.N, odt, x.device)) return none();
     const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device.index()).stream();
     const Answer a = ask(kLinear, x.M, w.N, w.K, w.group, zp_kind(w));
     Ref keep;
@@ -281,7 +305,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const uint8_t* const zp = w.z();
         void* const y = out.data_ptr();
         Py_BEGIN_ALLOW_THREADS
-        rc = p_slimk_w2a8_gemm_fused(x.p, x.ld, x.dtype, w_r, s_r, zp, w.zp_const, 1, w.N, w.K, w.group, y, w.N, odt, ws, ws_bytes, 0, stream);
+        rc = p_slimk_w2a8_gemm_fused_bias(x.p, x.ld, x.dtype, w_r, s_r, zp, w.zp_const, 1, w.N, w.K, w.group, y, w.N, odt, ws, ws_bytes, 0,
+                                          bias.p, stream);
         Py_END_ALLOW_THREADS
     } else if (a.digits) {
         Scratch scratch(a.act + a.ws, stream);
@@ -290,23 +315,24 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const uint8_t* const zp = w.z();
         void* const y = out.data_ptr();
         Py_BEGIN_ALLOW_THREADS
-        rc = p_slimk_w2a8_linear(x.p, x.ld, x.dtype, w_r, s_r, zp, w.zp_const, x.M, w.N, w.K, w.group, y, w.N, odt, scratch.p, a.act,
-                                 a.ws ? scratch.p + a.act : nullptr, a.ws, stream);
+        rc = p_slimk_w2a8_linear_bias(x.p, x.ld, x.dtype, w_r, s_r, zp, w.zp_const, x.M, w.N, w.K, w.group, y, w.N, odt, scratch.p, a.act,
+                                 a.ws ? scratch.p + a.act : nullptr, a.ws, bias.p, stream);
         Py_END_ALLOW_THREADS
     } else {
-        rc = quantise_and_gemm(x, w, 1, a, false, w.z(), out, odt, ws, ws_bytes, stream);
+        rc = quantise_and_gemm(x, w, 1, a, false, w.z(), out, odt, bias.p, ws, ws_bytes, stream);
     }
-    return finish(rc, std::move(out));
+    return finish(rc, std::move(out), &bias);
     END_HANDLE_TH_ERRORS
 }
 
-// linear16(x, weight, out_dtype): ops.w2a16_gemm with its own choice of a split; x of any number of dimensions
+// linear16(x, weight, out_dtype, bias): W2A16Linear (ops.w2a16_gemm with its own choice of a split)
 PyObject* linear16(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Rows x;
     Weight w;
-    const int odt = n == 3 ? dtype_code(args[2]) : -1;
-    if (odt < 0 || modes() || !x.of(args[0]) || !w.of(args[1]) || x.K != w.K) return none();
+    Bias bias;
+    const int odt = n == 4 ? dtype_code(args[2]) : -1;
+    if (odt < 0 || modes() || !x.of(args[0]) || !w.of(args[1]) || x.K != w.K || !bias.of(args[3], w.N, odt, x.device)) return none();
     const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device.index()).stream();
     const Answer a = ask(kW2A16, x.M, w.N, w.K, w.group, 0);
     at::Tensor out = output_like(args[0], w.N, odt, x.device);
@@ -317,24 +343,27 @@ PyObject* linear16(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void* const y = out.data_ptr();
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = p_slimk_w2a16_gemm(x.p, x.ld, x.dtype, w_r, s_r, zp, w.zp_const, x.M, w.N, w.K, w.group, y, w.N, odt, scratch.p, a.ws, 0, stream);
+    rc = p_slimk_w2a16_gemm_bias(x.p, x.ld, x.dtype, w_r, s_r, zp, w.zp_const, x.M, w.N, w.K, w.group, y, w.N, odt, scratch.p, a.ws, 0,
+                                 bias.p, stream);
     Py_END_ALLOW_THREADS
-    return finish(rc, std::move(out));
+    return finish(rc, std::move(out), &bias);
     END_HANDLE_TH_ERRORS
 }
 
-// linear4(x, weight, out_dtype): W4A8Linear without its bias (w4.w4a8_linear), more than one token row
+// linear4(x, weight, out_dtype, bias): W4A8Linear (w4.w4a8_linear) on more than one token row
 PyObject* linear4(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Rows x;
     Weight w;
     Ref planes, uniform;
     int N, K, group;
-    const int odt = n == 3 ? dtype_code(args[2]) : -1;
+    Bias bias;
+    const int odt = n == 4 ? dtype_code(args[2]) : -1;
     if (odt < 0 || modes() || !x.of(args[0]) || x.M == 1 || !get(args[1], n_planes, planes) || !w.of(planes.p) || !get_int(args[1], n_N, N) ||
         !get_int(args[1], n_K, K) || !get_int(args[1], n_group_size, group) || !get(args[1], n_uniform_zp8, uniform) || !PyBool_Check(uniform.p))
         return none();
-    if (x.K != K || w.N != N || w.K != 2 * K || w.group != group || K % group != 0 || !w.per_group()) return none();
+    if (x.K != K || w.N != N || w.K != 2 * K || w.group != group || K % group != 0 || !w.per_group() || !bias.of(args[3], N, odt, x.device))
+        return none();
     const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device.index()).stream();
     const bool one_pass = x.M >= 33 && K % 128 == 0 && (group == 64 || group == 128);   // (w4.one_pass_applies)
     Answer a = one_pass ? ask(kW4, x.M, N, K, group, 0) : ask(kGemm, x.M, N, 2 * K, group, zp_kind(w));
@@ -345,7 +374,8 @@ PyObject* linear4(PyObject*, PyObject* const* args, Py_ssize_t n) {
     size_t ws_bytes;
     if (!workspace(planes.p, stream, a.ws, keep, ws, ws_bytes)) return none();
     at::Tensor out = output_like(args[0], N, odt, x.device);
-    return finish(quantise_and_gemm(x, w, one_pass ? 1 : 2, a, one_pass, zp, out, odt, ws, ws_bytes, stream), std::move(out));
+    const int rc = quantise_and_gemm(x, w, one_pass ? 1 : 2, a, one_pass, zp, out, odt, bias.p, ws, ws_bytes, stream);
+    return finish(rc, std::move(out), &bias);
     END_HANDLE_TH_ERRORS
 }
 
@@ -423,8 +453,8 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void* const y = out.data_ptr();
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = p_slimk_w2a8_gemm(q, x.ldq, s_a, sums, x.ldr, w_r, s_r, zp, w.zp_const, x.M, w.N, w.K, w.group, y, w.N, odt, nullptr, SLIMK_DUMP_NONE,
-                           ws, ws_bytes, SLIMK_KERNEL_AUTO, 0, stream);
+    rc = p_slimk_w2a8_gemm_bias(q, x.ldq, s_a, sums, x.ldr, w_r, s_r, zp, w.zp_const, x.M, w.N, w.K, w.group, y, w.N, odt, ws, ws_bytes,
+                                SLIMK_KERNEL_AUTO, 0, nullptr, stream);
     Py_END_ALLOW_THREADS
     return finish(rc, std::move(out));
     END_HANDLE_TH_ERRORS
@@ -517,9 +547,9 @@ constexpr PyCFunction fast() { return reinterpret_cast<PyCFunction>(reinterpret_
 
 PyMethodDef g_methods[] = {
     {"bind", fast<bind>(), METH_FASTCALL, "bind(addresses, check)"},
-    {"linear", fast<linear>(), METH_FASTCALL, "linear(x, weight, out_dtype) -> tensor, or None for the general path"},
-    {"linear16", fast<linear16>(), METH_FASTCALL, "linear16(x, weight, out_dtype) -> tensor or None"},
-    {"linear4", fast<linear4>(), METH_FASTCALL, "linear4(x, weight, out_dtype) -> tensor or None"},
+    {"linear", fast<linear>(), METH_FASTCALL, "linear(x, weight, out_dtype, bias) -> tensor, or None for the general path"},
+    {"linear16", fast<linear16>(), METH_FASTCALL, "linear16(x, weight, out_dtype, bias) -> tensor or None"},
+    {"linear4", fast<linear4>(), METH_FASTCALL, "linear4(x, weight, out_dtype, bias) -> tensor or None"},
     {"quantize", fast<quantize>(), METH_FASTCALL, "quantize(x, group_size, copies, rowsum) -> (q, s_a, rowsum) or None"},
     {"gemm", fast<gemm>(), METH_FASTCALL, "gemm(qa, weight, out_dtype) -> tensor or None"},
     {"grouped", fast<grouped>(), METH_FASTCALL, "grouped(problems, out_dtype) -> list of tensors or None"},

@@ -390,7 +390,7 @@ def w2a16_gemm(x: torch.Tensor, w: W2A8Weight, out_dtype=torch.float16, *, split
     activation quantisation), the 2-bit codes widened in front of the fp16 resp. bf16 matrix cores, fp32 sums.
     Any number of token rows (above 32 a tiled kernel takes over where it is faster); K must be a multiple of 128."""
     if split_k == 0 and out is None and x.dim() == 2:
-        y = (_fast or _host()).linear16(x, w, out_dtype)
+        y = (_fast or _host()).linear16(x, w, out_dtype, None)
         if y is not None:
             return y
     L = _lib.lib()
@@ -600,9 +600,9 @@ class W2A8Linear(torch.nn.Module):
         return cls(load_w2_weight(path, device), bias, out_dtype)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        y = (_fast or _host()).linear(x, self.weight, self.out_dtype)
-        if y is not None and (self.bias is None or self.bias.dim() <= 1):
-            return y if self.bias is None else y + self.bias
+        y = (_fast or _host()).linear(x, self.weight, self.out_dtype, self.bias)
+        if y is not None:
+            return y
         x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         if x2.dtype not in _DT:
             x2 = x2.to(self.out_dtype)
@@ -626,9 +626,9 @@ class W2A16Linear(W2A8Linear):
     weight-only kernels, for any number of token rows; the weight object and the constructors are W2A8Linear's."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        y = (_fast or _host()).linear16(x, self.weight, self.out_dtype)
-        if y is not None and (self.bias is None or self.bias.dim() <= 1):
-            return y if self.bias is None else y + self.bias
+        y = (_fast or _host()).linear16(x, self.weight, self.out_dtype, self.bias)
+        if y is not None:
+            return y
         x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         if x2.dtype not in _DT:
             x2 = x2.to(torch.float16)

@@ -216,9 +216,9 @@ class W4A8Linear(torch.nn.Module):
         return cls(repack_w4(packed4, scales, zero, group_size, device=device), bias, out_dtype)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        y = (ops._fast or ops._host()).linear4(x, self.weight, self.out_dtype)
-        if y is not None and (self.bias is None or self.bias.dim() <= 1):
-            return y if self.bias is None else y + self.bias
+        y = (ops._fast or ops._host()).linear4(x, self.weight, self.out_dtype, self.bias)
+        if y is not None:
+            return y
         x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         if x2.dtype not in _DT:
             x2 = x2.to(self.out_dtype)

@@ -23,9 +23,9 @@ def test_cpu_tensors_and_other_objects_are_left_to_the_general_code():
     host = ops._host()
     x = torch.zeros((2, 128), dtype=torch.float16)
     w = ops.W2A8Weight(x, x, None, 2, 64, 128, 128)
-    assert host.linear(x, w, torch.float16) is None and host.linear16(x, w, torch.float16) is None
-    assert host.linear(None, w, torch.float16) is None and host.linear(x, w, "float16") is None and host.linear(x, w) is None
-    assert host.linear4(x, object(), torch.float16) is None and host.gemm(object(), w, torch.float16) is None
+    assert host.linear(x, w, torch.float16, None) is None and host.linear16(x, w, torch.float16, None) is None
+    assert host.linear(None, w, torch.float16, None) is None and host.linear(x, w, "float16", None) is None and host.linear(x, w) is None
+    assert host.linear4(x, object(), torch.float16, None) is None and host.gemm(object(), w, torch.float16) is None
     assert host.quantize(x, 128, 1, True) is None and host.quantize(3, 128, 1, True) is None
     assert host.grouped([], torch.float16) is None and host.grouped([(x, w)], torch.float16) is None
     assert host.grouped(iter([]), torch.float16) is None
@@ -62,12 +62,12 @@ def test_layers(gpu_ops, monkeypatch, kind, lead, N, K, g, mode, out, bias):
     want = _without_native(monkeypatch, lambda: layer(x))
     call = {"2": ops._host().linear, "4": ops._host().linear4, "16": ops._host().linear16}[kind]
     rows = x.numel() // K
-    y = call(x, layer.weight, dtype)
+    y = call(x, layer.weight, dtype, b)
     if kind == "4" and rows == 1:
         assert y is None                                       # (the row is laid down twice by the general code)
     else:
         assert y.shape == (*lead, N) and y.dtype == dtype and y.is_contiguous()
-        assert torch.equal(y if b is None else y + b, want)
+        assert torch.equal(y, want)
     assert torch.equal(layer(x), want)
     # layouts: rows of a wider tensor are read in place; what is not laid out for the kernels goes the general way
     x2 = x.reshape(-1, K)
@@ -77,16 +77,82 @@ def test_layers(gpu_ops, monkeypatch, kind, lead, N, K, g, mode, out, bias):
     odd[:, 1:] = x2
     for t, taken in ((wide[:, :K], not (kind == "4" and rows == 1)), (odd[:, 1:], False), (x2.t().contiguous().t(), rows == 1 and kind != "4")):
         if rows == 1 and t.stride(0) % 8:
-            assert call(t, layer.weight, dtype) is None        # (one row at an odd pitch: refused by both)
+            assert call(t, layer.weight, dtype, b) is None        # (one row at an odd pitch: refused by both)
             continue
-        assert (call(t, layer.weight, dtype) is not None) == taken
+        assert (call(t, layer.weight, dtype, b) is not None) == taken
         assert torch.equal(layer(t), want.reshape(-1, N))
-    assert call(x.float(), layer.weight, dtype) is None and call(x, layer.weight, torch.float32) is None
-    assert call(x[..., :K - 128], layer.weight, dtype) is None
+    assert call(x.float(), layer.weight, dtype, b) is None and call(x, layer.weight, torch.float32, b) is None
+    assert call(x[..., :K - 128], layer.weight, dtype, b) is None
     with pytest.raises(ValueError):
         layer(x[..., :K - 128])
     sub = x.as_subclass(type("Sub", (torch.Tensor,), {}))
-    assert call(sub, layer.weight, dtype) is None
+    assert call(sub, layer.weight, dtype, b) is None
+
+
+# every kernel that a layer call can end in, with and without whole 16-byte output rows (the W4 layer's K is the planes' half)
+BIASED = [("2", 1, 4096, 4096, 128, "sym"), ("2", 1, 1001, 16384, 64, "asym"), ("2", 3, 33000, 512, 64, "sym"), ("2", 14, 24640, 1024, 128, "asym"),
+          ("2", 16, 520, 14336, 256, "sym"), ("2", 24, 12288, 8192, 128, "sym"), ("2", 40, 28672, 4608, 64, "sym"), ("2", 80, 11009, 14336, 128, "asym"),
+          ("2", 60, 11008, 4096, 128, "asym"), ("2", 200, 1000, 4096, 128, "sym"), ("2", 600, 4100, 1024, 256, "asym"), ("2", 1025, 14600, 256, 128, "sym"),
+          ("2", 300, 4096, 8192, 128, "asym"), ("2", 520, 16640, 4096, 64, "sym"), ("2", 1025, 14601, 512, 128, "asym"),
+          ("16", 1, 14336, 4096, 128, "sym"), ("16", 6, 1001, 9216, 64, "asym"), ("16", 300, 4096, 8192, 128, "sym"), ("16", 700, 11009, 2048, 128, "asym"),
+          ("16", 1024, 14336, 1024, 128, "sym"), ("4", 1, 520, 2048, 128, "asym"), ("4", 20, 1001, 4096, 128, "sym"), ("4", 100, 1000, 4096, 64, "asym"),
+          ("4", 1000, 14408, 256, 128, "sym")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("out", ["float16", "bfloat16"])
+@pytest.mark.parametrize("kind,M,N,K,g,mode", BIASED)
+def test_bias_in_the_kernels(gpu_ops, kind, M, N, K, g, mode, out):
+    """Bit for bit the sum of two tensors, for values that round, vanish beside each other, overflow or are no numbers."""
+    print(f"bias {kind} M={M} N={N} K={K} g={g} {mode} {out}", flush=True)
+    dtype = getattr(torch, out)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + N + K)
+    weight = torch.randn((N, K), generator=gen, device="cuda", dtype=torch.float16) * 0.02
+    layer = LAYERS[kind].from_float(weight, g, mode, out_dtype=dtype)
+    x = torch.randn((M, K), generator=gen, device="cuda").to(dtype)
+    plain = layer(x)
+    b = (torch.randn((N,), generator=gen, device="cuda") * 2.0 ** torch.randint(-12, 8, (N,), generator=gen, device="cuda")).to(dtype)
+    b[:8] = torch.tensor([0.0, -0.0, float("inf"), float("-inf"), float("nan"), torch.finfo(dtype).max, torch.finfo(dtype).min, 1.0], dtype=dtype)
+    b[8:16] = -plain[0, 8:16]
+    want = plain + b
+    layer.bias = b
+    got = layer(x)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got.nan_to_num(0.0).view(torch.int16), want.nan_to_num(0.0).view(torch.int16))
+
+
+@pytest.mark.gpu
+def test_biases_that_the_kernels_do_not_add(gpu_ops):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    layer = gpu_ops.W2A8Linear.from_float(torch.randn((320, 512), generator=gen, device="cuda", dtype=torch.float16), 64, "sym")
+    x = torch.randn((4, 512), generator=gen, device="cuda", dtype=torch.float16)
+    plain = layer(x)
+    b = torch.randn((400,), generator=gen, device="cuda", dtype=torch.float16)
+    for bias in (b[1:321], b[:320].float(), torch.randn((640,), generator=gen, device="cuda", dtype=torch.float16)[::2], b[:1], b[0],
+                 b[:320].bfloat16(), b[:320].expand(4, 320), torch.randn((4, 1), device="cuda", dtype=torch.float16)):
+        layer.bias = bias
+        got, want = layer(x), plain + bias
+        assert got.dtype == want.dtype and torch.equal(got, want)
+    # a derivative is asked of it
+    p = torch.nn.Parameter(b[:320].clone())
+    layer.bias = p
+    y = layer(x)
+    assert y.requires_grad and torch.equal(y, plain + p)
+    y.sum().backward()
+    assert torch.equal(p.grad, torch.full_like(p, 4.0))
+    with torch.no_grad():
+        assert not layer(x).requires_grad and torch.equal(layer(x), plain + p)
+    import torch.autograd.forward_ad as fwd
+    with fwd.dual_level(), torch.no_grad():
+        layer.bias = None
+        del layer.bias
+        layer.bias = fwd.make_dual(b[:320].clone(), torch.ones_like(b[:320]))
+        assert torch.equal(fwd.unpack_dual(layer(x)).tangent, torch.ones_like(plain))
+    layer.bias = b[:300]
+    with pytest.raises(RuntimeError):
+        layer(x)
 
 
 @pytest.mark.gpu
