@@ -56,67 +56,70 @@ typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 constexpr int kFp6 = 2, kFp4 = 4;          // operand formats of the f8f6f4 instructions
 constexpr int kScaleOne = 127, kScale4 = 129;   // 2^(x - 127)
 
-// ---- activations: per-token quantisation straight into digit fragments.  One row per workgroup, 32 elements per
-// thread (an fp6 conversion takes 32), the row read once, whole cache lines at a time: a thread's 64 bytes are four
-// lines' worth of address work per lane otherwise, so the row turns through LDS, its 16-byte pieces rotated by c / 16
-// inside each set of four (the readers' pieces then lie in all banks).  The quotients are those of
-// act_quant_keep_kernel, bit for bit.  32 consecutive rows go to one XCD, so that the 16-byte pieces of a fragment meet
-// in one L2.
-template <bool BF16>
+// ---- activations: per-token quantisation straight into digit fragments.  R rows per workgroup, 32 elements per thread (an
+// fp6 conversion takes 32), R neighbouring lanes on the same elements of R rows: their pieces of a fragment are 16 * R bytes in
+// one run, where one row's pieces are 16 bytes at a time, 2560 apart (the times stand at mx_quant_plan).  The rows are read
+// once, whole cache lines at a time: a thread's 64 bytes are four lines' worth of address work per lane otherwise, so they turn
+// through LDS: piece i of a thread's four lies at i * pitch + its chunk.  With pitch = 4 and a row = 16 / R modulo 16 pieces the 16
+// lanes of a write's and of a read's phase fall into all banks.  The quotients are those of act_quant_keep_kernel, bit for
+// bit.  32 consecutive rows go to one XCD, so that the pieces of a fragment meet in one L2.
+template <bool BF16, int R>
 __global__ __launch_bounds__(1024) void mx_quant_kernel(const uint16_t* __restrict__ x, int ldx, int M, int K, int group_size,
                                                         uint8_t* __restrict__ frag, float* __restrict__ cs, float centre,
-                                                        float* __restrict__ s_a, unsigned* __restrict__ counters, int n_counters) {
-    __shared__ float red[16];
+                                                        float* __restrict__ s_a, unsigned* __restrict__ counters, int n_counters,
+                                                        int pitch, int row_pieces) {
+    __shared__ float red[16][R];
     const int xcd = blockIdx.x & 7, kth = blockIdx.x >> 3;
-    const int m = M >= 256 ? (((kth >> 5) << 3) + xcd) * 32 + (kth & 31) : (int)blockIdx.x;
-    if (m >= M) return;   // (uniform: the grid is rounded up to whole sets of rows)
+    constexpr int kSets = 32 / R;   // workgroups of 32 rows
+    const int m0 = M >= 256 ? ((kth / kSets) * 8 + xcd) * 32 + kth % kSets * R : (int)blockIdx.x * R;
+    if (m0 >= M) return;   // (uniform: the grid is rounded up to whole sets of rows)
     const int tid = threadIdx.x;
-    if (m == 0)   // the arrival counters of a split GEMM behind this launch
+    if (m0 == 0)   // the arrival counters of a split GEMM behind this launch
         for (int i = tid; i < n_counters; i += (int)blockDim.x) counters[i] = 0u;
-    const bool on = tid * 32 < K;
-    extern __shared__ __attribute__((aligned(16))) v4u row[];   // K / 8 pieces
+    const int r = tid % R, c = tid / R, m = m0 + r;
+    const bool on = c * 32 < K && m < M;
+    extern __shared__ __attribute__((aligned(16))) v4u row[];
     const int threads = (int)blockDim.x, pieces = K / 8;
-    const auto place = [](int c) { return (c & ~3) | ((c + (c >> 4)) & 3); };
     const auto widen = [](uint32_t w, float& a, float& b) {
         a = BF16 ? __uint_as_float(w << 16) : half_bits_to_float((uint16_t)(w & 0xffffu));
         b = BF16 ? __uint_as_float(w & 0xffff0000u) : half_bits_to_float((uint16_t)(w >> 16));
     };
-    float amax = 0.0f;
     {
-        const v4u* src = reinterpret_cast<const v4u*>(x + (size_t)m * ldx);
+        // (threads / R >= K / 32: four rounds of threads / R pieces cover a row, the R rows one after the other)
         v4u raw[4];
+        const int per = threads / R, lr = tid / per, lp = tid % per;   // the row and the piece this thread loads
+        const v4u* src = reinterpret_cast<const v4u*>(x + (size_t)min(m0 + lr, M - 1) * ldx);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) raw[i] = i * threads + tid < pieces ? src[i * threads + tid] : v4u{0, 0, 0, 0};
+        for (int i = 0; i < 4; ++i) raw[i] = i * per + lp < pieces ? src[i * per + lp] : v4u{0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int c = i * threads + tid;
-            if (c < pieces) row[place(c)] = raw[i];
+            const int p = i * per + lp;
+            if (p < pieces) row[lr * row_pieces + (p & 3) * pitch + (p >> 2)] = raw[i];
+        }
+    }
+    __syncthreads();
+    float f[32];
+    float amax = 0.0f;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                float a, b;
-                widen(raw[i][k], a, b);
-                amax = fmaxf(amax, fmaxf(fabsf(a), fabsf(b)));
-            }
+    for (int i = 0; i < 4; ++i) {
+        const v4u raw = on ? row[r * row_pieces + i * pitch + c] : v4u{0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            widen(raw[k], f[8 * i + 2 * k], f[8 * i + 2 * k + 1]);
+            amax = fmaxf(amax, fmaxf(fabsf(f[8 * i + 2 * k]), fabsf(f[8 * i + 2 * k + 1])));
         }
     }
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-    const int waves = (int)blockDim.x >> 6;
-    if ((tid & 63) == 0) red[tid >> 6] = amax;
+    for (int off = 32; off >= R; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+    const int waves = threads >> 6;
+    if ((tid & 63) < R) red[tid >> 6][r] = amax;
     __syncthreads();
-    amax = red[0];
-    for (int w = 1; w < waves; ++w) amax = fmaxf(amax, red[w]);
+    amax = red[0][r];
+    for (int w = 1; w < waves; ++w) amax = fmaxf(amax, red[w][r]);
     const float s = fmaxf(amax, 1e-9f) / 127.0f;
-    if (tid == 0) s_a[m] = s;
+    if (c == 0 && m < M) s_a[m] = s;
     const float inv_s = 1.0f / s;
 
-    float f[32];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const v4u raw = on ? row[place(tid * 4 + i)] : v4u{0, 0, 0, 0};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) widen(raw[k], f[8 * i + 2 * k], f[8 * i + 2 * k + 1]);
-    }
     float sumf = 0.0f;   // (whole numbers below 2^24: exact)
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
@@ -145,15 +148,15 @@ __global__ __launch_bounds__(1024) void mx_quant_kernel(const uint16_t* __restri
     const v6i lo = __builtin_bit_cast(v6i, __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(lo_even, lo_odd, 8.0f));
     if (on) {
         const int steps2 = mx_padded_steps(K);
-        uint8_t* dst = frag + ((size_t)(m >> 5) * steps2 + (tid >> 1)) * kFragBytes;
-        const int fl = (tid & 1) * 32 + (m & 31);
+        uint8_t* dst = frag + ((size_t)(m >> 5) * steps2 + (c >> 1)) * kFragBytes;
+        const int fl = (c & 1) * 32 + (m & 31);
         *reinterpret_cast<v4u*>(dst + fl * 16) = hi;
         *reinterpret_cast<v4i*>(dst + 1024 + fl * 16) = v4i{lo[0], lo[1], lo[2], lo[3]};
         *reinterpret_cast<v2i*>(dst + 2048 + fl * 8) = v2i{lo[4], lo[5]};
     }
-    const int tpd = group_size == 64 ? 2 : 4;   // threads per drain of the GEMM (all of a drain's threads are on or off)
-    for (int off = 1; off < tpd; off <<= 1) sumf += __shfl_xor(sumf, off, 64);
-    if (on && tid % tpd == 0) cs[(size_t)(tid / tpd) * M + m] = sumf * centre;
+    const int tpd = group_size == 64 ? 2 : 4;   // threads of a row per drain of the GEMM (all of a drain's are on or off)
+    for (int off = 1; off < tpd; off <<= 1) sumf += __shfl_xor(sumf, off * R, 64);
+    if (on && c % tpd == 0) cs[(size_t)(c / tpd) * M + m] = sumf * centre;
 }
 
 __device__ __forceinline__ v16f mfma_hi(v4i a, v4i b, v16f c) {   // 4 * a4 * c/2
@@ -690,12 +693,38 @@ MxPlan mx_plan(int M, int N, int K, int group_size) {
     return plan;
 }
 
+// How the quantising kernel's workgroups hold their rows in LDS (in pieces of 16 bytes), and how many rows they have.
+namespace {
+struct MxQuantPlan { int rows, pitch, row_pieces; };
+constexpr int kMxQuantLds = 65536 - 256;   // beside the waves' maxima
+MxQuantPlan mx_quant_layout(int K, int rows) {
+    const int chunks = K / 32, pitch = (chunks + 27) / 16 * 16 - 12;   // 4 modulo 16
+    const MxQuantPlan plan{rows, pitch, 4 * pitch + 16 / rows};
+    if (rows == 1 && plan.row_pieces * 16 > kMxQuantLds) return {1, chunks, 4 * chunks};   // (the longest rows: without the padding)
+    return plan;
+}
+}  // namespace
+// Two rows where there are more than 256 of them and two fit, with other workgroups beside them on the CU: 4096 x 4096 17.6 ->
+// 14.6 us, 2048 x 8192 17.9 -> 15.7, 1024 x 11008 15.1 -> 11.3; up to 256 rows one (256 x 6144 5.4 against 5.9), 2048 x 14336 27.9
+// against 29.0.  Four rows: level (4096 x 4096 15.4, 2048 x 8192 15.6).
+static MxQuantPlan mx_quant_plan(int M, int K) { return mx_quant_layout(K, M > 256 && K <= 11264 ? 2 : 1); }
+
 hipError_t launch_mx_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size, int centre, uint8_t* frag, float* cs,
                            float* s_a, unsigned* counters, int n_counters, hipStream_t stream) {
-    const dim3 grid((unsigned)(M >= 256 ? (M + 255) / 256 * 256 : M)), block((unsigned)((K / 32 + 63) / 64 * 64));
     const float f = -(float)centre / 16.0f;   // (the accumulators hold sums of q * code / 16)
-    if (x_bf16) mx_quant_kernel<true><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a, counters, n_counters);
-    else mx_quant_kernel<false><<<grid, block, (size_t)K * 2, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a, counters, n_counters);
+    const MxQuantPlan plan = mx_quant_plan(M, K);
+    const int rows = plan.rows;
+    const dim3 grid((unsigned)(M >= 256 ? (M + 255) / 256 * (256 / rows) : (M + rows - 1) / rows));
+    const dim3 block((unsigned)((K / 32 * rows + 63) / 64 * 64));
+    const size_t lds = (size_t)rows * plan.row_pieces * 16;
+#define SLIMK_MX_QUANT(R)                                                                                                            \
+    do {                                                                                                                             \
+        if (x_bf16) mx_quant_kernel<true, R><<<grid, block, lds, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a, counters, n_counters, plan.pitch, plan.row_pieces); \
+        else mx_quant_kernel<false, R><<<grid, block, lds, stream>>>((const uint16_t*)x, ldx, M, K, group_size, frag, cs, f, s_a, counters, n_counters, plan.pitch, plan.row_pieces);       \
+    } while (0)
+    if (rows == 2) SLIMK_MX_QUANT(2);
+    else SLIMK_MX_QUANT(1);
+#undef SLIMK_MX_QUANT
     return hipGetLastError();
 }
 

@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restri
 // between the absmax pass and the quantising pass, all of its loads in flight together.  With many rows the
 // two-pass kernel moves every row twice (the second time from L2) in phases that the workgroups of a round
 // go through together; this one moves it once.  Same arithmetic per element: bit-identical results.
-// THREADS: 256 in general (many rows: several workgroups per CU); 512 or 1024 for a few rows, where one row per
+// THREADS: 256 in general (many rows: several workgroups per CU); 512 or 1024 for few rows, where one row per
 // workgroup leaves most of the chip idle and a row's time is what its one CU needs for the arithmetic.  The IEEE
 // divisions (a dozen instructions each) were most of that arithmetic: rne_quotient() (w2a8_common.h) avoids nearly
 // all of them (32 rows x 28672: 8.2 -> 7.2 us; 4096 x 4096: 17.6 -> 15.2 us).
@@ -258,7 +258,12 @@ __global__ __launch_bounds__(THREADS) void act_quant_keep_kernel(const uint16_t*
     }
 }
 
-constexpr int kFewRows = 64;  // up to this many rows a long row gets 1024 threads
+// Up to this many rows (two workgroups a CU) a row of more than 4096 elements gets 1024 threads and one of more than 2048
+// 512: with group sums 65 x 14336 8.4 -> 5.0 us, 200 x 8192 6.1 -> 4.5, 512 x 4096 4.6 -> 4.2, 512 x 14336 10.7 -> 8.0.  With
+// 1024 rows the wide workgroups are behind on up to 8192 elements (1024 x 8192 9.2 / 9.6; 1024 x 14336 15.9 / 13.8).
+// A row of more than 16384 gets 1024 threads whatever their number, and is kept in registers too: 1024 x 20480 22.7 (in two
+// passes) -> 19.3, 100 x 28672 17.7 -> 8.4.
+constexpr int kFewRows = 512;
 
 template <bool BF16, bool SUMS>
 static void launch_act_quant_keep(const void* x, int ldx, int M, int K, int group_size, int8_t* q, int ldq, float* s_a,
@@ -268,7 +273,7 @@ static void launch_act_quant_keep(const void* x, int ldx, int M, int K, int grou
         act_quant_keep_kernel<BF16, 1, 512, SUMS><<<grid, dim3(512), 0, stream>>>((const uint16_t*)x, ldx, M, K, group_size, q, ldq, s_a, rowsum, ldr, copies);
         return;
     }
-    if (M <= kFewRows && K > 4096) {  // a few long rows: 1024 threads a row
+    if ((M <= kFewRows && K > 4096) || K > 16384) {  // few rows, or long ones: 1024 threads a row
         const dim3 wide(1024);
         if (K <= 8192)
             act_quant_keep_kernel<BF16, 1, 1024, SUMS><<<grid, wide, 0, stream>>>((const uint16_t*)x, ldx, M, K, group_size, q, ldq, s_a, rowsum, ldr, copies);
@@ -288,7 +293,7 @@ static void launch_act_quant_keep(const void* x, int ldx, int M, int K, int grou
 
 hipError_t launch_act_quant(const void* x, int ldx, bool x_bf16, int M, int K, int group_size,
                             int8_t* q, int ldq, float* s_a, int32_t* rowsum, int ldr, int copies, hipStream_t stream) {
-    if (K <= 16384 || (M <= kFewRows && K <= 32768)) {
+    if (K <= 32768) {
         if (rowsum) {
             if (x_bf16) launch_act_quant_keep<true, true>(x, ldx, M, K, group_size, q, ldq, s_a, rowsum, ldr, copies, stream);
             else launch_act_quant_keep<false, true>(x, ldx, M, K, group_size, q, ldq, s_a, rowsum, ldr, copies, stream);
