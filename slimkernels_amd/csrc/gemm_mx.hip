@@ -217,8 +217,12 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
     const int tiles_n = (p.strips + kStripsPerWg - 1) / kStripsPerWg, tiles_m = (p.M + kBM - 1) / kBM;
     const int total = tiles_m * tiles_n, per_xcd = (total + 7) / 8;
     const int xcd = (int)(blockIdx.x & 7), local = (int)(blockIdx.x >> 3);
-    int tile;
-    if (tiles_n % 8 == 0) {
+    int tile, split_idx = 0;
+    if (SPLIT) {
+        if (!split_tile_place((int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y, tiles_n, tiles_m, tile, split_idx)) return;
+        tile = __builtin_amdgcn_readfirstlane(tile);
+        split_idx = __builtin_amdgcn_readfirstlane(split_idx);
+    } else if (tiles_n % 8 == 0) {
         const int band = tiles_n / 8;
         tile = (local / band) * tiles_n + xcd * band + local % band;
     } else if (tiles_m >= 2 && tiles_m <= 4) {
@@ -228,7 +232,7 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
     } else {
         tile = xcd * per_xcd + local;
     }
-    if (local >= per_xcd || tile >= total) return;
+    if (!SPLIT && (local >= per_xcd || tile >= total)) return;
     const int m_tile = (tile / tiles_n) * kBM;
     const int strip_raw = (tile % tiles_n) * kStripsPerWg + wave;
     const int strip = min(strip_raw, p.strips - 1);   // a surplus wave recomputes the last strip and stores nothing
@@ -236,7 +240,7 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
 
     const int steps2 = (p.steps + 1) / 2 * 2;
     const int all_stages = steps2 / 2;
-    const int stage0 = SPLIT ? (int)blockIdx.y * p.stages_per_split : 0;
+    const int stage0 = SPLIT ? split_idx * p.stages_per_split : 0;
     const int n_stages = SPLIT ? min(p.stages_per_split, all_stages - stage0) : all_stages;
 
     const int row_blocks = (p.M + kFragRows - 1) / kFragRows;
@@ -509,7 +513,7 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
         uint32_t ws_off[RB];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            ws_off[rb] = ws_lane + rb * 8192 + blockIdx.y * ws_pitch + ws_tile;
+            ws_off[rb] = ws_lane + rb * 8192 + (uint32_t)split_idx * ws_pitch + ws_tile;
             asm volatile("" : "+v"(ws_off[rb]));
         }
         __builtin_amdgcn_sched_barrier(0);

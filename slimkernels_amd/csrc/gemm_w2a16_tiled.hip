@@ -70,14 +70,23 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
     const uint16_t* const bias = early_bias(p.bias);
     // token tiles of a channel tile next to each other on one XCD: they read the same weights
     const int tiles_n = (p.strips + kStripsPerWg - 1) / kStripsPerWg, tiles_m = (p.M + kBM - 1) / kBM;
-    int n_tile, m_tile_i;
-    if (!xcd_place((int)blockIdx.x, tiles_n, tiles_m, n_tile, m_tile_i)) return;
+    // ((split, channel tile) pairs dealt out together where split by split is uneven: 360 x 1584 x 11264 43.5 -> 28.1 us, 505 x
+    // 5360 x 11520 119 -> 84.  The partial sums meet in a second launch: no split has to share an XCD with another.)
+    int n_tile, m_tile_i, split_idx = PARTIAL ? (int)blockIdx.y : 0;
+    if (PARTIAL && splits_uneven(tiles_n * tiles_m, (int)gridDim.y)) {
+        int set;
+        if (!xcd_place((int)(blockIdx.y * gridDim.x + blockIdx.x), tiles_n * (int)gridDim.y, tiles_m, set, m_tile_i)) return;
+        split_idx = __builtin_amdgcn_readfirstlane(set / tiles_n);
+        n_tile = __builtin_amdgcn_readfirstlane(set % tiles_n);
+    } else if (!xcd_place((int)blockIdx.x, tiles_n, tiles_m, n_tile, m_tile_i)) {
+        return;
+    }
     const int m_tile = m_tile_i * kBM;
     const int strip_raw = n_tile * kStripsPerWg + wave;
     const int strip = min(strip_raw, p.strips - 1);   // a surplus wave recomputes the last strip and stores nothing
     const bool strip_ok = strip_raw < p.strips;
     // (KP = 2: an even number of steps in every split, so that the halves meet at the same barriers; no split is empty)
-    const int wg_step0 = PARTIAL ? (int)blockIdx.y * steps_per_split : 0;
+    const int wg_step0 = PARTIAL ? split_idx * steps_per_split : 0;
     const int wg_steps = PARTIAL ? min(steps_per_split, p.steps - wg_step0) : p.steps;
     const int n_steps = wg_steps / KP, step0 = wg_step0 + kh * n_steps;
 
@@ -258,7 +267,7 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
     if (!strip_ok) return;
 
     if constexpr (PARTIAL) {   // fp32 partial sums [split][M][N]: 128 bytes of a row per half-wave and store
-        float* ws = p.ws + (size_t)blockIdx.y * p.M * p.N;
+        float* ws = p.ws + (size_t)split_idx * p.M * p.N;
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll

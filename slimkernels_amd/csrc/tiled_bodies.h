@@ -98,8 +98,12 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
     const int total = tiles_m * tiles_n;
     const int per_xcd = (total + 7) / 8;
     const int xcd = (int)(blockIdx.x & 7), local = (int)(blockIdx.x >> 3);
-    int tile;
-    if (tiles_n % 8 == 0) {
+    int tile, split_idx = 0;
+    if (SPLIT) {
+        if (!split_tile_place((int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y, tiles_n, tiles_m, tile, split_idx)) return;
+        tile = __builtin_amdgcn_readfirstlane(tile);
+        split_idx = __builtin_amdgcn_readfirstlane(split_idx);
+    } else if (tiles_n % 8 == 0) {
         const int band = tiles_n / 8;
         tile = (local / band) * tiles_n + xcd * band + local % band;
     } else if (tiles_m >= 2 && tiles_m <= 4) {
@@ -109,17 +113,17 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
     } else {
         tile = xcd * per_xcd + local;
     }
-    if (local >= per_xcd || tile >= total) return;
+    if (!SPLIT && (local >= per_xcd || tile >= total)) return;
     const int m_tile = (tile / tiles_n) * kBM;
     const int strip0 = (tile % tiles_n) * kStrips;
     const int strip = min(strip0 + wave, p.strips - 1);  // clamped: a surplus wave recomputes the last strip, stores nothing
     const bool strip_ok = strip0 + wave < p.strips;
-    // this workgroup's share of K in stages (all of it unless K is split over blockIdx.y)
+    // this workgroup's share of K in stages (all of it unless K is split)
     // (an odd step count ends in a stage whose second step lies past the weights and the scales: both read as zero
     // through the range-checked buffer loads, so that step's group adds nothing)
     const int all_stages = (p.steps + kStageSteps - 1) / kStageSteps;
     const int stages_per_split = SPLIT ? p.groups_per_split * GS / kStageSteps : all_stages;
-    const int stage0 = SPLIT ? (int)blockIdx.y * stages_per_split : 0;
+    const int stage0 = SPLIT ? split_idx * stages_per_split : 0;
     const int n_stages = min(stages_per_split, all_stages - stage0);
 
     // ---- loads, one stage ahead, all through buffer instructions: a wave-uniform descriptor plus a
@@ -431,7 +435,7 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
         // zero, the form whose wait states the compiler inserts itself; every address is made before the first store
         // and each store is followed by two idle cycles written here (the wait the hardware needs, whatever the
         // scheduler and the register allocator do); and fences keep everything else out of the run of stores.
-        const uint32_t ws_base = blockIdx.y * ws_split_pitch + ws_tile;
+        const uint32_t ws_base = (uint32_t)split_idx * ws_split_pitch + ws_tile;
         uint32_t ws_off[kMB];
 #pragma unroll
         for (int mb = 0; mb < kMB; ++mb) {

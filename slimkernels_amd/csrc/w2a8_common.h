@@ -205,5 +205,49 @@ __host__ __device__ __forceinline__ bool xcd_place(const int local, const int se
     return true;
 }
 inline int xcd_grid(const int sets, const int members) { return (sets * members + 7) / 8 * 8; }
+// One contiguous run of `items` per XCD, the runs' lengths at most one apart; local as above, false: a padding workgroup.
+__host__ __device__ __forceinline__ bool xcd_run(const int local, const int items, int& item) {
+    const int xcd = local & 7;
+    item = items * xcd / 8 + (local >> 3);
+    return item < items * (xcd + 1) / 8;
+}
+
+// K splits of tiled kernels: grids of (tiles rounded up to eight, splits).  Dealt out split by split the XCDs that get the odd
+// tile get it in every split: 14 x 6 tiles in six splits put 66 workgroups on an XCD with room for 64.  Whether (split,
+// tile) pairs dealt out evenly load the fullest of an XCD's 32 CUs with fewer workgroups:
+__host__ __device__ __forceinline__ bool splits_uneven(const int total, const int splits) {
+    return ((total + 7) / 8 * splits + 31) / 32 > ((total * splits + 7) / 8 + 31) / 32;
+}
+// Which tile and K split workgroup (x, y) of the int8 or digit form takes.  Where that helps (splits_uneven), each XCD gets a
+// run of pairs, a tile's together: of 1466 drawn calls 32 int8 ones went 2..44 % faster (360 x 1584 x 11264 35.8 -> 28.0
+// us), 35 digit ones 3..31 % (795 x 3248 x 14080 89.0 -> 69.4).  Elsewhere split by split: a tile's splits share an XCD,
+// out of whose L2 the last of them to arrive reads the partial sums, and even dealing was up to 18 % slower.
+// Order within a split: channel tiles that divide by eight in bands, token tile major; with two to four token tiles those of a
+// channel tile on one XCD's queue; else one run of tiles per XCD, channel tile fastest.
+__host__ __device__ __forceinline__ bool split_tile_place(const int x, const int y, const int splits, const int tiles_n, const int tiles_m,
+                                                          int& tile, int& split) {
+    const int total = tiles_n * tiles_m, per_xcd = (total + 7) / 8, xcd = x & 7, slot = x >> 3;
+    const bool few = tiles_m >= 2 && tiles_m <= 4;
+    if (splits_uneven(total, splits)) {
+        int pair;
+        if (!xcd_run(y * per_xcd * 8 + x, total * splits, pair)) return false;
+        const int t = pair / splits;
+        split = pair % splits;
+        tile = few ? t % tiles_m * tiles_n + t / tiles_m : t;
+        return true;
+    }
+    split = y;
+    if (tiles_n % 8 == 0) {
+        const int band = tiles_n / 8;
+        tile = (slot / band) * tiles_n + xcd * band + slot % band;
+    } else if (few) {
+        int n_tile, m_tile;
+        if (!xcd_place(x, tiles_n, tiles_m, n_tile, m_tile)) return false;
+        tile = m_tile * tiles_n + n_tile;
+    } else {
+        tile = xcd * per_xcd + slot;
+    }
+    return tile < total;
+}
 
 }  // namespace w2a8
