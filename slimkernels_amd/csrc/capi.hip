@@ -165,12 +165,15 @@ int skinny_plain_split(int N, int K, int group_size) {
 // stay under 100 MiB).
 enum MidRoute { kMidPlain, kMidShared, kMidTiled, kMidStrips };
 int mid_split(int M, int N, int K, int group_size);
-// skinny_only: the faster of the two skinny forms (what an explicit request for the skinny kernel runs)
-MidRoute mid_route(int M, int N, int K, int group_size, bool skinny_only = false) {
+// skinny_only: the faster of the two skinny forms (what an explicit request for the skinny kernel runs).  cost: the
+// prediction for the form that is returned (33..256 rows)
+MidRoute mid_route(int M, int N, int K, int group_size, bool skinny_only = false, float* cost = nullptr) {
     if (M > kSkinnyMaxRows) return skinny_only ? kMidPlain : kMidTiled;
     const int strips = strips_of(N), steps = K / w2a8::kStepK, blocks = (M + 15) / 16;
     const size_t weight_bytes = (size_t)strips * 64 * (K / 4);
-    if (K <= 2048) return skinny_only || (size_t)blocks * weight_bytes <= ((size_t)100 << 20) ? kMidPlain : kMidTiled;
+    const bool by_size = K <= 2048;
+    const MidRoute sized = skinny_only || (size_t)blocks * weight_bytes <= ((size_t)100 << 20) ? kMidPlain : kMidTiled;
+    if (by_size && !cost) return sized;
     const float weight_mib = (float)weight_bytes / 1048576.0f;
     // a step costs more in groups of 64 and less in groups of 256 and more than in groups of 128: factors per form
     const auto by_group = [&](float of64, float of256) { return group_size == 64 ? of64 : (group_size >= 256 ? of256 : 1.0f); };
@@ -212,8 +215,11 @@ MidRoute mid_route(int M, int N, int K, int group_size, bool skinny_only = false
         }
     }
     const float skinny_cost = std::min(plain_cost, shared_cost), other_cost = std::min(tiled_cost, strips_cost);
-    if (skinny_cost <= other_cost) return plain_cost <= shared_cost ? kMidPlain : kMidShared;
-    return tiled_cost <= strips_cost ? kMidTiled : kMidStrips;
+    const MidRoute route = by_size                    ? sized
+                           : skinny_cost <= other_cost ? (plain_cost <= shared_cost ? kMidPlain : kMidShared)
+                                                       : (tiled_cost <= strips_cost ? kMidTiled : kMidStrips);
+    if (cost) *cost = route == kMidPlain ? plain_cost : route == kMidShared ? shared_cost : route == kMidTiled ? tiled_cost : strips_cost;
+    return route;
 }
 
 
@@ -650,10 +656,16 @@ size_t slimk_w2a8_linear_workspace_bytes(int M, int N, int K, int group_size) {
     return kCounterBlockBytes + (size_t)plan.split * plan.tiles * plan.rb * w2a8::mx::kFragRows * 256 * sizeof(float);
 }
 
-// What act_quant and the int8 tiled kernel take for more than 256 rows in fewer than 512 128-row tiles (64-row tiles,
-// the split tiled_fast_auto_split chooses), in the form of mx_predicted_time; 4.5 % rms on 364 timed calls, 4.2 % on 328
-// others.
+// What act_quant and the int8 path take.  Up to 256 rows: the form that mid_route chooses, by its own prediction; 5.1 %
+// rms on 320 timed calls (sixteen matrices, 96..256 rows).  More, in fewer than 512 128-row tiles: 64-row tiles, the split
+// tiled_fast_auto_split chooses, in the form of mx_predicted_time; 4.5 % rms on 364 timed calls, 4.2 % on 328 others.
 static float int8_layer_time(int M, int N, int K, int group_size, int per_group_zp) {
+    if (M <= kSkinnyMaxRows) {
+        static const float factor[4][2] = {{0.799f, 0.845f}, {0.963f, 0.995f}, {0.897f, 1.059f}, {0.984f, 1.106f}};
+        float cost = 0.0f;
+        const MidRoute form = mid_route(M, N, K, group_size, false, &cost);
+        return 4.489f + 1.843e-6f * (float)M * (float)K + factor[form][per_group_zp ? 1 : 0] * cost;
+    }
     const int strips = strips_of(N), steps = K / w2a8::kStepK, gs = group_size / w2a8::kStepK;
     const int split = w2a8::tiled_fast_auto_split(M, strips, steps, gs);
     const int wgs = (int)w2a8::tiled_fast_workspace_tiles(M, strips, gs) * split, n = (wgs + 255) / 256;
@@ -665,6 +677,23 @@ static float int8_layer_time(int M, int N, int K, int group_size, int per_group_
     return 5.57f + 1.104e-6f * (float)M * (float)K + sums + ((float)per + 3.4f) * each;
 }
 
+// What the digit form takes with its quantisation, to be held against int8_layer_time: 4.6 % rms on 576 timed calls
+// (sixteen matrices of 1024..28672 channels and K = 1536..28672, 96..700 rows, both group sizes and kinds of zero-points).
+// mx_predicted_time compares the plans of one call, this one the planned call with another path (the other is 2..4 % high on
+// average since the quantisation writes its fragments 32 bytes at a time, and 9 % rms off on 96..256 rows).
+static float digit_layer_time(int M, int N, int K, int group_size, int per_group_zp, const w2a8::MxPlan& plan) {
+    const int stages = w2a8::mx_padded_steps(K) / 2, per = (stages + plan.split - 1) / plan.split;
+    const int n = (plan.tiles * plan.split + 255) / 256;
+    static const float side_by_side[2][3] = {{0.7352f, 0.9788f, 1.4324f}, {1.141f, 1.6519f, 2.4685f}};
+    const float* const cu = side_by_side[plan.rb == 4];
+    float each = n <= 3 ? cu[n - 1] : cu[2] * (float)n / 3.0f;
+    if (group_size == 64) each *= 1.1753f;
+    if (per_group_zp) each *= group_size == 64 ? 1.1268f : 1.108f;
+    const float sums = plan.split > 1 ? 6.77f + 0.013e-6f * 8.0f * (float)plan.split * (float)M * (float)N : 0.0f;
+    const float many = plan.split > 3 ? 1.0f + 0.014f * (float)(plan.split - 3) : 1.0f;   // (what drawn calls beyond the fit took more)
+    return many * (4.363f + 1.2145e-6f * (float)M * (float)K + sums + ((float)per + 5.668f) * each);
+}
+
 // Where the digit form beats act_quant + the kernel that slimk_w2a8_gemm would take, both timed with their quantisation;
 // groups of 64 and 128 (with 256, where the int8 kernel drains half as often, they were level: 2048 x 14336 x 4096
 // 127 / 128 us).
@@ -673,26 +702,31 @@ static float int8_layer_time(int M, int N, int K, int group_size, int per_group_
 //    575 -> 512, but 4096 x 4096 x 14336 level at 257 (per-group zero-points: 301 -> 279).  Symmetric levels with K < 512 are mostly
 //    launch and quantisation: level at K = 384, up to 3 % slower at 256 (2317 x 8400 x 256 24.3 -> 25.1).  95 routed calls of 70 drawn
 //    shapes, K = 256..16384: 18 % faster on average, the slowest 2 % faster.
-//  * fewer tiles, more than 256 rows: the smaller predicted time, with 6 % in hand, inside the range the predictions were
-//    first fitted on, 4096 channels and elements and more.  200 routed calls of shapes that took no part in the fit: 16 %
-//    faster on average, the slowest level (264 x 14336 x 4096 with per-group zero-points 47.6 / 47.9 us); on normal
-//    activations without outliers (other toggling, another clock) 281 routed calls of thirteen decoder matrices 13 %
-//    faster, the slowest 1500 x 8192 x 8192 120.5 -> 124.0.  512 x 28672 x 8192 in
-//    groups of 64 184 -> 146, with per-group zero-points 236 -> 165.  (With 3 % in hand 1300 x 4096 x 11008 in groups of
-//    64 would go 111 -> 115.)
-//  * 96..256 rows: long reductions only, in groups of 128 (128 x 8192 x 28672 62 -> 54 us, 96 x 4096 x 28672 50 -> 41).
+//  * fewer tiles, 96 rows and more, 1024 channels and elements and more: the smaller predicted time, with 6 % in hand, 8 %
+//    for symmetric groups of 128 on more than 256 rows.  Of 9863 drawn calls that the int8 path had (96..1200 rows, odd widths
+//    among them), the 84 % this takes are 14 % faster on average, 1.1 % of them more than 3 % slower, the slowest 13 %
+//    (4311 x 9728 and 7881 x 11520 in eight splits); what it leaves would gain 5 %.  128 x 28672 x 8192 in groups of 64
+//    63.1 -> 56.7 us, with per-group zero-points 76 -> 64; 160 x 20480 x 2048 31 -> 23; 700 x 3072 x 24576 121 -> 105.
+//    4096 channels and elements and more, more than 256 rows: also where mx_predicted_time, the first fit, has 6 % in hand,
+//    as before (200 routed calls of shapes that took no part in it 16 % faster, the slowest level; 512 x 28672 x
+//    8192 in groups of 64 184 -> 146, with per-group zero-points 236 -> 165).
+//  * 96..256 rows, long reductions in groups of 128: without asking (128 x 8192 x 28672 62 -> 54 us, 96 x 4096 x 28672
+//    50 -> 41).
 int slimk_w2a8_linear_route(int M, int N, int K, int group_size, int per_group_zp) {
     if (slimk_w2a8_linear_activation_bytes(M, N, K, group_size) == 0) return 0;
     if (group_size > 128 || M < 96) return 0;
-    if (M <= 256) return group_size == 128 && K >= 20480 && N >= 4096 ? 1 : 0;
+    if (M <= 256 && group_size == 128 && K >= 20480 && N >= 4096) return 1;
     const w2a8::MxPlan plan = w2a8::mx_plan(M, N, K, group_size);
     if (plan.rb == 4 && plan.tiles >= 2 * 256) {
         if (!per_group_zp && K < 512) return 0;
         return N >= (group_size == 128 && !per_group_zp ? 5120 : 4096) ? 1 : 0;
     }
-    if (N < 4096 || K < 4096) return 0;
-    return w2a8::mx_predicted_time(M, N, K, group_size, per_group_zp, plan.rb, plan.split) <
-                   0.94f * int8_layer_time(M, N, K, group_size, per_group_zp) ? 1 : 0;
+    if (N < 1024 || K < 1024) return 0;
+    const float other = int8_layer_time(M, N, K, group_size, per_group_zp);
+    if (M > 256 && N >= 4096 && K >= 4096 &&
+        w2a8::mx_predicted_time(M, N, K, group_size, per_group_zp, plan.rb, plan.split) < 0.94f * other) return 1;
+    const float in_hand = M > 256 && group_size == 128 && !per_group_zp ? 0.92f : 0.94f;
+    return digit_layer_time(M, N, K, group_size, per_group_zp, plan) < in_hand * other ? 1 : 0;
 }
 
 int slimk_w2a8_linear_plan(int M, int N, int K, int group_size, int* tile_rows, int* splits) {

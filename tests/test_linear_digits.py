@@ -256,3 +256,27 @@ def test_route_knows_short_reductions_and_per_group_zero_points():
         assert [route(M, N, 512, g, zp) for zp in (0, 1)] == [1, 1]
     assert [route(600, 11008, 4096, 128, zp) for zp in (0, 1)] == [0, 1]
     assert [route(512, 28672, 8192, 64, zp) for zp in (0, 1)] == [1, 1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,g,mode,out", [
+    (96, 16384, 8192, 64, "asym", "bfloat16"),     # the fewest rows
+    (129, 16384, 1088, 64, "sym", "float16"),      # a short reduction of an odd number of steps, one row in the last tile
+    (255, 20481, 1024, 128, "asym", "float16"),    # the shortest; 2-byte stores
+    (513, 2056, 9728, 64, "asym", "bfloat16"),     # few channels, a last strip of eight
+])
+def test_newly_routed_calls_give_the_int8_paths_results(gpu_ops, M, N, K, g, mode, out):
+    """Calls of 96 rows and more below 4096 channels or elements, or up to 256 rows, that the layer takes through the digits:
+    exact group sums on both paths, fp32 folds in another order, outputs rounded once (2^-11 / 2^-8 of a value at most)."""
+    dtype = getattr(torch, out)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M)
+    weight = torch.randn((N, K), generator=gen, device="cuda", dtype=torch.float16) * 0.02
+    bias = torch.randn((N,), generator=gen, device="cuda").to(dtype)
+    layer = gpu_ops.W2A8Linear.from_float(weight, g, mode, bias=bias, out_dtype=dtype)
+    assert _lib.lib().slimk_w2a8_linear_route(M, N, K, g, int(mode == "asym"))
+    x = (torch.randn((M, K), generator=gen, device="cuda") + 0.3).to(dtype)
+    with torch.no_grad():
+        y = layer(x).double()
+    ref = (gpu_ops.w2a8_gemm(gpu_ops.quantize_act_int8(x, g), layer.weight, dtype) + bias).double()
+    assert (y - ref).norm() <= (3e-4 if dtype == torch.float16 else 2.4e-3) * ref.norm()
