@@ -422,6 +422,10 @@ hipError_t launch_w2a16(const W2A16Params& asked, int gs, bool out_bf16, hipStre
     const W2A16Plan plan = w2a16_plan(asked.M, asked.strips, asked.steps, gs, asked.split);
     W2A16Params p = asked;
     p.split = plan.split;   // (at most what was asked for, which the workspace was sized by)
+    // (the many-rows kernel reads its bias in pieces of eight channels: where output rows are not whole pieces a read would be
+    // misaligned, and with fewer than eight channels in front of the bias, so there it is added behind the kernel)
+    const bool bias_behind = plan.rb && p.split <= 1 && p.bias && !output_rows_whole(p.out, p.ldo, p.N);
+    if (bias_behind) p.bias = nullptr;
     if (plan.rb) {
         if (hipError_t e = launch_w2a16_tiled(p, plan.rb, plan.halves, gs, out_bf16, stream); e != hipSuccess) return e;
     } else {
@@ -439,8 +443,8 @@ hipError_t launch_w2a16(const W2A16Params& asked, int gs, bool out_bf16, hipStre
             w2a16_reduce_kernel<OutBF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo, p.bias);
         else
             w2a16_reduce_kernel<OutF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo, p.bias);
-    } else if (plan.rb && p.bias && !output_rows_whole(p.out, p.ldo, p.N)) {
-        return launch_add_bias(p.out, p.ldo, p.M, p.N, p.bias, out_bf16, stream);
+    } else if (bias_behind) {
+        return launch_add_bias(p.out, p.ldo, p.M, p.N, asked.bias, out_bf16, stream);
     }
     return hipGetLastError();
 }

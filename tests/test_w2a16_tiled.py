@@ -99,3 +99,20 @@ def test_w2a16_prompt_without_workspace(gpu_ops):
     _lib.check(L.slimk_w2a16_gemm(x.data_ptr(), K, _lib.F16, w.w_r.data_ptr(), w.s_r.data_ptr(), None, w.zp_const, M, N, K, g,
                                   out.data_ptr(), N, _lib.F16, None, 0, 0, stream.cuda_stream))
     assert torch.equal(out, gpu_ops.w2a16_gemm(x, w, split_k=1))
+
+
+@pytest.mark.parametrize("M,N,K,g,rows", [(16384, 1, 128, 128, 64), (16384, 4, 128, 64, 64), (16384, 7, 128, 128, 64), (16384, 8, 128, 128, 64),
+                                          (8192, 100, 128, 128, 64), (20000, 103, 128, 64, 128), (700, 14337, 2048, 128, 64)])
+def test_w2a16_bias_of_rows_that_are_no_whole_pieces(gpu_ops, M, N, K, g, rows):
+    """A bias of fewer than eight channels, or of a number that is no multiple of eight, in an unsplit call of the many-rows kernel:
+    the sum of two tensors, bit for bit.  (The bias lies inside a longer tensor.)"""
+    assert plan(M, N, K, g)[:2] == (rows, 1)
+    print(f"W2A16 bias M={M} N={N} K={K} g={g}", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(N)
+    layer = gpu_ops.W2A16Linear.from_float(torch.randn((N, K), generator=gen, device="cuda", dtype=torch.float16), g)
+    x = torch.randn((M, K), generator=gen, device="cuda", dtype=torch.float16)
+    bias = torch.randn((N + 128,), generator=gen, device="cuda", dtype=torch.float16)[64:64 + N]
+    plain = layer(x)
+    layer.bias = bias
+    assert torch.equal(layer(x).view(torch.int16), (plain + bias).view(torch.int16))
