@@ -87,9 +87,9 @@ class SlimkError(RuntimeError):
 
 
 def build(verbose=False):
-    """Compile the library in-tree with hipcc for gfx950 (cross-compiles without a GPU), and the native host side of the
-    torch calls beside it."""
-    subprocess.run(["make", "-C", _CSRC, "-B", "-j8", f"PYTHON={sys.executable}", "libslimk_w2a8.so", "../torch/_native.so"], check=True,
+    """Compile the library in-tree with hipcc for gfx950 (cross-compiles without a GPU), and where this Python's torch has
+    GPU support the native host side of the torch calls beside it."""
+    subprocess.run(["make", "-C", _CSRC, "-B", "-j8", f"PYTHON={sys.executable}", "all"], check=True,
                    stdout=None if verbose else subprocess.DEVNULL,
                    stderr=None if verbose else subprocess.DEVNULL)
     return LIB_PATH
