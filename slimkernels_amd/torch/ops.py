@@ -34,10 +34,18 @@ _DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 _fast = None
 
 
+class _NoGpuHost:
+    """On a torch without GPU support every tensor is one that the general code refuses, by a message of its own."""
+    linear = linear16 = linear4 = quantize = gemm = grouped = staticmethod(lambda *args: None)
+
+
 def _host():
     """The native host side, bound to the loaded library.  As with the library itself there is no doing without it."""
     global _fast
     if _fast is None:
+        if _raw_stream is None:
+            _fast = _NoGpuHost
+            return _fast
         L = _lib.lib()
         try:
             from . import _native
