@@ -182,7 +182,8 @@ struct Bias {
         Py_INCREF(o);
         keep.take(o);
         const at::Tensor& t = tensor(keep);
-        if (t.dim() > 1) return false;
+        // (another width: an error, or on a one-channel layer a wider result that the general code can only give for two dimensions)
+        if (t.dim() > 1 || (t.dim() == 1 && t.size(0) != N && t.size(0) != 1)) return false;
         p = t.data_ptr();
         behind = dtype_code(t.scalar_type()) != dtype || t.dim() != 1 || t.size(0) != N || (N > 1 && t.stride(0) != 1) || t.device() != device ||
                  (reinterpret_cast<uintptr_t>(p) & 15) != 0 || (t.requires_grad() && c10::GradMode::is_enabled()) || t._fw_grad(0).defined();

@@ -156,6 +156,26 @@ def test_biases_that_the_kernels_do_not_add(gpu_ops):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["2", "4", "16"])
+def test_a_wider_bias_on_a_layer_of_one_channel(gpu_ops, monkeypatch, kind):
+    """Token rows [M, 1] widen with the bias; of more (or fewer) dimensions the general code refuses it, and so does the layer."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    layer = LAYERS[kind].from_float(torch.randn((1, 256), generator=gen, device="cuda", dtype=torch.float16), 128, "sym")
+    x = torch.randn((2, 3, 256), generator=gen, device="cuda", dtype=torch.float16)
+    plain = layer(x)
+    layer.bias = torch.randn((5,), generator=gen, device="cuda", dtype=torch.float16)
+    assert torch.equal(layer(x[0]), plain[0] + layer.bias)
+    for t in (x, x[0, 0]):
+        with pytest.raises(RuntimeError):
+            _without_native(monkeypatch, lambda: layer(t))
+        with pytest.raises(RuntimeError):
+            layer(t)
+    layer.bias = layer.bias[:1]
+    assert torch.equal(layer(x), plain + layer.bias)
+
+
+@pytest.mark.gpu
 def test_quantise_gemm_and_grouped(gpu_ops, monkeypatch):
     host = ops._host()
     gen = torch.Generator(device="cuda")
