@@ -813,7 +813,9 @@ struct GroupedSmem {
 // partial tiles meet in the caller's workspace, the last workgroup of a unit to arrive adds them
 // up in split order and stores).
 // DUMP: verification instantiation, as in skinny_body: the int32 group sums are also written out, nothing else changes.
-template <int J, int GS, int NK, bool SHARE, bool ASYM, bool NT, bool SPLIT, typename OutT, bool DUMP = false>
+// BIAS: p.bias is added to the rounded outputs; instantiations of their own, as the branch for it cost unsplit calls without
+// one 3 to 6 % (in graphs: 184 x 11104 x 2560 20.05 -> 21.37 us, 89 x 20330 x 2304 14.67 -> 15.60).
+template <int J, int GS, int NK, bool SHARE, bool ASYM, bool NT, bool SPLIT, typename OutT, bool DUMP = false, bool BIAS = false>
 __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit, const int mblk, const int wave,
                                             GroupedSmem& sm, const int split = 0) {
     constexpr int NS = kGroupedWaves / NK;               // waves (strips) sharing one activation stream
@@ -843,7 +845,7 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
     uint16_t* const out = reinterpret_cast<uint16_t*>(p.out) + (size_t)m0 * p.ldo;
 
     // token scales for the epilogue, fetched first
-    const uint16_t* const bias_at = DUMP ? nullptr : early_bias(p.bias);
+    const uint16_t* const bias_at = BIAS ? early_bias(p.bias) : nullptr;
     float sa[NK == 1 && !SPLIT ? J : kOutPerThread];
     if (NK == 1 && !SPLIT) {
 #pragma unroll
@@ -1041,11 +1043,10 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
     }
 
     constexpr float kUnscale[4] = {1.0f, 0.25f, 0.0625f, 0.015625f};  // 4^-p, exact
-    const bool biased = __builtin_expect(bias_at != nullptr, 0);
     if (NK == 1 && !SPLIT) {
         if (active) {
             uint16_t bias[4] = {0, 0, 0, 0};
-            if (__builtin_expect(biased, 0)) {
+            if constexpr (BIAS) {
 #pragma unroll
                 for (int pp = 0; pp < 4; ++pp) bias[pp] = bias_at[min(strip * kStripN + pp * 16 + col, p.N - 1)];
             }
@@ -1057,7 +1058,7 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
                     const int n = strip * kStripN + pp * 16 + col;
                     if (m < M && n < p.N) {
                         uint16_t v = OutT::cast((t[pp][j] * kUnscale[pp]) * sa[j]);
-                        if (__builtin_expect(biased, 0)) v = add_bias<OutT>(v, bias[pp]);
+                        if constexpr (BIAS) v = add_bias<OutT>(v, bias[pp]);
                         out[(size_t)m * p.ldo + n] = v;
                     }
                 }
@@ -1067,9 +1068,11 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
 
     // ---- the k-parts of each strip meet in LDS (the metadata area is dead once every wave is here)
     uint16_t bias[kOutPerThread];
+    if constexpr (BIAS) {
 #pragma unroll
-    for (int i = 0; i < kOutPerThread; ++i)
-        bias[i] = __builtin_expect(biased, 0) ? bias_at[min((unit * NS + min((tid + kThreads * i) / kLive, NS - 1)) * kStripN + (tid & 63), p.N - 1)] : (uint16_t)0;
+        for (int i = 0; i < kOutPerThread; ++i)
+            bias[i] = bias_at[min((unit * NS + min((tid + kThreads * i) / kLive, NS - 1)) * kStripN + (tid & 63), p.N - 1)];
+    }
     __syncthreads();
 #pragma unroll
     for (int pp = 0; pp < 4; ++pp)
@@ -1090,7 +1093,7 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
 #pragma unroll
                 for (int kp = 1; kp < NK; ++kp) v += sm.red[kp * NS + sidx][m][nl];
                 uint16_t o = OutT::cast(v * sa[i]);
-                if (__builtin_expect(biased, 0)) o = add_bias<OutT>(o, bias[i]);
+                if constexpr (BIAS) o = add_bias<OutT>(o, bias[i]);
                 out[(size_t)m * p.ldo + n] = o;
             }
         }
@@ -1156,7 +1159,7 @@ __device__ __forceinline__ void shared_body(const GemmParams& p, const int unit,
         const int n = (unit * NS + sidx) * kStripN + nl;
         if (eon[i] && m < M && n < p.N) {
             uint16_t o = OutT::cast(v[i] * sa[i]);
-            if (__builtin_expect(biased, 0)) o = add_bias<OutT>(o, bias[i]);
+            if constexpr (BIAS) o = add_bias<OutT>(o, bias[i]);
             out[(size_t)m * p.ldo + n] = o;
         }
     }
@@ -1218,7 +1221,7 @@ __global__ __launch_bounds__(kGroupedWaves * 64, 4) void skinny_grouped_kernel(c
 // The grid is one-dimensional and placed by xcd_place: a set is a (unit, K split) pair, its members are its row
 // blocks.  (Dealing whole units out instead, K splits in blockIdx.y, left 5120 channels = 20 units at 96 rows in two
 // splits with 36 workgroups on four XCDs of 32 CUs and 24 on the others: 30.6 us, now 22.3 us.)
-template <int GS, int NK, bool ASYM, typename OutT, bool DUMP = false>
+template <int GS, int NK, bool ASYM, typename OutT, bool DUMP, bool BIAS>
 __global__ __launch_bounds__(kGroupedWaves * 64, 4) void skinny_shared_kernel(const GemmParams p) {
     __shared__ __attribute__((aligned(16))) GroupedSmem sm;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1231,13 +1234,13 @@ __global__ __launch_bounds__(kGroupedWaves * 64, 4) void skinny_shared_kernel(co
     at.unit = pair % units;
     at.split = pair / units;
     if (mblocks == 1) {  // one row block: every weight byte is used once (loads marked stream-once)
-        if (p.split > 1) shared_body<4, GS, NK, true, ASYM, true, true, OutT, DUMP>(p, at.unit, at.mblk, wave, sm, at.split);
-        else shared_body<4, GS, NK, true, ASYM, true, false, OutT, DUMP>(p, at.unit, at.mblk, wave, sm);
+        if (p.split > 1) shared_body<4, GS, NK, true, ASYM, true, true, OutT, DUMP, BIAS>(p, at.unit, at.mblk, wave, sm, at.split);
+        else shared_body<4, GS, NK, true, ASYM, true, false, OutT, DUMP, BIAS>(p, at.unit, at.mblk, wave, sm);
         return;
     }
     // several row blocks: all but the first read of the weights come from L2
-    if (p.split > 1) shared_body<4, GS, NK, true, ASYM, false, true, OutT, DUMP>(p, at.unit, at.mblk, wave, sm, at.split);
-    else shared_body<4, GS, NK, true, ASYM, false, false, OutT, DUMP>(p, at.unit, at.mblk, wave, sm);
+    if (p.split > 1) shared_body<4, GS, NK, true, ASYM, false, true, OutT, DUMP, BIAS>(p, at.unit, at.mblk, wave, sm, at.split);
+    else shared_body<4, GS, NK, true, ASYM, false, false, OutT, DUMP, BIAS>(p, at.unit, at.mblk, wave, sm);
 }
 
 template <int GS, int NK, bool DUMP>
@@ -1245,13 +1248,19 @@ static void launch_shared_nk(const GemmParams& p, bool asym, bool out_bf16, hipS
     const int per_unit = kGroupedWaves / NK;
     const int units = (p.strips + per_unit - 1) / per_unit;
     const dim3 grid(xcd_grid(units * (p.split > 1 ? p.split : 1), (p.M + 15) / 16)), block(kGroupedWaves * 64);
+#define SLIMK_SHARED_PICK(ASYMV, OUT)                                                                                       \
+    do {                                                                                                                    \
+        if (!DUMP && p.bias != nullptr) skinny_shared_kernel<GS, NK, ASYMV, OUT, DUMP, !DUMP><<<grid, block, 0, stream>>>(p); \
+        else skinny_shared_kernel<GS, NK, ASYMV, OUT, DUMP, false><<<grid, block, 0, stream>>>(p);                          \
+    } while (0)
     if (asym) {
-        if (out_bf16) skinny_shared_kernel<GS, NK, true, OutBF16, DUMP><<<grid, block, 0, stream>>>(p);
-        else skinny_shared_kernel<GS, NK, true, OutF16, DUMP><<<grid, block, 0, stream>>>(p);
+        if (out_bf16) SLIMK_SHARED_PICK(true, OutBF16);
+        else SLIMK_SHARED_PICK(true, OutF16);
     } else {
-        if (out_bf16) skinny_shared_kernel<GS, NK, false, OutBF16, DUMP><<<grid, block, 0, stream>>>(p);
-        else skinny_shared_kernel<GS, NK, false, OutF16, DUMP><<<grid, block, 0, stream>>>(p);
+        if (out_bf16) SLIMK_SHARED_PICK(false, OutBF16);
+        else SLIMK_SHARED_PICK(false, OutF16);
     }
+#undef SLIMK_SHARED_PICK
 }
 
 // kparts: k-parts per workgroup, kSharedParts (four strips share an activation stream) or twice that (two strips)
