@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kWaves * 64, XBF && GS < 4 ? 4 : 1) void w2a16_grou
 // Adds up the partial sums in split order: four neighbouring values of a row per thread, the splits' loads independent
 // of each other (one value per thread and its row and column by a 64-bit division: the second launch of a
 // 300 x 4096 x 14336 call).
-template <typename OutT>
+template <typename OutT, bool BIAS>
 __global__ __launch_bounds__(128) void w2a16_reduce_kernel(const float* __restrict__ ws, int split, int M, int N,
                                                            uint16_t* __restrict__ out, int ldo, const uint16_t* __restrict__ bias) {
     const size_t total = (size_t)M * N;
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(128) void w2a16_reduce_kernel(const float* __restri
             uint16_t o[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[i] = OutT::cast(v[i]);
-            if (bias) {
+            if constexpr (BIAS) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) o[i] = add_bias<OutT>(o[i], bias[t * 4 + i]);
             }
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(128) void w2a16_reduce_kernel(const float* __restri
 #pragma unroll 4
                 for (int s = 1; s < split; ++s) v += src[(size_t)s * total + n];
                 uint16_t o = OutT::cast(v);
-                if (bias) o = add_bias<OutT>(o, bias[n]);
+                if constexpr (BIAS) o = add_bias<OutT>(o, bias[n]);
                 dst[n] = o;
             }
         }
@@ -439,10 +439,15 @@ hipError_t launch_w2a16(const W2A16Params& asked, int gs, bool out_bf16, hipStre
     if (p.split > 1) {
         const int per_thread = p.N % 4 == 0 ? 4 : 1;
         const dim3 blocks((unsigned)((p.N + 128 * per_thread - 1) / (128 * per_thread)), (unsigned)std::min(p.M, 32768));
-        if (out_bf16)
-            w2a16_reduce_kernel<OutBF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo, p.bias);
-        else
-            w2a16_reduce_kernel<OutF16><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo, p.bias);
+#define SLIMK_W2A16_REDUCE(OUT, BIASV) w2a16_reduce_kernel<OUT, BIASV><<<blocks, dim3(128), 0, stream>>>(p.ws, p.split, p.M, p.N, (uint16_t*)p.out, p.ldo, p.bias)
+        if (p.bias) {
+            if (out_bf16) SLIMK_W2A16_REDUCE(OutBF16, true);
+            else SLIMK_W2A16_REDUCE(OutF16, true);
+        } else {
+            if (out_bf16) SLIMK_W2A16_REDUCE(OutBF16, false);
+            else SLIMK_W2A16_REDUCE(OutF16, false);
+        }
+#undef SLIMK_W2A16_REDUCE
     } else if (bias_behind) {
         return launch_add_bias(p.out, p.ldo, p.M, p.N, asked.bias, out_bf16, stream);
     }

@@ -52,7 +52,9 @@ __device__ __forceinline__ CodeTable code_table(int z) {
 
 // KP = 2: eight waves, the second four on the second half of the workgroup's steps in a ring of their own; the halves
 // meet in LDS (half the partial sums of a split launch with as many waves on a CU).
-template <int RB, int KP, bool ZP, bool PARTIAL, typename OutT, bool XBF>
+// BIAS: p.bias is added to the rounded outputs, on whole 16-byte output rows only (instantiations of their own: the branch for it
+// cost unsplit calls without one 1 to 4 %, in graphs 535 x 10024 x 4096 in asymmetric groups of 256 74.1 -> 77.3 us).
+template <int RB, int KP, bool ZP, bool PARTIAL, typename OutT, bool XBF, bool BIAS>
 __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int steps_per_split, const int group_shift) {
     constexpr int kBM = RB * 32;
     constexpr int kASlot = RB * 4096, kWSlot = kStripsPerWg * kUnitBytes, kSSlot = kStripsPerWg * 256;
@@ -67,7 +69,7 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & (kStripsPerWg - 1);
     uint8_t* const lds = lds_all + kh * kLds;
     const int col = lane & 31, half = lane >> 5, c16 = lane & 15, sub = (lane >> 4) & 1;
-    const uint16_t* const bias = early_bias(p.bias);
+    const uint16_t* const bias = BIAS ? early_bias(p.bias) : nullptr;
     // token tiles of a channel tile next to each other on one XCD: they read the same weights
     const int tiles_n = (p.strips + kStripsPerWg - 1) / kStripsPerWg, tiles_m = (p.M + kBM - 1) / kBM;
     // ((split, channel tile) pairs dealt out together where split by split is uneven: 360 x 1584 x 11264 43.5 -> 28.1 us, 505 x
@@ -283,7 +285,7 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
     const bool wide = (p.N & 7) == 0 && (p.ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
     float* stage_out = reinterpret_cast<float*>(lds) + wave * (32 * kPitch);
     out8 bias8 = {0, 0, 0, 0};
-    if (__builtin_expect(bias != nullptr, 0)) bias8 = *reinterpret_cast<const out8*>(bias + min(strip * kStripN + (lane & 7) * 8, p.N - 8));
+    if constexpr (BIAS) bias8 = *reinterpret_cast<const out8*>(bias + min(strip * kStripN + (lane & 7) * 8, p.N - 8));
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
         if (wide) {
@@ -303,7 +305,7 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
                 v.y = (uint32_t)OutT::cast(lo.z) | ((uint32_t)OutT::cast(lo.w) << 16);
                 v.z = (uint32_t)OutT::cast(hi.x) | ((uint32_t)OutT::cast(hi.y) << 16);
                 v.w = (uint32_t)OutT::cast(hi.z) | ((uint32_t)OutT::cast(hi.w) << 16);
-                if (__builtin_expect(bias != nullptr, 0)) v = add_bias8<OutT>(v, bias8);
+                if constexpr (BIAS) v = add_bias8<OutT>(v, bias8);
                 const int m = m_tile + rb * 32 + row, n = strip * kStripN + cg * 8;
                 if (m < p.M && n < p.N) *reinterpret_cast<v4u*>(out + (size_t)m * p.ldo + n) = v;
             }
@@ -320,17 +322,23 @@ __device__ __forceinline__ void w2a16_tiled_body(const W2A16Params& p, const int
 }
 
 // (four-wave workgroups: two of 128 or three of 64 rows per CU; eight-wave ones, 64 rows only: one)
-template <int RB, int KP, bool ZP, bool PARTIAL, typename OutT, bool XBF>
+template <int RB, int KP, bool ZP, bool PARTIAL, typename OutT, bool XBF, bool BIAS>
 __global__ __launch_bounds__(KP * 256, RB == 4 || KP == 2 ? 2 : 3) void w2a16_tiled_kernel(const W2A16Params p, const int steps_per_split, const int group_shift) {
-    w2a16_tiled_body<RB, KP, ZP, PARTIAL, OutT, XBF>(p, steps_per_split, group_shift);
+    w2a16_tiled_body<RB, KP, ZP, PARTIAL, OutT, XBF, BIAS>(p, steps_per_split, group_shift);
 }
 
 template <int RB, int KP, bool ZP, bool XBF>
 void launch_rb(const W2A16Params& p, bool out_bf16, dim3 grid, int sps, int shift, hipStream_t stream) {
     const dim3 block(KP * 256);
-    if (p.split > 1) w2a16_tiled_kernel<RB, KP, ZP, true, OutF16, XBF><<<grid, block, 0, stream>>>(p, sps, shift);
-    else if (out_bf16) w2a16_tiled_kernel<RB, KP, ZP, false, OutBF16, XBF><<<grid, block, 0, stream>>>(p, sps, shift);
-    else w2a16_tiled_kernel<RB, KP, ZP, false, OutF16, XBF><<<grid, block, 0, stream>>>(p, sps, shift);
+    if (p.split > 1) {   // (the sums' launch adds the bias)
+        w2a16_tiled_kernel<RB, KP, ZP, true, OutF16, XBF, false><<<grid, block, 0, stream>>>(p, sps, shift);
+    } else if (p.bias) {
+        if (out_bf16) w2a16_tiled_kernel<RB, KP, ZP, false, OutBF16, XBF, true><<<grid, block, 0, stream>>>(p, sps, shift);
+        else w2a16_tiled_kernel<RB, KP, ZP, false, OutF16, XBF, true><<<grid, block, 0, stream>>>(p, sps, shift);
+    } else {
+        if (out_bf16) w2a16_tiled_kernel<RB, KP, ZP, false, OutBF16, XBF, false><<<grid, block, 0, stream>>>(p, sps, shift);
+        else w2a16_tiled_kernel<RB, KP, ZP, false, OutF16, XBF, false><<<grid, block, 0, stream>>>(p, sps, shift);
+    }
 }
 
 }  // namespace

@@ -162,8 +162,8 @@ struct OutBF16 {
 
 // A layer's bias in the kernels' epilogues: the output is rounded, then the sum with the bias is, so the bits are those of
 // a separate addition of two tensors of the output's type (which reads and writes the output once more, and is a launch: 4 us
-// for 4 x 9312 outputs, 8 for 616 x 12120).  The int8 tiled kernels and the digit form have instantiations of their own for
-// it; in the few-rows and weight-only kernels it is a branch marked unlikely, so that its code lies behind the rest.
+// for 4 x 9312 outputs, 8 for 616 x 12120).  The many-rows kernels and the shared few-rows kernel have instantiations
+// of their own for it; in the other few-rows kernels it is a branch marked unlikely, so that its code lies behind the rest.
 template <typename OutT>
 __device__ __forceinline__ uint16_t add_bias(uint16_t out, uint16_t bias) {
     return OutT::cast(OutT::widen(out) + OutT::widen(bias));
