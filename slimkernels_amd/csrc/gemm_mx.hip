@@ -219,7 +219,8 @@ __device__ __forceinline__ void mx_body(const MxParams& p) {
     const int xcd = (int)(blockIdx.x & 7), local = (int)(blockIdx.x >> 3);
     int tile, split_idx = 0;
     if (SPLIT) {
-        if (!split_tile_place((int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y, tiles_n, tiles_m, tile, split_idx)) return;
+        const int counted = p.group_shift ? counted_splits((int)gridDim.y, (p.steps + 1) / 2, p.stages_per_split) : 0;
+        if (!split_tile_place((int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y, tiles_n, tiles_m, tile, split_idx, counted)) return;
         tile = __builtin_amdgcn_readfirstlane(tile);
         split_idx = __builtin_amdgcn_readfirstlane(split_idx);
     } else if (tiles_n % 8 == 0) {

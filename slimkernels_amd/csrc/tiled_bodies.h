@@ -100,7 +100,8 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
     const int xcd = (int)(blockIdx.x & 7), local = (int)(blockIdx.x >> 3);
     int tile, split_idx = 0;
     if (SPLIT) {
-        if (!split_tile_place((int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y, tiles_n, tiles_m, tile, split_idx)) return;
+        const int counted = kLong ? counted_splits((int)gridDim.y, (p.steps + kStageSteps - 1) / kStageSteps, p.groups_per_split * GS / kStageSteps) : 0;
+        if (!split_tile_place((int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y, tiles_n, tiles_m, tile, split_idx, counted)) return;
         tile = __builtin_amdgcn_readfirstlane(tile);
         split_idx = __builtin_amdgcn_readfirstlane(split_idx);
     } else if (tiles_n % 8 == 0) {

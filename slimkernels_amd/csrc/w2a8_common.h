@@ -218,17 +218,27 @@ __host__ __device__ __forceinline__ bool xcd_run(const int local, const int item
 __host__ __device__ __forceinline__ bool splits_uneven(const int total, const int splits) {
     return ((total + 7) / 8 * splits + 31) / 32 > ((total * splits + 7) / 8 + 31) / 32;
 }
-// Which tile and K split workgroup (x, y) of the int8 or digit form takes.  Where that helps (splits_uneven), each XCD gets a
-// run of pairs, a tile's together: of 1466 drawn calls 32 int8 ones went 2..44 % faster (360 x 1584 x 11264 35.8 -> 28.0
-// us), 35 digit ones 3..31 % (795 x 3248 x 14080 89.0 -> 69.4).  Elsewhere split by split: a tile's splits share an XCD,
-// out of whose L2 the last of them to arrive reads the partial sums, and even dealing was up to 18 % slower.
+// In groups of 256 a split owns pairs of stages and the last one is often short: up to half the length of the others its workgroups,
+// the last of a grid that is dealt out split by split, find room beside theirs.  Such splits do not count then, unless even
+// dealing leaves every CU with one workgroup.  With them counted, calls with two workgroups a CU ran at 0.92..1.06 of their speed
+// (257 x 4160 x 7936 28.0 -> 30.7 us; with one a CU 422 x 1344 x 6656 19.8 -> 19.6).
+__host__ __device__ __forceinline__ int counted_splits(const int splits, const int stages, const int stages_per_split) {
+    return 2 * (stages - (splits - 1) * stages_per_split) <= stages_per_split ? splits - 1 : splits;
+}
+__host__ __device__ __forceinline__ bool deal_evenly(const int total, const int splits, const int counted) {
+    return splits_uneven(total, splits) && (counted == splits || total * splits <= 8 * 32 || splits_uneven(total, counted));
+}
+// Which tile and K split workgroup (x, y) of the int8 or digit form takes.  Where that helps (deal_evenly; counted 0: all splits),
+// each XCD gets a run of pairs, a tile's together: of 1466 drawn calls 32 int8 ones went 2..44 % faster (360 x 1584 x 11264 35.8
+// -> 28.0 us), 35 digit ones 3..31 % (795 x 3248 x 14080 89.0 -> 69.4).  Elsewhere split by split: a tile's splits share an
+// XCD, out of whose L2 the last of them to arrive reads the partial sums, and even dealing was up to 18 % slower.
 // Order within a split: channel tiles that divide by eight in bands, token tile major; with two to four token tiles those of a
 // channel tile on one XCD's queue; else one run of tiles per XCD, channel tile fastest.
 __host__ __device__ __forceinline__ bool split_tile_place(const int x, const int y, const int splits, const int tiles_n, const int tiles_m,
-                                                          int& tile, int& split) {
+                                                          int& tile, int& split, const int counted = 0) {
     const int total = tiles_n * tiles_m, per_xcd = (total + 7) / 8, xcd = x & 7, slot = x >> 3;
     const bool few = tiles_m >= 2 && tiles_m <= 4;
-    if (splits_uneven(total, splits)) {
+    if (deal_evenly(total, splits, counted ? counted : splits)) {
         int pair;
         if (!xcd_run(y * per_xcd * 8 + x, total * splits, pair)) return false;
         const int t = pair / splits;
