@@ -58,9 +58,51 @@ int tiled_w4_auto_split(int M, int strips, int steps) {
     return (stages + sps - 1) / sps;
 }
 
+// 4-bit weights, one pass (64-row tiles: three stage buffers of 24 KiB leave room for two workgroups on a CU)
+template <int GS, bool SPLIT, bool ZP, typename OutT, bool BIAS>
+__global__ __launch_bounds__(256, 2) void tiled_kernel_w4(const GemmParams p) {
+    tiled_body<64, GS, SPLIT, ZP, OutT, true, false, BIAS>(p);
+}
+// ... and 128-row tiles, two workgroups on a CU as well
+template <int GS, bool ZP, typename OutT, bool BIAS>
+__global__ __launch_bounds__(256, 2) void tiled_kernel_w4_bm128(const GemmParams p) {
+    tiled_body<128, GS, false, ZP, OutT, true, false, BIAS>(p);
+}
+
 hipError_t launch_tiled_w4(const GemmParams& p, int gs, bool out_bf16, hipStream_t stream) {
-    if (p.acc_dump != nullptr && p.dump_mode != 0) return launch_tiled_w4_verify(p, gs, out_bf16, stream);
-    return launch_tiled_w4_impl<false>(p, gs, out_bf16, stream);
+    const bool biased = p.bias != nullptr && output_rows_whole(p.out, p.ldo, p.N);
+    const bool tall = p.split <= 1 && tiled_w4_tall(p.M, p.strips);
+    const int tiles = (int)tiled_w4_tiles(p.M, p.strips, tall ? 128 : 64);
+    const dim3 grid((tiles + 7) / 8 * 8, p.split > 1 ? p.split : 1), block(256);
+#define SLIMK_W4_PICK(KERNEL, ...)                                                \
+    do {                                                                          \
+        if (biased) KERNEL<__VA_ARGS__, true><<<grid, block, 0, stream>>>(p);     \
+        else KERNEL<__VA_ARGS__, false><<<grid, block, 0, stream>>>(p);           \
+    } while (0)
+#define SLIMK_W4_LAUNCH(GSV, ZPV)                                                 \
+    do {                                                                          \
+        if (tall) {                                                               \
+            if (out_bf16) SLIMK_W4_PICK(tiled_kernel_w4_bm128, GSV, ZPV, OutBF16);\
+            else SLIMK_W4_PICK(tiled_kernel_w4_bm128, GSV, ZPV, OutF16);          \
+        } else if (p.split > 1) {                                                 \
+            if (out_bf16) SLIMK_W4_PICK(tiled_kernel_w4, GSV, true, ZPV, OutBF16);\
+            else SLIMK_W4_PICK(tiled_kernel_w4, GSV, true, ZPV, OutF16);          \
+        } else {                                                                  \
+            if (out_bf16) SLIMK_W4_PICK(tiled_kernel_w4, GSV, false, ZPV, OutBF16);\
+            else SLIMK_W4_PICK(tiled_kernel_w4, GSV, false, ZPV, OutF16);         \
+        }                                                                         \
+    } while (0)
+    const bool zp = p.zp_r != nullptr;   // per-group zero-points: the planes' (rows 0..G-1 hi, G..2G-1 lo) and p.rowsum
+    if (gs == 1) {
+        if (zp) SLIMK_W4_LAUNCH(1, true);
+        else SLIMK_W4_LAUNCH(1, false);
+    } else {
+        if (zp) SLIMK_W4_LAUNCH(2, true);
+        else SLIMK_W4_LAUNCH(2, false);
+    }
+#undef SLIMK_W4_LAUNCH
+#undef SLIMK_W4_PICK
+    return hipGetLastError();
 }
 
 bool tiled_fast_supported(const GemmParams& p, int gs, bool asym) {

@@ -8,8 +8,4 @@ hipError_t launch_tiled_verify(const GemmParams& p, int gs, bool asym, bool out_
     return launch_tiled_impl<true>(p, gs, asym, out_bf16, stream);
 }
 
-hipError_t launch_tiled_w4_verify(const GemmParams& p, int gs, bool out_bf16, hipStream_t stream) {
-    return launch_tiled_w4_impl<true>(p, gs, out_bf16, stream);
-}
-
 }  // namespace w2a8

@@ -572,54 +572,12 @@ __global__ __launch_bounds__(256, DUMP || GS == 4 ? 2 : 3) void tiled_kernel_bm6
     tiled_body<64, GS, SPLIT, ZP, OutT, false, DUMP, BIAS>(p);
 }
 
-// 4-bit weights, one pass (64-row tiles: three stage buffers of 24 KiB leave room for two workgroups on a CU)
-template <int GS, bool SPLIT, bool ZP, typename OutT, bool DUMP, bool BIAS>
-__global__ __launch_bounds__(256, 2) void tiled_kernel_w4(const GemmParams p) {
-    tiled_body<64, GS, SPLIT, ZP, OutT, true, DUMP, BIAS>(p);
-}
-// ... and 128-row tiles, two workgroups on a CU as well
-template <int GS, bool ZP, typename OutT, bool DUMP, bool BIAS>
-__global__ __launch_bounds__(256, 2) void tiled_kernel_w4_bm128(const GemmParams p) {
-    tiled_body<128, GS, false, ZP, OutT, true, DUMP, BIAS>(p);
-}
-
 // the instantiation with or without a bias (a verification launch has none)
 #define SLIMK_TILED_PICK(KERNEL, ...)                                                     \
     do {                                                                                  \
         if (biased) KERNEL<__VA_ARGS__, DUMP, !DUMP><<<grid, block, 0, stream>>>(p);      \
         else KERNEL<__VA_ARGS__, DUMP, false><<<grid, block, 0, stream>>>(p);             \
     } while (0)
-
-template <bool DUMP>
-static hipError_t launch_tiled_w4_impl(const GemmParams& p, int gs, bool out_bf16, hipStream_t stream) {
-    const bool biased = !DUMP && p.bias != nullptr && output_rows_whole(p.out, p.ldo, p.N);
-    const bool tall = !DUMP && p.split <= 1 && tiled_w4_tall(p.M, p.strips);
-    const int tiles = (int)tiled_w4_tiles(p.M, p.strips, tall ? 128 : 64);
-    const dim3 grid((tiles + 7) / 8 * 8, p.split > 1 ? p.split : 1), block(256);
-#define SLIMK_W4_LAUNCH(GSV, ZPV)                                                                         \
-    do {                                                                                                  \
-        if (tall) {                                                                                       \
-            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel_w4_bm128, GSV, ZPV, OutBF16);        \
-            else SLIMK_TILED_PICK(tiled_kernel_w4_bm128, GSV, ZPV, OutF16);                  \
-        } else if (p.split > 1) {                                                                                \
-            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel_w4, GSV, true, ZPV, OutBF16);  \
-            else SLIMK_TILED_PICK(tiled_kernel_w4, GSV, true, ZPV, OutF16);            \
-        } else {                                                                                          \
-            if (out_bf16) SLIMK_TILED_PICK(tiled_kernel_w4, GSV, false, ZPV, OutBF16); \
-            else SLIMK_TILED_PICK(tiled_kernel_w4, GSV, false, ZPV, OutF16);           \
-        }                                                                                                 \
-    } while (0)
-    const bool zp = p.zp_r != nullptr;   // per-group zero-points: the planes' (rows 0..G-1 hi, G..2G-1 lo) and p.rowsum
-    if (gs == 1) {
-        if (zp) SLIMK_W4_LAUNCH(1, true);
-        else SLIMK_W4_LAUNCH(1, false);
-    } else {
-        if (zp) SLIMK_W4_LAUNCH(2, true);
-        else SLIMK_W4_LAUNCH(2, false);
-    }
-#undef SLIMK_W4_LAUNCH
-    return hipGetLastError();
-}
 
 // Tile height and tile count of the fast kernel for a problem: two workgroups fit a CU, so below
 // about two 128-row tiles per CU, 64-row tiles fill the chip better.  A group of 256 (gs = 4) has 64-row tiles only.

@@ -88,7 +88,6 @@ hipError_t launch_mid_verify(const GemmParams& p, int gs, bool asym, bool out_bf
 // p.split > 1: K split over blockIdx.y in whole 128-element stages (p.groups_per_split), workspace = one arrival
 // counter and p.split fp32 tiles of 64 x 256 per tile (tiled_w4_tiles)
 hipError_t launch_tiled_w4(const GemmParams& p, int gs, bool out_bf16, hipStream_t stream);
-hipError_t launch_tiled_w4_verify(const GemmParams& p, int gs, bool out_bf16, hipStream_t stream);
 size_t tiled_w4_tiles(int M, int strips, int rows = 64);
 bool tiled_w4_tall(int M, int strips);   // an unsplit launch runs on 128-row tiles
 int tiled_w4_auto_split(int M, int strips, int steps);
