@@ -703,10 +703,14 @@ static float digit_layer_time(int M, int N, int K, int group_size, int per_group
 //    launch and quantisation: level at K = 384, up to 3 % slower at 256 (2317 x 8400 x 256 24.3 -> 25.1).  95 routed calls of 70 drawn
 //    shapes, K = 256..16384: 18 % faster on average, the slowest 2 % faster.
 //  * fewer tiles, 96 rows and more, 1024 channels and elements and more: the smaller predicted time, with 6 % in hand, 8 %
-//    for symmetric groups of 128 on more than 256 rows.  Of 9863 drawn calls that the int8 path had (96..1200 rows, odd widths
-//    among them), the 84 % this takes are 14 % faster on average, 1.1 % of them more than 3 % slower, the slowest 13 %
-//    (4311 x 9728 and 7881 x 11520 in eight splits); what it leaves would gain 5 %.  128 x 28672 x 8192 in groups of 64
-//    63.1 -> 56.7 us, with per-group zero-points 76 -> 64; 160 x 20480 x 2048 31 -> 23; 700 x 3072 x 24576 121 -> 105.
+//    for symmetric groups of 128 on more than 256 rows, and more where a prediction is asked beyond its fit: 14 % for symmetric
+//    levels on more than 1200 rows (with per-group zero-points the digits gain more than the predictions miss), 11 % for up to
+//    2048 elements in an odd number of steps on up to 256 rows (mid_route's is 15 % high there).  Of 2081 drawn calls (96..16384
+//    rows, odd widths among them) that have the smaller predicted time with the 6 or 8 %, the 1803 it takes are 14 % faster on
+//    average, 0.9 % of them more than 3 % slower, the slowest 11 % (1075 x 4448 x 4608 50.4 -> 56.5 us); the 278 it leaves would be
+//    4 % faster on average, 11 % of them more than 3 % slower (4936 x 1024 x 18240 in groups of 64 193 -> 220, 134 x 23552 x
+//    1856 25.5 -> 28.2).  128 x 28672 x 8192 in groups of 64 63.1 -> 56.7 us, with per-group zero-points 76 -> 64; 160 x 20480 x
+//    2048 31 -> 23; 700 x 3072 x 24576 121 -> 105.
 //    4096 channels and elements and more, more than 256 rows: also where mx_predicted_time, the first fit, has 6 % in hand,
 //    as before (200 routed calls of shapes that took no part in it 16 % faster, the slowest level; 512 x 28672 x
 //    8192 in groups of 64 184 -> 146, with per-group zero-points 236 -> 165).
@@ -725,7 +729,8 @@ int slimk_w2a8_linear_route(int M, int N, int K, int group_size, int per_group_z
     const float other = int8_layer_time(M, N, K, group_size, per_group_zp);
     if (M > 256 && N >= 4096 && K >= 4096 &&
         w2a8::mx_predicted_time(M, N, K, group_size, per_group_zp, plan.rb, plan.split) < 0.94f * other) return 1;
-    const float in_hand = M > 256 && group_size == 128 && !per_group_zp ? 0.92f : 0.94f;
+    const bool odd = M <= 256 && K <= 2048 && K / w2a8::kStepK % 2 != 0, tall = M > 1200 && !per_group_zp;
+    const float in_hand = odd ? 0.89f : tall ? 0.86f : M > 256 && group_size == 128 && !per_group_zp ? 0.92f : 0.94f;
     return digit_layer_time(M, N, K, group_size, per_group_zp, plan) < in_hand * other ? 1 : 0;
 }
 

@@ -258,6 +258,20 @@ def test_route_knows_short_reductions_and_per_group_zero_points():
     assert [route(512, 28672, 8192, 64, zp) for zp in (0, 1)] == [1, 1]
 
 
+@pytest.mark.parametrize("M,N,K,g,zp,taken", [
+    (4936, 1024, 18240, 64, 0, 0),      # 220 us through the digits, 193 not
+    (3574, 2296, 28160, 128, 0, 0),     # 329 / 307
+    (134, 23552, 1856, 64, 0, 0),       # 28.2 / 25.5: an odd number of steps
+    (207, 12544, 1984, 64, 0, 0),       # 23.7 / 21.6
+    (4936, 1024, 18240, 64, 1, 1),      # per-group zero-points gain whatever the rows (1200..16384: 17 %)
+    (4096, 2048, 8192, 128, 1, 1),
+    (160, 20480, 2048, 128, 0, 1),      # 23 / 31
+    (700, 3072, 24576, 64, 0, 1),       # 105 / 121
+])
+def test_route_beyond_what_the_predictions_were_fitted_on(M, N, K, g, zp, taken):
+    assert _lib.lib().slimk_w2a8_linear_route(M, N, K, g, zp) == taken
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,g,mode,out", [
     (96, 16384, 8192, 64, "asym", "bfloat16"),     # the fewest rows
