@@ -4,7 +4,7 @@
 // A decode call's kernels run for 5 to 10 us; the same steps in Python (attribute reads, allocations, a ctypes call of
 // twenty arguments per launch) took 8 to 12 us for each launch, so the host was what a small call waited for.  A call among
 // others, us: 1 x 4096 x 4096 10.4 -> 6.3, the seven linears of a decoder block at 4 rows 90 -> 50, 1 x 14336 x 4096
-// weight-only 10.3 -> 7.6, 77 x 11008 x 4096 with a bias 28.8 -> 20.5.
+// weight-only 10.3 -> 7.6, 77 x 11008 x 4096 28.8 -> 20.5 with its bias in a launch behind (19.0 with it in the kernel).
 //
 // Every function here handles the plain form of its call (tensors of this device, of the types and layouts the kernels read
 // directly, no modes or transforms active) and returns None for anything else, which the Python functions of ops.py and
@@ -258,6 +258,7 @@ Answer ask(Question q, int M, int N, int K, int group, int zp) {
     return a;
 }
 int zp_kind(const Weight& w) { return w.per_group() ? 2 : w.zp_const != 2; }
+bool one_pass_w4(int M, int K, int group) { return M >= 33 && K % 128 == 0 && (group == 64 || group == 128); }   // (w4.one_pass_applies)
 
 // quantisation into scratch and the GEMM behind it
 int quantise_and_gemm(const Rows& x, const Weight& w, int copies, const Answer& a, bool one_pass_w4, const uint8_t* zp, at::Tensor& out,
@@ -366,7 +367,7 @@ PyObject* linear4(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (x.K != K || w.N != N || w.K != 2 * K || w.group != group || K % group != 0 || !w.per_group() || !bias.of(args[3], N, odt, x.device))
         return none();
     const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device.index()).stream();
-    const bool one_pass = x.M >= 33 && K % 128 == 0 && (group == 64 || group == 128);   // (w4.one_pass_applies)
+    const bool one_pass = one_pass_w4(x.M, K, group);
     Answer a = one_pass ? ask(kW4, x.M, N, K, group, 0) : ask(kGemm, x.M, N, 2 * K, group, zp_kind(w));
     const uint8_t* const zp = one_pass && uniform.p == Py_True ? nullptr : w.z();
     a.sums = !one_pass || zp != nullptr;
@@ -519,6 +520,20 @@ PyObject* grouped(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// rules(M, N, K, group_size, zp) -> (digits, sums, workspace, scratch, one_pass_w4): what the functions above decide by a call's
+// shape, to be held against ops.linear_digits_applies, ops.needs_rowsum, w4.one_pass_applies and the library's sizes
+PyObject* rules(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    int v[5];
+    for (int i = 0; i < 5; ++i)
+        if (n != 5 || !to_int(args[i], v[i])) return none();
+    if (!g_check) return none();
+    const Answer a = ask(kLinear, v[0], v[1], v[2], v[3], v[4]), b = ask(kGemm, v[0], v[1], v[2], v[3], v[4]);
+    return Py_BuildValue("(OOnnO)", a.digits ? Py_True : Py_False, b.sums ? Py_True : Py_False, (Py_ssize_t)a.ws, (Py_ssize_t)a.act,
+                         one_pass_w4(v[0], v[2], v[3]) ? Py_True : Py_False);
+    END_HANDLE_TH_ERRORS
+}
+
 // bind(addresses, check): the C ABI's functions by name, and what raises for their codes
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 2 || !PyDict_Check(args[0]) || !PyCallable_Check(args[1])) {
@@ -553,6 +568,7 @@ PyMethodDef g_methods[] = {
     {"linear4", fast<linear4>(), METH_FASTCALL, "linear4(x, weight, out_dtype, bias) -> tensor or None"},
     {"quantize", fast<quantize>(), METH_FASTCALL, "quantize(x, group_size, copies, rowsum) -> (q, s_a, rowsum) or None"},
     {"gemm", fast<gemm>(), METH_FASTCALL, "gemm(qa, weight, out_dtype) -> tensor or None"},
+    {"rules", fast<rules>(), METH_FASTCALL, "rules(M, N, K, group_size, zp) -> what a call's shape decides (zp 0: symmetric levels, 1: uniform, 2: per group)"},
     {"grouped", fast<grouped>(), METH_FASTCALL, "grouped(problems, out_dtype) -> list of tensors or None"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", "Native host side of the layer calls.", -1, g_methods, nullptr, nullptr, nullptr, nullptr};

@@ -1,10 +1,13 @@
 """The native host side of the calls (slimkernels_amd/torch/_native.cpp) against the general Python code of the same calls: the
 same bits wherever it takes a call, and None, which hands the call to that code, wherever it does not."""
+import math
+import random
 import types
 
 import pytest
 import torch
 
+from slimkernels_amd import _lib
 from slimkernels_amd.torch import ops, w4
 
 
@@ -35,6 +38,29 @@ def test_cpu_tensors_and_other_objects_are_left_to_the_general_code():
         host.bind({}, None)
     with pytest.raises(KeyError):
         host.bind({}, print)
+
+
+def test_the_same_rules_as_the_general_code():
+    """Which kernels a shape goes to, asked of the native host side and of the predicates of ops.py and w4.py: the layers' bits alone
+    would not show the two running different kernels."""
+    rules, rng = ops._host().rules, random.Random(3)
+    seen = set()
+    for _ in range(4000):
+        g = rng.choice([64, 128, 256])
+        M = int(math.exp(rng.uniform(0, math.log(6000))))
+        N, K = int(math.exp(rng.uniform(math.log(16), math.log(30000)))), g * rng.randint(1, 28672 // g)
+        zp = rng.randint(0, 2)
+        w = ops.W2A8Weight(None, None, object() if zp == 2 else None, 2 if zp != 1 else 1, N, K, g)
+        digits, sums, ws, act, one_pass = rules(M, N, K, g, zp)
+        assert digits == (M > 1 and ops.linear_digits_applies(M, w)) and sums == ops.needs_rowsum(M, w), (M, N, K, g, zp)
+        assert one_pass == w4.one_pass_applies(M, w4.W4A8Weight(w, N, K, g)), (M, K, g)
+        name, args = ("slimk_w2a8_gemm_fused_workspace_bytes", (0,)) if M == 1 and ops.fused_applies(1, K) else \
+            ("slimk_w2a8_linear_workspace_bytes", ()) if digits else ("slimk_w2a8_gemm_workspace_bytes", (_lib.KERNEL_AUTO, 0))
+        assert ws == ops._query(name, M, N, K, g, *args)
+        assert act == (ops._query("slimk_w2a8_linear_activation_bytes", M, N, K, g) if digits else 0)
+        seen.add((digits, sums, one_pass, ws > 0))
+    assert len(seen) >= 8
+    assert rules(1, 2, 3) is None and rules(1.0, 64, 64, 64, 0) is None
 
 
 LAYERS = {"2": ops.W2A8Linear, "16": ops.W2A16Linear, "4": w4.W4A8Linear}
