@@ -4,7 +4,7 @@
 // A decode call's kernels run for 5 to 10 us; the same steps in Python (attribute reads, allocations, a ctypes call of
 // twenty arguments per launch) took 8 to 12 us for each launch, so the host was what a small call waited for.  A call among
 // others, us: 1 x 4096 x 4096 10.4 -> 6.3, the seven linears of a decoder block at 4 rows 90 -> 50, 1 x 14336 x 4096
-// weight-only 10.3 -> 7.6, 77 x 11008 x 4096 28.8 -> 20.5 with its bias in a launch behind (19.0 with it in the kernel).
+// weight-only 10.3 -> 7.6, 77 x 11008 x 4096 28.8 -> 20.5 with its bias in a launch behind (17.5 with it in the kernel).
 //
 // Every function here handles the plain form of its call (tensors of this device, of the types and layouts the kernels read
 // directly, no modes or transforms active) and returns None for anything else, which the Python functions of ops.py and
