@@ -77,6 +77,7 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
     // second stages only, and the stage loop runs over pairs of stages.
     constexpr bool kLong = GS == 4;
     static_assert(!kLong || (BM == 64 && !W4), "a group of 256 runs on 64-row W2 tiles only");
+    static_assert(!(W4 && DUMP), "only 2-bit weights have a verification instantiation");
     constexpr int GSE = kLong ? kStageSteps : GS;       // steps of a group inside one stage
     constexpr int kGroupsPerStage = kStageSteps / GSE;  // 2 (group 64) or 1 (group 128, 256)
 
@@ -368,8 +369,8 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
                                 const int g_here = (stage0 + stage) * kStageSteps / GS;
                                 const int g_dump = kLong ? (u == 0 ? g_here - 1 : g_here) : g_here + (u == 0 ? -1 : pgi);
                                 if ((u > 0 || stage > 0) && strip_ok && g_dump < p.G)
-                                    dump_group_sum<W4>(p, m_tile + pmb * 16 + quad * 4 + e % 4, strip * kStripN + (e / 4) * 16 + col,
-                                                       g_dump, acc[prev][e / 4][e % 4] >> (W4 ? 4 : 6), W4 ? 8 : 2);
+                                    dump_group_sum(p, m_tile + pmb * 16 + quad * 4 + e % 4, strip * kStripN + (e / 4) * 16 + col,
+                                                       g_dump, acc[prev][e / 4][e % 4] >> 6, 2);
                             }
                         }
                     }
@@ -404,8 +405,8 @@ __device__ __forceinline__ void tiled_body(const GemmParams& p) {
             if constexpr (DUMP) {
                 const int g_dump = (stage0 + n_stages) * kStageSteps / GS - 1;
                 if (strip_ok && g_dump < p.G)
-                    dump_group_sum<W4>(p, m_tile + (kMB - 1) * 16 + quad * 4 + j, strip * kStripN + pp * 16 + col,
-                                       g_dump, acc[kLastSet][pp][j] >> (W4 ? 4 : 6), W4 ? 8 : 2);
+                    dump_group_sum(p, m_tile + (kMB - 1) * 16 + quad * 4 + j, strip * kStripN + pp * 16 + col,
+                                       g_dump, acc[kLastSet][pp][j] >> 6, 2);
             }
         }
 
